@@ -259,9 +259,8 @@ int vfg_batch_u_apply(vfg_batch *b, const double *const *x, double *const *y);
 int vfg_batch_u_apply_f32(vfg_batch *b, const float *const *x, float *const *y);
 /* times nrep persistent applies on internal vectors (HIP events), total ms */
 int vfg_batch_time_u_apply(vfg_batch *b, int fp32, int nrep, double *ms);
-/* picks the persistent apply's schedule (0: 16 x 16 element tiles on the
- * register march, 1: 8 x 8 tiles on the register march, 2: 16 x 16 tiles on
- * the LDS-ring march), z-chunk length (0.5 / 1 / 2 x the whole-round choice)
+/* picks the persistent apply's schedule (element tiles of 0: 16 x 16,
+ * 1: 8 x 8, 2: 16 x 8), z-chunk length (0.5 / 1 / 2 x the whole-round choice)
  * and grid size (one workgroup per item, one or two rounds of resident
  * workgroups) by timing every combination; best ms per apply */
 int vfg_batch_autotune(vfg_batch *b, int fp32, double *best_ms);

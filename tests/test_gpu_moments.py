@@ -1,0 +1,27 @@
+"""u-apply in moment form against the assembled oracle operator: grids whose
+last tile owns one node or all of them (7-, 15-node tiles), grids on both sides
+of the FP32 tile switch, cubic and non-cubic elements."""
+import numpy as np
+import pytest
+
+from . import scenarios as S
+
+pytestmark = pytest.mark.gpu
+
+GRIDS = [(8, 8, 3), (15, 9, 4), (22, 15, 5), (23, 16, 2), (61, 30, 3), (64, 8, 6), (65, 8, 3), (30, 61, 2)]
+
+
+@pytest.mark.parametrize("cubic", [True, False], ids=["cubic", "stretched"])
+@pytest.mark.parametrize("n", GRIDS, ids=["x".join(map(str, g)) for g in GRIDS])
+def test_u_apply_moment_form(oracle, n, cubic):
+    # an entry sums about 900 products of both signs: 900 eps = 2e-13 (FP64)
+    # at worst; FP32 rounds its inputs too, 1e-5 as for the other FP32 applies
+    l = tuple((m - 1) / 8.0 for m in n) if cubic else (1.0, 2.3, 0.6)
+    s = S.make(n=n, l=l, seed=3 * sum(n), nu=0.3, bcU=S.MIXED_U)
+    op, F = S.to_oracle(oracle, s)
+    P = S.to_gpu(s)
+    ref = oracle.u_jacobian(op, F) @ s["x"]
+    scale = np.abs(ref).max()
+    assert np.abs(P.UIJacobian_mult(s["x"]) - ref).max() <= 1e-12 * scale
+    assert np.abs(P.UIJacobian_mult(s["x"], fp32=True) - ref).max() <= 1e-5 * scale
+    P.close()

@@ -42,7 +42,7 @@ class Batch:
         self._c(self.L.vfg_batch_autotune(self.b, int(fp32), C.byref(ms)))
         return ms.value
 
-    SCHEDULES = {0: "16x16 tiles, register march", 1: "8x8 tiles, register march", 2: "16x16 tiles, LDS-ring march"}
+    SCHEDULES = {0: "16x16 tiles", 1: "8x8 tiles", 2: "16x8 tiles"}
 
     def tune_points(self):
         """The (schedule, z-chunk scale, grid, ms) points the last autotune timed."""

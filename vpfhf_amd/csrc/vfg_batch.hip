@@ -321,7 +321,7 @@ struct vfg_batch {
   double *d_part = nullptr, *d_sc = nullptr, *d_scale = nullptr, *d_iscale = nullptr;
   void *d_ops = nullptr, *d_ops32 = nullptr, *d_opsx = nullptr;
   int grid = 0;  // persistent grid size (0: one block per item)
-  int sched = 0;  // persistent-apply schedule (batch_tile, BATCH_SCHEDS)
+  int sched = 0;  // persistent-apply schedule (batch_tile_x, BATCH_SCHEDS)
   double oz_scale = 1.;
   std::vector<vfg_tune_point> tune;  // the last autotuning's measurements
   int graph_on = 1, graph_chunk = 10;
@@ -365,10 +365,10 @@ static int build_items(vfg_batch *b, int slots, double oz_scale) {
   b->items.clear();
   b->oz.assign(b->np, 1);
   b->oz_scale = oz_scale;
-  const int ow = batch_tile(b->sched) - 1;  // owned node columns per tile
+  const int ow = batch_tile_x(b->sched) - 1, oh = batch_tile_y(b->sched) - 1;  // owned node columns per tile
   for (int p = 0; p < b->np; p++) {
     const Grid &G = b->m[p]->P.G;
-    int tx = (G.nx + ow - 1) / ow, ty = (G.ny + ow - 1) / ow;
+    int tx = (G.nx + ow - 1) / ow, ty = (G.ny + oh - 1) / oh;
     int oz = choose_oz_pub(G, tx * ty, slots);
     oz = (int)(oz * oz_scale + .5);
     if (oz < 2) oz = 2;
@@ -435,7 +435,7 @@ int vfg_batch_create(vfg_handle *const *members, int n, vfg_batch **out) {
       (rc = balloc(b, (void **)&b->d_part, 16 * ch.size())) || (rc = balloc(b, (void **)&b->d_sc, 8 * B_NS * n)) ||
       (rc = balloc(b, (void **)&b->d_scale, 8 * n)) || (rc = balloc(b, (void **)&b->d_iscale, 8 * n)) ||
       (rc = balloc(b, &b->d_ops, batch_op_bytes(0) * n)) || (rc = balloc(b, &b->d_ops32, batch_op_bytes(1) * n)) ||
-      (rc = balloc(b, &b->d_opsx, batch_op_bytes(0) * n)) || (rc = build_items(b, batch_slots(), 1.0))) {
+      (rc = balloc(b, &b->d_opsx, batch_op_bytes(0) * n)) || (rc = build_items(b, batch_slots(0), 1.0))) {
     vfg_batch_destroy(b);
     return rc;
   }
@@ -514,8 +514,7 @@ int vfg_batch_time_u_apply(vfg_batch *b, int fp32, int nrep, double *ms) {
 }
 
 // Autotuner: times the persistent apply for every (schedule, z-chunk scale,
-// grid) point -- schedules: 16 x 16 element tiles on the register march, 8 x 8
-// tiles on the register march, 16 x 16 tiles on the LDS-ring march; z-chunk
+// grid) point -- schedules: 16 x 16, 8 x 8 and 16 x 8 element tiles; z-chunk
 // lengths 0.5, 1 and 2 times the whole-round choice; one workgroup per item,
 // or a persistent grid of one or two rounds of resident workgroups -- keeps the
 // fastest and records every point (vfg_batch_tune_points); best_ms receives
@@ -586,7 +585,7 @@ static void cg_iter(vfg_batch *b, int o, void *ops, int fp32, double rtol, int m
   const BChunk *ch = b->d_ch;
   // frozen members are skipped by the apply and the vector kernels
   const int g = b->grid > 0 && b->grid < b->nitems ? b->grid : b->nitems;
-  launch_engine_u_apply(fp32, b->sched, ops, b->d_items, 0, b->d_nitems, g, b->d_sc + B_ACTIVE, B_NS, s);
+  launch_engine_u_apply(fp32, b->sched, 0, ops, b->d_items, 0, b->d_nitems, g, b->d_sc + B_ACTIVE, B_NS, s);
   hipLaunchKernelGGL(k_bdot<T>, dim3(b->nch), dim3(BRB), 0, s, (const BVec *)b->d_vt, o + VP, o + VQ, ch,
                      (const double *)b->d_sc, b->d_part);
   hipLaunchKernelGGL(k_bscalar, dim3(b->np), dim3(BRB), 0, s, (const double *)b->d_part, (const int *)b->d_first,

@@ -212,8 +212,8 @@ int bmg_rebuild(BatchMG *g, hipStream_t s, bool *grew) {
     if (l >= Lmax && !P.dcnt) continue;  // nothing on this level, ever
     if (!P.dcnt && (rc = galloc(g, (void **)&P.dcnt, 8 * sizeof(int)))) break;
     if (!P.ops && (rc = galloc(g, &P.ops, batch_op_bytes(1) * g->np))) break;
-    if (!P.ops_pre && (rc = galloc(g, &P.ops_pre, mg_smooth_op_bytes(0) * g->np))) break;
-    if (!P.ops_post && (rc = galloc(g, &P.ops_post, mg_smooth_op_bytes(1) * g->np))) break;
+    if (!P.ops_pre && (rc = galloc(g, &P.ops_pre, mg_smooth_op_bytes() * g->np))) break;
+    if (!P.ops_post && (rc = galloc(g, &P.ops_post, mg_smooth_op_bytes() * g->np))) break;
     BmgList *ls[3] = {&P.M, &P.D, &P.C};
     for (int k = 0; k < 3 && !rc; k++)
       if ((rc = grow(g, ls[k]->items, grew)) || (rc = grow(g, ls[k]->ch, grew))) break;
@@ -251,14 +251,14 @@ static int bmg_alloc(int np, BatchMG **out) {
   g->m.assign(np, nullptr);
   g->r32.assign(np, nullptr);
   g->z32.assign(np, nullptr);
-  g->slots = batch_slots();
+  g->slots = batch_slots(1);
   g->L.assign(np, 0);
   g->oz.assign(np, std::vector<int>(BML, 2));
   g->h_lvt.assign((size_t)np * BML, BmgVec{});
   g->h_coef.assign((size_t)np * BML * 2 * BMK, BmgCoef{0.f, 0.f});
   g->h_ops.assign(BML, std::vector<char>(batch_op_bytes(1) * np, 0));
-  g->h_pre.assign(BML, std::vector<char>(mg_smooth_op_bytes(0) * np, 0));
-  g->h_post.assign(BML, std::vector<char>(mg_smooth_op_bytes(1) * np, 0));
+  g->h_pre.assign(BML, std::vector<char>(mg_smooth_op_bytes() * np, 0));
+  g->h_post.assign(BML, std::vector<char>(mg_smooth_op_bytes() * np, 0));
   int rc = galloc(g, (void **)&g->d_lvt, sizeof(BmgVec) * np * BML);
   if (!rc) rc = galloc(g, (void **)&g->d_coef, sizeof(BmgCoef) * np * BML * 2 * BMK);
   if (rc) {
@@ -330,9 +330,9 @@ static void stage_member(BatchMG *g, int p) {
     // descending levels: pre-smoothing from 0 into d (A d into y), post-smoothing d -> x
     static_assert(MG_SMOOTH == 1, "the fused smoothing records do one Chebyshev step");
     make_mg_smooth_op(V.P, 0, v.b, v.dinv, cf[0].c2, nullptr, v.d, v.y, g->oz[p][l],
-                      g->h_pre[l].data() + mg_smooth_op_bytes(0) * p);
+                      g->h_pre[l].data() + mg_smooth_op_bytes() * p);
     make_mg_smooth_op(V.P, 1, v.b, v.dinv, cf[0].c2, v.d, v.x, nullptr, g->oz[p][l],
-                      g->h_post[l].data() + mg_smooth_op_bytes(1) * p);
+                      g->h_post[l].data() + mg_smooth_op_bytes() * p);
   }
 }
 static int upload_member(BatchMG *g, int p, hipStream_t s) {
@@ -342,7 +342,7 @@ static int upload_member(BatchMG *g, int p, hipStream_t s) {
       hipMemcpyAsync(g->d_coef + (size_t)p * BML * 2 * BMK, &g->h_coef[(size_t)p * BML * 2 * BMK],
                      sizeof(BmgCoef) * BML * 2 * BMK, hipMemcpyHostToDevice, s) != hipSuccess)
     return VFG_E_HIP;
-  const size_t pb = mg_smooth_op_bytes(0), qb = mg_smooth_op_bytes(1);
+  const size_t pb = mg_smooth_op_bytes(), qb = mg_smooth_op_bytes();
   for (int l = 0; l < g->L[p]; l++)
     if (!g->lv[l].ops || !g->lv[l].ops_pre || !g->lv[l].ops_post ||
         hipMemcpyAsync((char *)g->lv[l].ops + ob * p, g->h_ops[l].data() + ob * p, ob, hipMemcpyHostToDevice, s) !=
@@ -384,7 +384,7 @@ int bmg_setup_member(BatchMG *g, int p, const double *dinv64, hipStream_t s) {
 static void apply(BatchMG *g, int l, const BmgList &L, int which, const double *flags, int fstride, hipStream_t s) {
   if (!L.items.cap) return;
   const int grid = L.items.cap < g->slots ? L.items.cap : g->slots;
-  launch_engine_u_apply(1, 0, g->lv[l].ops, L.items.d, 0, g->lv[l].dcnt + 2 * which, grid, flags, fstride, s);
+  launch_engine_u_apply(1, 0, l > 0, g->lv[l].ops, L.items.d, 0, g->lv[l].dcnt + 2 * which, grid, flags, fstride, s);
 }
 static void cheb(BatchMG *g, int l, const BmgList &L, int which, int step, int use_y, int xzero, const double *flags,
                  int fstride, hipStream_t s) {
@@ -397,7 +397,7 @@ static void cheb(BatchMG *g, int l, const BmgList &L, int which, int step, int u
 static void smooth(BatchMG *g, int l, const BmgList &L, int post, const double *flags, int fstride, hipStream_t s) {
   if (!L.items.cap) return;
   const int grid = L.items.cap < g->slots ? L.items.cap : g->slots;
-  launch_batch_mg_smooth(post, post ? g->lv[l].ops_post : g->lv[l].ops_pre, L.items.d, g->lv[l].dcnt + 2, grid, flags,
+  launch_batch_mg_smooth(post, l > 0, post ? g->lv[l].ops_post : g->lv[l].ops_pre, L.items.d, g->lv[l].dcnt + 2, grid, flags,
                          fstride, s);
 }
 

@@ -705,7 +705,7 @@ static int advance(vfg_engine *e, int p) {
 static int rebuild_lists(vfg_engine *e) {
   for (int k = 0; k < 3; k++) e->h_it[k].clear();
   for (int k = 0; k < 2; k++) e->h_ch[k].clear();
-  const int slots = batch_slots();
+  const int slots = batch_slots(e->o.precision == VFG_PREC_MIXED);
   int pi = 0;
   for (int p = 0; p < e->ns; p++) e->h_first[p] = e->h_nch[p] = 0;
   for (int pass = 0; pass < 2; pass++)  // FP32 chunks first, then FP64: partial indices follow
@@ -764,9 +764,9 @@ static void e_iter(vfg_engine *e, bool with_mg) {
   hipStream_t s = e->s;
   const double *fl = e->d_sc + E_ACTIVE;
   if (e->o.precision == VFG_PREC_MIXED)
-    launch_engine_u_apply(1, 0, e->d_uop, e->d_it[0], 0, e->d_cnt + C_U32, e->grid_apply, fl, E_NS, s);
+    launch_engine_u_apply(1, 0, 0, e->d_uop, e->d_it[0], 0, e->d_cnt + C_U32, e->grid_apply, fl, E_NS, s);
   else
-    launch_engine_u_apply(0, 0, e->d_uop, e->d_it[1], 0, e->d_cnt + C_U64, e->grid_apply, fl, E_NS, s);
+    launch_engine_u_apply(0, 0, 0, e->d_uop, e->d_it[1], 0, e->d_cnt + C_U64, e->grid_apply, fl, E_NS, s);
   launch_engine_v_apply(e->d_vop, e->d_it[2], e->d_cnt + C_V, e->grid_vapply, fl, E_NS, s);
   hipLaunchKernelGGL(k_e_dot, dim3(e->grid_vec), dim3(ERB), 0, s, (const EVec *)e->d_vt, (const EChunk *)e->d_ch[0],
                      (const EChunk *)e->d_ch[1], (const int *)e->d_cnt, (const double *)e->d_sc, e->d_part);
@@ -872,7 +872,7 @@ int vfg_engine_create(const vfg_engine_opts *o, vfg_engine **out) {
   hipDeviceProp_t prop;
   int cus = 256;
   if (hipGetDeviceProperties(&prop, dev) == hipSuccess) cus = prop.multiProcessorCount;
-  e->grid_apply = batch_slots();
+  e->grid_apply = batch_slots(o->precision == VFG_PREC_MIXED);
   e->grid_vapply = 3 * cus;
   e->grid_vec = 4 * cus;
   bool ok = hipStreamCreateWithFlags(&e->s, hipStreamNonBlocking) == hipSuccess &&
@@ -944,7 +944,7 @@ int vfg_engine_submit(vfg_engine *e, vfg_handle *h, double *U, const double *BCU
   q.st = ST_U_BEGIN;
   const int mixed = e->o.precision == VFG_PREC_MIXED;
   const Grid &G = h->P.G;
-  const int oz = choose_oz_pub(G, ((G.nx + 14) / 15) * ((G.ny + 14) / 15), batch_slots());
+  const int oz = choose_oz_pub(G, ((G.nx + 14) / 15) * ((G.ny + 14) / 15), batch_slots(mixed));
   make_uop(h->P, mixed ? (const void *)h->wf[QP32 - QX32] : (const void *)h->w[QP],
            mixed ? (void *)h->wf[QQ32 - QX32] : (void *)h->w[QQ], mixed, oz, &e->h_uop[(size_t)p * e->uop_sz]);
   e->dirty_uop = true;

@@ -21,6 +21,7 @@ struct DevProblem {
   double E, nu, lam1, mu1, alpha, beta, Gc, eta, eps, irrevtol, atcv;
   int atnum, hasCrackPressure;
   int unilateral;   // VFG_UNILATERAL_*
+  int unit;         // a coarse multigrid level: V = 1, eta = 0 (the degradation is 1)
   uint32_t *cmask;  // per element: Gauss points where tr(eps(U_J)) < 0 (Jacobian state)
   BcMask bcU, bcV;
   vfg_bc hbcU[3], hbcV;

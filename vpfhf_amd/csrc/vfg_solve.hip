@@ -646,6 +646,7 @@ int mg_build(vfg_handle *h) {
     Pc.G = Gc;
     Pc.nn = (int64_t)Gc.nx * Gc.ny * Gc.nz;
     Pc.ne = (int64_t)Gc.nex * Gc.ney * Gc.nez;
+    Pc.unit = 1;
     lc.n = 3 * Pc.nn;
     if ((rc = vfg_alloc(h, (void **)&Pc.E_elem, 8 * (size_t)Pc.ne)) ||
         (rc = vfg_alloc(h, (void **)&Pc.V, 8 * (size_t)Pc.nn)) ||

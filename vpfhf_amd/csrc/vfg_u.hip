@@ -11,6 +11,7 @@
 // factorisation with the 1-D Gauss tables; d_x u_c is constant along x, so it
 // takes 9 distinct values per component.
 #include "vfg_internal.h"
+#include "vfg_umodal.h"
 #include "vfg_kernels.h"
 #include "vfg_batch_apply.h"
 #include "vfg_handle.h"
@@ -193,15 +194,12 @@ __device__ __forceinline__ void u_elem_apply(const T (&X)[2][4][4], T cE, T lam1
 // their z-differences (Dz); x-derivatives Gx[c][gy] for the layer; then
 // gx-outer, gy-inner over the 9 points, with interpolation written as
 // a + p1 (b - a) (one FMA per point and value).  Accumulation and the final
-// projections are those of u_elem_apply.  UNILATERAL_NONE only: the
-// NOCOMPRESSION apply keeps the register march.
-// QS != nullptr (stored coefficients): the 27 products W_g s_g E_e vol of the
-// element are read from QS[g * QSTRIDE], g = (gz * 3 + gy) * 3 + gx, instead
-// of being formed from the nodal v (then xs needs no field 3).
-template <typename T, typename XS, typename OUT, int QSTRIDE>
-__device__ __forceinline__ void u_elem_lds_impl(const XS &xs, T cE, T lam1, T mu1, T eta, T ihx, T ihy, T ihz,
-                                                const OUT &out, const T *__restrict__ QS) {
-  constexpr bool STORED = QSTRIDE > 0;
+// projections are those of u_elem_apply.  Stored coefficients: the 27 products
+// W_g s_g E_e vol of the element are read from QS[g * QSTRIDE],
+// g = (gz * 3 + gy) * 3 + gx.
+template <int QSTRIDE, typename T, typename XS, typename OUT>
+__device__ __forceinline__ void u_elem_apply_lds_stored(const XS &xs, T lam1, T mu1, T ihx, T ihy, T ihz,
+                                                        const OUT &out, const T *__restrict__ QS) {
   const T lr = lam1 / mu1;
   const T mx = mu1 * ihx, my = mu1 * ihy, mz = mu1 * ihz;
   // Rx[c][k][j], Ry[c][k][i]; Sz[c][gy][i]: the z-stress summed over the Gauss
@@ -225,14 +223,12 @@ __device__ __forceinline__ void u_elem_lds_impl(const XS &xs, T cE, T lam1, T mu
     // compiler barrier: the corners are read again from LDS for this layer
     // rather than kept live across layers
     asm volatile("" ::: "memory");
-    T Dz[4][3], Vz[4], Gx[3][3], by0[3], byd[3];
+    T Dz[4][3], Gx[3][3], by0[3], byd[3];
     T Ql[3][3];  // stored coefficients of the layer [gx][gy]
-    if constexpr (STORED) {
 #pragma unroll
-      for (int gx = 0; gx < 3; gx++)
+    for (int gx = 0; gx < 3; gx++)
 #pragma unroll
-        for (int gy = 0; gy < 3; gy++) Ql[gx][gy] = QS[((gz * 3 + gy) * 3 + gx) * QSTRIDE];
-    }
+      for (int gy = 0; gy < 3; gy++) Ql[gx][gy] = QS[((gz * 3 + gy) * 3 + gx) * QSTRIDE];
     {
       T Uz[4][3];
 #pragma unroll
@@ -242,10 +238,6 @@ __device__ __forceinline__ void u_elem_lds_impl(const XS &xs, T cE, T lam1, T mu
           const T a = xs(0, q, c), d = xs(1, q, c) - a;
           Uz[q][c] = a + pz1 * d;
           Dz[q][c] = d * mz;
-        }
-        if constexpr (!STORED) {
-          const T a = xs(0, q, 3);
-          Vz[q] = a + pz1 * (xs(1, q, 3) - a);
         }
       }
 #pragma unroll
@@ -263,8 +255,6 @@ __device__ __forceinline__ void u_elem_lds_impl(const XS &xs, T cE, T lam1, T mu
       Dzx0[c] = Dz[1][c] - Dz[0][c];
       Dzx2[c] = Dz[3][c] - Dz[2][c];
     }
-    T vdx0 = T(0), vdx2 = T(0);
-    if constexpr (!STORED) { vdx0 = Vz[1] - Vz[0]; vdx2 = Vz[3] - Vz[2]; }
     T Sx[3][3], ay[3][2];  // Sx[c][gy] = sum_gx sigma_c0; ay[c][i] = y-projection of sum_gy sigma_c1
 #pragma unroll
     for (int c = 0; c < 3; c++) {
@@ -272,7 +262,6 @@ __device__ __forceinline__ void u_elem_lds_impl(const XS &xs, T cE, T lam1, T mu
       for (int g = 0; g < 3; g++) Sx[c][g] = T(0);
       ay[c][0] = ay[c][1] = T(0);
     }
-    const T wz = cE * T(gW(gz));
 #pragma unroll
     for (int gx = 0; gx < 3; gx++) {
       const T px = T(gP1(gx));
@@ -284,22 +273,9 @@ __device__ __forceinline__ void u_elem_lds_impl(const XS &xs, T cE, T lam1, T mu
         azd[c] = Dz[2][c] + px * Dzx2[c] - az0[c];
         Sy[c] = T(0);
       }
-      T av0 = T(0), avd = T(0), w0 = T(0), w1 = T(0);
-      if constexpr (!STORED) {
-        av0 = Vz[0] + px * vdx0;
-        avd = Vz[2] + px * vdx2 - av0;
-        const T wzx = wz * T(gW(gx));
-        w0 = wzx * T(gW(0));
-        w1 = wzx * T(gW(1));
-      }
 #pragma unroll
       for (int gy = 0; gy < 3; gy++) {
-        T cq;
-        if constexpr (STORED) cq = Ql[gx][gy];
-        else {
-          const T v = av0 + T(gP1(gy)) * avd;
-          cq = (gy == 1 ? w1 : w0) * (v * v + eta);
-        }
+        const T cq = Ql[gx][gy];
         const T H00 = Gx[0][gy], H01 = Gy[0], H02 = az0[0] + T(gP1(gy)) * azd[0];
         const T H10 = Gx[1][gy], H11 = Gy[1], H12 = az0[1] + T(gP1(gy)) * azd[1];
         const T H20 = Gx[2][gy], H21 = Gy[2], H22 = az0[2] + T(gP1(gy)) * azd[2];
@@ -355,65 +331,31 @@ __device__ __forceinline__ void u_elem_lds_impl(const XS &xs, T cE, T lam1, T mu
   }
 }
 
-// recomputing form: s_g = v_g^2 + eta from the staged nodal v (field 3)
-template <typename T, typename XS, typename OUT>
-__device__ __forceinline__ void u_elem_apply_lds_out(const XS &xs, T cE, T lam1, T mu1, T eta, T ihx, T ihy, T ihz,
-                                                     const OUT &out) {
-  u_elem_lds_impl<T, XS, OUT, 0>(xs, cE, lam1, mu1, eta, ihx, ihy, ihz, out, nullptr);
-}
-// stored form: the 27 weights W_g s_g E_e vol at QS[g * QSTRIDE]
-template <int QSTRIDE, typename T, typename XS, typename OUT>
-__device__ __forceinline__ void u_elem_apply_lds_stored(const XS &xs, T lam1, T mu1, T ihx, T ihy, T ihz,
-                                                        const OUT &out, const T *__restrict__ QS) {
-  static_assert(QSTRIDE > 0, "stored weights need their stride");
-  u_elem_lds_impl<T, XS, OUT, QSTRIDE>(xs, T(0), lam1, mu1, T(0), ihx, ihy, ihz, out, QS);
-}
-// the same with the 24 outputs in registers
-template <typename T, typename XS>
-__device__ __forceinline__ void u_elem_apply_lds(const XS &xs, T cE, T lam1, T mu1, T eta, T ihx, T ihy, T ihz,
-                                                 T (&r)[8][3]) {
-  u_elem_apply_lds_out<T>(xs, cE, lam1, mu1, eta, ihx, ihy, ihz, [&](int a, int c, T v) { r[a][c] = v; });
-}
-
+// NOCOMPRESSION apply (Gauss-point form: its branch is per point)
 template <typename T>
 struct UAuxM {
   T E;
   uint32_t m;  // compressed Gauss points of the Jacobian state
 };
 
-template <typename T, bool UNI = false>
-struct UApplyOp {
+template <typename T>
+struct UApplyUniOp {
   static constexpr int NF = 4, NC = 3;
   const T *x;
   T *y;
   const T *v;
   const double *E_elem;
-  const uint32_t *cmask;  // UNI only
+  const uint32_t *cmask;
   Grid G;
   BcMask bc;
   T E, lam1, mu1, eta, vol, ihx, ihy, ihz;
   __device__ T load(int f, int64_t n) const { return f < 3 ? x[3 * n + f] : v[n]; }
-  __device__ auto aux(int ex, int ey, int ek) const {
+  __device__ UAuxM<T> aux(int ex, int ey, int ek) const {
     const int64_t c = cell_id(G, ex, ey, ek);
-    const T Ee = E_elem ? T(E_elem[c]) : E;
-    if constexpr (UNI) return UAuxM<T>{Ee, cmask[c]};
-    else return Ee;
+    return UAuxM<T>{E_elem ? T(E_elem[c]) : E, cmask[c]};
   }
-  template <typename A>
-  __device__ void element(int, int, int, const T (&xin)[2][4][4], A a, T (&r)[8][3]) const {
-    if constexpr (UNI) u_elem_apply<T, true>(xin, a.E * vol, lam1, mu1, eta, ihx, ihy, ihz, r, a.m);
-    else u_elem_apply<T>(xin, a * vol, lam1, mu1, eta, ihx, ihy, ihz, r);
-  }
-  template <typename XS, typename A>
-  __device__ void element_lds(int, int, int, const XS &xs, A a, T (&r)[8][3]) const {
-    static_assert(!UNI, "the NOCOMPRESSION apply uses the register march");
-    u_elem_apply_lds<T>(xs, a * vol, lam1, mu1, eta, ihx, ihy, ihz, r);
-  }
-  // the element's outputs handed to out(corner, component, value) as they are formed
-  template <typename XS, typename A, typename OUT>
-  __device__ void element_out(int, int, int, const XS &xs, A a, const OUT &out) const {
-    static_assert(!UNI, "the NOCOMPRESSION apply uses the register march");
-    u_elem_apply_lds_out<T>(xs, a * vol, lam1, mu1, eta, ihx, ihy, ihz, out);
+  __device__ void element(int, int, int, const T (&xin)[2][4][4], UAuxM<T> a, T (&r)[8][3]) const {
+    u_elem_apply<T, true>(xin, a.E * vol, lam1, mu1, eta, ihx, ihy, ihz, r, a.m);
   }
   __device__ void store(int i, int j, int k, const T (&acc)[3], const T (&own)[4]) const {
     int64_t n = node_id(G, i, j, k);
@@ -422,11 +364,56 @@ struct UApplyOp {
       y[3 * n + c] = on_dirichlet(G, bc.face[c], bc.vert[c], i, j, k) ? own[c] : acc[c];
   }
 };
-
 // FP32: at most 256 registers, two waves per SIMD
-template <typename T, int TX, int TY, bool UNI = false>
-__global__ __launch_bounds__(TX *TY, sizeof(T) == 4 ? 2 : 1) void k_u_apply(UApplyOp<T, UNI> op, int OZ) {
+template <typename T, int TX, int TY>
+__global__ __launch_bounds__(TX *TY, sizeof(T) == 4 ? 2 : 1) void k_u_apply_uni(UApplyUniOp<T> op, int OZ) {
   march<T, TX, TY>(op.G, op, OZ, xcd_block());
+}
+
+// Apply in moment form (UNILATERAL_NONE).  UNIT: s = 1, the coarse multigrid
+// levels; the record is the same for both, the kernel chooses.
+template <typename T>
+struct UModRec {
+  const T *x;
+  T *y;
+  const T *v;
+  const double *E_elem;
+  Grid G;
+  BcMask bc;
+  T E;
+  UModal<T> m;
+};
+template <typename T, bool UNIT_>
+struct UModOp : UModRec<T> {
+  static constexpr bool UNIT = UNIT_;
+  __device__ T load(int f, int64_t n) const { return f < 3 ? this->x[3 * n + f] : this->v[n]; }
+  __device__ T young(int ex, int ey, int ek) const {
+    return this->E_elem ? T(this->E_elem[cell_id(this->G, ex, ey, ek)]) : this->E;
+  }
+  __device__ bool dirichlet(int c, uint32_t fb) const { return face_dirichlet(this->bc.face[c], this->bc.vert[c], fb); }
+  __device__ void store(int64_t n, uint32_t fb, const T (&acc)[3], const T (&own)[3]) const {
+#pragma unroll
+    for (int c = 0; c < 3; c++) this->y[3 * n + c] = dirichlet(c, fb) ? own[c] : acc[c];
+  }
+};
+template <typename T>
+static void umod_fill(UModRec<T> &r, const DevProblem &P, const T *x, T *y) {
+  r.x = x;
+  r.y = y;
+  r.v = sizeof(T) == 4 ? (const T *)(const void *)P.V32 : (const T *)(const void *)P.V;
+  r.E_elem = P.E_elem;
+  r.G = P.G;
+  r.bc = P.bcU;
+  r.E = T(P.E);
+  r.m = make_umodal<T>(P.G, P.lam1, P.mu1, P.eta, P.unit != 0);
+}
+
+// waves per SIMD asked of the compiler: FP64 two (256 registers), FP32 three
+template <typename T>
+constexpr int um_waves() { return sizeof(T) == 8 ? 2 : 3; }
+template <typename T, int TX, int TY, bool UNIT>
+__global__ __launch_bounds__(TX *TY, um_waves<T>()) void k_u_apply(UModOp<T, UNIT> op, int OZ) {
+  march_modal<T, TX, TY>(op.G, op, OZ, xcd_block());
 }
 
 // FP32 multigrid apply fused with its Chebyshev(1)-Jacobi step (mg_cheb_entry
@@ -438,13 +425,19 @@ __global__ __launch_bounds__(TX *TY, sizeof(T) == 4 ? 2 : 1) void k_u_apply(UApp
 //        of the owned node are loaded a node plane ahead (own_load).  The
 //        rz form also reduces r . xo (r: the FP64 residual the V-cycle
 //        preconditions) over the owned rows, one partial per workgroup.
-struct UMgPreOp : UApplyOp<float, false> {
+struct UMgRec : UModRec<float> {
   const float *b, *dinv;
   float *xo, *ro;
   float c2;
+  const double *r64;  // rz form
+  double *part;       // rz form
+};
+template <bool UNIT_>
+struct UMgPreOp : UMgRec {
+  static constexpr bool UNIT = UNIT_;
   __device__ float load(int f, int64_t n) const { return f == 3 ? v[n] : c2 * dinv[3 * n + f] * b[3 * n + f]; }
-  __device__ void store(int i, int j, int k, const float (&acc)[3], const float (&own)[4]) const {
-    const int64_t n = node_id(G, i, j, k);
+  __device__ float young(int ex, int ey, int ek) const { return E_elem ? float(E_elem[cell_id(G, ex, ey, ek)]) : E; }
+  __device__ void store(int64_t n, uint32_t, const float (&acc)[3], const float (&own)[3]) const {
 #pragma unroll
     for (int c = 0; c < 3; c++) {
       xo[3 * n + c] = own[c];
@@ -459,15 +452,12 @@ struct MgOwnR {
   float b[3], di[3];
   double r[3];
 };
-template <bool RZ>
-struct UMgPostOp : UApplyOp<float, false> {
-  const float *b, *dinv;
-  float *xo;
-  float c2;
-  const double *r64;  // RZ
-  double *part;       // RZ
-  __device__ auto own_load(int i, int j, int k) const {
-    const int64_t n = node_id(G, i, j, k);
+template <bool UNIT_, bool RZ>
+struct UMgPostOp : UMgRec {
+  static constexpr bool UNIT = UNIT_;
+  __device__ float load(int f, int64_t n) const { return f < 3 ? x[3 * n + f] : v[n]; }
+  __device__ float young(int ex, int ey, int ek) const { return E_elem ? float(E_elem[cell_id(G, ex, ey, ek)]) : E; }
+  __device__ auto own_load(int64_t n) const {
     std::conditional_t<RZ, MgOwnR, MgOwn> o;
 #pragma unroll
     for (int c = 0; c < 3; c++) {
@@ -478,12 +468,11 @@ struct UMgPostOp : UApplyOp<float, false> {
     return o;
   }
   template <typename O>
-  __device__ auto store(int i, int j, int k, const float (&acc)[3], const float (&own)[4], const O &o) const {
-    const int64_t n = node_id(G, i, j, k);
+  __device__ auto store(int64_t n, uint32_t fb, const float (&acc)[3], const float (&own)[3], const O &o) const {
     double rz = 0.;
 #pragma unroll
     for (int c = 0; c < 3; c++) {
-      const float yv = on_dirichlet(G, bc.face[c], bc.vert[c], i, j, k) ? own[c] : acc[c];
+      const float yv = face_dirichlet(bc.face[c], bc.vert[c], fb) ? own[c] : acc[c];
       const float z = own[c] + c2 * o.di[c] * (o.b[c] - yv);
       xo[3 * n + c] = z;
       if constexpr (RZ) rz += o.r[c] * (double)z;
@@ -491,40 +480,23 @@ struct UMgPostOp : UApplyOp<float, false> {
     if constexpr (RZ) return rz;
   }
 };
-struct UMgPostRzOp : UMgPostOp<true> {
+struct UMgPostRzOp : UMgPostOp<false, true> {
   __device__ void partial(int slot, double v) const { part[slot] = v; }
 };
-template <int TX, int TY>
-__global__ __launch_bounds__(TX *TY, 2) void k_u_mg_pre(UMgPreOp op, int OZ) {
-  march<float, TX, TY>(op.G, op, OZ, xcd_block());
-}
-template <int TX, int TY>
-__global__ __launch_bounds__(TX *TY, 2) void k_u_mg_post(UMgPostOp<false> op, int OZ) {
-  march<float, TX, TY>(op.G, op, OZ, xcd_block());
-}
-template <int TX, int TY>
-__global__ __launch_bounds__(TX *TY, 2) void k_u_mg_post_rz(UMgPostRzOp op, int OZ) {
-  march<float, TX, TY>(op.G, op, OZ, xcd_block(), blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));
+template <class Op, int TX, int TY>
+__global__ __launch_bounds__(TX *TY, 3) void k_u_mg(Op op, int OZ) {
+  march_modal<float, TX, TY>(op.G, op, OZ, xcd_block(), blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));
 }
 
-// FP64 apply with the corners in LDS: at most 256 registers, two waves per
-// SIMD; the next plane is loaded at the start of its layer (the other
-// resident workgroup covers the latency; a register prefetch measured slower)
-__global__ __launch_bounds__(256, 2) void k_u_apply_lds(UApplyOp<double, false> op, int OZ) {
-  const Blk3 b = xcd_block();
-  march_lds<double, 16, 16, false>(op.G, op, OZ, b.x, b.y, b.z);
-}
-
-// the same apply, also reducing p.q (p = the input, q = the output, every
+// the FP64 apply also reducing p.q (p = the input, q = the output, every
 // row) to one partial per workgroup: the CG's p.q without another pass
-struct UApplyDotOp : UApplyOp<double, false> {
+struct UApplyDotOp : UModOp<double, false> {
   double *part;
-  __device__ double store(int i, int j, int k, const double (&acc)[3], const double (&own)[4]) const {
-    const int64_t n = node_id(G, i, j, k);
+  __device__ double store(int64_t n, uint32_t fb, const double (&acc)[3], const double (&own)[3]) const {
     double d = 0.;
 #pragma unroll
     for (int c = 0; c < 3; c++) {
-      const double yv = on_dirichlet(G, bc.face[c], bc.vert[c], i, j, k) ? own[c] : acc[c];
+      const double yv = dirichlet(c, fb) ? own[c] : acc[c];
       y[3 * n + c] = yv;
       d += own[c] * yv;
     }
@@ -532,10 +504,9 @@ struct UApplyDotOp : UApplyOp<double, false> {
   }
   __device__ void partial(int slot, double v) const { part[slot] = v; }
 };
-__global__ __launch_bounds__(256, 2) void k_u_apply_lds_dot(UApplyDotOp op, int OZ) {
-  const Blk3 b = xcd_block();
-  march_lds<double, 16, 16, false>(op.G, op, OZ, b.x, b.y, b.z,
-                                   blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));
+__global__ __launch_bounds__(256, 2) void k_u_apply_dot(UApplyDotOp op, int OZ) {
+  march_modal<double, 16, 16>(op.G, op, OZ, xcd_block(),
+                              blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));
 }
 
 // ------------------------------------------------ stored-form FP64 apply
@@ -1093,13 +1064,11 @@ static int device_slots(K kernel, int threads) {
 }
 
 // FP32 grids of 16-64 nodes in x (coarse multigrid levels) march 8 x 8 tiles
-// of 7 x 7 owned nodes: more, shorter workgroups, and no row of two 15-node
-// tiles whose second owns 1-2 nodes (16-17 nodes in x), which runs the
-// 16 x 16 apply at 34-37 us against 14 us (five times the memory waits)
+// of 7 x 7 owned nodes: more, shorter workgroups
 constexpr int SMALL_NX_LO = 16, SMALL_NX_HI = 64;
-template <typename T, bool UNI>
-static void launch_u_apply_u(const DevProblem &P, const T *x, T *y, const T *v, hipStream_t s) {
-  UApplyOp<T, UNI> op;
+template <typename T>
+static void launch_u_apply_uni(const DevProblem &P, const T *x, T *y, const T *v, hipStream_t s) {
+  UApplyUniOp<T> op;
   op.x = x; op.y = y; op.v = v;
   op.E_elem = P.E_elem;
   op.cmask = P.cmask;
@@ -1107,40 +1076,44 @@ static void launch_u_apply_u(const DevProblem &P, const T *x, T *y, const T *v, 
   op.E = T(P.E); op.lam1 = T(P.lam1); op.mu1 = T(P.mu1); op.eta = T(P.eta);
   op.vol = T(P.G.hx * P.G.hy * P.G.hz);
   op.ihx = T(1. / P.G.hx); op.ihy = T(1. / P.G.hy); op.ihz = T(1. / P.G.hz);
-  int tiles = ((P.G.nx + 14) / 15) * ((P.G.ny + 14) / 15);
-  if constexpr (sizeof(T) == 8 && !UNI) {
+  const int tiles = ((P.G.nx + 14) / 15) * ((P.G.ny + 14) / 15);
+  static int slots = device_slots(k_u_apply_uni<T, 16, 16>, 256);
+  const int OZ = choose_oz(P.G, tiles, slots);
+  hipLaunchKernelGGL((k_u_apply_uni<T, 16, 16>), march_grid(P.G, 16, 16, OZ), dim3(256), 0, s, op, OZ);
+}
+template <typename T, int W, bool UNIT>
+static void launch_u_apply_w(const DevProblem &P, const T *x, T *y, hipStream_t s) {
+  UModOp<T, UNIT> op;
+  umod_fill<T>(op, P, x, y);
+  static int slots = device_slots(k_u_apply<T, W, W, UNIT>, W * W);
+  const int OZ = choose_oz(P.G, ((P.G.nx + W - 2) / (W - 1)) * ((P.G.ny + W - 2) / (W - 1)), slots);
+  hipLaunchKernelGGL((k_u_apply<T, W, W, UNIT>), march_grid(P.G, W, W, OZ), dim3(W * W), 0, s, op, OZ);
+}
+
+template <typename T>
+static void launch_u_apply_t(const DevProblem &P, const T *x, T *y, const T *v, hipStream_t s) {
+  if (P.unilateral) {
+    launch_u_apply_uni<T>(P, x, y, v, s);
+    return;
+  }
+  if constexpr (sizeof(T) == 8) {
     if (P.uq) {
       UApplyLdsqOp<false> q;
       q.x = (const double *)x; q.y = (double *)y; q.part = nullptr; q.uq = P.uq;
       q.G = P.G; q.bc = P.bcU; q.lam1 = P.lam1; q.mu1 = P.mu1;
       q.ihx = 1. / P.G.hx; q.ihy = 1. / P.G.hy; q.ihz = 1. / P.G.hz;
+      const int tiles = ((P.G.nx + 14) / 15) * ((P.G.ny + 14) / 15);
       static int lqslots = device_slots(k_u_apply_ldsq, 256);
       const int OZ = choose_oz(P.G, tiles, lqslots);
       hipLaunchKernelGGL(k_u_apply_ldsq, march_grid(P.G, 16, 16, OZ), dim3(256), 0, s, q, OZ);
       return;
     }
-    static int slots = device_slots(k_u_apply_lds, 256);
-    int OZ = choose_oz(P.G, tiles, slots);
-    hipLaunchKernelGGL(k_u_apply_lds, march_grid(P.G, 16, 16, OZ), dim3(256), 0, s, op, OZ);
+    launch_u_apply_w<T, 16, false>(P, x, y, s);
   } else {
-    if constexpr (sizeof(T) == 4 && !UNI) {
-      if (P.G.nx >= SMALL_NX_LO && P.G.nx <= SMALL_NX_HI) {
-        static int slots = device_slots(k_u_apply<T, 8, 8, false>, 64);
-        int OZ = choose_oz(P.G, ((P.G.nx + 6) / 7) * ((P.G.ny + 6) / 7), slots);
-        hipLaunchKernelGGL((k_u_apply<T, 8, 8, false>), march_grid(P.G, 8, 8, OZ), dim3(64), 0, s, op, OZ);
-        return;
-      }
-    }
-    static int slots = device_slots(k_u_apply<T, 16, 16, UNI>, 256);
-    int OZ = choose_oz(P.G, tiles, slots);
-    hipLaunchKernelGGL((k_u_apply<T, 16, 16, UNI>), march_grid(P.G, 16, 16, OZ), dim3(256), 0, s, op, OZ);
+    const bool small = P.G.nx >= SMALL_NX_LO && P.G.nx <= SMALL_NX_HI;
+    if (P.unit) small ? launch_u_apply_w<T, 8, true>(P, x, y, s) : launch_u_apply_w<T, 16, true>(P, x, y, s);
+    else small ? launch_u_apply_w<T, 8, false>(P, x, y, s) : launch_u_apply_w<T, 16, false>(P, x, y, s);
   }
-}
-
-template <typename T>
-static void launch_u_apply_t(const DevProblem &P, const T *x, T *y, const T *v, hipStream_t s) {
-  if (P.unilateral) launch_u_apply_u<T, true>(P, x, y, v, s);
-  else launch_u_apply_u<T, false>(P, x, y, v, s);
 }
 
 // per element: the Gauss points where tr(eps(U)) < 0
@@ -1164,20 +1137,27 @@ void launch_u_cmask(const DevProblem &P, const double *U, hipStream_t s) {
 // (the coarsest multigrid level, at most MGC_NE elements): x, d and the
 // operator output stay in LDS.  An apply is an element pass (one element per
 // thread, its 24 outputs to LDS) and a node pass that adds each node's eight
-// element contributions in the order of the marching apply (x-pairs, then
-// y-pairs, the lower element layer before the upper), so it gives the values
-// of launch_u_apply_f32; the step is mg_cheb_entry, as in the multi-launch
-// smoother.
+// element contributions in a fixed order (x-pairs, then y-pairs, the lower
+// element layer before the upper); the step is mg_cheb_entry, as in the
+// multi-launch smoother.
 // one apply record of the batched / engine applies
 template <typename T>
 struct BApply {
-  UApplyOp<T> op;
+  UModRec<T> op;
   int OZ;
 };
+// the kernel's op from a record
+template <class Op, class Rec>
+__device__ __forceinline__ Op op_of(const Rec &r) {
+  Op o;
+  static_cast<Rec &>(o) = r;
+  return o;
+}
 
 constexpr int MGC_T = 512, MGC_NE = 512, MGC_NN = 729;
 
-__device__ __forceinline__ void mg_coarse_cheb_body(const UApplyOp<float, false> &op, const float *__restrict__ b,
+template <bool UNIT>
+__device__ __forceinline__ void mg_coarse_cheb_body(const UModOp<float, UNIT> &op, const float *__restrict__ b,
                                                     const float *__restrict__ dinv, float *__restrict__ xout,
                                                     const MgChebCoefs &cc) {
   __shared__ float sx[3 * MGC_NN], sd[3 * MGC_NN], sy[3 * MGC_NN];
@@ -1197,22 +1177,39 @@ __device__ __forceinline__ void mg_coarse_cheb_body(const UApplyOp<float, false>
     if (i > 0) {
       for (int e = tid; e < ne; e += MGC_T) {
         const int ex = e % G.nex, ey = (e / G.nex) % G.ney, ez = e / (G.nex * G.ney);
-        float xin[2][4][4];
+        UFace<float> fb, ft;
+        float U[3][8], M[3][3][3];
+        const int64_t n0 = node_id(G, ex, ey, ez), nr = G.nx, np = (int64_t)G.nx * G.ny;
 #pragma unroll
-        for (int kz = 0; kz < 2; kz++)
+        for (int c = 0; c < 3; c++) {
+          const float *xb = sx + 3 * n0 + c, *xt = xb + 3 * np;
+          uface_set<float>(fb, c, xb[0], xb[3], xb[3 * nr], xb[3 * nr + 3]);
+          uface_set<float>(ft, c, xt[0], xt[3], xt[3 * nr], xt[3 * nr + 3]);
+        }
+        const float Ek = op.young(ex, ey, ez) * op.m.kap;
+        if constexpr (!UNIT) {
+          const float *vp = op.v + n0, *vq = vp + np;
+          const float vb[4] = {vp[0], vp[1], vp[nr], vp[nr + 1]}, vt[4] = {vq[0], vq[1], vq[nr], vq[nr + 1]};
+          um_moments<float>(vb, vt, Ek, op.m.eta4, M);
+        }
+        um_modes<float>(fb, ft, U);
 #pragma unroll
-          for (int q = 0; q < 4; q++) {
-            const int64_t n = node_id(G, ex + (q & 1), ey + (q >> 1), ez + kz);
+        for (int c = 0; c < 3; c++) {
+          float R[8];
+          if constexpr (UNIT) um_force_unit<float>(Ek, U, op.m, c, R);
+          else um_force<float>(M, U, op.m, c, R);
 #pragma unroll
-            for (int f = 0; f < 3; f++) xin[kz][q][f] = sx[3 * n + f];
-            xin[kz][q][3] = op.v[n];
+          for (int kz = 0; kz < 2; kz++) {
+            const float z = kz ? 1.f : -1.f;
+            const float t0 = z * R[4], t1 = R[1] + z * R[5], t2 = R[2] + z * R[6], t3 = R[3] + z * R[7];
+            const float e0 = t0 - t1, e1 = t0 + t1, f0 = t2 - t3, f1 = t2 + t3;
+            float *o = sr + e * 24 + kz * 12 + c;
+            o[0] = e0 - f0;
+            o[3] = e1 - f1;
+            o[6] = e0 + f0;
+            o[9] = e1 + f1;
           }
-        float r[8][3];
-        op.element(ex, ey, ez, xin, op.aux(ex, ey, ez), r);
-#pragma unroll
-        for (int a = 0; a < 8; a++)
-#pragma unroll
-          for (int c = 0; c < 3; c++) sr[e * 24 + a * 3 + c] = r[a][c];
+        }
       }
       __syncthreads();
       for (int n = tid; n < nn; n += MGC_T) {
@@ -1237,15 +1234,16 @@ __device__ __forceinline__ void mg_coarse_cheb_body(const UApplyOp<float, false>
   for (int t = tid; t < 3 * nn; t += MGC_T) xout[t] = sx[t];
 }
 
-__global__ __launch_bounds__(MGC_T) void k_mg_coarse_cheb(UApplyOp<float, false> op, const float *__restrict__ b,
+__global__ __launch_bounds__(MGC_T) void k_mg_coarse_cheb(UModOp<float, true> op, const float *__restrict__ b,
                                                           const float *__restrict__ dinv, float *__restrict__ xout,
                                                           MgChebCoefs cc) {
-  mg_coarse_cheb_body(op, b, dinv, xout, cc);
+  mg_coarse_cheb_body<true>(op, b, dinv, xout, cc);
 }
 
 // the batched form: one workgroup per listed member (its first chunk), the
 // member's level operator, vectors and coarsest-level coefficients from the
 // engine's tables
+template <bool UNIT>
 __global__ __launch_bounds__(MGC_T) void k_bmg_coarse_cheb(const BApply<float> *__restrict__ ops,
                                                            const BmgVec *__restrict__ lvt, int level,
                                                            const BmgChunk *__restrict__ ch, const int *__restrict__ dn,
@@ -1263,7 +1261,7 @@ __global__ __launch_bounds__(MGC_T) void k_bmg_coarse_cheb(const BApply<float> *
     cc.c1[i] = k.c1;
     cc.c2[i] = k.c2;
   }
-  mg_coarse_cheb_body(ops[c.p].op, v.b, v.dinv, v.x, cc);
+  mg_coarse_cheb_body<UNIT>(op_of<UModOp<float, UNIT>>(ops[c.p].op), v.b, v.dinv, v.x, cc);
 }
 
 bool mg_coarse_fits(const DevProblem &P) {
@@ -1272,22 +1270,21 @@ bool mg_coarse_fits(const DevProblem &P) {
 
 void launch_mg_coarse_cheb(const DevProblem &P, const float *b, const float *dinv, float *x, const MgChebCoefs &cc,
                            hipStream_t s) {
-  UApplyOp<float, false> op;
-  op.x = nullptr; op.y = nullptr; op.v = P.V32;
-  op.E_elem = P.E_elem;
-  op.cmask = nullptr;
-  op.G = P.G; op.bc = P.bcU;
-  op.E = float(P.E); op.lam1 = float(P.lam1); op.mu1 = float(P.mu1); op.eta = float(P.eta);
-  op.vol = float(P.G.hx * P.G.hy * P.G.hz);
-  op.ihx = float(1. / P.G.hx); op.ihy = float(1. / P.G.hy); op.ihz = float(1. / P.G.hz);
+  UModOp<float, true> op;  // a coarse level: s = 1
+  umod_fill<float>(op, P, nullptr, nullptr);
   hipLaunchKernelGGL(k_mg_coarse_cheb, dim3(1), dim3(MGC_T), 0, s, op, b, dinv, x, cc);
 }
 
 void launch_bmg_coarse_cheb(const void *ops, const BmgVec *lvt, int level, const BmgChunk *ch, const int *dn,
                             int grid, const BmgCoef *coef, const double *flags, int fstride, hipStream_t s) {
   if (grid <= 0) return;
-  hipLaunchKernelGGL(k_bmg_coarse_cheb, dim3(grid), dim3(MGC_T), 0, s, (const BApply<float> *)ops, lvt, level, ch,
-                     dn, coef, flags, fstride);
+  // level 0: a problem small enough to be its own coarsest level
+  if (level > 0)
+    hipLaunchKernelGGL(k_bmg_coarse_cheb<true>, dim3(grid), dim3(MGC_T), 0, s, (const BApply<float> *)ops, lvt, level,
+                       ch, dn, coef, flags, fstride);
+  else
+    hipLaunchKernelGGL(k_bmg_coarse_cheb<false>, dim3(grid), dim3(MGC_T), 0, s, (const BApply<float> *)ops, lvt,
+                       level, ch, dn, coef, flags, fstride);
 }
 
 void launch_u_apply(const DevProblem &P, const double *x, double *y, hipStream_t s) {
@@ -1297,13 +1294,7 @@ void launch_u_apply(const DevProblem &P, const double *x, double *y, hipStream_t
 int launch_u_apply_dot(const DevProblem &P, const double *x, double *y, double *part, hipStream_t s) {
   if (P.unilateral) return 0;
   UApplyDotOp op;
-  op.x = x; op.y = y; op.v = P.V;
-  op.E_elem = P.E_elem;
-  op.cmask = nullptr;
-  op.G = P.G; op.bc = P.bcU;
-  op.E = P.E; op.lam1 = P.lam1; op.mu1 = P.mu1; op.eta = P.eta;
-  op.vol = P.G.hx * P.G.hy * P.G.hz;
-  op.ihx = 1. / P.G.hx; op.ihy = 1. / P.G.hy; op.ihz = 1. / P.G.hz;
+  umod_fill<double>(op, P, x, y);
   op.part = part;
   if (P.uq) {
     UApplyLdsqDotOp q;
@@ -1317,68 +1308,59 @@ int launch_u_apply_dot(const DevProblem &P, const double *x, double *y, double *
     hipLaunchKernelGGL(k_u_apply_ldsq_dot, g, dim3(256), 0, s, q, OZ);
     return (int)(g.x * g.y * g.z);
   }
-  static int slots = device_slots(k_u_apply_lds_dot, 256);
+  static int slots = device_slots(k_u_apply_dot, 256);
   const int tiles = ((P.G.nx + 14) / 15) * ((P.G.ny + 14) / 15);
   const int OZ = choose_oz(P.G, tiles, slots);
   const dim3 g = march_grid(P.G, 16, 16, OZ);
-  hipLaunchKernelGGL(k_u_apply_lds_dot, g, dim3(256), 0, s, op, OZ);
+  hipLaunchKernelGGL(k_u_apply_dot, g, dim3(256), 0, s, op, OZ);
   return (int)(g.x * g.y * g.z);
 }
 void launch_u_apply_f32(const DevProblem &P, const float *x, float *y, hipStream_t s) {
   launch_u_apply_t<float>(P, x, y, P.V32, s);
 }
 
-template <class Op>
-static void mg_op_fill(Op &op, const DevProblem &P, const float *b, const float *dinv, float c2) {
-  op.y = nullptr; op.v = P.V32;
-  op.E_elem = P.E_elem;
-  op.cmask = nullptr;
-  op.G = P.G; op.bc = P.bcU;
-  op.E = float(P.E); op.lam1 = float(P.lam1); op.mu1 = float(P.mu1); op.eta = float(P.eta);
-  op.vol = float(P.G.hx * P.G.hy * P.G.hz);
-  op.ihx = float(1. / P.G.hx); op.ihy = float(1. / P.G.hy); op.ihz = float(1. / P.G.hz);
+static void mg_op_fill(UMgRec &op, const DevProblem &P, const float *b, const float *dinv, float c2) {
+  umod_fill<float>(op, P, nullptr, nullptr);
   op.b = b; op.dinv = dinv; op.c2 = c2;
+  op.xo = nullptr; op.ro = nullptr; op.r64 = nullptr; op.part = nullptr;
 }
-// launches kernel 8x8 or 16x16 by the grid's x extent; returns the workgroup
+// launches 8 x 8 or 16 x 16 tiles by the grid's x extent; returns the workgroup
 // count, or 0 without launching when it would exceed max_wg
-template <class Op, class K8, class K16>
-static int mg_launch(const DevProblem &P, const Op &op, K8 k8, K16 k16, int &slots8, int &slots16, hipStream_t s,
-                     int64_t max_wg = INT32_MAX) {
-  const bool small = P.G.nx >= SMALL_NX_LO && P.G.nx <= SMALL_NX_HI;
-  if (small && !slots8) slots8 = device_slots(k8, 64);
-  if (!small && !slots16) slots16 = device_slots(k16, 256);
-  const int T = small ? 8 : 16;
-  const int OZ = choose_oz(P.G, ((P.G.nx + T - 2) / (T - 1)) * ((P.G.ny + T - 2) / (T - 1)), small ? slots8 : slots16);
-  const dim3 g = march_grid(P.G, T, T, OZ);
+template <class Op, int W>
+static int mg_launch_w(const DevProblem &P, const Op &op, hipStream_t s, int64_t max_wg) {
+  static int slots = device_slots(k_u_mg<Op, W, W>, W * W);
+  const int OZ = choose_oz(P.G, ((P.G.nx + W - 2) / (W - 1)) * ((P.G.ny + W - 2) / (W - 1)), slots);
+  const dim3 g = march_grid(P.G, W, W, OZ);
   const int64_t nwg = (int64_t)g.x * g.y * g.z;
   if (nwg > max_wg) return 0;
-  if (small) hipLaunchKernelGGL(k8, g, dim3(64), 0, s, op, OZ);
-  else hipLaunchKernelGGL(k16, g, dim3(256), 0, s, op, OZ);
+  hipLaunchKernelGGL((k_u_mg<Op, W, W>), g, dim3(W * W), 0, s, op, OZ);
   return (int)nwg;
+}
+template <class Op>
+static int mg_launch(const DevProblem &P, const UMgRec &r, hipStream_t s, int64_t max_wg = INT32_MAX) {
+  Op op;
+  static_cast<UMgRec &>(op) = r;
+  const bool small = P.G.nx >= SMALL_NX_LO && P.G.nx <= SMALL_NX_HI;
+  return small ? mg_launch_w<Op, 8>(P, op, s, max_wg) : mg_launch_w<Op, 16>(P, op, s, max_wg);
 }
 void launch_mg_presmooth(const DevProblem &P, const float *b, const float *dinv, float c2, float *x, float *r,
                          hipStream_t s) {
-  UMgPreOp op;
+  UMgRec op;
   mg_op_fill(op, P, b, dinv, c2);
-  op.x = nullptr; op.xo = x; op.ro = r;
-  static int s8 = 0, s16 = 0;
-  mg_launch(P, op, k_u_mg_pre<8, 8>, k_u_mg_pre<16, 16>, s8, s16, s);
+  op.xo = x; op.ro = r;
+  if (P.unit) mg_launch<UMgPreOp<true>>(P, op, s);
+  else mg_launch<UMgPreOp<false>>(P, op, s);
 }
 int launch_mg_postsmooth(const DevProblem &P, const float *b, const float *dinv, float c2, const float *x, float *xo,
                          const double *r64, double *part, hipStream_t s) {
+  UMgRec op;
+  mg_op_fill(op, P, b, dinv, c2);
+  op.x = x; op.xo = xo; op.r64 = r64; op.part = part;
   if (r64) {
-    UMgPostRzOp op;
-    mg_op_fill(op, P, b, dinv, c2);
-    op.x = x; op.xo = xo; op.r64 = r64; op.part = part;
-    static int s8 = 0, s16 = 0;
-    const int n = mg_launch(P, op, k_u_mg_post_rz<8, 8>, k_u_mg_post_rz<16, 16>, s8, s16, s, 2 * 65536);
+    const int n = mg_launch<UMgPostRzOp>(P, op, s, 2 * 65536);
     if (n) return n;  // else too many workgroups for the partials: the plain form
   }
-  UMgPostOp<false> op;
-  mg_op_fill(op, P, b, dinv, c2);
-  op.x = x; op.xo = xo; op.r64 = nullptr; op.part = nullptr;
-  static int s8 = 0, s16 = 0;
-  return mg_launch(P, op, k_u_mg_post<8, 8>, k_u_mg_post<16, 16>, s8, s16, s);
+  return P.unit ? mg_launch<UMgPostOp<true, false>>(P, op, s) : mg_launch<UMgPostOp<false, false>>(P, op, s);
 }
 
 void launch_u_diag(const DevProblem &P, double *d, hipStream_t s) {
@@ -1452,30 +1434,29 @@ namespace vfg {
 // the device, so a captured graph follows a list that changes between replays;
 // flags (optional) skip items of members whose flags[p * fstride] is 0.
 // Schedules (the autotuner's choice): TX x TY element tiles of (TX-1) x (TY-1)
-// owned node columns, on the register march or the LDS-ring march.
-template <typename T, int TX, int TY, bool LDS>
-__global__ __launch_bounds__(TX *TY, (sizeof(T) == 4 || LDS) ? 2 : 1) void k_batch_u_apply(
+// owned node columns.  UNIT: the records are coarse multigrid levels.
+template <typename T, int TX, int TY, bool UNIT>
+__global__ __launch_bounds__(TX *TY, um_waves<T>()) void k_batch_u_apply(
     const BApply<T> *__restrict__ probs, const BItem *__restrict__ items, int nitems, const int *__restrict__ dcount,
     const double *__restrict__ flags, int fstride) {
   const int n = dcount ? *dcount : nitems;
   for (int it = blockIdx.x; it < n; it += gridDim.x) {
     const BItem w = items[it];
     if (flags && flags[(int64_t)w.p * fstride] == 0.) continue;  // uniform per block
-    const UApplyOp<T> op = probs[w.p].op;
+    const auto op = op_of<UModOp<T, UNIT>>(probs[w.p].op);
     const int OZ = probs[w.p].OZ;
     __syncthreads();  // LDS of the previous item is free
-    if constexpr (LDS) march_lds<T, TX, TY, false>(op.G, op, OZ, w.bx, w.by, w.bz);
-    else march<T, TX, TY>(op.G, op, OZ, w.bx, w.by, w.bz);
+    march_modal<T, TX, TY>(op.G, op, OZ, w.bx, w.by, w.bz);
   }
 }
 
-// schedule -> tile width and threads: 0: 16 x 16 register march, 1: 8 x 8
-// register march, 2: 16 x 16 LDS-ring march
-int batch_tile(int sched) { return sched == 1 ? 8 : 16; }
+// schedule -> tile: 0: 16 x 16, 1: 8 x 8, 2: 16 x 8
+int batch_tile_x(int sched) { return sched == 1 ? 8 : 16; }
+int batch_tile_y(int sched) { return sched == 0 ? 16 : 8; }
 template <typename T>
 static int batch_slots_t(int sched) {
   if (sched == 1) return device_slots(k_batch_u_apply<T, 8, 8, false>, 64);
-  if (sched == 2) return device_slots(k_batch_u_apply<T, 16, 16, true>, 256);
+  if (sched == 2) return device_slots(k_batch_u_apply<T, 16, 8, false>, 128);
   return device_slots(k_batch_u_apply<T, 16, 16, false>, 256);
 }
 int batch_slots_s(int fp32, int sched) {
@@ -1489,7 +1470,7 @@ size_t batch_op_bytes(int fp32) { return fp32 ? sizeof(BApply<float>) : sizeof(B
 
 int choose_oz_pub(const Grid &G, int tiles_xy, int slots) { return choose_oz(G, tiles_xy, slots); }
 
-int batch_slots() { return batch_slots_s(0, 0); }
+int batch_slots(int fp32) { return batch_slots_s(fp32, 0); }
 
 template <typename T>
 static void fill_ops_t(const std::vector<vfg_handle *> &m, const void *const *x, void *const *y,
@@ -1497,16 +1478,7 @@ static void fill_ops_t(const std::vector<vfg_handle *> &m, const void *const *x,
   std::vector<BApply<T>> ops(m.size());
   for (size_t p = 0; p < m.size(); p++) {
     const DevProblem &P = m[p]->P;
-    UApplyOp<T> &op = ops[p].op;
-    op.x = (const T *)x[p];
-    op.y = (T *)y[p];
-    op.v = sizeof(T) == 4 ? (const T *)(const void *)P.V32 : (const T *)(const void *)P.V;
-    op.E_elem = P.E_elem;
-    op.G = P.G;
-    op.bc = P.bcU;
-    op.E = T(P.E); op.lam1 = T(P.lam1); op.mu1 = T(P.mu1); op.eta = T(P.eta);
-    op.vol = T(P.G.hx * P.G.hy * P.G.hz);
-    op.ihx = T(1. / P.G.hx); op.ihy = T(1. / P.G.hy); op.ihz = T(1. / P.G.hz);
+    umod_fill<T>(ops[p].op, P, (const T *)x[p], (T *)y[p]);
     ops[p].OZ = oz[p];
   }
   hipStreamSynchronize(s);  // no kernel of the previous call still reads d_ops
@@ -1522,96 +1494,80 @@ void fill_ops(const std::vector<vfg_handle *> &m, const void *const *x, void *co
 void launch_batch_apply(int fp32, int sched, const void *d_ops, const BItem *items, int nitems, int grid,
                         hipStream_t s) {
   const int g = grid > 0 && grid < nitems ? grid : nitems;
-  launch_engine_u_apply(fp32, sched, d_ops, items, nitems, nullptr, g, nullptr, 0, s);
+  launch_engine_u_apply(fp32, sched, 0, d_ops, items, nitems, nullptr, g, nullptr, 0, s);
 }
 
-template <typename T>
-static void launch_batch_t(int sched, const void *d_ops, const BItem *items, int nitems, const int *dcount, int grid,
+template <typename T, int TX, int TY, bool UNIT>
+static void launch_batch_t(const void *d_ops, const BItem *items, int nitems, const int *dcount, int grid,
                            const double *flags, int fstride, hipStream_t s) {
-  const BApply<T> *ops = (const BApply<T> *)d_ops;
-  if (sched == 1)
-    hipLaunchKernelGGL((k_batch_u_apply<T, 8, 8, false>), dim3(grid), dim3(64), 0, s, ops, items, nitems, dcount,
-                       flags, fstride);
-  else if (sched == 2)
-    hipLaunchKernelGGL((k_batch_u_apply<T, 16, 16, true>), dim3(grid), dim3(256), 0, s, ops, items, nitems, dcount,
-                       flags, fstride);
-  else
-    hipLaunchKernelGGL((k_batch_u_apply<T, 16, 16, false>), dim3(grid), dim3(256), 0, s, ops, items, nitems, dcount,
-                       flags, fstride);
+  hipLaunchKernelGGL((k_batch_u_apply<T, TX, TY, UNIT>), dim3(grid), dim3(TX * TY), 0, s, (const BApply<T> *)d_ops,
+                     items, nitems, dcount, flags, fstride);
 }
-void launch_engine_u_apply(int fp32, int sched, const void *d_ops, const BItem *items, int nitems,
+template <typename T>
+static void launch_batch_s(int sched, const void *d_ops, const BItem *items, int nitems, const int *dcount, int grid,
+                           const double *flags, int fstride, hipStream_t s) {
+  if (sched == 1) launch_batch_t<T, 8, 8, false>(d_ops, items, nitems, dcount, grid, flags, fstride, s);
+  else if (sched == 2) launch_batch_t<T, 16, 8, false>(d_ops, items, nitems, dcount, grid, flags, fstride, s);
+  else launch_batch_t<T, 16, 16, false>(d_ops, items, nitems, dcount, grid, flags, fstride, s);
+}
+void launch_engine_u_apply(int fp32, int sched, int unit, const void *d_ops, const BItem *items, int nitems,
                            const int *dcount, int grid, const double *flags, int fstride, hipStream_t s) {
-  if (fp32) launch_batch_t<float>(sched, d_ops, items, nitems, dcount, grid, flags, fstride, s);
-  else launch_batch_t<double>(sched, d_ops, items, nitems, dcount, grid, flags, fstride, s);
+  if (unit) launch_batch_t<float, 16, 16, true>(d_ops, items, nitems, dcount, grid, flags, fstride, s);
+  else if (fp32) launch_batch_s<float>(sched, d_ops, items, nitems, dcount, grid, flags, fstride, s);
+  else launch_batch_s<double>(sched, d_ops, items, nitems, dcount, grid, flags, fstride, s);
 }
 
 // multigrid smoothing records and their persistent launch
-template <class OpT>
 struct BSmooth {
-  OpT op;
+  UMgRec op;
   int OZ;
 };
-using BMgPre = BSmooth<UMgPreOp>;
-using BMgPost = BSmooth<UMgPostOp<false>>;
-template <class Rec>
-__global__ __launch_bounds__(256, 2) void k_batch_mg_smooth(const Rec *__restrict__ recs, const BItem *__restrict__ items,
+template <class Op>
+__global__ __launch_bounds__(256, 3) void k_batch_mg_smooth(const BSmooth *__restrict__ recs,
+                                                            const BItem *__restrict__ items,
                                                             const int *__restrict__ dcount,
                                                             const double *__restrict__ flags, int fstride) {
   const int n = *dcount;
   for (int it = blockIdx.x; it < n; it += gridDim.x) {
     const BItem w = items[it];
     if (flags && flags[(int64_t)w.p * fstride] == 0.) continue;  // uniform per block
-    const auto op = recs[w.p].op;
+    const Op op = op_of<Op>(recs[w.p].op);
     const int OZ = recs[w.p].OZ;
     __syncthreads();  // LDS of the previous item is free
-    march<float, 16, 16>(op.G, op, OZ, w.bx, w.by, w.bz);
+    march_modal<float, 16, 16>(op.G, op, OZ, w.bx, w.by, w.bz);
   }
 }
-size_t mg_smooth_op_bytes(int post) { return post ? sizeof(BMgPost) : sizeof(BMgPre); }
+size_t mg_smooth_op_bytes() { return sizeof(BSmooth); }
 void make_mg_smooth_op(const DevProblem &P, int post, const float *b, const float *dinv, float c2, const float *xin,
                        float *xo, float *ro, int OZ, void *out) {
-  if (post) {
-    BMgPost r;
-    mg_op_fill(r.op, P, b, dinv, c2);
-    r.op.x = xin; r.op.xo = xo; r.op.r64 = nullptr; r.op.part = nullptr;
-    r.OZ = OZ;
-    *(decltype(r) *)out = r;
-  } else {
-    BMgPre r;
-    mg_op_fill(r.op, P, b, dinv, c2);
-    r.op.x = nullptr; r.op.xo = xo; r.op.ro = ro;
-    r.OZ = OZ;
-    *(decltype(r) *)out = r;
-  }
+  BSmooth r;
+  mg_op_fill(r.op, P, b, dinv, c2);
+  r.op.x = post ? xin : nullptr;
+  r.op.xo = xo;
+  r.op.ro = post ? nullptr : ro;
+  r.OZ = OZ;
+  *(BSmooth *)out = r;
 }
-void launch_batch_mg_smooth(int post, const void *d_ops, const BItem *items, const int *dcount, int grid,
+void launch_batch_mg_smooth(int post, int unit, const void *d_ops, const BItem *items, const int *dcount, int grid,
                             const double *flags, int fstride, hipStream_t s) {
-  if (post)
-    hipLaunchKernelGGL(k_batch_mg_smooth<BMgPost>, dim3(grid), dim3(256), 0, s, (const BMgPost *)d_ops, items, dcount,
-                       flags, fstride);
-  else
-    hipLaunchKernelGGL(k_batch_mg_smooth<BMgPre>, dim3(grid), dim3(256), 0, s, (const BMgPre *)d_ops, items, dcount,
-                       flags, fstride);
+  auto go = [&](auto k) {
+    hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, s, (const BSmooth *)d_ops, items, dcount, flags, fstride);
+  };
+  if (post) unit ? go(k_batch_mg_smooth<UMgPostOp<true, false>>) : go(k_batch_mg_smooth<UMgPostOp<false, false>>);
+  else unit ? go(k_batch_mg_smooth<UMgPreOp<true>>) : go(k_batch_mg_smooth<UMgPreOp<false>>);
 }
 
 // one member's operator entry for a persistent list (host memory `out`)
 void make_uop(const DevProblem &P, const void *x, void *y, int fp32, int OZ, void *out) {
-  auto fill = [&](auto *b, auto one) {
-    using T = decltype(one);
-    UApplyOp<T> &op = b->op;
-    op.x = (const T *)x;
-    op.y = (T *)y;
-    op.v = sizeof(T) == 4 ? (const T *)(const void *)P.V32 : (const T *)(const void *)P.V;
-    op.E_elem = P.E_elem;
-    op.G = P.G;
-    op.bc = P.bcU;
-    op.E = T(P.E); op.lam1 = T(P.lam1); op.mu1 = T(P.mu1); op.eta = T(P.eta);
-    op.vol = T(P.G.hx * P.G.hy * P.G.hz);
-    op.ihx = T(1. / P.G.hx); op.ihy = T(1. / P.G.hy); op.ihz = T(1. / P.G.hz);
+  if (fp32) {
+    BApply<float> *b = (BApply<float> *)out;
+    umod_fill<float>(b->op, P, (const float *)x, (float *)y);
     b->OZ = OZ;
-  };
-  if (fp32) fill((BApply<float> *)out, 0.f);
-  else fill((BApply<double> *)out, 0.);
+  } else {
+    BApply<double> *b = (BApply<double> *)out;
+    umod_fill<double>(b->op, P, (const double *)x, (double *)y);
+    b->OZ = OZ;
+  }
 }
 
 }  // namespace vfg
