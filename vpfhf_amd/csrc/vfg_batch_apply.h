@@ -39,6 +39,7 @@ void launch_batch_mg_smooth(int post, int unit, const void *d_ops, const BItem *
                             const double *flags, int fstride, hipStream_t s);
 size_t vop_bytes();
 int v_oz(const Grid &G);
+int v_apply_slots();  // resident workgroups of the V apply on the device
 void make_vop(const DevProblem &P, const double *x, double *y, const uint8_t *mask, void *out);
 void launch_engine_v_apply(const void *d_ops, const BItem *items, const int *dcount, int grid, const double *flags,
                            int fstride, hipStream_t s);

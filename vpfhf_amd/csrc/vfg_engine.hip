@@ -873,7 +873,7 @@ int vfg_engine_create(const vfg_engine_opts *o, vfg_engine **out) {
   int cus = 256;
   if (hipGetDeviceProperties(&prop, dev) == hipSuccess) cus = prop.multiProcessorCount;
   e->grid_apply = batch_slots(o->precision == VFG_PREC_MIXED);
-  e->grid_vapply = 3 * cus;
+  e->grid_vapply = v_apply_slots();
   e->grid_vec = 4 * cus;
   bool ok = hipStreamCreateWithFlags(&e->s, hipStreamNonBlocking) == hipSuccess &&
             hipMalloc((void **)&e->d_sc, 8 * E_NS * (size_t)e->ns) == hipSuccess &&

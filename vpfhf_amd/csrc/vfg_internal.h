@@ -144,11 +144,6 @@ template <class Op, class = void>
 struct is_tiled : std::false_type {};
 template <class Op>
 struct is_tiled<Op, std::void_t<decltype(Op::TILED)>> : std::true_type {};
-// tile-blocked layout: [tile][element layer][coefficient][TX*TY slots]
-__host__ __device__ inline int64_t tiled_index(int tile, int ek, int nez, int ncoef, int slot, int coef, int nslot) {
-  return (((int64_t)tile * nez + ek) * ncoef + coef) * nslot + slot;
-}
-
 // Ops whose store also reads data of the owned node that is not staged define
 //   __device__ O own_load(int i, int j, int k)      (O trivially copyable)
 //   store(i, j, k, acc, own, O o)

@@ -31,7 +31,7 @@ struct DevProblem {
   double *zero3;                          // 3*nn zeros
   // V-subproblem state, refreshed by vfg_v_set_u
   double *uq;      // FP64 u-apply, stored form: W_g s_g E_e vol per element (uq_doubles); null: recomputed
-  double *Vq;      // W_g * (c_AT/eps [AT2] + 2 W^el_g), tile-blocked (vq_doubles)
+  double *Vq;      // 27 moments per element of W_g (c_AT/eps [AT2] + 2 W^el_g), tile-blocked (vq_doubles)
   double *bV;      // V load vector (nn)
   uint8_t *vfix;   // fixed V rows/cols (Dirichlet + AT2 irreversibility)
 };

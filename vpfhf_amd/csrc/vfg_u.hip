@@ -383,17 +383,65 @@ struct UModRec {
   T E;
   UModal<T> m;
 };
-template <typename T, bool UNIT_>
-struct UModOp : UModRec<T> {
-  static constexpr bool UNIT = UNIT_;
-  __device__ T load(int f, int64_t n) const { return f < 3 ? this->x[3 * n + f] : this->v[n]; }
-  __device__ T young(int ex, int ey, int ek) const {
+// the parts of the march's interface that every moment-form operator shares
+// (Rec: UModRec<T> or a record derived from it)
+template <typename T_, bool UNIT, class Rec>
+struct UModBase : Rec {
+  using T = T_;
+  using Record = Rec;
+  static constexpr int NF = UNIT ? 3 : 4, NC = 3;
+  struct Face {
+    UFace<T> f;
+    T v[UNIT ? 1 : 4], own[3];
+  };
+  struct Own {
+    T x[3];
+  };
+  using Aux = T;  // E_e
+  using Raw = T;
+  static __device__ T off() { return T(0); }
+  __device__ T stage(int, T v) const { return v; }
+  template <class RD>
+  __device__ void face(const RD &rd, Face &F) const {
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      const T x3 = rd(c, 3);
+      uface_set<T>(F.f, c, rd(c, 0), rd(c, 1), rd(c, 2), x3);
+      F.own[c] = x3;
+    }
+    if constexpr (!UNIT)
+#pragma unroll
+      for (int q = 0; q < 4; q++) F.v[q] = rd(NF - 1, q);
+  }
+  __device__ Own own(const Face &F) const { return Own{{F.own[0], F.own[1], F.own[2]}}; }
+  __device__ T aux(int ex, int ey, int ek, int, int) const {
     return this->E_elem ? T(this->E_elem[cell_id(this->G, ex, ey, ek)]) : this->E;
   }
-  __device__ bool dirichlet(int c, uint32_t fb) const { return face_dirichlet(this->bc.face[c], this->bc.vert[c], fb); }
-  __device__ void store(int64_t n, uint32_t fb, const T (&acc)[3], const T (&own)[3]) const {
+  __device__ void element(T Ee, const Face &B, const Face &F, T (&tot)[3][4], T (&carry)[3][4]) const {
+    um_layer<T, UNIT>(B.f, F.f, B.v, F.v, Ee, this->m, tot, carry);
+  }
+  // A x of a node: the displacement itself on the Dirichlet rows (a wavefront
+  // without a boundary node skips the tests)
+  __device__ void rows(uint32_t fb, const T (&acc)[3], const Own &own, T (&yv)[3]) const {
 #pragma unroll
-    for (int c = 0; c < 3; c++) this->y[3 * n + c] = dirichlet(c, fb) ? own[c] : acc[c];
+    for (int c = 0; c < 3; c++) yv[c] = acc[c];
+    if (__builtin_amdgcn_ballot_w64(fb != 0u) != 0) {
+      __asm__ __volatile__("");  // keeps the tests inside the branch
+#pragma unroll
+      for (int c = 0; c < 3; c++)
+        if (face_dirichlet(this->bc.face[c], this->bc.vert[c], fb)) yv[c] = own.x[c];
+    }
+  }
+};
+template <typename T, bool UNIT>
+struct UModOp : UModBase<T, UNIT, UModRec<T>> {
+  using typename UModBase<T, UNIT, UModRec<T>>::Own;
+  __device__ T load(int f, int64_t n) const { return f < 3 ? this->x[3 * n + f] : this->v[n]; }
+  __device__ void store(int64_t n, uint32_t fb, const T (&acc)[3], const Own &own) const {
+    T yv[3];
+    this->rows(fb, acc, own, yv);
+#pragma unroll
+    for (int c = 0; c < 3; c++) this->y[3 * n + c] = yv[c];
   }
 };
 template <typename T>
@@ -413,7 +461,7 @@ template <typename T>
 constexpr int um_waves() { return sizeof(T) == 8 ? 2 : 3; }
 template <typename T, int TX, int TY, bool UNIT>
 __global__ __launch_bounds__(TX *TY, um_waves<T>()) void k_u_apply(UModOp<T, UNIT> op, int OZ) {
-  march_modal<T, TX, TY>(op.G, op, OZ, xcd_block());
+  march_modal<TX, TY>(op.G, op, OZ, xcd_block());
 }
 
 // FP32 multigrid apply fused with its Chebyshev(1)-Jacobi step (mg_cheb_entry
@@ -432,16 +480,23 @@ struct UMgRec : UModRec<float> {
   const double *r64;  // rz form
   double *part;       // rz form
 };
-template <bool UNIT_>
-struct UMgPreOp : UMgRec {
-  static constexpr bool UNIT = UNIT_;
-  __device__ float load(int f, int64_t n) const { return f == 3 ? v[n] : c2 * dinv[3 * n + f] * b[3 * n + f]; }
-  __device__ float young(int ex, int ey, int ek) const { return E_elem ? float(E_elem[cell_id(G, ex, ey, ek)]) : E; }
-  __device__ void store(int64_t n, uint32_t, const float (&acc)[3], const float (&own)[3]) const {
+template <bool UNIT>
+struct UMgPreOp : UModBase<float, UNIT, UMgRec> {
+  using typename UModBase<float, UNIT, UMgRec>::Own;
+  struct Raw {
+    float b, di;
+  };
+  static __device__ Raw off() { return Raw{0.f, 0.f}; }
+  __device__ Raw load(int f, int64_t n) const {
+    if (f == 3) return Raw{this->v[n], 0.f};
+    return Raw{this->b[3 * n + f], this->dinv[3 * n + f]};
+  }
+  __device__ float stage(int f, const Raw &r) const { return f == 3 ? r.b : this->c2 * r.di * r.b; }
+  __device__ void store(int64_t n, uint32_t, const float (&acc)[3], const Own &own) const {
 #pragma unroll
     for (int c = 0; c < 3; c++) {
-      xo[3 * n + c] = own[c];
-      ro[3 * n + c] = acc[c];
+      this->xo[3 * n + c] = own.x[c];
+      this->ro[3 * n + c] = acc[c];
     }
   }
 };
@@ -452,29 +507,29 @@ struct MgOwnR {
   float b[3], di[3];
   double r[3];
 };
-template <bool UNIT_, bool RZ>
-struct UMgPostOp : UMgRec {
-  static constexpr bool UNIT = UNIT_;
-  __device__ float load(int f, int64_t n) const { return f < 3 ? x[3 * n + f] : v[n]; }
-  __device__ float young(int ex, int ey, int ek) const { return E_elem ? float(E_elem[cell_id(G, ex, ey, ek)]) : E; }
+template <bool UNIT, bool RZ>
+struct UMgPostOp : UModBase<float, UNIT, UMgRec> {
+  using typename UModBase<float, UNIT, UMgRec>::Own;
+  __device__ float load(int f, int64_t n) const { return f < 3 ? this->x[3 * n + f] : this->v[n]; }
   __device__ auto own_load(int64_t n) const {
     std::conditional_t<RZ, MgOwnR, MgOwn> o;
 #pragma unroll
     for (int c = 0; c < 3; c++) {
-      o.b[c] = b[3 * n + c];
-      o.di[c] = dinv[3 * n + c];
-      if constexpr (RZ) o.r[c] = r64[3 * n + c];
+      o.b[c] = this->b[3 * n + c];
+      o.di[c] = this->dinv[3 * n + c];
+      if constexpr (RZ) o.r[c] = this->r64[3 * n + c];
     }
     return o;
   }
   template <typename O>
-  __device__ auto store(int64_t n, uint32_t fb, const float (&acc)[3], const float (&own)[3], const O &o) const {
+  __device__ auto store(int64_t n, uint32_t fb, const float (&acc)[3], const Own &own, const O &o) const {
     double rz = 0.;
+    float yv[3];
+    this->rows(fb, acc, own, yv);
 #pragma unroll
     for (int c = 0; c < 3; c++) {
-      const float yv = face_dirichlet(bc.face[c], bc.vert[c], fb) ? own[c] : acc[c];
-      const float z = own[c] + c2 * o.di[c] * (o.b[c] - yv);
-      xo[3 * n + c] = z;
+      const float z = own.x[c] + this->c2 * o.di[c] * (o.b[c] - yv[c]);
+      this->xo[3 * n + c] = z;
       if constexpr (RZ) rz += o.r[c] * (double)z;
     }
     if constexpr (RZ) return rz;
@@ -485,28 +540,28 @@ struct UMgPostRzOp : UMgPostOp<false, true> {
 };
 template <class Op, int TX, int TY>
 __global__ __launch_bounds__(TX *TY, 3) void k_u_mg(Op op, int OZ) {
-  march_modal<float, TX, TY>(op.G, op, OZ, xcd_block(), blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));
+  march_modal<TX, TY>(op.G, op, OZ, xcd_block(), blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));
 }
 
 // the FP64 apply also reducing p.q (p = the input, q = the output, every
 // row) to one partial per workgroup: the CG's p.q without another pass
 struct UApplyDotOp : UModOp<double, false> {
   double *part;
-  __device__ double store(int64_t n, uint32_t fb, const double (&acc)[3], const double (&own)[3]) const {
-    double d = 0.;
+  __device__ double store(int64_t n, uint32_t fb, const double (&acc)[3], const Own &own) const {
+    double d = 0., yv[3];
+    rows(fb, acc, own, yv);
 #pragma unroll
     for (int c = 0; c < 3; c++) {
-      const double yv = dirichlet(c, fb) ? own[c] : acc[c];
-      y[3 * n + c] = yv;
-      d += own[c] * yv;
+      y[3 * n + c] = yv[c];
+      d += own.x[c] * yv[c];
     }
     return d;
   }
   __device__ void partial(int slot, double v) const { part[slot] = v; }
 };
 __global__ __launch_bounds__(256, 2) void k_u_apply_dot(UApplyDotOp op, int OZ) {
-  march_modal<double, 16, 16>(op.G, op, OZ, xcd_block(),
-                              blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));
+  march_modal<16, 16>(op.G, op, OZ, xcd_block(),
+                      blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));
 }
 
 // ------------------------------------------------ stored-form FP64 apply
@@ -1049,8 +1104,7 @@ int choose_oz(const Grid &G, int tiles_xy, int slots) {
 }
 
 // resident workgroups of a kernel on the whole device (occupancy x CUs)
-template <typename K>
-static int device_slots(K kernel, int threads) {
+int device_slots_of(const void *kernel, int threads) {
   static int cus = 0;
   if (!cus) {
     int dev = 0;
@@ -1061,6 +1115,10 @@ static int device_slots(K kernel, int threads) {
   int per = 0;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, threads, 0) != hipSuccess || per < 1) per = 1;
   return per * cus;
+}
+template <typename K>
+static int device_slots(K kernel, int threads) {
+  return device_slots_of((const void *)kernel, threads);
 }
 
 // FP32 grids of 16-64 nodes in x (coarse multigrid levels) march 8 x 8 tiles
@@ -1147,10 +1205,10 @@ struct BApply {
   int OZ;
 };
 // the kernel's op from a record
-template <class Op, class Rec>
-__device__ __forceinline__ Op op_of(const Rec &r) {
+template <class Op>
+__device__ __forceinline__ Op op_of(const typename Op::Record &r) {
   Op o;
-  static_cast<Rec &>(o) = r;
+  static_cast<typename Op::Record &>(o) = r;
   return o;
 }
 
@@ -1178,7 +1236,6 @@ __device__ __forceinline__ void mg_coarse_cheb_body(const UModOp<float, UNIT> &o
       for (int e = tid; e < ne; e += MGC_T) {
         const int ex = e % G.nex, ey = (e / G.nex) % G.ney, ez = e / (G.nex * G.ney);
         UFace<float> fb, ft;
-        float U[3][8], M[3][3][3];
         const int64_t n0 = node_id(G, ex, ey, ez), nr = G.nx, np = (int64_t)G.nx * G.ny;
 #pragma unroll
         for (int c = 0; c < 3; c++) {
@@ -1186,30 +1243,28 @@ __device__ __forceinline__ void mg_coarse_cheb_body(const UModOp<float, UNIT> &o
           uface_set<float>(fb, c, xb[0], xb[3], xb[3 * nr], xb[3 * nr + 3]);
           uface_set<float>(ft, c, xt[0], xt[3], xt[3 * nr], xt[3 * nr + 3]);
         }
-        const float Ek = op.young(ex, ey, ez) * op.m.kap;
+        float vb[4] = {}, vt[4] = {}, t[2][3][4] = {};
         if constexpr (!UNIT) {
           const float *vp = op.v + n0, *vq = vp + np;
-          const float vb[4] = {vp[0], vp[1], vp[nr], vp[nr + 1]}, vt[4] = {vq[0], vq[1], vq[nr], vq[nr + 1]};
-          um_moments<float>(vb, vt, Ek, op.m.eta4, M);
+#pragma unroll
+          for (int q = 0; q < 4; q++) {
+            vb[q] = vp[(q >> 1) * nr + (q & 1)];
+            vt[q] = vq[(q >> 1) * nr + (q & 1)];
+          }
         }
-        um_modes<float>(fb, ft, U);
+        um_layer<float, UNIT>(fb, ft, vb, vt, op.aux(ex, ey, ez, 0, 0), op.m, t[0], t[1]);
 #pragma unroll
-        for (int c = 0; c < 3; c++) {
-          float R[8];
-          if constexpr (UNIT) um_force_unit<float>(Ek, U, op.m, c, R);
-          else um_force<float>(M, U, op.m, c, R);
+        for (int kz = 0; kz < 2; kz++)
 #pragma unroll
-          for (int kz = 0; kz < 2; kz++) {
-            const float z = kz ? 1.f : -1.f;
-            const float t0 = z * R[4], t1 = R[1] + z * R[5], t2 = R[2] + z * R[6], t3 = R[3] + z * R[7];
-            const float e0 = t0 - t1, e1 = t0 + t1, f0 = t2 - t3, f1 = t2 + t3;
+          for (int c = 0; c < 3; c++) {
+            const float(&u)[4] = t[kz][c];
+            const float e0 = u[0] - u[1], e1 = u[0] + u[1], f0 = u[2] - u[3], f1 = u[2] + u[3];
             float *o = sr + e * 24 + kz * 12 + c;
             o[0] = e0 - f0;
             o[3] = e1 - f1;
             o[6] = e0 + f0;
             o[9] = e1 + f1;
           }
-        }
       }
       __syncthreads();
       for (int n = tid; n < nn; n += MGC_T) {
@@ -1446,7 +1501,7 @@ __global__ __launch_bounds__(TX *TY, um_waves<T>()) void k_batch_u_apply(
     const auto op = op_of<UModOp<T, UNIT>>(probs[w.p].op);
     const int OZ = probs[w.p].OZ;
     __syncthreads();  // LDS of the previous item is free
-    march_modal<T, TX, TY>(op.G, op, OZ, w.bx, w.by, w.bz);
+    march_modal<TX, TY>(op.G, op, OZ, w.bx, w.by, w.bz);
   }
 }
 
@@ -1534,7 +1589,7 @@ __global__ __launch_bounds__(256, 3) void k_batch_mg_smooth(const BSmooth *__res
     const Op op = op_of<Op>(recs[w.p].op);
     const int OZ = recs[w.p].OZ;
     __syncthreads();  // LDS of the previous item is free
-    march_modal<float, 16, 16>(op.G, op, OZ, w.bx, w.by, w.bz);
+    march_modal<16, 16>(op.G, op, OZ, w.bx, w.by, w.bz);
   }
 }
 size_t mg_smooth_op_bytes() { return sizeof(BSmooth); }

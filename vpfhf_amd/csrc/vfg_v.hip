@@ -4,51 +4,37 @@
 //   K[a][b] = c sum_g W_g (phi_a phi_b / eps [AT2 only] + eps grad phi_a . grad phi_b)
 //           + sum_g W_g phi_a phi_b 2 W^el_g,            c = Gc / atCv / 2,
 //   W^el_g = 1/2 sigma(e~):e~,  e~ = e(u) - alpha dtheta I  (VFMech.c:32-106).
-// Split as K = ks * L + M_q with the constant Q1 stiffness L (8x8, exact for
-// the 27-point rule) and the point-weighted mass M_q, q_g = W_g (c/eps [AT2] +
-// 2 W^el_g) precomputed once per U (vfg_v_set_u) and stored [27][N_e].
-#include "vfg_internal.h"
+// Split as K = ks * L + M_q with the Q1 stiffness L and the point-weighted mass
+// M_q, q_g = W_g (c/eps [AT2] + 2 W^el_g).  A product of two trilinear functions
+// has degree 2 per variable, so M_q depends on the q_g only through their 27
+// moments
+//   Q_pqr = sum_g q_g xi_g^p eta_g^q zeta_g^r / 64,  p, q, r <= 2,
+// precomputed once per U (vfg_v_set_u): (M_q x)_abc = sum Q_(a+a',b+b',c+c') x_a'b'c'
+// in modal sums (vfg_modal.h), 64 FMAs per element, and L is diagonal there.
+#include "vfg_modal.h"
 #include "vfg_kernels.h"
 
 namespace vfg {
 
 struct VConst {
-  double L[64];     // sum_g W_g grad phi_a . grad phi_b (element of size h)
-  double ks;        // c * eps
+  double ks[8];     // ks L in modal sums: c eps vol / 16 sum_d (1/h_d^2) (1/3)^(other powers)
   double crhs;      // Gc/atCv/eps * (.5 AT2 | .25 AT1), VFMech.c:2350-2384
 };
 
 static VConst make_vconst(const DevProblem &P) {
   VConst C;
-  const double h[3] = {P.G.hx, P.G.hy, P.G.hz};
-  for (int a = 0; a < 8; a++)
-    for (int b = 0; b < 8; b++) {
-      double s = 0.;
-      for (int g = 0; g < 27; g++) {
-        int gx = g % 3, gy = (g / 3) % 3, gz = g / 9;
-        const int ga[3] = {gx, gy, gz};
-        double W = h[0] * h[1] * h[2] * gW(gx) * gW(gy) * gW(gz);
-        double da[3], db[3];
-        for (int d = 0; d < 3; d++) {
-          double pa = 1., pb = 1.;
-          for (int e = 0; e < 3; e++) {
-            int ia = (a >> e) & 1, ib = (b >> e) & 1;
-            if (e == d) {
-              pa *= (ia ? 1. : -1.) / h[e];
-              pb *= (ib ? 1. : -1.) / h[e];
-            } else {
-              pa *= ia ? gP1(ga[e]) : gP0(ga[e]);
-              pb *= ib ? gP1(ga[e]) : gP0(ga[e]);
-            }
-          }
-          da[d] = pa; db[d] = pb;
-        }
-        s += W * (da[0] * db[0] + da[1] * db[1] + da[2] * db[2]);
-      }
-      C.L[a * 8 + b] = s;
+  const double h[3] = {P.G.hx, P.G.hy, P.G.hz}, c = P.Gc / P.atcv * .5;
+  for (int i = 0; i < 8; i++) {
+    double t = 0.;
+    for (int d = 0; d < 3; d++) {
+      if (!um_pow(i, d)) continue;
+      double w = 1. / (h[d] * h[d]);
+      for (int e = 0; e < 3; e++)
+        if (e != d && um_pow(i, e)) w /= 3.;
+      t += w;
     }
-  double c = P.Gc / P.atcv * .5;
-  C.ks = c * P.eps;
+    C.ks[i] = c * P.eps * h[0] * h[1] * h[2] / 16. * t;
+  }
   C.crhs = P.atnum == 2 ? P.Gc / P.atcv / P.eps * .5 : P.Gc / P.atcv / P.eps * .25;
   return C;
 }
@@ -58,7 +44,8 @@ static VConst make_vconst(const DevProblem &P) {
 // (15 bx - 1 + tx, 15 by - 1 + ty) of the V operator's tile-blocked layout
 // (halo elements are computed by every tile that holds them), so each
 // coefficient is written as one aligned, contiguous 512-byte segment per
-// wavefront.  Gauss-point values by sum factorisation (gauss_walk).
+// wavefront.  Gauss-point values by sum factorisation (gauss_walk); the
+// moments are summed row by row as the walk visits the points.
 __global__ __launch_bounds__(256) void k_v_setup(DevProblem P, const double *__restrict__ U) {
   const Grid &G = P.G;
   const int tid = threadIdx.x;
@@ -79,8 +66,16 @@ __global__ __launch_bounds__(256) void k_v_setup(DevProblem P, const double *__r
   }
   const double Ee = P.E_elem ? P.E_elem[e] : P.E;
   const double lam = P.lam1 * Ee, mu = P.mu1 * Ee;
-  const double vol = G.hx * G.hy * G.hz;
+  const double vol = G.hx * G.hy * G.hz / 64.;
   const double cm = P.atnum == 2 ? P.Gc / P.atcv * .5 / P.eps : 0.;
+  constexpr double X1 = VFG_SQ35, X2 = .6;  // Gauss point +1 and its square (point -1: -X1; the middle one 0)
+  double Q[3][3][3], Y[3][3], row[3];       // [r][q][p]; [q][p] of the layer; the row's points
+#pragma unroll
+  for (int q = 0; q < 9; q++) {
+    Y[q / 3][q % 3] = 0.;
+#pragma unroll
+    for (int r = 0; r < 3; r++) Q[r][q / 3][q % 3] = 0.;
+  }
   gauss_walk<3, 1>(fld, 1. / G.hx, 1. / G.hy, 1. / G.hz,
                    [&](int gx, int gy, int gz, const double (&val)[4], const double (&H)[3][3]) {
     const double t = val[3];
@@ -100,9 +95,38 @@ __global__ __launch_bounds__(256) void k_v_setup(DevProblem P, const double *__r
     } else {
       W = (s11 * e11 + s22 * e22 + s33 * e33) * .5 + 2. * mu * (e12 * e12 + e23 * e23 + e13 * e13);
     }
-    const double Wg = vol * gW(gx) * gW(gy) * gW(gz);
-    out[((gz * 3 + gy) * 3 + gx) * 256] = Wg * (cm + 2. * W);
+    row[gx] = gW(gx) * (cm + 2. * W);
+    if (gx == 2) {  // end of a row (gy, gz)
+      const double S = row[0] + row[2], w = vol * gW(gy) * gW(gz);
+      const double m[3] = {w * (S + row[1]), (w * X1) * (row[2] - row[0]), (w * X2) * S};
+#pragma unroll
+      for (int p = 0; p < 3; p++) {
+        Y[0][p] += m[p];
+        if (gy != 1) {
+          Y[1][p] += gy ? X1 * m[p] : -X1 * m[p];
+          Y[2][p] += X2 * m[p];
+        }
+      }
+      if (gy == 2)  // end of a layer gz
+#pragma unroll
+        for (int q = 0; q < 3; q++)
+#pragma unroll
+          for (int p = 0; p < 3; p++) {
+            Q[0][q][p] += Y[q][p];
+            if (gz != 1) {
+              Q[1][q][p] += gz ? X1 * Y[q][p] : -X1 * Y[q][p];
+              Q[2][q][p] += X2 * Y[q][p];
+            }
+            Y[q][p] = 0.;
+          }
+    }
   });
+#pragma unroll
+  for (int r = 0; r < 3; r++)
+#pragma unroll
+    for (int q = 0; q < 3; q++)
+#pragma unroll
+      for (int p = 0; p < 3; p++) out[((r * 3 + q) * 3 + p) * 256] = Q[r][q][p];
 }
 
 int64_t vq_doubles(const Grid &G) {
@@ -120,155 +144,180 @@ __global__ void k_v_fixmask(DevProblem P) {
 }
 
 // ------------------------------------------------------------------- apply
-// the 27 coupling weights of one element, read one layer ahead by the march
+// the 27 moments of one element, read one layer ahead by the march
 struct VQ {
-  double q[27];
+  double q[27];  // [r][q][p]
 };
-__device__ __forceinline__ VQ load_vq(const double *__restrict__ Vq, int tile, int slot, int ek, int nez) {
-  VQ a;
-  const double *b = Vq + tiled_index(tile, ek, nez, 27, slot, 0, 256);
-#pragma unroll
-  for (int g = 0; g < 27; g++) a.q[g] = b[g * 256];
-  return a;
-}
-
-// y_a = ks sum_b L[a][b] x_b + sum_g q_g phi_a(g) x(g); the weights are read
-// one Gauss plane (9 values) at a time, the next plane's loads in flight while
-// the current one is used (keeps the register count at four waves per SIMD)
-__device__ __forceinline__ void v_elem_apply_qp(const double (&x)[8], const double *__restrict__ qb,
-                                                const VConst &C, double (&r)[8]) {
-  double qa[9], qn[9];
-#pragma unroll
-  for (int g = 0; g < 9; g++) qa[g] = qb[g * 256];
-#pragma unroll
-  for (int a = 0; a < 8; a++) {
-    double s = 0.;
-#pragma unroll
-    for (int b = 0; b < 8; b++) s += C.L[a * 8 + b] * x[b];
-    r[a] = C.ks * s;
-  }
-  double ax[2][2][3];  // [k][j][gx]
-#pragma unroll
-  for (int k = 0; k < 2; k++)
-#pragma unroll
-    for (int j = 0; j < 2; j++)
-#pragma unroll
-      for (int gx = 0; gx < 3; gx++) ax[k][j][gx] = interp<double>(gx, x[(k * 2 + j) * 2], x[(k * 2 + j) * 2 + 1]);
-  double bz[2][2][3];
-#pragma unroll
-  for (int k = 0; k < 2; k++)
-#pragma unroll
-    for (int j = 0; j < 2; j++)
-#pragma unroll
-      for (int gx = 0; gx < 3; gx++) bz[k][j][gx] = 0.;
-#pragma unroll
-  for (int gz = 0; gz < 3; gz++) {
-    if (gz < 2)
-#pragma unroll
-      for (int g = 0; g < 9; g++) qn[g] = qb[((gz + 1) * 9 + g) * 256];
-#pragma unroll
-    for (int gy = 0; gy < 3; gy++)
-#pragma unroll
-      for (int gx = 0; gx < 3; gx++) {
-        double a0 = interp<double>(gy, ax[0][0][gx], ax[0][1][gx]);
-        double a1 = interp<double>(gy, ax[1][0][gx], ax[1][1][gx]);
-        double xv = interp<double>(gz, a0, a1);
-        double f = qa[gy * 3 + gx] * xv;
-        double f0 = gP0(gz) * f, f1 = gP1(gz) * f;
-        bz[0][0][gx] += gP0(gy) * f0; bz[0][1][gx] += gP1(gy) * f0;
-        bz[1][0][gx] += gP0(gy) * f1; bz[1][1][gx] += gP1(gy) * f1;
-      }
-#pragma unroll
-    for (int g = 0; g < 9; g++) qa[g] = qn[g];
-  }
-#pragma unroll
-  for (int k = 0; k < 2; k++)
-#pragma unroll
-    for (int j = 0; j < 2; j++) {
-      double s0 = 0., s1 = 0.;
-#pragma unroll
-      for (int gx = 0; gx < 3; gx++) { s0 += gP0(gx) * bz[k][j][gx]; s1 += gP1(gx) * bz[k][j][gx]; }
-      r[(k * 2 + j) * 2] += s0;
-      r[(k * 2 + j) * 2 + 1] += s1;
-    }
-}
-
-struct VApplyOp {
+// the parts of the march's interface that the V operators share: one nodal
+// field, the moments of the tile-blocked layout
+struct VModBase {
+  using T = double;
   static constexpr int NF = 1, NC = 1;
-  static constexpr bool TILED = true;  // element(tile, slot, ek, ...): q is tile-blocked
-  const double *x;
-  double *y;
-  const double *q, *bV, *VIrrev;
+  struct Face {
+    double m[4], own;  // modal sums of the face; the thread's own node
+  };
+  struct Own {
+    double x;
+  };
+  using Aux = VQ;
+  const double *q;
   const uint8_t *vfix;
   Grid G;
-  int64_t ne;
   VConst C;
+  template <class RD>
+  __device__ void face(const RD &rd, Face &F) const {
+    const double x0 = rd(0, 0), x1 = rd(0, 1), x2 = rd(0, 2), x3 = rd(0, 3);
+    const double a = x0 + x1, b = x2 + x3, e = x1 - x0, f = x3 - x2;
+    F.m[0] = a + b;
+    F.m[1] = e + f;
+    F.m[2] = b - a;
+    F.m[3] = f - e;
+    F.own = x3;
+  }
+  __device__ Own own(const Face &F) const { return Own{F.own}; }
+  // NT: streamed past the caches
+  template <bool NT>
+  __device__ VQ moments(int ek, int tile, int slot) const {
+    VQ a;
+    const double *b = q + tiled_index(tile, ek, G.nez, 27, 0, 0, 256);  // uniform in the workgroup
+#pragma unroll
+    for (int g = 0; g < 27; g++) {
+      const double *p = b + g * 256 + (unsigned)slot;
+      a.q[g] = NT ? __builtin_nontemporal_load(p) : *p;
+    }
+    return a;
+  }
+  __device__ VQ aux(int, int, int ek, int tile, int slot) const { return moments<false>(ek, tile, slot); }
+};
+// adds the modal forces y[8] of a layer to the planes below and above it
+__device__ __forceinline__ void v_planes(const double (&y)[8], double (&tot)[1][4], double (&carry)[1][4]) {
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    tot[0][i] += y[i] - y[i + 4];
+    carry[0][i] = y[i] + y[i + 4];
+  }
+}
+
+// an owned node's data, read a layer before its store: a load issued there
+// would wait for the next layer's moments, which are in flight by then
+struct VOwn {
+  double x, b, irr;
+  uint8_t fix;
+};
+// MODE 0: masked Jacobian; 1: VF_VResidual; 2: plain K x
+struct VApplyRec : VModBase {
+  const double *x;
+  double *y;
+  const double *bV, *VIrrev;
   BcMask bc;
   uint8_t ftype[6], vtype[8];
-  int mode, atnum;
+  int atnum;
   double irrevtol;
-  __device__ double load(int, int64_t n) const { return (mode == 0 && vfix[n]) ? 0. : x[n]; }
-  // mode 0: masked Jacobian; 1: VF_VResidual; 2: plain K x
-  // the coupling weights are read inside the layer: prefetching them a layer
-  // ahead costs a wave of occupancy and is slower
-  __device__ void element(int tile, int slot, int ek, const double (&xin)[2][4][1], double (&r)[8][1]) const {
-    double xe[8], re[8];
-#pragma unroll
-    for (int a = 0; a < 8; a++) xe[a] = xin[a >> 2][a & 3][0];
-    v_elem_apply_qp(xe, q + tiled_index(tile, ek, G.nez, 27, slot, 0, 256), C, re);
-#pragma unroll
-    for (int a = 0; a < 8; a++) r[a][0] = re[a];
+};
+struct VRaw {
+  double x;
+  uint8_t fix;
+};
+template <int MODE>
+struct VApplyOp : VApplyRec {
+  using Raw = VRaw;
+  static __device__ VRaw off() { return VRaw{0., 1}; }
+  __device__ VRaw load(int, int64_t n) const { return VRaw{x[n], MODE == 0 ? vfix[n] : (uint8_t)0}; }
+  __device__ double stage(int, const VRaw &r) const { return r.fix ? 0. : r.x; }
+  __device__ VOwn own_load(int64_t n) const {
+    VOwn o{};
+    if constexpr (MODE == 0) {
+      o.fix = vfix[n];
+      o.x = x[n];
+    }
+    if constexpr (MODE == 1) {
+      o.b = bV[n];
+      if (atnum == 2) o.irr = VIrrev[n];
+    }
+    return o;
   }
-  __device__ void store(int i, int j, int k, const double (&acc)[1], const double (&)[1]) const {
-    int64_t n = node_id(G, i, j, k);
-    if (mode == 0) {
-      y[n] = vfix[n] ? x[n] : acc[0];
-      return;
+  __device__ void element(const VQ &Q, const Face &B, const Face &F, double (&tot)[1][4], double (&carry)[1][4]) const {
+    double X[8], R[8];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      X[i] = B.m[i] + F.m[i];
+      X[i + 4] = F.m[i] - B.m[i];
     }
-    if (mode == 2) {
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      R[i] = C.ks[i] * X[i];
+#pragma unroll
+      for (int j = 0; j < 8; j++)
+        R[i] += Q.q[(um_pow(i, 0) + um_pow(j, 0)) + 3 * (um_pow(i, 1) + um_pow(j, 1)) +
+                    9 * (um_pow(i, 2) + um_pow(j, 2))] * X[j];
+    }
+    v_planes(R, tot, carry);
+  }
+  __device__ void store(int64_t n, uint32_t fb, const double (&acc)[1], const Own &own, const VOwn &o) const {
+    if constexpr (MODE == 0) {
+      y[n] = o.fix ? o.x : acc[0];
+    } else if constexpr (MODE == 2) {
       y[n] = acc[0];
-      return;
+    } else {
+      // VF_VResidual: F = K V - b; AT2 irreversible rows -> 0 (VF_IrrevApplyEQVec);
+      // then ResidualApplyDirichletBC with V as its own BC vector.
+      double F = acc[0] - o.b;
+      if (atnum == 2 && o.irr <= irrevtol) F = 0.;
+      if (face_dirichlet(bc.face[0], bc.vert[0], fb)) {
+        int t = 0;
+        for (int f = 0; f < 6; f++)
+          if (ftype[f] && (fb >> f & 1u)) t = ftype[f];
+        const int v = face_vertex(fb);
+        if (v >= 0 && vtype[v]) t = vtype[v];
+        F = t == 2 ? own.x - 1. : t == 3 ? 0. : own.x;
+      }
+      y[n] = F;
     }
-    // VF_VResidual: F = K V - b; AT2 irreversible rows -> 0 (VF_IrrevApplyEQVec);
-    // then ResidualApplyDirichletBC with V as its own BC vector.
-    double F = acc[0] - bV[n];
-    if (atnum == 2 && VIrrev[n] <= irrevtol) F = 0.;
-    if (on_dirichlet(G, bc.face[0], bc.vert[0], i, j, k)) {
-      int t = 0;
-      const bool onf[6] = {i == 0, i == G.nx - 1, j == 0, j == G.ny - 1, k == 0, k == G.nz - 1};
-      for (int f = 0; f < 6; f++)
-        if (ftype[f] && onf[f]) t = ftype[f];
-      int ix = (i == 0) ? 0 : (i == G.nx - 1) ? 1 : -1;
-      int iy = (j == 0) ? 0 : (j == G.ny - 1) ? 1 : -1;
-      int iz = (k == 0) ? 0 : (k == G.nz - 1) ? 1 : -1;
-      if (ix >= 0 && iy >= 0 && iz >= 0 && vtype[ix + 2 * iy + 4 * iz]) t = vtype[ix + 2 * iy + 4 * iz];
-      double v = x[n];
-      F = t == 2 ? v - 1. : t == 3 ? 0. : v;
-    }
-    y[n] = F;
   }
 };
 
-// CG-fused masked apply (mode 0): stages p = z + beta p_old off the mask, writes
-// p and q = K p, one partial of p.q per workgroup; p_old and p are different
+// CG-fused masked apply: stages p = z + beta p_old off the mask, writes
+// p and q = K p, one partial of p.q per workgroup; p_old (x) and p are different
 // arrays (neighbouring workgroups still read p_old at their halo nodes)
-struct VApplyCgOp : VApplyOp {
+struct VApplyCgOp : VApplyOp<0> {
   const double *z;
   const double *beta;
   double *pw;
   double *part;
-  __device__ double load(int, int64_t n) const { return vfix[n] ? 0. : z[n] + *beta * x[n]; }
-  __device__ double store(int i, int j, int k, const double (&acc)[1], const double (&own)[1]) const {
-    const int64_t n = node_id(G, i, j, k);
-    const double yv = vfix[n] ? own[0] : acc[0];
+  double bval;  // *beta, read once by the kernel
+  struct Raw {
+    double z, x;
+    uint8_t fix;
+  };
+  static __device__ Raw off() { return Raw{0., 0., 1}; }
+  __device__ Raw load(int, int64_t n) const { return Raw{z[n], x[n], vfix[n]}; }
+  __device__ double stage(int, const Raw &r) const { return r.fix ? 0. : r.z + bval * r.x; }
+  __device__ uint8_t own_load(int64_t n) const { return vfix[n]; }
+  __device__ double store(int64_t n, uint32_t, const double (&acc)[1], const Own &own, uint8_t fix) const {
+    const double yv = fix ? own.x : acc[0];
     y[n] = yv;
-    pw[n] = own[0];
-    return own[0] * yv;
+    pw[n] = own.x;
+    return own.x * yv;
   }
   __device__ void partial(int slot, double v) const { part[slot] = v; }
 };
 
-__global__ __launch_bounds__(256, 3) void k_v_apply(VApplyOp op, int OZ) { march<double, 16, 16>(op.G, op, OZ, xcd_block()); }
+// Bound by the read of the moments (216 B per element, 1.27 x with the halo
+// slots at 128^3): 128^3 120 us = 5.1 TB/s, 141 us for the 27 Gauss weights read
+// a plane at a time.  All 27 of the next layer are in flight during a layer;
+// the 176 registers that takes leave two waves per SIMD (three spill: 151 us).
+// NT: a moment array well over the 256 MB last-level cache is streamed past
+// it (128^3, 579 MB: 120 against 127 us); one that fits is kept there for the
+// next product (96^3, 260 MB: 46 against 56 us).
+constexpr int64_t V_STREAM_BYTES = 400ll << 20;
+template <int MODE, bool NT>
+struct VApplyStreamOp : VApplyOp<MODE> {
+  __device__ VQ aux(int, int, int ek, int tile, int slot) const { return this->template moments<NT>(ek, tile, slot); }
+};
+template <int MODE, bool NT>
+__global__ __launch_bounds__(256, 2) void k_v_apply(VApplyStreamOp<MODE, NT> op, int OZ) {
+  march_modal<16, 16>(op.G, op, OZ, xcd_block());
+}
 
 // The same over a list of workgroups.  The reduced Newton systems of the
 // V-solve live on the free nodes, a thin band around the cracks: a workgroup
@@ -281,19 +330,21 @@ struct VChunk {
 };
 __device__ __forceinline__ VChunk chunk_at(const Grid &G, const int *__restrict__ list, int cap, int w) {
   const int gx = (G.nx + 14) / 15, txy = gx * ((G.ny + 14) / 15);
-  const int c = list[w], t = c % txy;
-  return VChunk{t % gx, t / gx, c / txy, list[cap + 1]};
+  const int c = __builtin_amdgcn_readfirstlane(list[w]), t = c % txy;  // uniform: the moments' base address too
+  return VChunk{t % gx, t / gx, c / txy, __builtin_amdgcn_readfirstlane(list[cap + 1])};
 }
-__global__ __launch_bounds__(256, 3) void k_v_apply_cg_list(VApplyCgOp op, const int *__restrict__ list, int cap,
+__global__ __launch_bounds__(256, 2) void k_v_apply_cg_list(VApplyCgOp op, const int *__restrict__ list, int cap,
                                                            const double *__restrict__ done) {
   if (done && *done != 0.) return;  // the CG has converged
+  op.bval = *op.beta;
   const VChunk q = chunk_at(op.G, list, cap, blockIdx.x);
-  march<double, 16, 16>(op.G, op, q.L, q.bx, q.by, q.bz, blockIdx.x);
+  march_modal<16, 16>(op.G, op, q.L, q.bx, q.by, q.bz, blockIdx.x);
 }
-// the plain apply (any mode) over the listed chunks
-__global__ __launch_bounds__(256, 3) void k_v_apply_list(VApplyOp op, const int *__restrict__ list, int cap) {
+// the plain apply over the listed chunks
+template <int MODE>
+__global__ __launch_bounds__(256, 2) void k_v_apply_list(VApplyOp<MODE> op, const int *__restrict__ list, int cap) {
   const VChunk q = chunk_at(op.G, list, cap, blockIdx.x);
-  march<double, 16, 16>(op.G, op, q.L, q.bx, q.by, q.bz);
+  march_modal<16, 16>(op.G, op, q.L, q.bx, q.by, q.bz);
 }
 
 __global__ void k_fill_u32(uint32_t *a, uint32_t v, int64_t n) {
@@ -430,68 +481,64 @@ __global__ __launch_bounds__(256) void k_v_xr_list(Grid G, const int *__restrict
 }
 
 // ---------------------------------------------------------------- diagonal
-struct VDiagOp {
-  static constexpr int NF = 1, NC = 1;
-  static constexpr bool TILED = true;
+// d_a = sum over modal pairs of signs times Q and ks: per direction
+// Q_0 + 2 s Q_1 + Q_2 with s = -1, 1 the corner's side
+struct VDiagOp : VModBase {
   double *d;
-  const double *q;
-  const uint8_t *vfix;
-  Grid G;
-  int64_t ne;
-  VConst C;
+  using Raw = double;
+  static __device__ double off() { return 0.; }
   __device__ double load(int, int64_t) const { return 0.; }
-  __device__ VQ aux(int tile, int slot, int ek) const { return load_vq(q, tile, slot, ek, G.nez); }
-  // d_a = ks L[a][a] + sum_g q_g phi_a(g)^2, phi_a^2 = P_i(gx)^2 P_j(gy)^2 P_k(gz)^2:
-  // contracted direction by direction (x, then y, then z)
-  __device__ void element(int, int, int, const double (&)[2][4][1], const VQ &Q, double (&r)[8][1]) const {
-    double bx[3][3][2];  // [gz][gy][i]
+  __device__ double stage(int, double v) const { return v; }
+  __device__ void element(const VQ &Q, const Face &, const Face &, double (&tot)[1][4], double (&carry)[1][4]) const {
+    double a[3][3][2], b[3][2][2], r[2][2][2], L = 0.;
 #pragma unroll
-    for (int gz = 0; gz < 3; gz++)
+    for (int i = 0; i < 8; i++) L += C.ks[i];
 #pragma unroll
-      for (int gy = 0; gy < 3; gy++) {
-        double s0 = 0., s1 = 0.;
+    for (int k = 0; k < 3; k++)
 #pragma unroll
-        for (int gx = 0; gx < 3; gx++) {
-          const double qv = Q.q[(gz * 3 + gy) * 3 + gx];
-          s0 += gP0(gx) * gP0(gx) * qv;
-          s1 += gP1(gx) * gP1(gx) * qv;
-        }
-        bx[gz][gy][0] = s0;
-        bx[gz][gy][1] = s1;
+      for (int j = 0; j < 3; j++) {
+        const double *m = Q.q + (k * 3 + j) * 3;
+        const double S = m[0] + m[2];
+        a[k][j][0] = S - 2. * m[1];
+        a[k][j][1] = S + 2. * m[1];
       }
-    double by[3][2][2];  // [gz][j][i]
 #pragma unroll
-    for (int gz = 0; gz < 3; gz++)
+    for (int k = 0; k < 3; k++)
 #pragma unroll
       for (int i = 0; i < 2; i++) {
-        double s0 = 0., s1 = 0.;
-#pragma unroll
-        for (int gy = 0; gy < 3; gy++) {
-          s0 += gP0(gy) * gP0(gy) * bx[gz][gy][i];
-          s1 += gP1(gy) * gP1(gy) * bx[gz][gy][i];
-        }
-        by[gz][0][i] = s0;
-        by[gz][1][i] = s1;
+        const double S = a[k][0][i] + a[k][2][i];
+        b[k][0][i] = S - 2. * a[k][1][i];
+        b[k][1][i] = S + 2. * a[k][1][i];
       }
 #pragma unroll
-    for (int a = 0; a < 8; a++) {
-      const int i = a & 1, j = (a >> 1) & 1, k = a >> 2;
-      double s = 0.;
+    for (int j = 0; j < 2; j++)
 #pragma unroll
-      for (int gz = 0; gz < 3; gz++) s += (k ? gP1(gz) * gP1(gz) : gP0(gz) * gP0(gz)) * by[gz][j][i];
-      r[a][0] = C.ks * C.L[a * 9] + s;
+      for (int i = 0; i < 2; i++) {
+        const double S = b[0][j][i] + b[2][j][i];
+        r[0][j][i] = L + (S - 2. * b[1][j][i]);
+        r[1][j][i] = L + (S + 2. * b[1][j][i]);
+      }
+    // the corner values as modal sums of the two faces
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+      const double s0 = .25 * (r[k][0][0] + r[k][0][1]), s1 = .25 * (r[k][1][0] + r[k][1][1]);
+      const double e0 = .25 * (r[k][0][1] - r[k][0][0]), e1 = .25 * (r[k][1][1] - r[k][1][0]);
+      double(&o)[4] = k ? carry[0] : tot[0];
+      const double m[4] = {s0 + s1, e0 + e1, s1 - s0, e1 - e0};
+#pragma unroll
+      for (int q = 0; q < 4; q++) o[q] = k ? m[q] : o[q] + m[q];
     }
   }
-  __device__ void store(int i, int j, int k, const double (&acc)[1], const double (&)[1]) const {
-    int64_t n = node_id(G, i, j, k);
-    d[n] = vfix[n] ? 1. : acc[0];
+  __device__ uint8_t own_load(int64_t n) const { return vfix[n]; }
+  __device__ void store(int64_t n, uint32_t, const double (&acc)[1], const Own &, uint8_t fix) const {
+    d[n] = fix ? 1. : acc[0];
   }
 };
 
-__global__ __launch_bounds__(256) void k_v_diag(VDiagOp op, int OZ) { march<double, 16, 16>(op.G, op, OZ, xcd_block()); }
-__global__ __launch_bounds__(256) void k_v_diag_list(VDiagOp op, const int *__restrict__ list, int cap) {
+__global__ __launch_bounds__(256, 2) void k_v_diag(VDiagOp op, int OZ) { march_modal<16, 16>(op.G, op, OZ, xcd_block()); }
+__global__ __launch_bounds__(256, 2) void k_v_diag_list(VDiagOp op, const int *__restrict__ list, int cap) {
   const VChunk q = chunk_at(op.G, list, cap, blockIdx.x);
-  march<double, 16, 16>(op.G, op, q.L, q.bx, q.by, q.bz);
+  march_modal<16, 16>(op.G, op, q.L, q.bx, q.by, q.bz);
 }
 
 // ------------------------------------------------------------ load vector
@@ -585,9 +632,14 @@ static dim3 mgrid(const Grid &G, int OZ) {
   return dim3((G.nx + 14) / 15, (G.ny + 14) / 15, (G.nz + OZ - 1) / OZ);
 }
 int choose_oz(const Grid &G, int tiles_xy, int slots);
-// z-chunk length of the V kernels (three workgroups per CU): whole rounds of
-// workgroups, as for the u kernels; a partial last round costs a full one.
-static int oz_for(const Grid &G) { return choose_oz(G, ((G.nx + 14) / 15) * ((G.ny + 14) / 15), 768); }
+// z-chunk length of the V kernels: whole rounds of resident workgroups, as for
+// the u kernels; a partial last round costs a full one
+int device_slots_of(const void *kernel, int threads);
+static int v_slots() {
+  static int n = device_slots_of((const void *)k_v_apply<0, false>, 256);
+  return n;
+}
+static int oz_for(const Grid &G) { return choose_oz(G, ((G.nx + 14) / 15) * ((G.ny + 14) / 15), v_slots()); }
 
 void launch_v_setup(const DevProblem &P, const double *U, hipStream_t s) {
   hipLaunchKernelGGL(k_v_setup, dim3((P.G.nx + 14) / 15, (P.G.ny + 14) / 15, P.G.nez), dim3(256), 0, s, P, U);
@@ -603,28 +655,55 @@ void launch_v_fixmask(const DevProblem &P, hipStream_t s) {
   hipLaunchKernelGGL(k_v_fixmask, dim3((unsigned)((P.nn + 255) / 256)), dim3(256), 0, s, P);
 }
 
-static VApplyOp make_vapply_op(const DevProblem &P, const double *x, double *y, int mode, const uint8_t *mask) {
-  VApplyOp op;
-  op.x = x; op.y = y; op.q = P.Vq; op.bV = P.bV; op.VIrrev = P.VIrrev; op.vfix = mask ? mask : P.vfix;
-  op.G = P.G; op.ne = P.ne; op.C = make_vconst(P); op.bc = P.bcV;
+static void v_fill(VModBase &op, const DevProblem &P, const uint8_t *mask) {
+  op.q = P.Vq;
+  op.vfix = mask ? mask : P.vfix;
+  op.G = P.G;
+  op.C = make_vconst(P);
+}
+static void vapply_fill(VApplyRec &op, const DevProblem &P, const double *x, double *y, const uint8_t *mask) {
+  v_fill(op, P, mask);
+  op.x = x; op.y = y; op.bV = P.bV; op.VIrrev = P.VIrrev; op.bc = P.bcV;
   for (int f = 0; f < 6; f++) op.ftype[f] = (uint8_t)P.hbcV.face[f];
   for (int v = 0; v < 8; v++) op.vtype[v] = (uint8_t)P.hbcV.vertex[v];
-  op.mode = mode; op.atnum = P.atnum; op.irrevtol = P.irrevtol;
+  op.atnum = P.atnum; op.irrevtol = P.irrevtol;
+}
+template <class Op>
+static Op vapply_op(const VApplyRec &r) {
+  Op op;
+  static_cast<VApplyRec &>(op) = r;
   return op;
+}
+template <int MODE>
+static void launch_v_apply_m(const VApplyRec &r, const dim3 &g, int OZ, bool stream, hipStream_t s) {
+  if (stream)
+    hipLaunchKernelGGL((k_v_apply<MODE, true>), g, dim3(256), 0, s, (vapply_op<VApplyStreamOp<MODE, true>>(r)), OZ);
+  else
+    hipLaunchKernelGGL((k_v_apply<MODE, false>), g, dim3(256), 0, s, (vapply_op<VApplyStreamOp<MODE, false>>(r)), OZ);
 }
 
 void launch_v_apply(const DevProblem &P, const double *x, double *y, int mode, hipStream_t s,
                     const uint8_t *mask) {
-  const VApplyOp op = make_vapply_op(P, x, y, mode, mask);
-  int OZ = oz_for(P.G);
-  hipLaunchKernelGGL(k_v_apply, mgrid(P.G, OZ), dim3(256), 0, s, op, OZ);
+  VApplyRec r;
+  vapply_fill(r, P, x, y, mask);
+  const int OZ = oz_for(P.G);
+  const dim3 g = mgrid(P.G, OZ);
+  const bool stream = 8 * vq_doubles(P.G) > V_STREAM_BYTES;
+  if (mode == 0) launch_v_apply_m<0>(r, g, OZ, stream, s);
+  else if (mode == 1) launch_v_apply_m<1>(r, g, OZ, stream, s);
+  else launch_v_apply_m<2>(r, g, OZ, stream, s);
 }
 
 void launch_v_apply_list(const DevProblem &P, const double *x, double *y, int mode, const int *list, int count,
                          hipStream_t s, const uint8_t *mask) {
   if (count <= 0) return;
-  const VApplyOp op = make_vapply_op(P, x, y, mode, mask);
-  hipLaunchKernelGGL(k_v_apply_list, dim3((unsigned)count), dim3(256), 0, s, op, list, v_chunk_cap(P.G));
+  VApplyRec r;
+  vapply_fill(r, P, x, y, mask);
+  const dim3 g((unsigned)count);
+  const int cap = v_chunk_cap(P.G);
+  if (mode == 0) hipLaunchKernelGGL(k_v_apply_list<0>, g, dim3(256), 0, s, vapply_op<VApplyOp<0>>(r), list, cap);
+  else if (mode == 1) hipLaunchKernelGGL(k_v_apply_list<1>, g, dim3(256), 0, s, vapply_op<VApplyOp<1>>(r), list, cap);
+  else hipLaunchKernelGGL(k_v_apply_list<2>, g, dim3(256), 0, s, vapply_op<VApplyOp<2>>(r), list, cap);
 }
 
 // ------------------------------------------------ persistent multi-problem apply
@@ -632,10 +711,10 @@ void launch_v_apply_list(const DevProblem &P, const double *x, double *y, int mo
 // a work list of (member, tile x, tile y, z-chunk); the item count lives on the
 // device and members whose flags[p * fstride] is 0 are skipped.
 struct BVApply {
-  VApplyOp op;
+  VApplyOp<0> op;
   int OZ;
 };
-__global__ __launch_bounds__(256, 3) void k_batch_v_apply(const BVApply *__restrict__ probs,
+__global__ __launch_bounds__(256, 2) void k_batch_v_apply(const BVApply *__restrict__ probs,
                                                        const BItem *__restrict__ items,
                                                        const int *__restrict__ dcount,
                                                        const double *__restrict__ flags, int fstride) {
@@ -643,22 +722,18 @@ __global__ __launch_bounds__(256, 3) void k_batch_v_apply(const BVApply *__restr
   for (int it = blockIdx.x; it < n; it += gridDim.x) {
     const BItem w = items[it];
     if (flags[(int64_t)w.p * fstride] == 0.) continue;  // uniform per block
-    const VApplyOp &op = probs[w.p].op;  // read in place: the record is large
+    const VApplyOp<0> &op = probs[w.p].op;  // read in place: the record is large
     const int OZ = probs[w.p].OZ;
     __syncthreads();  // LDS of the previous item is free
-    march<double, 16, 16>(op.G, op, OZ, w.bx, w.by, w.bz);
+    march_modal<16, 16>(op.G, op, OZ, w.bx, w.by, w.bz);
   }
 }
 size_t vop_bytes() { return sizeof(BVApply); }
 int v_oz(const Grid &G) { return oz_for(G); }
+int v_apply_slots() { return v_slots(); }
 void make_vop(const DevProblem &P, const double *x, double *y, const uint8_t *mask, void *out) {
   BVApply *b = (BVApply *)out;
-  VApplyOp &op = b->op;
-  op.x = x; op.y = y; op.q = P.Vq; op.bV = P.bV; op.VIrrev = P.VIrrev; op.vfix = mask ? mask : P.vfix;
-  op.G = P.G; op.ne = P.ne; op.C = make_vconst(P); op.bc = P.bcV;
-  for (int f = 0; f < 6; f++) op.ftype[f] = (uint8_t)P.hbcV.face[f];
-  for (int v = 0; v < 8; v++) op.vtype[v] = (uint8_t)P.hbcV.vertex[v];
-  op.mode = 0; op.atnum = P.atnum; op.irrevtol = P.irrevtol;
+  vapply_fill(b->op, P, x, y, mask);
   b->OZ = oz_for(P.G);
 }
 void launch_engine_v_apply(const void *d_ops, const BItem *items, const int *dcount, int grid, const double *flags,
@@ -670,11 +745,7 @@ void launch_engine_v_apply(const void *d_ops, const BItem *items, const int *dco
 static VApplyCgOp make_vcg_op(const DevProblem &P, const double *pold, double *p, const double *z,
                               const double *beta, double *q, double *part, const uint8_t *mask) {
   VApplyCgOp op;
-  op.x = pold; op.y = q; op.q = P.Vq; op.bV = P.bV; op.VIrrev = P.VIrrev; op.vfix = mask ? mask : P.vfix;
-  op.G = P.G; op.ne = P.ne; op.C = make_vconst(P); op.bc = P.bcV;
-  for (int f = 0; f < 6; f++) op.ftype[f] = (uint8_t)P.hbcV.face[f];
-  for (int v = 0; v < 8; v++) op.vtype[v] = (uint8_t)P.hbcV.vertex[v];
-  op.mode = 0; op.atnum = P.atnum; op.irrevtol = P.irrevtol;
+  vapply_fill(op, P, pold, q, mask);
   op.z = z; op.beta = beta; op.pw = p; op.part = part;
   return op;
 }
@@ -720,7 +791,8 @@ int launch_v_xr_list(const Grid &G, const int *list, int count, double *x, doubl
 
 void launch_v_diag(const DevProblem &P, double *d, hipStream_t s, const uint8_t *mask) {
   VDiagOp op;
-  op.d = d; op.q = P.Vq; op.vfix = mask ? mask : P.vfix; op.G = P.G; op.ne = P.ne; op.C = make_vconst(P);
+  v_fill(op, P, mask);
+  op.d = d;
   int OZ = oz_for(P.G);
   hipLaunchKernelGGL(k_v_diag, mgrid(P.G, OZ), dim3(256), 0, s, op, OZ);
 }
@@ -729,7 +801,8 @@ void launch_v_diag_list(const DevProblem &P, double *d, const uint8_t *mask, con
                         hipStream_t s) {
   if (count <= 0) return;
   VDiagOp op;
-  op.d = d; op.q = P.Vq; op.vfix = mask ? mask : P.vfix; op.G = P.G; op.ne = P.ne; op.C = make_vconst(P);
+  v_fill(op, P, mask);
+  op.d = d;
   hipLaunchKernelGGL(k_v_diag_list, dim3((unsigned)count), dim3(256), 0, s, op, list, v_chunk_cap(P.G));
 }
 
