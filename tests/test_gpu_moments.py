@@ -25,3 +25,21 @@ def test_u_apply_moment_form(oracle, n, cubic):
     assert np.abs(P.UIJacobian_mult(s["x"]) - ref).max() <= 1e-12 * scale
     assert np.abs(P.UIJacobian_mult(s["x"], fp32=True) - ref).max() <= 1e-5 * scale
     P.close()
+
+
+@pytest.mark.parametrize("n", [(66, 60, 58), (65, 97, 81), (9, 40, 23)], ids=["non-nested", "nested", "flat"])
+def test_vcycle_transfers(n):
+    """The V-cycle is symmetric only if restriction and prolongation are each
+    other's transpose and every level's operator is symmetric: one entry per
+    thread (more than 2^16 coarse entries), four lanes per entry, directions
+    that are not coarsened."""
+    s = S.make(n=n, seed=sum(n), nu=0.3, bcU=S.MIXED_U)
+    P = S.to_gpu(s)
+    free = 1.0 - P.bc_mask("U")
+    rng = np.random.default_rng(n[0])
+    a, b = (rng.standard_normal(3 * P.nn) * free for _ in range(2))
+    Ma, Mb = P.u_pc_apply(a), P.u_pc_apply(b)
+    # FP32 throughout: 1e-5 of the norms, as for one FP32 apply
+    assert abs(a @ Mb - b @ Ma) <= 1e-5 * np.linalg.norm(a) * np.linalg.norm(Mb)
+    assert a @ Ma > 0.0
+    P.close()

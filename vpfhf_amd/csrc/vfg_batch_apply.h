@@ -30,8 +30,8 @@ void launch_engine_u_apply(int fp32, int sched, int unit, const void *d_ops, con
 void make_uop(const DevProblem &P, const void *x, void *y, int fp32, int OZ, void *out);  // host record
 // multigrid smoothing fused with the level apply, one record per member
 // (launch_mg_presmooth / launch_mg_postsmooth of every listed member at once;
-// 16 x 16 tiles): post = 0: x = c2 D^-1 b into xo, A x into
-// ro; post = 1: xo = xin + c2 D^-1 (b - A xin); unit: coarse levels
+// 16 x 16 tiles): post = 0: x = c2 D^-1 b into xo, b - A x
+// (0 on the Dirichlet rows) into ro; post = 1: xo = xin + c2 D^-1 (b - A xin); unit: coarse levels
 size_t mg_smooth_op_bytes();
 void make_mg_smooth_op(const DevProblem &P, int post, const float *b, const float *dinv, float c2, const float *xin,
                        float *xo, float *ro, int OZ, void *out);  // host record

@@ -22,7 +22,7 @@
 namespace vfg {
 
 constexpr int BCH = 4096;  // entries per Chebyshev chunk
-constexpr int BTR = 256;   // threads per transfer chunk: one fine node each (prolongation), four per coarse dof (restriction)
+constexpr int BTR = 256;   // threads per transfer chunk: one fine node each (prolongation), four per coarse entry (restriction)
 
 
 // Launch grids are list capacities; dn holds the live chunk count, so a
@@ -40,10 +40,8 @@ __global__ __launch_bounds__(256) void k_bmg_cheb(const BmgVec *__restrict__ lvt
     mg_cheb_entry(v.b, use_y ? v.y : nullptr, v.dinv, v.d, v.x, k.c1, k.c2, step == 0, xzero, c.start + t);
 }
 
-// chunks of BTR / 4 coarse dofs (level + 1) of members that descend, four
-// lanes per dof: lane kk sums the fine planes kk, kk + 4, ... of the gather
-// and the four are added by shuffles in lane order (as k_mg_restrict4), so a
-// thread's serial gather is a quarter as long
+// chunks of BTR / 4 coarse entries (level + 1) of members that descend, four
+// lanes each
 __global__ __launch_bounds__(256) void k_bmg_restrict(const BmgVec *__restrict__ lvt, int level,
                                                       const BmgChunk *__restrict__ ch, const int *__restrict__ dn,
                                                       const double *__restrict__ flags, int fstride) {
@@ -52,25 +50,32 @@ __global__ __launch_bounds__(256) void k_bmg_restrict(const BmgVec *__restrict__
   if (flags[(int64_t)c.p * fstride] == 0.) return;
   const BmgVec &f = lvt[c.p * BML + level];
   const BmgVec &g = lvt[c.p * BML + level + 1];
-  const int t = (int)threadIdx.x >> 2, kk = (int)threadIdx.x & 3;
-  const bool ok = t < c.len;
-  const int64_t dof = c.start + (ok ? t : 0), N = dof / 3;
-  const float v = ok ? mg_restrict_dof_plane(f.G, g.G, f.bc, f.b, f.y, N, (int)(dof - 3 * N), kk) : 0.f;
-  const float v1 = __shfl_down(v, 1, 4), v2 = __shfl_down(v, 2, 4), v3 = __shfl_down(v, 3, 4);
-  if (ok && kk == 0) g.b[dof] = ((v + v1) + v2) + v3;
+  const Grid &G = g.G;
+  const int l = (int)threadIdx.x >> 2, kk = (int)threadIdx.x & 3;
+  const bool ok = l < c.len;
+  const int64_t t = c.start + (ok ? l : 0);
+  const unsigned N = (unsigned)(t / 3), np = (unsigned)(G.nx * G.ny);
+  const int K = (int)(N / np), m = (int)(N - K * np), J = m / G.nx, I = m - J * G.nx, cc = (int)(t - 3 * (int64_t)N);
+  const float v = mg_lanes(mg_nested_grids(f.G, G) ? mg_restrict_plane<3>(f.G, G, f.bc, f.y, I, J, K, cc, kk)
+                                                   : mg_restrict_plane<4>(f.G, G, f.bc, f.y, I, J, K, cc, kk));
+  if (ok && kk == 0) g.b[t] = v;
 }
 
-// chunks over the fine nodes (level) of members that descend: the coarse
+// chunks of the fine nodes (level) of members that descend: the coarse
 // correction is added to the level's iterate d (the post-smoothing leaves x)
 __global__ __launch_bounds__(256) void k_bmg_prolong(const BmgVec *__restrict__ lvt, int level,
                                                      const BmgChunk *__restrict__ ch, const int *__restrict__ dn,
                                                      const double *__restrict__ flags, int fstride) {
   if ((int)blockIdx.x >= *dn) return;
   const BmgChunk c = ch[blockIdx.x];
-  if (flags[(int64_t)c.p * fstride] == 0.) return;
+  if (flags[(int64_t)c.p * fstride] == 0. || (int)threadIdx.x >= c.len) return;
   const BmgVec &f = lvt[c.p * BML + level];
   const BmgVec &g = lvt[c.p * BML + level + 1];
-  for (int t = threadIdx.x; t < c.len; t += 256) mg_prolong_node(f.G, g.G, f.bc, g.x, f.d, c.start + t);
+  const Grid &G = f.G;
+  const unsigned n = (unsigned)(c.start + threadIdx.x), np = (unsigned)(G.nx * G.ny);
+  const int k = (int)(n / np), m = (int)(n - k * np), j = m / G.nx, i = m - j * G.nx;
+  if (mg_nested_grids(G, g.G)) mg_prolong_node<true>(G, g.G, f.bc, g.x, f.d, i, j, k);
+  else mg_prolong_node<false>(G, g.G, f.bc, g.x, f.d, i, j, k);
 }
 
 // ------------------------------------------------------------------ host side
@@ -90,7 +95,7 @@ struct BmgPlan {
   void *ops = nullptr;  // one FP32 apply record per member (level operator, x -> y)
   void *ops_pre = nullptr, *ops_post = nullptr;  // fused smoothing records per member
   BmgList M, D, C;      // members with this level / that descend from it / whose coarsest it is
-  Grow<BmgChunk> rch;   // restriction: coarse dofs of the descending members
+  Grow<BmgChunk> rch;   // restriction: coarse entries of the descending members
   Grow<BmgChunk> pch;   // prolongation: fine nodes of the descending members
   // live counts: M items, M chunks, D items, D chunks, C items, C chunks, rch, pch
   int *dcnt = nullptr;
@@ -205,7 +210,7 @@ int bmg_rebuild(BatchMG *g, hipStream_t s, bool *grew) {
       if (g->L[p] - 1 <= l) continue;
       const Grid &Gf = level_grid(g, p, l), &Gc = level_grid(g, p, l + 1);
       const int64_t nc = 3 * (int64_t)Gc.nx * Gc.ny * Gc.nz, nf = (int64_t)Gf.nx * Gf.ny * Gf.nz;
-      constexpr int RC = BTR / 4;  // four lanes per coarse dof
+      constexpr int RC = BTR / 4;  // four lanes per coarse entry
       for (int64_t st = 0; st < nc; st += RC) P.rch.h.push_back({p, st, (int)(nc - st < RC ? nc - st : RC)});
       for (int64_t st = 0; st < nf; st += BTR) P.pch.h.push_back({p, st, (int)(nf - st < BTR ? nf - st : BTR)});
     }
@@ -327,7 +332,7 @@ static void stage_member(BatchMG *g, int p) {
     cheb_coefs(V.lmax / 11., V.lmax, MG_SMOOTH, cf);           // smoother
     cheb_coefs(V.lmax / 30., V.lmax, MG_COARSE_DEG, cf + BMK);  // coarsest level
     make_uop(V.P, v.x, v.y, 1, g->oz[p][l], g->h_ops[l].data() + batch_op_bytes(1) * p);
-    // descending levels: pre-smoothing from 0 into d (A d into y), post-smoothing d -> x
+    // descending levels: pre-smoothing from 0 into d (b - A d into y), post-smoothing d -> x
     static_assert(MG_SMOOTH == 1, "the fused smoothing records do one Chebyshev step");
     make_mg_smooth_op(V.P, 0, v.b, v.dinv, cf[0].c2, nullptr, v.d, v.y, g->oz[p][l],
                       g->h_pre[l].data() + mg_smooth_op_bytes() * p);
@@ -402,7 +407,7 @@ static void smooth(BatchMG *g, int l, const BmgList &L, int post, const double *
 }
 
 // Descending members: one Chebyshev-Jacobi step from 0 fused with its apply
-// (d, A d), restriction of b - A d, the coarse correction added to d, one step
+// (d, b - A d), restriction, the coarse correction added to d, one step
 // fused with its apply (d -> x) -- the single-problem V-cycle's kernels over
 // the work list.  Members whose coarsest level this is: the one-launch
 // Chebyshev solve, or Chebyshev steps with separate applies.

@@ -43,11 +43,11 @@ void launch_u_qsetup(const DevProblem &P, double *uq, hipStream_t s);
 void launch_u_apply(const DevProblem &P, const double *x, double *y, hipStream_t s);
 void launch_u_apply_f32(const DevProblem &P, const float *x, float *y, hipStream_t s);
 // FP32 multigrid level: one Chebyshev-Jacobi step from x = 0 fused with its
-// apply (x = c2 D^-1 b, y = A x: the restriction forms b - y on the free
-// rows), and one step from x fused with its apply (xo = x + c2 D^-1 (b - A x));
+// apply (x = c2 D^-1 b, r = b - A x, 0 on the Dirichlet rows: what the
+// restriction reads), and one step from x fused with its apply (xo = x + c2 D^-1 (b - A x));
 // xo must not alias x.  With r64 the post-smoothing also writes one partial of
 // r64 . xo per workgroup to part and returns their number (else 0 partials).
-void launch_mg_presmooth(const DevProblem &P, const float *b, const float *dinv, float c2, float *x, float *y,
+void launch_mg_presmooth(const DevProblem &P, const float *b, const float *dinv, float c2, float *x, float *r,
                          hipStream_t s);
 int launch_mg_postsmooth(const DevProblem &P, const float *b, const float *dinv, float c2, const float *x, float *xo,
                          const double *r64, double *part, hipStream_t s);
@@ -127,11 +127,9 @@ void launch_energies(const DevProblem &P, const double *U, const double *V, doub
 // geometric multigrid pieces (vfg_mg.hip)
 void launch_mg_elem_coef(const DevProblem &P, double *out, hipStream_t s);
 void launch_mg_coarsen(const Grid &Gf, const double *cf, const Grid &Gc, double *cc, hipStream_t s);
-// tmp (optional, mg_restrict_tmp_floats entries): work space of the
-// separable restriction between nested large levels
-void launch_mg_restrict(const Grid &Gf, const Grid &Gc, const BcMask &bc, const float *b, const float *y,
-                        float *bcoarse, hipStream_t s, float *tmp = nullptr);
-int64_t mg_restrict_tmp_floats(const Grid &Gf, const Grid &Gc);
+// r: the residual, zero on the Dirichlet rows
+void launch_mg_restrict(const Grid &Gf, const Grid &Gc, const BcMask &bc, const float *r, float *bcoarse,
+                        hipStream_t s);
 void launch_mg_prolong(const Grid &Gf, const Grid &Gc, const BcMask &bc, const float *xc, float *xf,
                        hipStream_t s);
 void launch_mg_cheb(const float *b, const float *y, const float *dinv, float *d, float *x, float c1, float c2,

@@ -14,102 +14,129 @@ namespace vfg {
 //   restriction: its transpose (the same weights, gathered per coarse node);
 //   coefficients: the overlap-weighted mean of the fine elements under each
 //     coarse element.
-__device__ __forceinline__ double mg_xi(int i, int nf, int nc) { return (double)i * (double)nc / (double)nf; }
-__device__ __forceinline__ float mg_w(double xi, int I) {
-  const double d = fabs(xi - (double)I);
-  return d < 1. ? (float)(1. - d) : 0.f;
+// The weights are formed from integers, (nf - |i nc - I nf|) / nf, and written
+// out (1/2, 1, 1/2) where the grids are nested.
+__device__ __forceinline__ bool mg_nested_grids(const Grid &Gf, const Grid &Gc) {
+  return Gf.nex == 2 * Gc.nex && Gf.ney == 2 * Gc.ney && Gf.nez == 2 * Gc.nez;
 }
 
 // ------------------------------------------------- restriction / prolongation
-// fine nodes i of one axis that coarse node I gathers from, with weights
-__device__ __forceinline__ int mg_gather(int I, int nf, int nc, int *i0, float *w) {
-  const int lo = max(0, (int)floor((double)(I - 1) * nf / nc));
-  const int hi = min(nf, (int)ceil((double)(I + 1) * nf / nc));
-  int m = 0;
-  for (int i = lo; i <= hi && m < 6; i++) {
-    const float wi = mg_w(mg_xi(i, nf, nc), I);
-    if (wi > 0.f) {
-      if (m == 0) *i0 = i;
-      w[m++] = wi;
+// both transfers take their weights from here, so they are each other's transpose
+__device__ __forceinline__ float mg_wt(int n, int nf) { return (float)n / (float)nf; }
+// The fine nodes i0 .. i0 + M - 1 of one axis that coarse node I gathers from,
+// with weights, zero off the axis and outside the hat (i is clamped to the
+// axis, so every load is in range).  M = 3: nested; 4: nf / nc <= 2.
+template <int M>
+__device__ __forceinline__ void mg_gather(int I, int nf, int nc, int (&i)[M], float (&w)[M]) {
+  if constexpr (M == 3) {
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+      i[q] = 2 * I - 1 + q;
+      w[q] = i[q] < 0 || i[q] > nf ? 0.f : q == 1 ? 1.f : .5f;
+    }
+  } else {
+    const int lo = I > 0 ? (I - 1) * nf / nc + 1 : 0;  // first i with i nc > (I - 1) nf
+#pragma unroll
+    for (int q = 0; q < M; q++) {
+      i[q] = lo + q;
+      const int m = i[q] * nc - I * nf, n = nf - (m < 0 ? -m : m);
+      w[q] = n <= 0 || i[q] > nf ? 0.f : mg_wt(n, nf);
     }
   }
-  return m;
+#pragma unroll
+  for (int q = 0; q < M; q++) i[q] = i[q] < 0 ? 0 : i[q] > nf ? nf : i[q];
 }
 
-// coarse rhs entry (node N, component c) = P^T (b - y) over the free fine rows
-// (y = nullptr: b already holds the residual); zero on coarse Dirichlet rows
-__device__ __forceinline__ float mg_restrict_dof(const Grid &Gf, const Grid &Gc, const BcMask &bc,
-                                                 const float *__restrict__ b, const float *__restrict__ y,
-                                                 int64_t N, int c) {
-  const int I = (int)(N % Gc.nx), J = (int)((N / Gc.nx) % Gc.ny), K = (int)(N / ((int64_t)Gc.nx * Gc.ny));
+// Lane kk (< 4) of coarse rhs entry (node (I, J, K), component c) = P^T r, r
+// zero on the fine Dirichlet rows: fine plane kk of the gather.  The entry is
+// the sum over the four lanes (mg_lanes), 0 on the coarse Dirichlet rows.  All
+// M^2 loads of a lane are independent of each other.
+template <int M>
+__device__ __forceinline__ float mg_restrict_plane(const Grid &Gf, const Grid &Gc, const BcMask &bc,
+                                                   const float *__restrict__ r, int I, int J, int K, int c, int kk) {
   if (on_dirichlet(Gc, bc.face[c], bc.vert[c], I, J, K)) return 0.f;
-  int i0 = 0, j0 = 0, k0 = 0;
-  float wx[6], wy[6], wz[6];
-  const int mx = mg_gather(I, Gf.nex, Gc.nex, &i0, wx);
-  const int my = mg_gather(J, Gf.ney, Gc.ney, &j0, wy);
-  const int mz = mg_gather(K, Gf.nez, Gc.nez, &k0, wz);
-  float acc = 0.f;
-  for (int kk = 0; kk < mz; kk++)
-    for (int jj = 0; jj < my; jj++) {
-      float row = 0.f;
-      for (int ii = 0; ii < mx; ii++) {
-        const int i = i0 + ii, j = j0 + jj, k = k0 + kk;
-        if (on_dirichlet(Gf, bc.face[c], bc.vert[c], i, j, k)) continue;
-        const int64_t n = 3 * node_id(Gf, i, j, k) + c;
-        row += wx[ii] * (y ? b[n] - y[n] : b[n]);
-      }
-      acc += wy[jj] * wz[kk] * row;
+  int i[M], j[M], k[M];
+  float wx[M], wy[M], wz[M];
+  mg_gather<M>(I, Gf.nex, Gc.nex, i, wx);
+  mg_gather<M>(J, Gf.ney, Gc.ney, j, wy);
+  mg_gather<M>(K, Gf.nez, Gc.nez, k, wz);
+  int kp = 0;
+  float wp = 0.f;
+#pragma unroll
+  for (int q = 0; q < M; q++)
+    if (q == kk) {
+      kp = k[q];
+      wp = wz[q];
     }
-  return acc;
+  float pl = 0.f;
+#pragma unroll
+  for (int jj = 0; jj < M; jj++) {
+    const float *__restrict__ row = r + 3 * ((int64_t)Gf.nx * (j[jj] + (int64_t)Gf.ny * kp)) + c;
+    float s = 0.f;
+#pragma unroll
+    for (int ii = 0; ii < M; ii++) s += wx[ii] * row[3 * i[ii]];
+    pl += wy[jj] * s;
+  }
+  return wp * pl;
+}
+// one thread per entry: the same value (planes summed in lane order)
+template <int M>
+__device__ __forceinline__ float mg_restrict_entry(const Grid &Gf, const Grid &Gc, const BcMask &bc,
+                                                   const float *__restrict__ r, int I, int J, int K, int c) {
+  float v = 0.f;
+#pragma unroll
+  for (int kk = 0; kk < M; kk++) v += mg_restrict_plane<M>(Gf, Gc, bc, r, I, J, K, c, kk);
+  return v;
+}
+// sum over four lanes in lane order, in the first of them
+__device__ __forceinline__ float mg_lanes(float v) {
+  const float v1 = __shfl_down(v, 1, 4), v2 = __shfl_down(v, 2, 4), v3 = __shfl_down(v, 3, 4);
+  return ((v + v1) + v2) + v3;
 }
 
-// The same entry split over the fine planes: lane kk of four sums planes
-// k0 + kk, k0 + kk + 4, ...; the four lanes' values add up to the entry.
-__device__ __forceinline__ float mg_restrict_dof_plane(const Grid &Gf, const Grid &Gc, const BcMask &bc,
-                                                       const float *__restrict__ b, const float *__restrict__ y,
-                                                       int64_t N, int c, int kk) {
-  const int I = (int)(N % Gc.nx), J = (int)((N / Gc.nx) % Gc.ny), K = (int)(N / ((int64_t)Gc.nx * Gc.ny));
-  if (on_dirichlet(Gc, bc.face[c], bc.vert[c], I, J, K)) return 0.f;
-  int i0 = 0, j0 = 0, k0 = 0;
-  float wx[6], wy[6], wz[6];
-  const int mx = mg_gather(I, Gf.nex, Gc.nex, &i0, wx);
-  const int my = mg_gather(J, Gf.ney, Gc.ney, &j0, wy);
-  const int mz = mg_gather(K, Gf.nez, Gc.nez, &k0, wz);
-  float acc = 0.f;
-  for (int kp = kk; kp < mz; kp += 4)
-    for (int jj = 0; jj < my; jj++) {
-      float row = 0.f;
-      for (int ii = 0; ii < mx; ii++) {
-        const int i = i0 + ii, j = j0 + jj, k = k0 + kp;
-        if (on_dirichlet(Gf, bc.face[c], bc.vert[c], i, j, k)) continue;
-        const int64_t n = 3 * node_id(Gf, i, j, k) + c;
-        row += wx[ii] * (y ? b[n] - y[n] : b[n]);
-      }
-      acc += wy[jj] * wz[kp] * row;
-    }
-  return acc;
+// the two coarse nodes around fine node i of one axis, with weights (the second
+// is the first again where its weight is 0)
+template <bool NESTED>
+__device__ __forceinline__ void mg_bracket(int i, int nf, int nc, int (&I)[2], float (&w)[2]) {
+  if constexpr (NESTED) {
+    I[0] = i >> 1;
+    I[1] = I[0] + (i & 1);
+    w[0] = i & 1 ? .5f : 1.f;
+    w[1] = i & 1 ? .5f : 0.f;
+  } else {
+    const int q = i * nc / nf, m = i * nc - q * nf;
+    I[0] = q;
+    I[1] = q + (m > 0);
+    w[0] = mg_wt(nf - m, nf);
+    w[1] = mg_wt(m, nf);
+  }
 }
-
-// x_fine(node n) += P x_coarse on the free fine rows
+// x_fine(node (i, j, k)) += P x_coarse on the free fine rows
+template <bool NESTED>
 __device__ __forceinline__ void mg_prolong_node(const Grid &Gf, const Grid &Gc, const BcMask &bc,
-                                                const float *__restrict__ xc, float *__restrict__ xf, int64_t n) {
-  const int i = (int)(n % Gf.nx), j = (int)((n / Gf.nx) % Gf.ny), k = (int)(n / ((int64_t)Gf.nx * Gf.ny));
-  const double xi = mg_xi(i, Gf.nex, Gc.nex), yj = mg_xi(j, Gf.ney, Gc.ney), zk = mg_xi(k, Gf.nez, Gc.nez);
-  const int I0 = min((int)floor(xi), Gc.nex - 1), J0 = min((int)floor(yj), Gc.ney - 1),
-            K0 = min((int)floor(zk), Gc.nez - 1);
-  const float wx[2] = {mg_w(xi, I0), mg_w(xi, I0 + 1)}, wy[2] = {mg_w(yj, J0), mg_w(yj, J0 + 1)},
-              wz[2] = {mg_w(zk, K0), mg_w(zk, K0 + 1)};
-  float acc[3] = {0.f, 0.f, 0.f};
+                                                const float *__restrict__ xc, float *__restrict__ xf, int i, int j,
+                                                int k) {
+  int I[2], J[2], K[2];
+  float wx[2], wy[2], wz[2];
+  mg_bracket<NESTED>(i, Gf.nex, Gc.nex, I, wx);
+  mg_bracket<NESTED>(j, Gf.ney, Gc.ney, J, wy);
+  mg_bracket<NESTED>(k, Gf.nez, Gc.nez, K, wz);
+  float *__restrict__ p = xf + 3 * node_id(Gf, i, j, k);
+  float x[3], acc[3] = {0.f, 0.f, 0.f};
+#pragma unroll
+  for (int c = 0; c < 3; c++) x[c] = p[c];
+#pragma unroll
   for (int c3 = 0; c3 < 2; c3++)
-    for (int c2 = 0; c2 < 2; c2++)
-      for (int c1 = 0; c1 < 2; c1++) {
-        const float w = wx[c1] * wy[c2] * wz[c3];
-        if (w == 0.f) continue;
-        const int64_t N = node_id(Gc, I0 + c1, J0 + c2, K0 + c3);
-        for (int c = 0; c < 3; c++) acc[c] += w * xc[3 * N + c];
-      }
+#pragma unroll
+    for (int c2 = 0; c2 < 2; c2++) {
+      const float *__restrict__ row = xc + 3 * ((int64_t)Gc.nx * (J[c2] + (int64_t)Gc.ny * K[c3]));
+      const float w = wz[c3] * wy[c2];
+#pragma unroll
+      for (int c = 0; c < 3; c++) acc[c] += w * (wx[0] * row[3 * I[0] + c] + wx[1] * row[3 * I[1] + c]);
+    }
+#pragma unroll
   for (int c = 0; c < 3; c++)
-    if (!on_dirichlet(Gf, bc.face[c], bc.vert[c], i, j, k)) xf[3 * n + c] += acc[c];
+    if (!on_dirichlet(Gf, bc.face[c], bc.vert[c], i, j, k)) p[c] = x[c] + acc[c];
 }
 
 // one Chebyshev step on the Jacobi-scaled system, entry i:

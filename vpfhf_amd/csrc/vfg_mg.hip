@@ -86,157 +86,36 @@ __global__ void k_mg_coarsen(Grid Gf, const double *__restrict__ cf, Grid Gc, do
   cc[c] = acc / wsum;
 }
 
-// one thread per coarse (node, component)
-__global__ __launch_bounds__(256) void k_mg_restrict(Grid Gf, Grid Gc, BcMask bc, const float *__restrict__ b,
-                                                     const float *__restrict__ y, float *__restrict__ bcoarse) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= 3 * (int64_t)Gc.nx * Gc.ny * Gc.nz) return;
-  const int64_t N = t / 3;
-  bcoarse[t] = mg_restrict_dof(Gf, Gc, bc, b, y, N, (int)(t - 3 * N));
-}
-
-// small coarse grids: four lanes per (node, component), each over every
-// fourth fine plane (one plane each under ceil(n/2) coarsening), summed in
-// lane order
-__global__ __launch_bounds__(256) void k_mg_restrict4(Grid Gf, Grid Gc, BcMask bc, const float *__restrict__ b,
-                                                      const float *__restrict__ y, float *__restrict__ bcoarse) {
-  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, t = g >> 2;
-  const int kk = (int)(g & 3);
-  const bool ok = t < 3 * (int64_t)Gc.nx * Gc.ny * Gc.nz;
-  const int64_t N = ok ? t / 3 : 0;
-  float v = ok ? mg_restrict_dof_plane(Gf, Gc, bc, b, y, N, (int)(t - 3 * N), kk) : 0.f;
-  const float v1 = __shfl_down(v, 1, 4), v2 = __shfl_down(v, 2, 4), v3 = __shfl_down(v, 3, 4);
-  if (ok && kk == 0) bcoarse[t] = ((v + v1) + v2) + v3;
-}
-
-// Nested levels (nf = 2 nc in every direction): the same transfers with the
-// weights of the 1-D map xi = i / 2 written out -- fine node 2I gets coarse
-// node I with weight 1, fine node 2I + 1 gets I and I + 1 with 1/2 each --
-// and one thread per node doing all three components (the general kernels
-// form the weights from the map in FP64 per entry).
-__device__ __forceinline__ float mg_w2(int d) { return d == 0 ? 1.f : .5f; }
-// grid (ceil(nx * ny / 256), nz): node (i, j) of plane blockIdx.y from a
-// 32-bit index (no 64-bit division per thread)
-__global__ __launch_bounds__(256) void k_mg_restrict2(Grid Gf, Grid Gc, BcMask bc, const float *__restrict__ b,
-                                                      const float *__restrict__ y, float *__restrict__ bcoarse) {
-  const int t = blockIdx.x * 256 + threadIdx.x;
-  if (t >= Gc.nx * Gc.ny) return;
-  const int J = t / Gc.nx, I = t - J * Gc.nx, K = blockIdx.y;
-  float acc[3] = {0.f, 0.f, 0.f};
-  for (int dk = -1; dk <= 1; dk++) {
-    const int k = 2 * K + dk;
-    if (k < 0 || k >= Gf.nz) continue;
-    for (int dj = -1; dj <= 1; dj++) {
-      const int j = 2 * J + dj;
-      if (j < 0 || j >= Gf.ny) continue;
-      float row[3] = {0.f, 0.f, 0.f};
-      for (int di = -1; di <= 1; di++) {
-        const int i = 2 * I + di;
-        if (i < 0 || i >= Gf.nx) continue;
-        const int64_t n = 3 * node_id(Gf, i, j, k);
-#pragma unroll
-        for (int c = 0; c < 3; c++)
-          if (!on_dirichlet(Gf, bc.face[c], bc.vert[c], i, j, k))
-            row[c] += mg_w2(di) * (y ? b[n + c] - y[n + c] : b[n + c]);
-      }
-      const float w = mg_w2(dj) * mg_w2(dk);
-#pragma unroll
-      for (int c = 0; c < 3; c++) acc[c] += w * row[c];
-    }
+// Transfers, plane blockIdx.y (so that indices are 32-bit): restriction one
+// thread per (coarse node, component), on small levels (latency-bound) four,
+// one per fine plane of the gather; prolongation one thread per fine node.
+// Restriction, mean of the 129^3 -> 65^3 -> 33^3 nodes 9.7 us (25 us as three
+// separable passes that formed b - A x and the Dirichlet tests themselves), of
+// 33^3 -> 17^3 -> 9^3 3.2 us (8.8 us with FP64 weights); prolongation, mean of
+// the four levels of 128^3 8.0 us (9.8).
+template <int M, int LANES>
+__global__ __launch_bounds__(256) void k_mg_restrict(Grid Gf, Grid Gc, BcMask bc, const float *__restrict__ r,
+                                                     float *__restrict__ bcoarse) {
+  const int g = blockIdx.x * 256 + threadIdx.x, t = g / LANES, np = 3 * Gc.nx * Gc.ny;
+  const bool ok = t < np;
+  const int N = ok ? t / 3 : 0, c = ok ? t - 3 * N : 0, J = N / Gc.nx, I = N - J * Gc.nx, K = blockIdx.y;
+  if constexpr (LANES == 1) {
+    if (ok) bcoarse[t + (int64_t)np * K] = mg_restrict_entry<M>(Gf, Gc, bc, r, I, J, K, c);
+  } else {
+    const float v = mg_lanes(mg_restrict_plane<M>(Gf, Gc, bc, r, I, J, K, c, g & 3));
+    if (ok && (g & 3) == 0) bcoarse[t + (int64_t)np * K] = v;
   }
-  const int64_t N = node_id(Gc, I, J, K);
-#pragma unroll
-  for (int c = 0; c < 3; c++) bcoarse[3 * N + c] = on_dirichlet(Gc, bc.face[c], bc.vert[c], I, J, K) ? 0.f : acc[c];
 }
-__global__ __launch_bounds__(256) void k_mg_prolong2(Grid Gf, Grid Gc, BcMask bc, const float *__restrict__ xc,
-                                                     float *__restrict__ xf) {
+template <bool NESTED>
+__global__ __launch_bounds__(256) void k_mg_prolong(Grid Gf, Grid Gc, BcMask bc, const float *__restrict__ xc,
+                                                    float *__restrict__ xf) {
   const int t = blockIdx.x * 256 + threadIdx.x;
   if (t >= Gf.nx * Gf.ny) return;
-  const int j = t / Gf.nx, i = t - j * Gf.nx, k = blockIdx.y;
-  const int I0 = i >> 1, J0 = j >> 1, K0 = k >> 1;
-  const int mi = i & 1, mj = j & 1, mk = k & 1;  // odd: between I0 and I0 + 1
-  const float wx = mi ? .5f : 1.f, wy = mj ? .5f : 1.f, wz = mk ? .5f : 1.f;
-  float acc[3] = {0.f, 0.f, 0.f};
-  for (int c3 = 0; c3 <= mk; c3++)
-    for (int c2 = 0; c2 <= mj; c2++)
-      for (int c1 = 0; c1 <= mi; c1++) {
-        const float w = wx * wy * wz;
-        const int64_t N = 3 * node_id(Gc, I0 + c1, J0 + c2, K0 + c3);
-#pragma unroll
-        for (int c = 0; c < 3; c++) acc[c] += w * xc[N + c];
-      }
-  const int64_t n = node_id(Gf, i, j, k);
-#pragma unroll
-  for (int c = 0; c < 3; c++)
-    if (!on_dirichlet(Gf, bc.face[c], bc.vert[c], i, j, k)) xf[3 * n + c] += acc[c];
-}
-// Nested restriction in three separable passes (large levels): x, then y,
-// then z, each a contiguous sweep.  t1 holds (Gc.nx, Gf.ny, Gf.nz) nodes, t2
-// (Gc.nx, Gc.ny, Gf.nz); the fine Dirichlet rows are zeroed in the x pass,
-// the coarse ones in the z pass.
-__global__ __launch_bounds__(256) void k_mg_rsx(Grid Gf, Grid Gc, BcMask bc, const float *__restrict__ b,
-                                                const float *__restrict__ y, float *__restrict__ t1) {
-  const int t = blockIdx.x * 256 + threadIdx.x;
-  if (t >= Gc.nx * Gf.ny) return;
-  const int j = t / Gc.nx, I = t - j * Gc.nx, k = blockIdx.y;
-  float acc[3] = {0.f, 0.f, 0.f};
-  for (int di = -1; di <= 1; di++) {
-    const int i = 2 * I + di;
-    if (i < 0 || i >= Gf.nx) continue;
-    const int64_t n = 3 * node_id(Gf, i, j, k);
-#pragma unroll
-    for (int c = 0; c < 3; c++)
-      if (!on_dirichlet(Gf, bc.face[c], bc.vert[c], i, j, k)) acc[c] += mg_w2(di) * (y ? b[n + c] - y[n + c] : b[n + c]);
-  }
-  const int64_t o = 3 * ((int64_t)I + (int64_t)Gc.nx * (j + (int64_t)Gf.ny * k));
-#pragma unroll
-  for (int c = 0; c < 3; c++) t1[o + c] = acc[c];
-}
-__global__ __launch_bounds__(256) void k_mg_rsy(Grid Gf, Grid Gc, const float *__restrict__ t1, float *__restrict__ t2) {
-  const int t = blockIdx.x * 256 + threadIdx.x;
-  if (t >= Gc.nx * Gc.ny) return;
-  const int J = t / Gc.nx, I = t - J * Gc.nx, k = blockIdx.y;
-  float acc[3] = {0.f, 0.f, 0.f};
-  for (int dj = -1; dj <= 1; dj++) {
-    const int j = 2 * J + dj;
-    if (j < 0 || j >= Gf.ny) continue;
-    const int64_t n = 3 * ((int64_t)I + (int64_t)Gc.nx * (j + (int64_t)Gf.ny * k));
-#pragma unroll
-    for (int c = 0; c < 3; c++) acc[c] += mg_w2(dj) * t1[n + c];
-  }
-  const int64_t o = 3 * ((int64_t)I + (int64_t)Gc.nx * (J + (int64_t)Gc.ny * k));
-#pragma unroll
-  for (int c = 0; c < 3; c++) t2[o + c] = acc[c];
-}
-__global__ __launch_bounds__(256) void k_mg_rsz(Grid Gf, Grid Gc, BcMask bc, const float *__restrict__ t2,
-                                                float *__restrict__ bcoarse) {
-  const int t = blockIdx.x * 256 + threadIdx.x;
-  if (t >= Gc.nx * Gc.ny) return;
-  const int J = t / Gc.nx, I = t - J * Gc.nx, K = blockIdx.y;
-  float acc[3] = {0.f, 0.f, 0.f};
-  for (int dk = -1; dk <= 1; dk++) {
-    const int k = 2 * K + dk;
-    if (k < 0 || k >= Gf.nz) continue;
-    const int64_t n = 3 * ((int64_t)I + (int64_t)Gc.nx * (J + (int64_t)Gc.ny * k));
-#pragma unroll
-    for (int c = 0; c < 3; c++) acc[c] += mg_w2(dk) * t2[n + c];
-  }
-  const int64_t N = node_id(Gc, I, J, K);
-#pragma unroll
-  for (int c = 0; c < 3; c++) bcoarse[3 * N + c] = on_dirichlet(Gc, bc.face[c], bc.vert[c], I, J, K) ? 0.f : acc[c];
-}
-int64_t mg_restrict_tmp_floats(const Grid &Gf, const Grid &Gc) {
-  return 3 * ((int64_t)Gc.nx * Gf.ny * Gf.nz + (int64_t)Gc.nx * Gc.ny * Gf.nz);
+  const int j = t / Gf.nx;
+  mg_prolong_node<NESTED>(Gf, Gc, bc, xc, xf, t - j * Gf.nx, j, (int)blockIdx.y);
 }
 static bool mg_nested(const Grid &Gf, const Grid &Gc) {
   return Gf.nex == 2 * Gc.nex && Gf.ney == 2 * Gc.ney && Gf.nez == 2 * Gc.nez;
-}
-
-__global__ __launch_bounds__(256) void k_mg_prolong(Grid Gf, Grid Gc, BcMask bc, const float *__restrict__ xc,
-                                                    float *__restrict__ xf) {
-  const int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= (int64_t)Gf.nx * Gf.ny * Gf.nz) return;
-  mg_prolong_node(Gf, Gc, bc, xc, xf, n);
 }
 
 // ----------------------------------------------------------------- smoother
@@ -279,28 +158,20 @@ void launch_mg_coarsen(const Grid &Gf, const double *cf, const Grid &Gc, double 
   const int64_t ne = (int64_t)Gc.nex * Gc.ney * Gc.nez;
   hipLaunchKernelGGL(k_mg_coarsen, dim3(nbm(ne)), dim3(256), 0, s, Gf, cf, Gc, cc);
 }
-void launch_mg_restrict(const Grid &Gf, const Grid &Gc, const BcMask &bc, const float *b, const float *y,
-                        float *bcoarse, hipStream_t s, float *tmp) {
-  const int64_t n3 = 3 * (int64_t)Gc.nx * Gc.ny * Gc.nz;
-  // few coarse entries: latency-bound, split each over its fine planes
-  if (n3 <= (1 << 16)) hipLaunchKernelGGL(k_mg_restrict4, dim3(nbm(4 * n3)), dim3(256), 0, s, Gf, Gc, bc, b, y, bcoarse);
-  else if (mg_nested(Gf, Gc) && tmp) {
-    float *t1 = tmp, *t2 = tmp + 3 * (int64_t)Gc.nx * Gf.ny * Gf.nz;
-    hipLaunchKernelGGL(k_mg_rsx, dim3(nbm((int64_t)Gc.nx * Gf.ny), Gf.nz), dim3(256), 0, s, Gf, Gc, bc, b, y, t1);
-    hipLaunchKernelGGL(k_mg_rsy, dim3(nbm((int64_t)Gc.nx * Gc.ny), Gf.nz), dim3(256), 0, s, Gf, Gc, (const float *)t1, t2);
-    hipLaunchKernelGGL(k_mg_rsz, dim3(nbm((int64_t)Gc.nx * Gc.ny), Gc.nz), dim3(256), 0, s, Gf, Gc, bc, (const float *)t2,
-                       bcoarse);
-  } else if (mg_nested(Gf, Gc))
-    hipLaunchKernelGGL(k_mg_restrict2, dim3(nbm((int64_t)Gc.nx * Gc.ny), Gc.nz), dim3(256), 0, s, Gf, Gc, bc, b, y,
-                       bcoarse);
-  else hipLaunchKernelGGL(k_mg_restrict, dim3(nbm(n3)), dim3(256), 0, s, Gf, Gc, bc, b, y, bcoarse);
+void launch_mg_restrict(const Grid &Gf, const Grid &Gc, const BcMask &bc, const float *r, float *bcoarse,
+                        hipStream_t s) {
+  const int64_t np = 3 * (int64_t)Gc.nx * Gc.ny;
+  const bool small = np * Gc.nz <= (1 << 16);  // few entries: split each over its fine planes
+  const dim3 g(nbm(small ? 4 * np : np), Gc.nz);
+  auto go = [&](auto k) { hipLaunchKernelGGL(k, g, dim3(256), 0, s, Gf, Gc, bc, r, bcoarse); };
+  if (mg_nested(Gf, Gc)) small ? go(k_mg_restrict<3, 4>) : go(k_mg_restrict<3, 1>);
+  else small ? go(k_mg_restrict<4, 4>) : go(k_mg_restrict<4, 1>);
 }
 void launch_mg_prolong(const Grid &Gf, const Grid &Gc, const BcMask &bc, const float *xc, float *xf,
                        hipStream_t s) {
-  const int64_t nn = (int64_t)Gf.nx * Gf.ny * Gf.nz;
-  if (mg_nested(Gf, Gc))
-    hipLaunchKernelGGL(k_mg_prolong2, dim3(nbm((int64_t)Gf.nx * Gf.ny), Gf.nz), dim3(256), 0, s, Gf, Gc, bc, xc, xf);
-  else hipLaunchKernelGGL(k_mg_prolong, dim3(nbm(nn)), dim3(256), 0, s, Gf, Gc, bc, xc, xf);
+  const dim3 g(nbm((int64_t)Gf.nx * Gf.ny), Gf.nz);
+  if (mg_nested(Gf, Gc)) hipLaunchKernelGGL(k_mg_prolong<true>, g, dim3(256), 0, s, Gf, Gc, bc, xc, xf);
+  else hipLaunchKernelGGL(k_mg_prolong<false>, g, dim3(256), 0, s, Gf, Gc, bc, xc, xf);
 }
 void launch_mg_cheb(const float *b, const float *y, const float *dinv, float *d, float *x, float c1, float c2,
                     int dfirst, int xzero, int64_t n, hipStream_t s) {

@@ -777,13 +777,11 @@ static int mg_vcycle(vfg_handle *h, int l, const double *r64 = nullptr, double *
   // one Chebyshev-Jacobi step from x = 0 fused with its apply, restriction of
   // b - A x, coarse correction, and one step fused with its apply: the values
   // of mg_smooth(1) + apply + restrict ... + mg_smooth(1) in three passes less.
-  // The level iterates in d (A d in y) and leaves its result in x.
+  // The level iterates in d (b - A d in y) and leaves its result in x.
   float c1[1], c2[1];
   cheb_step_coefs(1, L.lmax / 11., L.lmax, c1, c2);
   launch_mg_presmooth(L.P, L.b, L.dinv, c2[0], L.d, L.y, s);
-  // L.x is written only by the post-smoothing: it is the restriction's work space
-  float *tmp = mg_restrict_tmp_floats(L.P.G, C.P.G) <= L.n ? L.x : nullptr;
-  launch_mg_restrict(L.P.G, C.P.G, L.P.bcU, L.b, L.y, C.b, s, tmp);
+  launch_mg_restrict(L.P.G, C.P.G, L.P.bcU, L.y, C.b, s);
   mg_vcycle(h, l + 1);
   launch_mg_prolong(L.P.G, C.P.G, L.P.bcU, C.x, L.d, s);
   return launch_mg_postsmooth(L.P, L.b, L.dinv, c2[0], L.d, L.x, r64, part, s);

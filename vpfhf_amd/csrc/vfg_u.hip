@@ -466,8 +466,8 @@ __global__ __launch_bounds__(TX *TY, um_waves<T>()) void k_u_apply(UModOp<T, UNI
 
 // FP32 multigrid apply fused with its Chebyshev(1)-Jacobi step (mg_cheb_entry
 // with one step, vfg_solve.hip's V-cycle):
-//   pre  (from x = 0): x = c2 D^-1 b staged on the fly; stores x and A x (the
-//        restriction forms b - A x on the free rows);
+//   pre  (from x = 0): x = c2 D^-1 b staged on the fly; stores x and the
+//        residual b - A x (0 on the Dirichlet rows) for the restriction;
 //   post: xo = x + c2 D^-1 (b - A x), A x = x on Dirichlet rows, into a
 //        buffer other than x (neighbouring tiles still stage x); b and D^-1
 //        of the owned node are loaded a node plane ahead (own_load).  The
@@ -492,11 +492,18 @@ struct UMgPreOp : UModBase<float, UNIT, UMgRec> {
     return Raw{this->b[3 * n + f], this->dinv[3 * n + f]};
   }
   __device__ float stage(int f, const Raw &r) const { return f == 3 ? r.b : this->c2 * r.di * r.b; }
-  __device__ void store(int64_t n, uint32_t, const float (&acc)[3], const Own &own) const {
+  struct OwnB {
+    float b[3];
+  };
+  __device__ OwnB own_load(int64_t n) const { return OwnB{{this->b[3 * n], this->b[3 * n + 1], this->b[3 * n + 2]}}; }
+  __device__ void store(int64_t n, uint32_t fb, const float (&acc)[3], const Own &own, const OwnB &o) const {
+    const Own rhs{{o.b[0], o.b[1], o.b[2]}};
+    float yv[3];
+    this->rows(fb, acc, rhs, yv);  // b itself on the Dirichlet rows
 #pragma unroll
     for (int c = 0; c < 3; c++) {
       this->xo[3 * n + c] = own.x[c];
-      this->ro[3 * n + c] = acc[c];
+      this->ro[3 * n + c] = o.b[c] - yv[c];
     }
   }
 };
@@ -1191,13 +1198,6 @@ void launch_u_cmask(const DevProblem &P, const double *U, hipStream_t s) {
   hipLaunchKernelGGL(k_u_cmask, dim3((unsigned)((P.ne + 255) / 256)), dim3(256), 0, s, P.G, U, P.cmask);
 }
 
-// Chebyshev-Jacobi solve of a small FP32 level from x = 0 in one workgroup
-// (the coarsest multigrid level, at most MGC_NE elements): x, d and the
-// operator output stay in LDS.  An apply is an element pass (one element per
-// thread, its 24 outputs to LDS) and a node pass that adds each node's eight
-// element contributions in a fixed order (x-pairs, then y-pairs, the lower
-// element layer before the upper); the step is mg_cheb_entry, as in the
-// multi-launch smoother.
 // one apply record of the batched / engine applies
 template <typename T>
 struct BApply {
@@ -1212,87 +1212,130 @@ __device__ __forceinline__ Op op_of(const typename Op::Record &r) {
   return o;
 }
 
+// Chebyshev-Jacobi solve of a small FP32 level from x = 0 in one workgroup
+// (the coarsest multigrid level, at most MGC_NE elements).  A thread owns one
+// element (its modulus, face sums of v and place are read once) and up to MGC_Q
+// entries (node, component), whose b, D^-1, x and direction stay in its
+// registers; only the iterate and the element forces go through LDS, component
+// by component so that consecutive lanes touch consecutive words.  A step is an
+// element pass and an entry pass that adds each node's eight element forces in
+// a fixed order (x-pairs, then y-pairs, the lower element layer before the
+// upper); the step itself is mg_cheb_entry's.  Latency-bound on one CU: 9^3
+// nodes 15 us, 27 us with E, b and D^-1 re-read from memory in every step and
+// the forces interleaved by element (eight-way bank conflicts).
 constexpr int MGC_T = 512, MGC_NE = 512, MGC_NN = 729;
+constexpr int MGC_Q = (3 * MGC_NN + MGC_T - 1) / MGC_T;
 
-template <bool UNIT>
+// coef(i): the step's coefficients {c1, c2}
+template <bool UNIT, class Coef>
 __device__ __forceinline__ void mg_coarse_cheb_body(const UModOp<float, UNIT> &op, const float *__restrict__ b,
                                                     const float *__restrict__ dinv, float *__restrict__ xout,
-                                                    const MgChebCoefs &cc) {
-  __shared__ float sx[3 * MGC_NN], sd[3 * MGC_NN], sy[3 * MGC_NN];
-  __shared__ float sr[MGC_NE * 24];
+                                                    int steps, const Coef &coef) {
+  __shared__ float sx[3 * MGC_NN];
+  __shared__ float sr[24 * MGC_NE + 1];  // [corner * 3 + component][element]; the last word stays 0
   const Grid &G = op.G;
   const int tid = threadIdx.x;
   const int nn = G.nx * G.ny * G.nz, ne = G.nex * G.ney * G.nez;
-  auto R = [&](int ex, int ey, int ez, int corner, int c) -> float {
-    if (ex < 0 || ex >= G.nex || ey < 0 || ey >= G.ney || ez < 0 || ez >= G.nez) return 0.f;
-    return sr[(ex + G.nex * (ey + G.ney * ez)) * 24 + corner * 3 + c];
-  };
-  // corner (i, J, K) of element (ex, ey, ez) plus corner (0, J, K) of its +x neighbour
-  auto cx = [&](int ex, int ey, int ez, int J, int K, int c) {
-    return R(ex, ey, ez, (K * 2 + J) * 2 + 1, c) + R(ex + 1, ey, ez, (K * 2 + J) * 2, c);
-  };
-  for (int i = 0; i < cc.k; i++) {
+  if (tid == 0) sr[24 * MGC_NE] = 0.f;
+  // the entries t = tid + q MGC_T, component t / nn
+  float eb[MGC_Q], ed[MGC_Q], ex_[MGC_Q], dir[MGC_Q];
+  int src[MGC_Q][8];  // where the eight forces of the entry lie in sr
+  bool fixed[MGC_Q];
+#pragma unroll
+  for (int q = 0; q < MGC_Q; q++) {
+    const int t = tid + q * MGC_T;
+    eb[q] = ed[q] = ex_[q] = dir[q] = 0.f;
+    fixed[q] = false;
+#pragma unroll
+    for (int a = 0; a < 8; a++) src[q][a] = 24 * MGC_NE;
+    if (t >= 3 * nn) continue;
+    const int c = t / nn, n = t - c * nn, ni = n % G.nx, nj = (n / G.nx) % G.ny, nk = n / (G.nx * G.ny);
+    eb[q] = b[3 * n + c];
+    ed[q] = dinv[3 * n + c];
+    fixed[q] = on_dirichlet(G, op.bc.face[c], op.bc.vert[c], ni, nj, nk);
+#pragma unroll
+    for (int a = 0; a < 8; a++) {
+      const int ei = ni - (a & 1), ej = nj - ((a >> 1) & 1), ek = nk - (a >> 2);  // the node is its corner a
+      if (ei >= 0 && ei < G.nex && ej >= 0 && ej < G.ney && ek >= 0 && ek < G.nez)
+        src[q][a] = (a * 3 + c) * MGC_NE + ei + G.nex * (ej + G.ney * ek);
+    }
+  }
+  // the thread's element
+  const bool el = tid < ne;
+  float E = 0.f, vb[4] = {}, vt[4] = {};
+  int n0 = 0;
+  const int nr = G.nx, np = G.nx * G.ny;
+  if (el) {
+    const int ex = tid % G.nex, ey = (tid / G.nex) % G.ney, ez = tid / (G.nex * G.ney);
+    n0 = ex + nr * ey + np * ez;
+    E = op.aux(ex, ey, ez, 0, 0);
+    if constexpr (!UNIT)
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        vb[q] = op.v[n0 + (q >> 1) * nr + (q & 1)];
+        vt[q] = op.v[n0 + np + (q >> 1) * nr + (q & 1)];
+      }
+  }
+  for (int i = 0; i < steps; i++) {
+    const BmgCoef cf = coef(i);
     if (i > 0) {
-      for (int e = tid; e < ne; e += MGC_T) {
-        const int ex = e % G.nex, ey = (e / G.nex) % G.ney, ez = e / (G.nex * G.ney);
+#pragma unroll
+      for (int q = 0; q < MGC_Q; q++)
+        if (tid + q * MGC_T < 3 * nn) sx[tid + q * MGC_T] = ex_[q];
+      __syncthreads();
+      if (el) {
         UFace<float> fb, ft;
-        const int64_t n0 = node_id(G, ex, ey, ez), nr = G.nx, np = (int64_t)G.nx * G.ny;
+        float t[2][3][4] = {};
 #pragma unroll
         for (int c = 0; c < 3; c++) {
-          const float *xb = sx + 3 * n0 + c, *xt = xb + 3 * np;
-          uface_set<float>(fb, c, xb[0], xb[3], xb[3 * nr], xb[3 * nr + 3]);
-          uface_set<float>(ft, c, xt[0], xt[3], xt[3 * nr], xt[3 * nr + 3]);
+          const float *xb = sx + c * nn + n0, *xt = xb + np;
+          uface_set<float>(fb, c, xb[0], xb[1], xb[nr], xb[nr + 1]);
+          uface_set<float>(ft, c, xt[0], xt[1], xt[nr], xt[nr + 1]);
         }
-        float vb[4] = {}, vt[4] = {}, t[2][3][4] = {};
-        if constexpr (!UNIT) {
-          const float *vp = op.v + n0, *vq = vp + np;
-#pragma unroll
-          for (int q = 0; q < 4; q++) {
-            vb[q] = vp[(q >> 1) * nr + (q & 1)];
-            vt[q] = vq[(q >> 1) * nr + (q & 1)];
-          }
-        }
-        um_layer<float, UNIT>(fb, ft, vb, vt, op.aux(ex, ey, ez, 0, 0), op.m, t[0], t[1]);
+        um_layer<float, UNIT>(fb, ft, vb, vt, E, op.m, t[0], t[1]);
 #pragma unroll
         for (int kz = 0; kz < 2; kz++)
 #pragma unroll
           for (int c = 0; c < 3; c++) {
             const float(&u)[4] = t[kz][c];
             const float e0 = u[0] - u[1], e1 = u[0] + u[1], f0 = u[2] - u[3], f1 = u[2] + u[3];
-            float *o = sr + e * 24 + kz * 12 + c;
+            float *o = sr + (kz * 12 + c) * MGC_NE + tid;
             o[0] = e0 - f0;
-            o[3] = e1 - f1;
-            o[6] = e0 + f0;
-            o[9] = e1 + f1;
+            o[3 * MGC_NE] = e1 - f1;
+            o[6 * MGC_NE] = e0 + f0;
+            o[9 * MGC_NE] = e1 + f1;
           }
       }
       __syncthreads();
-      for (int n = tid; n < nn; n += MGC_T) {
-        const int ni = n % G.nx, nj = (n / G.nx) % G.ny, nk = n / (G.nx * G.ny);
-        const int ex = ni - 1, ey = nj - 1;
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-          // element layer nk - 1 (corners K = 1), then layer nk (K = 0); in
-          // each, element row ey (corners J = 1) before row ey + 1 (J = 0)
-          const float carry = cx(ex, ey, nk - 1, 1, 1, c) + cx(ex, ey + 1, nk - 1, 0, 1, c);
-          const float acc = carry + (cx(ex, ey, nk, 1, 0, c) + cx(ex, ey + 1, nk, 0, 0, c));
-          sy[3 * n + c] = on_dirichlet(G, op.bc.face[c], op.bc.vert[c], ni, nj, nk) ? sx[3 * n + c] : acc;
-        }
-      }
-      __syncthreads();
     }
-    const float c1 = cc.c1[i], c2 = cc.c2[i];
-    for (int t = tid; t < 3 * nn; t += MGC_T)
-      mg_cheb_entry(b, i > 0 ? sy : nullptr, dinv, sd, sx, c1, c2, i == 0, i == 0, t);
-    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < MGC_Q; q++) {
+      float res = eb[q];
+      if (i > 0) {
+        const int(&s)[8] = src[q];
+        // corners a = 4 K + 2 J + I: the element layer below (K = 1), then the layer above
+        const float lo = (sr[s[7]] + sr[s[6]]) + (sr[s[5]] + sr[s[4]]);
+        const float y = lo + ((sr[s[3]] + sr[s[2]]) + (sr[s[1]] + sr[s[0]]));
+        res -= fixed[q] ? ex_[q] : y;
+      }
+      dir[q] = (i > 0 ? cf.c1 * dir[q] : 0.f) + cf.c2 * ed[q] * res;
+      ex_[q] += dir[q];
+    }
   }
-  for (int t = tid; t < 3 * nn; t += MGC_T) xout[t] = sx[t];
+#pragma unroll
+  for (int q = 0; q < MGC_Q; q++) {
+    const int t = tid + q * MGC_T;
+    if (t < 3 * nn) {
+      const int c = t / nn;
+      xout[3 * (t - c * nn) + c] = ex_[q];
+    }
+  }
 }
 
 __global__ __launch_bounds__(MGC_T) void k_mg_coarse_cheb(UModOp<float, true> op, const float *__restrict__ b,
                                                           const float *__restrict__ dinv, float *__restrict__ xout,
                                                           MgChebCoefs cc) {
-  mg_coarse_cheb_body<true>(op, b, dinv, xout, cc);
+  mg_coarse_cheb_body<true>(op, b, dinv, xout, cc.k, [&](int i) { return BmgCoef{cc.c1[i], cc.c2[i]}; });
 }
 
 // the batched form: one workgroup per listed member (its first chunk), the
@@ -1308,15 +1351,9 @@ __global__ __launch_bounds__(MGC_T) void k_bmg_coarse_cheb(const BApply<float> *
   const BmgChunk c = ch[blockIdx.x];
   if (c.start != 0 || flags[(int64_t)c.p * fstride] == 0.) return;  // uniform in the workgroup
   const BmgVec &v = lvt[c.p * BML + level];
-  MgChebCoefs cc;
-  cc.k = MG_COARSE_DEG;
-#pragma unroll
-  for (int i = 0; i < MG_COARSE_DEG; i++) {
-    const BmgCoef k = coef[((c.p * BML + level) * 2 + 1) * BMK + i];
-    cc.c1[i] = k.c1;
-    cc.c2[i] = k.c2;
-  }
-  mg_coarse_cheb_body<UNIT>(op_of<UModOp<float, UNIT>>(ops[c.p].op), v.b, v.dinv, v.x, cc);
+  const BmgCoef *__restrict__ cf = coef + ((c.p * BML + level) * 2 + 1) * BMK;
+  mg_coarse_cheb_body<UNIT>(op_of<UModOp<float, UNIT>>(ops[c.p].op), v.b, v.dinv, v.x, MG_COARSE_DEG,
+                            [&](int i) { return cf[i]; });
 }
 
 bool mg_coarse_fits(const DevProblem &P) {
