@@ -43,3 +43,29 @@ def test_vcycle_transfers(n):
     assert abs(a @ Mb - b @ Ma) <= 1e-5 * np.linalg.norm(a) * np.linalg.norm(Mb)
     assert a @ Ma > 0.0
     P.close()
+
+
+@pytest.mark.parametrize("unilateral", [0, 1], ids=["linear", "nocompression"])
+@pytest.mark.parametrize("n", [(2, 2, 2), (17, 18, 3), (18, 33, 20), (115, 114, 10)], ids=lambda n: "x".join(map(str, n)))
+def test_energies_modal_form(oracle, n, unilateral):
+    """Element tiles that are full, have one element or end in a ragged layer
+    group, on both sides of the layer-group switch; AT1 and AT2."""
+    # per-cell sums of 27 terms of order one operation each, 1e-12 as for the
+    # other diagnostics; signed totals against the sum of their magnitudes
+    for atnum in (1, 2):
+        s = S.make(n=n, l=(1.0, 2.3, 0.6), seed=sum(n) + atnum, nu=0.3, atnum=atnum, unilateral=unilateral)
+        s["theta"] = s["theta"] + 50.0
+        op, F = S.to_oracle(oracle, s)
+        P = S.to_gpu(s)
+        ref = oracle.energy_fields(op, F, s["U"], s["V"])
+        ef = P.energy_fields(s["U"], s["V"])
+        for c in range(3):
+            assert np.abs(ef[:, c] - ref[:, c]).max() <= 1e-12 * np.abs(ref[:, c]).max(), c
+        el, _, pw, se = P.energies(s["U"], s["V"])
+        for got, r in zip((el, pw, se), ref.T):
+            assert abs(got - r.sum()) <= 1e-12 * np.abs(r).sum()
+        vol, cf = P.VolumetricCrackOpening(s["U"], s["V"], cellfield=True)
+        rvol, rcf = oracle.crack_volume(op, s["U"], s["V"], cellfield=True)
+        assert np.abs(cf - rcf).max() <= 1e-12 * np.abs(rcf).max()
+        assert abs(vol - rvol) <= 1e-12 * np.abs(rcf).mean() * np.prod(s["l"])
+        P.close()

@@ -463,8 +463,9 @@ int vfg_vec_apply_dirichlet(vfg_handle *h, int which, double *vec, const double 
 }
 
 // ------------------------------------------------------------- diagnostics
+// volume_only: out[3] (and cellfield) alone
 static int energies_(vfg_handle *h, const double *U, const double *V, double *cellfield, double *efield,
-                     double out[4], int loc) {
+                     double out[4], int loc, bool volume_only = false) {
   DevProblem &P = h->P;
   int rc;
   int nb = energy_blocks(P);
@@ -482,7 +483,8 @@ static int energies_(vfg_handle *h, const double *U, const double *V, double *ce
     dcell = cellfield ? h->stage + 4 * P.nn : nullptr;
     deng = efield ? h->stage + 4 * P.nn + P.ne : nullptr;
   }
-  launch_energies(P, dU, dV, part, dcell, deng, h->scal, h->stream);
+  if (volume_only) launch_crack_volume(P, dU, dV, part, dcell, h->scal + 3, h->stream);
+  else launch_energies(P, dU, dV, part, dcell, deng, h->scal, h->stream);
   HIPCHK(h, hipMemcpyAsync(out, h->scal, 32, hipMemcpyDeviceToHost, h->stream));
   if (loc == VFG_HOST && cellfield)
     HIPCHK(h, hipMemcpyAsync(cellfield, dcell, 8 * P.ne, hipMemcpyDeviceToHost, h->stream));
@@ -508,7 +510,7 @@ int vfg_crack_volume(vfg_handle *h, const double *U, const double *V, double *vo
   NEED_H(h);
   if (!U || !V || !vol) return vfg_fail(h, VFG_E_ARG, "vfg_crack_volume: NULL array");
   double r[4];
-  int rc = energies_(h, U, V, cellfield, nullptr, r, loc);
+  int rc = energies_(h, U, V, cellfield, nullptr, r, loc, true);
   if (rc) return rc;
   *vol = r[3];
   return VFG_OK;

@@ -124,6 +124,9 @@ void launch_vec_apply_dirichlet(const DevProblem &P, int which, double *vec, con
 int energy_blocks(const DevProblem &P);
 void launch_energies(const DevProblem &P, const double *U, const double *V, double *partials,
                      double *cellfield, double *efield, double *result4, hipStream_t s);
+// crack volume alone (one partial per block of energy_blocks)
+void launch_crack_volume(const DevProblem &P, const double *U, const double *V, double *partials, double *cellfield,
+                         double *result, hipStream_t s);
 // geometric multigrid pieces (vfg_mg.hip)
 void launch_mg_elem_coef(const DevProblem &P, double *out, hipStream_t s);
 void launch_mg_coarsen(const Grid &Gf, const double *cf, const Grid &Gc, double *cc, hipStream_t s);
