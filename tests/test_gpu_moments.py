@@ -69,3 +69,19 @@ def test_energies_modal_form(oracle, n, unilateral):
         assert np.abs(cf - rcf).max() <= 1e-12 * np.abs(rcf).max()
         assert abs(vol - rvol) <= 1e-12 * np.abs(rcf).mean() * np.prod(s["l"])
         P.close()
+
+
+@pytest.mark.parametrize("pressurize", [True, False], ids=["pressure", "dry"])
+@pytest.mark.parametrize("n", [(2, 2, 2), (15, 9, 4), (16, 31, 3), (23, 16, 5), (61, 30, 3)], ids=lambda n: "x".join(map(str, n)))
+def test_u_loads_moment_form(oracle, n, pressurize):
+    # b sums 8 elements of some 30 terms each, the residual about 900 products
+    # more: 900 eps = 2e-13, 1e-12 as for the other operators
+    s = S.make(n=n, l=(1.0, 2.3, 0.6), seed=5 * sum(n), nu=0.3, bcU=S.MIXED_U, pressurize=pressurize, alpha=1e-3)
+    op, F = S.to_oracle(oracle, s)
+    P = S.to_gpu(s)
+    b, ref = P.u_rhs(), oracle.u_rhs(op, F)
+    assert np.abs(b - ref).max() <= 1e-12 * np.abs(ref).max()
+    U, BCU = s["U"], 0.3 * s["x"]
+    r, rref = P.VF_UResidual(U, BCU), oracle.u_residual(op, F, U, BCU)
+    assert np.abs(r - rref).max() <= 1e-12 * np.abs(rref).max()
+    P.close()

@@ -109,36 +109,6 @@ int energy_blocks(const DevProblem &P) {
   return (int)(g.x * g.y * g.z);
 }
 
-// the modal sums of the corner values cv(a), derivatives from nodal differences
-template <typename CV>
-__device__ __forceinline__ void modal_sums(const CV &cv, double (&m)[8]) {
-  double f[2][5];  // per face: first corner, and of the differences to it the sum, x, y, twist
-#pragma unroll
-  for (int k = 0; k < 2; k++) {
-    const double x0 = cv(k * 4), b = cv(k * 4 + 1) - x0, e = cv(k * 4 + 2) - x0, d = cv(k * 4 + 3) - x0, t = d - e;
-    f[k][0] = x0;
-    f[k][2] = t + b;
-    f[k][4] = t - b;
-    f[k][3] = 2. * d - f[k][2];
-    f[k][1] = 2. * d - f[k][4];
-  }
-  m[0] = 4. * (f[0][0] + f[1][0]) + (f[0][1] + f[1][1]);
-  m[4] = 4. * (f[1][0] - f[0][0]) + (f[1][1] - f[0][1]);
-#pragma unroll
-  for (int q = 1; q < 4; q++) {
-    m[q] = f[1][q + 1] + f[0][q + 1];
-    m[q + 4] = f[1][q + 1] - f[0][q + 1];
-  }
-}
-// modal index with power t of variable d and powers b, c of the two others
-constexpr int modal_at(int d, int t, int b, int c) {
-  const int o1 = d == 0 ? 1 : 0, o2 = d == 2 ? 1 : 2;
-  return t << d | b << o1 | c << o2;
-}
-constexpr double gX(int g) { return (g - 1) * VFG_SQ35; }  // Gauss point of [-1, 1]
-// a + b x at Gauss point g
-__device__ __forceinline__ double at_gauss(int g, double a, double b) { return g == 1 ? a : a + gX(g) * b; }
-
 // the operators' constants, formed once on the host (kernel arguments sit in
 // scalar registers; formed in the kernel they take vector ones)
 struct EnergyConst {

@@ -15,6 +15,53 @@ namespace vfg {
 // modal index i = a + 2 b + 4 c of xi^a eta^b zeta^c: power of variable d
 constexpr int um_pow(int i, int d) { return (i >> d) & 1; }
 
+// the modal sums of the corner values cv(a), derivatives from nodal differences
+template <typename CV>
+__device__ __forceinline__ void modal_sums(const CV &cv, double (&m)[8]) {
+  double f[2][5];  // per face: first corner, and of the differences to it the sum, x, y, twist
+#pragma unroll
+  for (int k = 0; k < 2; k++) {
+    const double x0 = cv(k * 4), b = cv(k * 4 + 1) - x0, e = cv(k * 4 + 2) - x0, d = cv(k * 4 + 3) - x0, t = d - e;
+    f[k][0] = x0;
+    f[k][2] = t + b;
+    f[k][4] = t - b;
+    f[k][3] = 2. * d - f[k][2];
+    f[k][1] = 2. * d - f[k][4];
+  }
+  m[0] = 4. * (f[0][0] + f[1][0]) + (f[0][1] + f[1][1]);
+  m[4] = 4. * (f[1][0] - f[0][0]) + (f[1][1] - f[0][1]);
+#pragma unroll
+  for (int q = 1; q < 4; q++) {
+    m[q] = f[1][q + 1] + f[0][q + 1];
+    m[q + 4] = f[1][q + 1] - f[0][q + 1];
+  }
+}
+// modal index with power t of variable d and powers b, c of the two others
+constexpr int modal_at(int d, int t, int b, int c) {
+  const int o1 = d == 0 ? 1 : 0, o2 = d == 2 ? 1 : 2;
+  return t << d | b << o1 | c << o2;
+}
+constexpr double gX(int g) { return (g - 1) * VFG_SQ35; }  // Gauss point of [-1, 1]
+// a + b x at Gauss point g
+__device__ __forceinline__ double at_gauss(int g, double a, double b) { return g == 1 ? a : a + gX(g) * b; }
+// the averages of P D x^a y^b over the square, a, b <= 1, of two bilinear
+// functions given by their coefficients, each still to be divided by 3^(a + b)
+__device__ __forceinline__ void bilinear_moments(const double (&P)[2][2], const double (&D)[2][2], double (&M)[2][2]) {
+  double c[2][2][2];  // [power of x][power of y in P][in D]
+#pragma unroll
+  for (int b = 0; b < 2; b++)
+#pragma unroll
+    for (int e = 0; e < 2; e++) {
+      c[0][b][e] = P[0][b] * D[0][e] + (1. / 3.) * (P[1][b] * D[1][e]);
+      c[1][b][e] = P[0][b] * D[1][e] + P[1][b] * D[0][e];
+    }
+#pragma unroll
+  for (int a = 0; a < 2; a++) {
+    M[a][0] = c[a][0][0] + (1. / 3.) * c[a][1][1];
+    M[a][1] = c[a][0][1] + c[a][1][0];
+  }
+}
+
 // tile-blocked coefficients: [tile][element layer][coefficient][16 x 16 slots];
 // a wavefront reads each coefficient as one aligned 512-byte segment, halo
 // elements are stored in every tile that computes them

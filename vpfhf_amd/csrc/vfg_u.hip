@@ -20,18 +20,19 @@
 
 namespace vfg {
 
-// Apply of one element: xin holds (x0,x1,x2,v) at the 8 corners.
-// cE = E_e * hx*hy*hz; lam1/mu1 are the Lame constants for E = 1.
-// The gradients are carried pre-scaled by mu (H' = mu H), so that
+// Apply of one element under UNILATERAL_NOCOMPRESSION (VFMech.c:299-376): X
+// holds (x0,x1,x2,v) at the 8 corners, cE = E_e * hx*hy*hz, lam1/mu1 are the
+// Lame constants for E = 1.  The gradients are carried pre-scaled by mu
+// (H' = mu H), so that
 //   sigma / (W s cE) = lr tr(H') I + H' + H'^T,  lr = lam / mu,
-// and each stress entry is accumulated with one FMA by its weight W s cE.
-// UNI (UNILATERAL_NOCOMPRESSION, VFMech.c:299-376): at the Gauss points set in
-// cm the spherical part keeps kappa (1 + eta) instead of kappa s, i.e.
+// and each stress entry is accumulated with one FMA by its weight W s cE; at
+// the Gauss points set in cm the spherical part keeps kappa (1 + eta) instead
+// of kappa s, i.e.
 //   sigma / (W cE) = (kr - 2 s / 3) tr(H') I + s (H' + H'^T),
 //   kr = kappa (1 + eta) / mu = (lr + 2/3)(1 + eta).
-template <typename T, bool UNI = false>
+template <typename T>
 __device__ __forceinline__ void u_elem_apply(const T (&X)[2][4][4], T cE, T lam1, T mu1, T eta,
-                                             T ihx, T ihy, T ihz, T (&r)[8][3], uint32_t cm = 0u) {
+                                             T ihx, T ihy, T ihz, T (&r)[8][3], uint32_t cm) {
   const T lr = lam1 / mu1;
   const T kr = (lr + T(2. / 3.)) * (T(1) + eta);
   const T mx = mu1 * ihx, my = mu1 * ihy, mz = mu1 * ihz;
@@ -117,21 +118,13 @@ __device__ __forceinline__ void u_elem_apply(const T (&X)[2][4][4], T cE, T lam1
         const T H10 = Gx[1][gy], H11 = Gy[1][gx], H12 = Gz[1][gy][gx];
         const T H20 = Gx[2][gy], H21 = Gy[2][gx], H22 = Gz[2][gy][gx];
         const T t01 = H01 + H10, t02 = H02 + H20, t12 = H12 + H21;
-        if constexpr (UNI) {
-          const bool comp = (cm >> ((gz * 3 + gy) * 3 + gx)) & 1u;
-          const T lw = comp ? wq * (kr - T(2. / 3.) * (v * v + eta)) : cq * lr;
-          const T L = lw * (H00 + H11 + H22);
-          const T c2 = cq + cq;
-          Sx[0][gy] += L + c2 * H00; Sx[1][gy] += cq * t01; Sx[2][gy] += cq * t02;
-          Sy[0][gx] += cq * t01; Sy[1][gx] += L + c2 * H11; Sy[2][gx] += cq * t12;
-          Sz[0][gy][gx] += cq * t02; Sz[1][gy][gx] += cq * t12; Sz[2][gy][gx] += L + c2 * H22;
-        } else {
-          const T lt = lr * (H00 + H11 + H22);
-          const T t00 = lt + T(2) * H00, t11 = lt + T(2) * H11, t22 = lt + T(2) * H22;
-          Sx[0][gy] += cq * t00; Sx[1][gy] += cq * t01; Sx[2][gy] += cq * t02;
-          Sy[0][gx] += cq * t01; Sy[1][gx] += cq * t11; Sy[2][gx] += cq * t12;
-          Sz[0][gy][gx] += cq * t02; Sz[1][gy][gx] += cq * t12; Sz[2][gy][gx] += cq * t22;
-        }
+        const bool comp = (cm >> ((gz * 3 + gy) * 3 + gx)) & 1u;
+        const T lw = comp ? wq * (kr - T(2. / 3.) * (v * v + eta)) : cq * lr;
+        const T L = lw * (H00 + H11 + H22);
+        const T c2 = cq + cq;
+        Sx[0][gy] += L + c2 * H00; Sx[1][gy] += cq * t01; Sx[2][gy] += cq * t02;
+        Sy[0][gx] += cq * t01; Sy[1][gx] += L + c2 * H11; Sy[2][gx] += cq * t12;
+        Sz[0][gy][gx] += cq * t02; Sz[1][gy][gx] += cq * t12; Sz[2][gy][gx] += L + c2 * H22;
       }
     }
     const T pz0 = T(gP0(gz)), pz1 = T(gP1(gz));
@@ -355,7 +348,7 @@ struct UApplyUniOp {
     return UAuxM<T>{E_elem ? T(E_elem[c]) : E, cmask[c]};
   }
   __device__ void element(int, int, int, const T (&xin)[2][4][4], UAuxM<T> a, T (&r)[8][3]) const {
-    u_elem_apply<T, true>(xin, a.E * vol, lam1, mu1, eta, ihx, ihy, ihz, r, a.m);
+    u_elem_apply<T>(xin, a.E * vol, lam1, mu1, eta, ihx, ihy, ihz, r, a.m);
   }
   __device__ void store(int i, int j, int k, const T (&acc)[3], const T (&own)[4]) const {
     int64_t n = node_id(G, i, j, k);
@@ -754,7 +747,6 @@ __global__ __launch_bounds__(256) void k_u_diag(UDiagOp op, int OZ) { march<doub
 // pressure term cp grad(v) (times N_a), both scaled by sgn, added into r.
 // The fields are interpolated along x first, and the projection is contracted
 // over gx, then gy, then added per gz.
-template <bool UNI>
 __device__ __forceinline__ void rhs_loads(const double (&X)[2][4][6], double coefalpha, double beta, double eta,
                                           double vol, bool crack, const double (&ih)[3], uint32_t cm, double sgn,
                                           double (&r)[8][3]) {
@@ -800,7 +792,7 @@ __device__ __forceinline__ void rhs_loads(const double (&X)[2][4][6], double coe
         const double gvz = ih[2] * (gP0(gy) * (f1[0][1][0][gx] - f1[0][0][0][gx]) +
                                     gP1(gy) * (f1[0][1][1][gx] - f1[0][0][1][gx]));
         const double W = vol * gW(gx) * gW(gy) * gW(gz);
-        const bool comp = UNI && ((cm >> ((gz * 3 + gy) * 3 + gx)) & 1u);  // VFMech.c:505-513
+        const bool comp = (cm >> ((gz * 3 + gy) * 3 + gx)) & 1u;  // VFMech.c:505-513
         const double tp = sgn * (comp ? W * (coefalpha * th * (1. + eta) + beta * pr)
                                       : W * (coefalpha * th * (vv * vv + eta) + beta * pr * vv));
         const double cp = crack ? sgn * W * pr : 0.;
@@ -849,7 +841,8 @@ __device__ __forceinline__ void rhs_loads(const double (&X)[2][4][6], double coe
   }
 }
 
-template <bool UNI>
+// residual and loads under UNILATERAL_NOCOMPRESSION in one pass: both follow
+// the branch of every Gauss point
 struct URhsOp {
   static constexpr int NF = 6, NC = 3;  // u0,u1,u2,v,dth,p
   const double *U, *v, *dth, *p, *BCU;
@@ -868,24 +861,21 @@ struct URhsOp {
     double Ee = E_elem ? E_elem[cell_id(G, ex, ey, ek)] : E;
     double lam = lam1 * Ee, mu = mu1 * Ee;
     const double ih[3] = {1. / G.hx, 1. / G.hy, 1. / G.hz};
-    // UNILATERAL_NOCOMPRESSION: the branch of every Gauss point follows U itself
-    // (VFMech.c:1566-1615: VF_UResidual evaluates both terms at the iterate)
-    uint32_t cm = 0u;
-    if constexpr (UNI) {
-      double u[8][3];
-      for (int a = 0; a < 8; a++)
-        for (int c = 0; c < 3; c++) u[a][c] = X[a >> 2][a & 3][c];
-      cm = compression_mask(u, ih[0], ih[1], ih[2]);
-    }
+    // the branch of every Gauss point follows U itself (VFMech.c:1566-1615:
+    // VF_UResidual evaluates both terms at the iterate)
+    double u[8][3];
+    for (int a = 0; a < 8; a++)
+      for (int c = 0; c < 3; c++) u[a][c] = X[a >> 2][a & 3][c];
+    const uint32_t cm = compression_mask(u, ih[0], ih[1], ih[2]);
     if (mode == 1) {
       double Xa[2][4][4];
       for (int k = 0; k < 2; k++)
         for (int q = 0; q < 4; q++)
           for (int f = 0; f < 4; f++) Xa[k][q][f] = X[k][q][f];
-      u_elem_apply<double, UNI>(Xa, Ee * vol, lam1, mu1, eta, ih[0], ih[1], ih[2], r, cm);
+      u_elem_apply<double>(Xa, Ee * vol, lam1, mu1, eta, ih[0], ih[1], ih[2], r, cm);
     }
     const double coefalpha = (3. * lam + 2. * mu) * alpha;
-    rhs_loads<UNI>(X, coefalpha, beta, eta, vol, crack != 0, ih, cm, mode == 1 ? -1. : 1., r);
+    rhs_loads(X, coefalpha, beta, eta, vol, crack != 0, ih, cm, mode == 1 ? -1. : 1., r);
   }
   // value written by ResidualApplyDirichletBC: traversal order X0..Z1 then
   // vertices, later writers win (VFCartFE.c:747-999)
@@ -910,119 +900,25 @@ struct URhsOp {
   }
 };
 
-// Load vector of one element under UNILATERAL_NONE, sum-factorised over two
-// Gauss-point walks (values of v, dth, p; then v with its gradient and p,
-// kept apart so that each walk's accumulators fit the registers of two waves
-// per SIMD):
-//   thermo-poro (VFMech.c:386-447): b[a][c] += sum_g W d_c phi_a T,
-//     T = (3 lam + 2 mu) alpha dth (v^2 + eta) + beta p v  -- the x-, y- and
-//     z-derivative projections of one scalar: T summed over gx per (gy, gz),
-//     over gy per (gx, gz), over gz per (gx, gy);
-//   crack pressure (VFMech.c:533-589): b[a][c] += sum_g W p (d_c v) phi_a --
-//     a value projection, summed over gx, then gy, then gz.
-// Every contribution is multiplied by sgn (-1 for the residual).
-template <typename CV>
-__device__ __forceinline__ void u_loads_elem(const CV &cv, double coefalpha, double beta, double eta,
-                                             double vol, bool crack, double ihx, double ihy, double ihz, double sgn,
-                                             double (&r)[8][3]) {
-  // thermo-poro: values of v, dth, p (fields 0-2)
-  {
-    double Tx = 0., Ty[3] = {0., 0., 0.}, Tz[3][3], Rx[2][2] = {{0., 0.}, {0., 0.}}, Ry[2][2] = {{0., 0.}, {0., 0.}};
-#pragma unroll
-    for (int q = 0; q < 3; q++)
-#pragma unroll
-      for (int w = 0; w < 3; w++) Tz[q][w] = 0.;
-    gauss_walk_cv<0, 3>(cv, ihx, ihy, ihz, [&](int gx, int gy, int gz, const double (&val)[3], const double (&)[1][3]) {
-      const double W = vol * gW(gx) * gW(gy) * gW(gz);
-      const double v = val[0];
-      const double T = sgn * (W * (coefalpha * val[1] * (v * v + eta) + beta * val[2] * v));
-      Tx += T;
-      Ty[gx] += T;
-      Tz[gy][gx] += T;
-      if (gx == 2) {  // end of a row (gy, gz)
-#pragma unroll
-        for (int k = 0; k < 2; k++)
-#pragma unroll
-          for (int j = 0; j < 2; j++) Rx[k][j] += (k ? gP1(gz) : gP0(gz)) * (j ? gP1(gy) : gP0(gy)) * Tx;
-        Tx = 0.;
-      }
-      if (gx == 2 && gy == 2) {  // end of a layer gz
-#pragma unroll
-        for (int q = 0; q < 3; q++) {
-#pragma unroll
-          for (int k = 0; k < 2; k++)
-#pragma unroll
-            for (int i = 0; i < 2; i++) Ry[k][i] += (k ? gP1(gz) : gP0(gz)) * (i ? gP1(q) : gP0(q)) * Ty[q];
-          Ty[q] = 0.;
-        }
-      }
-    });
-#pragma unroll
-    for (int a = 0; a < 8; a++) {
-      const int i = a & 1, j = (a >> 1) & 1, k = a >> 2;
-      double rz = 0.;
-#pragma unroll
-      for (int gy = 0; gy < 3; gy++)
-#pragma unroll
-        for (int gx = 0; gx < 3; gx++) rz += (j ? gP1(gy) : gP0(gy)) * (i ? gP1(gx) : gP0(gx)) * Tz[gy][gx];
-      r[a][0] += (i ? ihx : -ihx) * Rx[k][j];
-      r[a][1] += (j ? ihy : -ihy) * Ry[k][i];
-      r[a][2] += (k ? ihz : -ihz) * rz;
-    }
-  }
-  if (!crack) return;
-  // crack pressure: v with its gradient (field 0) and p (field 2); the value
-  // projection summed over gx (Vx), gy (Vy), then gz straight into r
-  double Vx[3][2], Vy[3][2][2];
-#pragma unroll
-  for (int c = 0; c < 3; c++)
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-      Vx[c][i] = 0.;
-#pragma unroll
-      for (int j = 0; j < 2; j++) Vy[c][j][i] = 0.;
-    }
-  gauss_walk_cv<1, 1>([&](int q, int a) { return cv(q ? 2 : 0, a); }, ihx, ihy, ihz,
-                      [&](int gx, int gy, int gz, const double (&val)[2], const double (&gv)[1][3]) {
-    const double cp = sgn * (vol * gW(gx) * gW(gy) * gW(gz)) * val[1];
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-      const double Gc = cp * gv[0][c];
-      Vx[c][0] += gP0(gx) * Gc;
-      Vx[c][1] += gP1(gx) * Gc;
-    }
-    if (gx == 2) {  // end of a row (gy, gz)
-#pragma unroll
-      for (int c = 0; c < 3; c++)
-#pragma unroll
-        for (int i = 0; i < 2; i++) {
-          Vy[c][0][i] += gP0(gy) * Vx[c][i];
-          Vy[c][1][i] += gP1(gy) * Vx[c][i];
-          Vx[c][i] = 0.;
-        }
-    }
-    if (gx == 2 && gy == 2) {  // end of a layer gz: into the corners (j, i) of both node planes
-#pragma unroll
-      for (int c = 0; c < 3; c++)
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-          for (int i = 0; i < 2; i++) {
-            r[(0 * 2 + j) * 2 + i][c] += gP0(gz) * Vy[c][j][i];
-            r[(1 * 2 + j) * 2 + i][c] += gP1(gz) * Vy[c][j][i];
-            Vy[c][j][i] = 0.;
-          }
-    }
-  });
-}
-
 // The load vector alone (UNILATERAL_NONE: the loads do not depend on U):
 // mode 0 stores b; mode 1 finishes the residual F = K U - b over an output
 // that already holds K U (the FP64 apply), and writes the Dirichlet rows'
 // ResidualApplyDirichletBC values from U (read there only); mode 2 stores b
 // with the Dirichlet rows' targets instead, so that F(U) = A U - b for the
 // MatShell operator A.
+//
+// With R the modal duals of the nodal loads (x mono = the monomial of a mode):
+//   thermo-poro (VFMech.c:386-447): R_d,i = vol / (4 h_d) <T mono_i / x_d> for
+//     the modes i with variable d, T = (3 lam + 2 mu) alpha dth (v^2 + eta) +
+//     beta p v: 7 moments of T, summed over its 27 Gauss points;
+//   crack pressure (VFMech.c:533-589): R_d,i = vol / 8 <p (d_d v) mono_i>, in
+//     closed form (d_d v does not depend on x_d).
+// Bound by issue, about 500 FP64 operations per element against 1300 of two
+// walks over the Gauss points into the corners: 101 x 88 x 95 in 45 us (first
+// touch), 72 us so; in small grids apply + loads 27 us against 47 us of both
+// in one spilling kernel.
 struct ULoadsOp {
+  using T = double;
   static constexpr int NF = 3, NC = 3;  // v, dth, p
   const double *U, *v, *dth, *p, *BCU;
   double *out;
@@ -1031,58 +927,169 @@ struct ULoadsOp {
   BcMask bc;
   uint8_t ftype[3][6];
   uint8_t vtype[3][8];
-  double E, lam1, mu1, eta, vol, alpha, beta;
+  double E, ca, beta, eta64;  // (3 lam + 2 mu) alpha / 8 for E = 1; eta of 8 v
+  double kt[3][3], kp[3];     // per component: thermo-poro (by odd powers), crack pressure
   int crack, mode;
+  struct Face {
+    double v[5], t[4], p[4];  // v: first corner, then s, x, y, w of the differences to it
+  };
+  struct Own {};
+  using Aux = double;  // E_e
+  using Raw = double;
+  static __device__ double off() { return 0.; }
   __device__ double load(int f, int64_t n) const { return f == 0 ? v[n] : f == 1 ? dth[n] : p[n]; }
-  __device__ double aux(int ex, int ey, int ek) const { return E_elem ? E_elem[cell_id(G, ex, ey, ek)] : E; }
-  __device__ void element(int, int, int, const double (&X)[2][4][3], double Ee, double (&r)[8][3]) const {
-    double fld[3][8];
+  __device__ double stage(int, double x) const { return x; }
+  template <class RD>
+  __device__ void face(const RD &rd, Face &F) const {
+    {
+      const double x0 = rd(0, 0), b = rd(0, 1) - x0, e = rd(0, 2) - x0, d = rd(0, 3) - x0, t = d - e;
+      F.v[0] = x0;
+      F.v[2] = t + b;
+      F.v[4] = t - b;
+      F.v[3] = 2. * d - F.v[2];
+      F.v[1] = 2. * d - F.v[4];
+    }
 #pragma unroll
-    for (int a = 0; a < 8; a++)
-#pragma unroll
-      for (int f = 0; f < 3; f++) fld[f][a] = X[a >> 2][a & 3][f];
-    const double coefalpha = (3. * lam1 + 2. * mu1) * Ee * alpha;
-    u_loads_elem([&](int q, int a) { return fld[q][a]; }, coefalpha, beta, eta, vol, crack != 0, 1. / G.hx,
-                 1. / G.hy, 1. / G.hz, mode == 1 ? -1. : 1., r);
-  }
-  template <typename XS>
-  __device__ void element_lds(int, int, int, const XS &xs, double Ee, double (&r)[8][3]) const {
-    const double coefalpha = (3. * lam1 + 2. * mu1) * Ee * alpha;
-    u_loads_elem([&](int q, int a) { return xs(a >> 2, a & 3, q); }, coefalpha, beta, eta, vol, crack != 0, 1. / G.hx, 1. / G.hy, 1. / G.hz, mode == 1 ? -1. : 1., r);
-  }
-  __device__ void store(int i, int j, int k, const double (&acc)[3], const double (&)[3]) const {
-    const int64_t n = node_id(G, i, j, k);
-    for (int c = 0; c < 3; c++) {
-      double val = acc[c];
-      if (mode == 2 && on_dirichlet(G, bc.face[c], bc.vert[c], i, j, k)) {
-        // the value the residual's Dirichlet row subtracts from U
-        val = dirichlet_value(i, j, k, c, n);
-      } else if (mode == 1) {
-        if (on_dirichlet(G, bc.face[c], bc.vert[c], i, j, k)) val = U[3 * n + c] - dirichlet_value(i, j, k, c, n);
-        else val = out[3 * n + c] + acc[c];  // K U - b
-      }
-      out[3 * n + c] = val;
+    for (int f = 1; f < 3; f++) {
+      double(&o)[4] = f == 1 ? F.t : F.p;
+      const double x0 = rd(f, 0), x1 = rd(f, 1), x2 = rd(f, 2), x3 = rd(f, 3);
+      const double s0 = x0 + x1, s1 = x2 + x3, d0 = x1 - x0, d1 = x3 - x2;
+      o[0] = s0 + s1;
+      o[1] = d0 + d1;
+      o[2] = s1 - s0;
+      o[3] = d1 - d0;
     }
   }
+  __device__ Own own(const Face &) const { return Own{}; }
+  __device__ double aux(int ex, int ey, int ek, int, int) const {
+    return E_elem ? E_elem[cell_id(G, ex, ey, ek)] : E;
+  }
+  __device__ void element(double Ee, const Face &B, const Face &F, double (&tot)[3][4], double (&carry)[3][4]) const {
+    double V[8], Th[8], Pm[8], m[8];
+    V[0] = 4. * (F.v[0] + B.v[0]) + (F.v[1] + B.v[1]);
+    V[4] = 4. * (F.v[0] - B.v[0]) + (F.v[1] - B.v[1]);
+#pragma unroll
+    for (int q = 1; q < 4; q++) {
+      V[q] = F.v[q + 1] + B.v[q + 1];
+      V[q + 4] = F.v[q + 1] - B.v[q + 1];
+    }
+    const double ce = ca * Ee;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      Th[q] = ce * (F.t[q] + B.t[q]);
+      Th[q + 4] = ce * (F.t[q] - B.t[q]);
+      Pm[q] = F.p[q] + B.p[q];
+      Pm[q + 4] = F.p[q] - B.p[q];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; i++) m[i] = 0.;  // moments of 64 T; the common weight is in kt
+#pragma unroll
+    for (int gz = 0; gz < 3; gz++) {
+      double f[3][4], L[4] = {0., 0., 0., 0.};
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        f[0][q] = at_gauss(gz, V[q], V[q + 4]);
+        f[1][q] = at_gauss(gz, Th[q], Th[q + 4]);
+        f[2][q] = beta * at_gauss(gz, Pm[q], Pm[q + 4]);
+      }
+#pragma unroll
+      for (int gy = 0; gy < 3; gy++) {
+        double t[3], r[3][2];
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+          r[c][0] = at_gauss(gy, f[c][0], f[c][2]);
+          r[c][1] = at_gauss(gy, f[c][1], f[c][3]);
+        }
+#pragma unroll
+        for (int gx = 0; gx < 3; gx++) {
+          const double vg = at_gauss(gx, r[0][0], r[0][1]);
+          t[gx] = at_gauss(gx, r[1][0], r[1][1]) * (vg * vg + eta64) + at_gauss(gx, r[2][0], r[2][1]) * vg;
+        }
+        const double s = (t[0] + t[2]) + 1.6 * t[1], o = t[2] - t[0];  // weights 5 : 8 : 5
+        L[0] += gy == 1 ? 1.6 * s : s;
+        L[1] += gy == 1 ? 1.6 * o : o;
+        if (gy != 1) {
+          L[2] += gy ? s : -s;
+          L[3] += gy ? o : -o;
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        m[q] += gz == 1 ? 1.6 * L[q] : L[q];
+        if (gz != 1 && q < 3) m[q + 4] += gz ? L[q] : -L[q];
+      }
+    }
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+      double R[8];
+#pragma unroll
+      for (int i = 0; i < 8; i++)
+        R[i] = um_pow(i, d) ? kt[d][__builtin_popcount(i) - 1] * m[i & ~(1 << d)] : 0.;
+      if (crack) {
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+          double p2[2][2], v2[2][2], M[2][2];
+#pragma unroll
+          for (int q = 0; q < 4; q++) {
+            p2[q & 1][q >> 1] = Pm[modal_at(d, t, q & 1, q >> 1)];
+            v2[q & 1][q >> 1] = kp[d] * V[modal_at(d, 1, q & 1, q >> 1)];
+          }
+          bilinear_moments(p2, v2, M);
+#pragma unroll
+          for (int q = 0; q < 4; q++) {
+            const int o = t + (q & 1) + (q >> 1);
+            R[modal_at(d, t, q & 1, q >> 1)] +=
+                (o == 0 ? 1. : o == 1 ? 1. / 3. : o == 2 ? 1. / 9. : 1. / 27.) * M[q & 1][q >> 1];
+          }
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        tot[d][q] += R[q] - R[q + 4];
+        carry[d][q] = R[q] + R[q + 4];
+      }
+    }
+  }
+  struct OwnKU {
+    double f[3];
+  };
+  __device__ OwnKU own_load(int64_t n) const {
+    OwnKU o{};
+    if (mode == 1)
+#pragma unroll
+      for (int c = 0; c < 3; c++) o.f[c] = out[3 * n + c];
+    return o;
+  }
+  __device__ void store(int64_t n, uint32_t fb, const double (&acc)[3], const Own &, const OwnKU &o) const {
+    double val[3];
+#pragma unroll
+    for (int c = 0; c < 3; c++) val[c] = o.f[c] + acc[c];  // mode 1: K U - b
+    if (mode != 0 && fb) {
+#pragma unroll
+      for (int c = 0; c < 3; c++)
+        if (face_dirichlet(bc.face[c], bc.vert[c], fb)) {
+          const double w = dirichlet_value(fb, c, n);
+          val[c] = mode == 1 ? U[3 * n + c] - w : w;
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < 3; c++) out[3 * n + c] = val[c];
+  }
   // ResidualApplyDirichletBC's target on a Dirichlet row: BCU (type 3), 1 (type 2), else 0
-  __device__ double dirichlet_value(int i, int j, int k, int c, int64_t n) const {
+  __device__ double dirichlet_value(uint32_t fb, int c, int64_t n) const {
     int t = 0;
-    const bool onf[6] = {i == 0, i == G.nx - 1, j == 0, j == G.ny - 1, k == 0, k == G.nz - 1};
     for (int f = 0; f < 6; f++)
-      if (ftype[c][f] && onf[f]) t = ftype[c][f];
-    const int ix = (i == 0) ? 0 : (i == G.nx - 1) ? 1 : -1;
-    const int iy = (j == 0) ? 0 : (j == G.ny - 1) ? 1 : -1;
-    const int iz = (k == 0) ? 0 : (k == G.nz - 1) ? 1 : -1;
-    if (ix >= 0 && iy >= 0 && iz >= 0 && vtype[c][ix + 2 * iy + 4 * iz]) t = vtype[c][ix + 2 * iy + 4 * iz];
+      if (ftype[c][f] && (fb >> f & 1u)) t = ftype[c][f];
+    const int q = face_vertex(fb);
+    if (q >= 0 && vtype[c][q]) t = vtype[c][q];
     return t == 3 ? BCU[3 * n + c] : t == 2 ? 1. : 0.;
   }
 };
 __global__ __launch_bounds__(256, 2) void k_u_loads(ULoadsOp op, int OZ) {
-  march_lds<double, 16, 16, false>(op.G, op, OZ, xcd_block());
+  march_modal<16, 16>(op.G, op, OZ, xcd_block());
 }
 
-template <bool UNI>
-__global__ __launch_bounds__(256) void k_u_rhs(URhsOp<UNI> op, int OZ) {
+__global__ __launch_bounds__(256) void k_u_rhs(URhsOp op, int OZ) {
   march<double, 16, 16>(op.G, op, OZ, xcd_block());
 }
 
@@ -1467,10 +1474,9 @@ void launch_u_diag(const DevProblem &P, double *d, hipStream_t s) {
   hipLaunchKernelGGL(k_u_diag, march_grid(P.G, 16, 16, OZ), dim3(256), 0, s, op, OZ);
 }
 
-template <bool UNI>
-static void launch_u_rhs_t(const DevProblem &P, const double *U, const double *BCU, double *out, int mode,
-                           hipStream_t s) {
-  URhsOp<UNI> op;
+static void launch_u_rhs_uni(const DevProblem &P, const double *U, const double *BCU, double *out, int mode,
+                             hipStream_t s) {
+  URhsOp op;
   op.U = U ? U : P.zero3; op.v = P.V; op.dth = P.dth; op.p = P.p; op.BCU = BCU;
   op.out = out; op.E_elem = P.E_elem; op.G = P.G; op.bc = P.bcU;
   for (int c = 0; c < 3; c++) {
@@ -1481,21 +1487,15 @@ static void launch_u_rhs_t(const DevProblem &P, const double *U, const double *B
   op.vol = P.G.hx * P.G.hy * P.G.hz; op.alpha = P.alpha; op.beta = P.beta;
   op.crack = P.hasCrackPressure; op.mode = mode;
   int tiles = ((P.G.nx + 14) / 15) * ((P.G.ny + 14) / 15);
-  static int slots = device_slots(k_u_rhs<UNI>, 256);
+  static int slots = device_slots(k_u_rhs, 256);
   int OZ = choose_oz(P.G, tiles, slots);
-  hipLaunchKernelGGL(k_u_rhs<UNI>, march_grid(P.G, 16, 16, OZ), dim3(256), 0, s, op, OZ);
+  hipLaunchKernelGGL(k_u_rhs, march_grid(P.G, 16, 16, OZ), dim3(256), 0, s, op, OZ);
 }
 
 void launch_u_rhs(const DevProblem &P, const double *U, const double *BCU, double *out, int mode,
                   hipStream_t s) {
   if (P.unilateral) {  // (mode 2 is not used with NOCOMPRESSION: its load depends on U)
-    launch_u_rhs_t<true>(P, U, BCU, out, mode, s);
-    return;
-  }
-  // small grids (ensemble members, served requests): the apply and the loads
-  // in one launch, which is latency-bound there
-  if (mode != 2 && P.nn < (1 << 19)) {
-    launch_u_rhs_t<false>(P, U, BCU, out, mode, s);
+    launch_u_rhs_uni(P, U, BCU, out, mode, s);
     return;
   }
   // UNILATERAL_NONE: K U by the FP64 apply, then the loads
@@ -1507,9 +1507,17 @@ void launch_u_rhs(const DevProblem &P, const double *U, const double *BCU, doubl
     for (int f = 0; f < 6; f++) op.ftype[c][f] = (uint8_t)P.hbcU[c].face[f];
     for (int v = 0; v < 8; v++) op.vtype[c][v] = (uint8_t)P.hbcU[c].vertex[v];
   }
-  op.E = P.E; op.lam1 = P.lam1; op.mu1 = P.mu1; op.eta = P.eta;
-  op.vol = P.G.hx * P.G.hy * P.G.hz; op.alpha = P.alpha; op.beta = P.beta;
+  op.E = P.E; op.beta = P.beta; op.eta64 = 64. * P.eta;
+  op.ca = (3. * P.lam1 + 2. * P.mu1) * P.alpha / 8.;
   op.crack = P.hasCrackPressure; op.mode = mode;
+  const double h[3] = {P.G.hx, P.G.hy, P.G.hz}, w = (mode == 1 ? -1. : 1.) * h[0] * h[1] * h[2];
+  for (int d = 0; d < 3; d++) {
+    const double k = w / (4. * 64. * h[d]) * (125. / 5832.);  // (5/18)^3
+    op.kt[d][0] = k;
+    op.kt[d][1] = k * VFG_SQ35;
+    op.kt[d][2] = k * .6;
+    op.kp[d] = w / (256. * h[d]);
+  }
   const int tiles = ((P.G.nx + 14) / 15) * ((P.G.ny + 14) / 15);
   static int slots = device_slots(k_u_loads, 256);
   const int OZ = choose_oz(P.G, tiles, slots);
