@@ -85,3 +85,21 @@ def test_u_loads_moment_form(oracle, n, pressurize):
     r, rref = P.VF_UResidual(U, BCU), oracle.u_residual(op, F, U, BCU)
     assert np.abs(r - rref).max() <= 1e-12 * np.abs(rref).max()
     P.close()
+
+
+@pytest.mark.parametrize("unilateral", [0, 1], ids=["linear", "nocompression"])
+@pytest.mark.parametrize("n", [(2, 2, 2), (15, 16, 4), (31, 9, 5), (46, 17, 3)], ids=lambda n: "x".join(map(str, n)))
+def test_v_setup_moment_form(oracle, n, unilateral):
+    # energies of 27 points with mixed-sign strains, then 8 x 8 products per
+    # row entry: 1e-12 as for the other operators
+    for atnum in (1, 2):
+        s = S.make(n=n, l=(1.0, 2.3, 0.6), seed=7 * sum(n) + atnum, nu=0.3, atnum=atnum, unilateral=unilateral,
+                   bcV=S.MIXED_V)
+        op, F = S.to_oracle(oracle, s)
+        P = S.to_gpu(s)
+        P.VIJacobian_setup(s["U"])
+        b, rb = P.v_rhs(), oracle.v_rhs(op, F, s["U"])
+        assert np.abs(b - rb).max() <= 1e-12 * np.abs(rb).max()
+        y, ry = P.VIJacobian_mult(s["xv"]), oracle.v_jacobian(op, F, s["U"]) @ s["xv"]
+        assert np.abs(y - ry).max() <= 1e-12 * np.abs(ry).max()
+        P.close()

@@ -40,64 +40,121 @@ static VConst make_vconst(const DevProblem &P) {
 }
 
 // -------------------------------------------------------------- setup: Vq
+// launch constants: strains are formed times 4 hz, so that d_z takes the modal
+// sums as they are
+struct VSetup {
+  double kx, ky;    // hz / hx, hz / hy
+  double kth;       // alpha dtheta of a modal sum, times 4 hz
+  double lam, mu2;  // lam, 2 mu for E = 1, over (4 hz)^2
+  double cm, vol;   // AT2 mass term; vol / 64
+};
+static VSetup make_vsetup(const DevProblem &P) {
+  const Grid &G = P.G;
+  const double s = 16. * G.hz * G.hz;
+  VSetup C;
+  C.kx = G.hz / G.hx;
+  C.ky = G.hz / G.hy;
+  C.kth = P.alpha * G.hz / 2.;
+  C.lam = P.lam1 / s;
+  C.mu2 = 2. * P.mu1 / s;
+  C.cm = P.atnum == 2 ? P.Gc / P.atcv * .5 / P.eps : 0.;
+  C.vol = G.hx * G.hy * G.hz / 64.;
+  return C;
+}
+
 // One block per (tile, element layer), one thread per tile slot: element
 // (15 bx - 1 + tx, 15 by - 1 + ty) of the V operator's tile-blocked layout
 // (halo elements are computed by every tile that holds them), so each
 // coefficient is written as one aligned, contiguous 512-byte segment per
-// wavefront.  Gauss-point values by sum factorisation (gauss_walk); the
-// moments are summed row by row as the walk visits the points.
-__global__ __launch_bounds__(256) void k_v_setup(DevProblem P, const double *__restrict__ U) {
+// wavefront.  The strains at the Gauss points come from the modal sums of the
+// corners; the moments are summed row by row.
+// UNI: UNILATERAL_NOCOMPRESSION (VFMech.c:183-208, 2125-2153), 1/2 sigma(eps -
+// e0) : eps, less kappa tr^2 / 2 where tr(eps) < 0.
+// Bound by issue and the write of the moments, which do not overlap (128^3:
+// about 105 us without the stores, 79 us for a fill of their 515 MB): about 950
+// FP64 operations per element against 2400 interpolating values and gradients
+// at each point; 128^3 187 -> 173 us.  Staging the node planes in LDS over
+// several layers, or storing each third of the moments when complete, is no
+// faster (164 us, and the apply after it loses as much to the caches).
+template <bool UNI>
+__global__ __launch_bounds__(256, 2) void k_v_setup(DevProblem P, VSetup C, const double *__restrict__ U) {
   const Grid &G = P.G;
   const int tid = threadIdx.x;
   const Blk3 b = xcd_block();
   const int ei = b.x * 15 - 1 + tid % 16, ej = b.y * 15 - 1 + tid / 16, ek = b.z;
   const int tile = b.x + gridDim.x * b.y;
-  double *out = P.Vq + tiled_index(tile, ek, G.nez, 27, tid, 0, 256);
+  double *out = P.Vq + tiled_index(tile, ek, G.nez, 27, tid);
   if (ei < 0 || ei >= G.nex || ej < 0 || ej >= G.ney) {
-    for (int g = 0; g < 27; g++) out[g * 256] = 0.;
+    for (int g = 0; g < 27; g++) out[g * 64] = 0.;
     return;
   }
-  const int64_t e = cell_id(G, ei, ej, ek);
-  double fld[4][8];  // u_c (values and gradients), theta - thetaRef (values)
-  for (int a = 0; a < 8; a++) {
-    int64_t n = node_id(G, ei + (a & 1), ej + ((a >> 1) & 1), ek + (a >> 2));
-    for (int c = 0; c < 3; c++) fld[c][a] = U[3 * n + c];
-    fld[3][a] = P.dth[n];
-  }
-  const double Ee = P.E_elem ? P.E_elem[e] : P.E;
-  const double lam = P.lam1 * Ee, mu = P.mu1 * Ee;
-  const double vol = G.hx * G.hy * G.hz / 64.;
-  const double cm = P.atnum == 2 ? P.Gc / P.atcv * .5 / P.eps : 0.;
-  constexpr double X1 = VFG_SQ35, X2 = .6;  // Gauss point +1 and its square (point -1: -X1; the middle one 0)
-  double Q[3][3][3], Y[3][3], row[3];       // [r][q][p]; [q][p] of the layer; the row's points
+  double M[3][8], Th[8];  // modal sums of u_c and of alpha dtheta
+  {
+    double fld[4][8];
 #pragma unroll
-  for (int q = 0; q < 9; q++) {
-    Y[q / 3][q % 3] = 0.;
+    for (int a = 0; a < 8; a++) {
+      const int64_t n = node_id(G, ei + (a & 1), ej + ((a >> 1) & 1), ek + (a >> 2));
+#pragma unroll
+      for (int c = 0; c < 3; c++) fld[c][a] = U[3 * n + c];
+      fld[3][a] = P.dth[n];
+    }
+#pragma unroll
+    for (int c = 0; c < 3; c++) modal_sums([&](int a) { return fld[c][a]; }, M[c]);
+    modal_sums([&](int a) { return fld[3][a]; }, Th);
+  }
+  const double Ee = P.E_elem ? P.E_elem[cell_id(G, ei, ej, ek)] : P.E;
+  const double lam = C.lam * Ee, mu2 = C.mu2 * Ee, kap = lam + mu2 * (1. / 3.);
+#pragma unroll
+  for (int q = 0; q < 8; q++) Th[q] *= C.kth;
+  constexpr double X1 = VFG_SQ35, X2 = .6;  // Gauss point +1 and its square (point -1: -X1; the middle one 0)
+  double Q[3][3][3];                        // [r][q][p]
+#pragma unroll
+  for (int q = 0; q < 9; q++)
 #pragma unroll
     for (int r = 0; r < 3; r++) Q[r][q / 3][q % 3] = 0.;
-  }
-  gauss_walk<3, 1>(fld, 1. / G.hx, 1. / G.hy, 1. / G.hz,
-                   [&](int gx, int gy, int gz, const double (&val)[4], const double (&H)[3][3]) {
-    const double t = val[3];
-    double e11 = H[0][0] - P.alpha * t, e22 = H[1][1] - P.alpha * t, e33 = H[2][2] - P.alpha * t;
-    double e12 = (H[1][0] + H[0][1]) * .5, e23 = (H[2][1] + H[1][2]) * .5, e13 = (H[2][0] + H[0][2]) * .5;
-    double s11 = (lam + 2. * mu) * e11 + lam * e22 + lam * e33;
-    double s22 = lam * e11 + (lam + 2. * mu) * e22 + lam * e33;
-    double s33 = lam * e11 + lam * e22 + (lam + 2. * mu) * e33;
-    double W;
-    if (P.unilateral) {
-      // ElasticEnergyDensitySphericalDeviatoricNoCompression3D_local
-      // (VFMech.c:183-208): 1/2 sigma(eps - e0) : eps, less kappa tr^2 / 2
-      // where tr(eps) < 0 (S + D of VFMech.c:2125-2153)
-      const double tr = (H[0][0] + H[1][1]) + H[2][2];
-      W = (s11 * H[0][0] + s22 * H[1][1] + s33 * H[2][2]) * .5 + 2. * mu * (e12 * e12 + e23 * e23 + e13 * e13);
-      if (tr < 0.) W -= (lam + 2. * mu / 3.) * tr * tr * .5;
-    } else {
-      W = (s11 * e11 + s22 * e22 + s33 * e33) * .5 + 2. * mu * (e12 * e12 + e23 * e23 + e13 * e13);
+#pragma unroll
+  for (int gz = 0; gz < 3; gz++) {
+    double dx[3][2], dy[3][3], th[4], Y[3][3];  // Y: [q][p] of the layer
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+#pragma unroll
+      for (int q = 0; q < 2; q++) dx[c][q] = C.kx * at_gauss(gz, M[c][1 + 2 * q], M[c][5 + 2 * q]);
+      const double y0 = C.ky * at_gauss(gz, M[c][2], M[c][6]), y1 = C.ky * at_gauss(gz, M[c][3], M[c][7]);
+#pragma unroll
+      for (int gx = 0; gx < 3; gx++) dy[c][gx] = at_gauss(gx, y0, y1);
+#pragma unroll
+      for (int p = 0; p < 3; p++) Y[c][p] = 0.;
     }
-    row[gx] = gW(gx) * (cm + 2. * W);
-    if (gx == 2) {  // end of a row (gy, gz)
-      const double S = row[0] + row[2], w = vol * gW(gy) * gW(gz);
+#pragma unroll
+    for (int q = 0; q < 4; q++) th[q] = at_gauss(gz, Th[q], Th[q + 4]);
+#pragma unroll
+    for (int gy = 0; gy < 3; gy++) {
+      double hx[3], z0[3], z1[3], row[3];
+#pragma unroll
+      for (int c = 0; c < 3; c++) {
+        hx[c] = at_gauss(gy, dx[c][0], dx[c][1]);
+        z0[c] = at_gauss(gy, M[c][4], M[c][6]);
+        z1[c] = at_gauss(gy, M[c][5], M[c][7]);
+      }
+      const double th0 = at_gauss(gy, th[0], th[2]), th1 = at_gauss(gy, th[1], th[3]);
+#pragma unroll
+      for (int gx = 0; gx < 3; gx++) {
+        const double t = at_gauss(gx, th0, th1), f11 = hx[0], f22 = dy[1][gx], f33 = at_gauss(gx, z0[2], z1[2]);
+        const double t01 = dy[0][gx] + hx[1], t02 = at_gauss(gx, z0[0], z1[0]) + hx[2],
+                     t12 = at_gauss(gx, z0[1], z1[1]) + dy[2][gx];
+        const double e11 = f11 - t, e22 = f22 - t, e33 = f33 - t, tr = (e11 + e22) + e33;
+        const double sh = .5 * (t01 * t01 + t02 * t02 + t12 * t12);
+        double W2;  // 2 W
+        if constexpr (UNI) {
+          const double trf = (f11 + f22) + f33;
+          W2 = C.cm + lam * (tr * trf) + mu2 * (sh + (e11 * f11 + e22 * f22 + e33 * f33));
+          if (trf < 0.) W2 -= kap * (trf * trf);
+        } else {
+          W2 = C.cm + lam * (tr * tr) + mu2 * (sh + (e11 * e11 + e22 * e22 + e33 * e33));
+        }
+        row[gx] = gW(gx) * W2;
+      }
+      const double S = row[0] + row[2], w = C.vol * gW(gy) * gW(gz);
       const double m[3] = {w * (S + row[1]), (w * X1) * (row[2] - row[0]), (w * X2) * S};
 #pragma unroll
       for (int p = 0; p < 3; p++) {
@@ -107,26 +164,24 @@ __global__ __launch_bounds__(256) void k_v_setup(DevProblem P, const double *__r
           Y[2][p] += X2 * m[p];
         }
       }
-      if (gy == 2)  // end of a layer gz
-#pragma unroll
-        for (int q = 0; q < 3; q++)
-#pragma unroll
-          for (int p = 0; p < 3; p++) {
-            Q[0][q][p] += Y[q][p];
-            if (gz != 1) {
-              Q[1][q][p] += gz ? X1 * Y[q][p] : -X1 * Y[q][p];
-              Q[2][q][p] += X2 * Y[q][p];
-            }
-            Y[q][p] = 0.;
-          }
     }
-  });
+#pragma unroll
+    for (int q = 0; q < 3; q++)
+#pragma unroll
+      for (int p = 0; p < 3; p++) {
+        Q[0][q][p] += Y[q][p];
+        if (gz != 1) {
+          Q[1][q][p] += gz ? X1 * Y[q][p] : -X1 * Y[q][p];
+          Q[2][q][p] += X2 * Y[q][p];
+        }
+      }
+  }
 #pragma unroll
   for (int r = 0; r < 3; r++)
 #pragma unroll
     for (int q = 0; q < 3; q++)
 #pragma unroll
-      for (int p = 0; p < 3; p++) out[((r * 3 + q) * 3 + p) * 256] = Q[r][q][p];
+      for (int p = 0; p < 3; p++) out[((r * 3 + q) * 3 + p) * 64] = Q[r][q][p];
 }
 
 int64_t vq_doubles(const Grid &G) {
@@ -179,10 +234,10 @@ struct VModBase {
   template <bool NT>
   __device__ VQ moments(int ek, int tile, int slot) const {
     VQ a;
-    const double *b = q + tiled_index(tile, ek, G.nez, 27, 0, 0, 256);  // uniform in the workgroup
+    const double *b = q + tiled_index(tile, ek, G.nez, 27, 0);  // uniform in the workgroup
 #pragma unroll
     for (int g = 0; g < 27; g++) {
-      const double *p = b + g * 256 + (unsigned)slot;
+      const double *p = b + g * 64 + (unsigned)(slot / 64 * (27 * 64) + slot % 64);
       a.q[g] = NT ? __builtin_nontemporal_load(p) : *p;
     }
     return a;
@@ -543,89 +598,87 @@ __global__ __launch_bounds__(256, 2) void k_v_diag_list(VDiagOp op, const int *_
 
 // ------------------------------------------------------------ load vector
 // b_a = crhs sum_g W phi_a + [pressurize] sum_g W p (u . grad phi_a)
+// In modal duals R: R_0 = crhs vol / 8 (the rule integrates phi_a exactly) and,
+// for the modes i with variable d, R_i += vol / (4 h_d) <p u_d mono_i / x_d> in
+// closed form.
+// About 230 FP64 operations per element, against 700 of a walk over the Gauss
+// points; 97 x 131 x 76 39 -> 23 us (near the read of U and p).
 struct VRhsOp {
+  using T = double;
   static constexpr int NF = 4, NC = 1;
   const double *U, *p;
   double *b;
   Grid G;
-  double crhs;
+  double at, kf[3];  // crhs vol / 8; vol / (256 h_d)
   int crack;
+  struct Face {
+    double f[4][4];  // u_c, p: s, x, y, w
+  };
+  struct Own {};
+  struct Aux {};
+  using Raw = double;
+  static __device__ double off() { return 0.; }
   __device__ double load(int f, int64_t n) const { return f < 3 ? U[3 * n + f] : p[n]; }
-  // AT part: c_rhs sum_g W_g phi_a(g) = c_rhs vol / 8 for every corner (the
-  // 3-point rule integrates phi_a exactly).  Crack-pressure part: the flux
-  // F(g) = W_g p_g u_g projected on grad phi_a, sum-factorised: the x-flux
-  // summed over gx per (gy, gz), the y-flux over gy per (gx, gz), the z-flux
-  // over gz per (gx, gy), each then projected on the two other axes.
-  __device__ void element(int, int, int, const double (&X)[2][4][4], double (&r)[8][1]) const {
-    const double vol = G.hx * G.hy * G.hz;
-    const double at = crhs * vol * .125;
-    if (!crack) {
+  __device__ double stage(int, double x) const { return x; }
+  template <class RD>
+  __device__ void face(const RD &rd, Face &F) const {
 #pragma unroll
-      for (int a = 0; a < 8; a++) r[a][0] += at;
-      return;
+    for (int f = 0; f < 4; f++) {
+      const double x0 = rd(f, 0), x1 = rd(f, 1), x2 = rd(f, 2), x3 = rd(f, 3);
+      const double s0 = x0 + x1, s1 = x2 + x3, d0 = x1 - x0, d1 = x3 - x2;
+      F.f[f][0] = s0 + s1;
+      F.f[f][1] = d0 + d1;
+      F.f[f][2] = s1 - s0;
+      F.f[f][3] = d1 - d0;
     }
-    double fld[4][8];
+  }
+  __device__ Own own(const Face &) const { return Own{}; }
+  __device__ Aux aux(int, int, int, int, int) const { return Aux{}; }
+  __device__ void element(const Aux &, const Face &B, const Face &F, double (&tot)[1][4], double (&carry)[1][4]) const {
+    double R[8] = {at, 0., 0., 0., 0., 0., 0., 0.};
+    if (crack) {
+      double Pm[8], Um[3][8];
 #pragma unroll
-    for (int a = 0; a < 8; a++)
+      for (int q = 0; q < 4; q++) {
+        Pm[q] = F.f[3][q] + B.f[3][q];
+        Pm[q + 4] = F.f[3][q] - B.f[3][q];
 #pragma unroll
-      for (int f = 0; f < 4; f++) fld[f][a] = X[a >> 2][a & 3][f];
-    double Rx[2][2] = {{0., 0.}, {0., 0.}}, Ry[2][2] = {{0., 0.}, {0., 0.}}, Sz[3][3], Sy[3], Sx = 0.;
-#pragma unroll
-    for (int q = 0; q < 3; q++) {
-      Sy[q] = 0.;
-#pragma unroll
-      for (int w = 0; w < 3; w++) Sz[q][w] = 0.;
-    }
-    gauss_walk<0, 4>(fld, 0., 0., 0., [&](int gx, int gy, int gz, const double (&val)[4], const double (&)[1][3]) {
-      const double wp = vol * gW(gx) * gW(gy) * gW(gz) * val[3];
-      Sx += wp * val[0];
-      Sy[gx] += wp * val[1];
-      Sz[gy][gx] += wp * val[2];
-      if (gx == 2) {  // end of a row: the x-flux of (gy, gz) onto phi_j(y) phi_k(z)
-#pragma unroll
-        for (int k = 0; k < 2; k++)
-#pragma unroll
-          for (int j = 0; j < 2; j++) Rx[k][j] += (k ? gP1(gz) : gP0(gz)) * (j ? gP1(gy) : gP0(gy)) * Sx;
-        Sx = 0.;
-      }
-      if (gx == 2 && gy == 2) {  // end of a layer: the y-flux of (gx, gz) onto phi_i(x) phi_k(z)
-#pragma unroll
-        for (int q = 0; q < 3; q++) {
-#pragma unroll
-          for (int k = 0; k < 2; k++)
-#pragma unroll
-            for (int i = 0; i < 2; i++) Ry[k][i] += (k ? gP1(gz) : gP0(gz)) * (i ? gP1(q) : gP0(q)) * Sy[q];
-          Sy[q] = 0.;
+        for (int c = 0; c < 3; c++) {
+          Um[c][q] = F.f[c][q] + B.f[c][q];
+          Um[c][q + 4] = F.f[c][q] - B.f[c][q];
         }
       }
-    });
-    double Rz[2][2];  // [j][i]
 #pragma unroll
-    for (int j = 0; j < 2; j++)
+      for (int d = 0; d < 3; d++) {
+        double M[2][2][2];  // by the power of variable d in p and u
 #pragma unroll
-      for (int i = 0; i < 2; i++) {
-        double acc = 0.;
+        for (int t = 0; t < 2; t++) {
+          double p2[2][2], u2[2][2];
 #pragma unroll
-        for (int gy = 0; gy < 3; gy++)
+          for (int q = 0; q < 4; q++) {
+            p2[q & 1][q >> 1] = Pm[modal_at(d, t, q & 1, q >> 1)];
+            u2[q & 1][q >> 1] = Um[d][modal_at(d, t, q & 1, q >> 1)];
+          }
+          bilinear_moments(p2, u2, M[t]);
+        }
 #pragma unroll
-          for (int gx = 0; gx < 3; gx++) acc += (j ? gP1(gy) : gP0(gy)) * (i ? gP1(gx) : gP0(gx)) * Sz[gy][gx];
-        Rz[j][i] = acc;
+        for (int q = 0; q < 4; q++) {
+          const int i = q & 1, j = q >> 1;
+          R[modal_at(d, 1, i, j)] += (kf[d] * (i + j == 2 ? 1. / 9. : i + j ? 1. / 3. : 1.)) *
+                                     (M[0][i][j] + (1. / 3.) * M[1][i][j]);
+        }
       }
-    const double ihx = 1. / G.hx, ihy = 1. / G.hy, ihz = 1. / G.hz;
+    }
 #pragma unroll
-    for (int a = 0; a < 8; a++) {
-      const int i = a & 1, j = (a >> 1) & 1, k = a >> 2;
-      const double vx = (i ? ihx : -ihx) * Rx[k][j], vy = (j ? ihy : -ihy) * Ry[k][i],
-                   vz = (k ? ihz : -ihz) * Rz[j][i];
-      r[a][0] += at + (vx + vy + vz);
+    for (int q = 0; q < 4; q++) {
+      tot[0][q] += R[q] - R[q + 4];
+      carry[0][q] = R[q] + R[q + 4];
     }
   }
-  __device__ void store(int i, int j, int k, const double (&acc)[1], const double (&)[4]) const {
-    b[node_id(G, i, j, k)] = acc[0];
-  }
+  __device__ void store(int64_t n, uint32_t, const double (&acc)[1], const Own &) const { b[n] = acc[0]; }
 };
 
-__global__ __launch_bounds__(256) void k_v_rhs(VRhsOp op, int OZ) { march<double, 16, 16>(op.G, op, OZ, xcd_block()); }
+__global__ __launch_bounds__(256, 2) void k_v_rhs(VRhsOp op, int OZ) { march_modal<16, 16>(op.G, op, OZ, xcd_block()); }
 
 // ------------------------------------------------------------ launchers
 static dim3 mgrid(const Grid &G, int OZ) {
@@ -642,10 +695,14 @@ static int v_slots() {
 static int oz_for(const Grid &G) { return choose_oz(G, ((G.nx + 14) / 15) * ((G.ny + 14) / 15), v_slots()); }
 
 void launch_v_setup(const DevProblem &P, const double *U, hipStream_t s) {
-  hipLaunchKernelGGL(k_v_setup, dim3((P.G.nx + 14) / 15, (P.G.ny + 14) / 15, P.G.nez), dim3(256), 0, s, P, U);
+  const dim3 g((P.G.nx + 14) / 15, (P.G.ny + 14) / 15, P.G.nez);
+  if (P.unilateral) hipLaunchKernelGGL(k_v_setup<true>, g, dim3(256), 0, s, P, make_vsetup(P), U);
+  else hipLaunchKernelGGL(k_v_setup<false>, g, dim3(256), 0, s, P, make_vsetup(P), U);
   VRhsOp op;
   op.U = U; op.p = P.p; op.b = P.bV; op.G = P.G;
-  op.crhs = make_vconst(P).crhs;
+  const double h[3] = {P.G.hx, P.G.hy, P.G.hz}, vol = h[0] * h[1] * h[2];
+  op.at = make_vconst(P).crhs * vol / 8.;
+  for (int d = 0; d < 3; d++) op.kf[d] = vol / (256. * h[d]);
   op.crack = P.hasCrackPressure;
   int OZ = oz_for(P.G);
   hipLaunchKernelGGL(k_v_rhs, mgrid(P.G, OZ), dim3(256), 0, s, op, OZ);
