@@ -364,7 +364,9 @@ int bmg_setup(BatchMG *g, const double *const *dinv64, hipStream_t s) {
   if (hipStreamSynchronize(s) != hipSuccess) return VFG_E_HIP;  // dinv64 is written on the batch stream
   int rc;
   for (int p = 0; p < g->np; p++)
-    if (g->m[p] && (rc = mg_setup(g->m[p], dinv64[p]))) return rc;
+    if (g->m[p] && (rc = mg_setup_begin(g->m[p], dinv64[p]))) return rc;
+  for (int p = 0; p < g->np; p++)
+    if (g->m[p] && (rc = mg_setup_end(g->m[p]))) return rc;
   for (int p = 0; p < g->np; p++)
     if (g->m[p] && hipStreamSynchronize(g->m[p]->stream) != hipSuccess) return VFG_E_HIP;
   for (int p = 0; p < g->np; p++)

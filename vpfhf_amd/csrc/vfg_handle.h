@@ -21,6 +21,7 @@ struct MgHier {
   int L = 0;
   MgLevel lv[MAXL];
   int setups = 0;          // smoother bounds are re-estimated on every 16th set-up
+  bool estimate = false;   // and are on their way in this one
   double *dtmp = nullptr;  // FP64 diagonal of level 1 (largest coarse level)
 };
 }  // namespace vfg
@@ -38,7 +39,7 @@ struct vfg_handle {
   double *part = nullptr;      // reduction partials (4 x 65536)
   double *part_big = nullptr;  // partials for very large grids
   double *scal = nullptr;      // device scalars (64)
-  double *abh = nullptr;       // CG coefficient history of an eigenvalue estimate (3 x 64)
+  double *abh = nullptr;       // CG coefficient histories of eigenvalue estimates
   uint32_t *vflag = nullptr;   // V-solve: node-plane chunks holding free nodes (v_chunk_cap flags)
   int *vlist = nullptr;        //          and their list, count and chunk length (v_chunk_cap + 2)
   uint32_t *vflag2 = nullptr;  // the same dilated by one tile and one plane,
@@ -61,6 +62,8 @@ namespace vfg {
 constexpr int MG_SMOOTH = 1, MG_COARSE_DEG = 6, MG_COARSEST = 8;
 int mg_build(vfg_handle *h);                      // hierarchy shape and buffers (once)
 int mg_setup(vfg_handle *h, const double *dinv64);  // coefficients, diagonals, bounds (per solve)
+int mg_setup_begin(vfg_handle *h, const double *dinv64);  // the same in two parts: enqueue, read back
+int mg_setup_end(vfg_handle *h);
 }  // namespace vfg
 
 int vfg_fail(vfg_handle *h, int code, const char *fmt, ...);

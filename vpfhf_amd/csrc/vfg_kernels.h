@@ -139,7 +139,6 @@ void launch_mg_cheb(const float *b, const float *y, const float *dinv, float *d,
                     int dfirst, int xzero, int64_t n, hipStream_t s);
 void launch_mg_recip32(const double *d, float *dinv, int64_t n, hipStream_t s);
 void launch_mg_fill32(float *x, float v, int64_t n, hipStream_t s);
-void launch_mg_seed(float *x, int64_t n, hipStream_t s);
 void launch_cell_to_node(const DevProblem &P, double lx, double ly, double lz, const double *cell, double *node,
                          int dof, hipStream_t s);
 void launch_penny(const DevProblem &P, double *V, const double c[3], double r, double theta,

@@ -136,17 +136,6 @@ __global__ void k_mg_fill32(float *x, float v, int64_t n) {
   if (i < n) x[i] = v;
 }
 
-// deterministic start vector in [-1, 1) for the eigenvalue estimates
-__global__ void k_mg_seed(float *x, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  uint64_t z = (uint64_t)i * 0x9E3779B97F4A7C15ull + 0x632BE59BD9B4E019ull;
-  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
-  z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
-  z ^= z >> 31;
-  x[i] = (float)((double)(z >> 11) * (2.0 / 9007199254740992.0) - 1.0);
-}
-
 static unsigned nbm(int64_t n) { return (unsigned)((n + 255) / 256); }
 
 void launch_mg_elem_coef(const DevProblem &P, double *out, hipStream_t s) {
@@ -183,8 +172,4 @@ void launch_mg_recip32(const double *d, float *dinv, int64_t n, hipStream_t s) {
 void launch_mg_fill32(float *x, float v, int64_t n, hipStream_t s) {
   hipLaunchKernelGGL(k_mg_fill32, dim3(nbm(n)), dim3(256), 0, s, x, v, n);
 }
-void launch_mg_seed(float *x, int64_t n, hipStream_t s) {
-  hipLaunchKernelGGL(k_mg_seed, dim3(nbm(n)), dim3(256), 0, s, x, n);
-}
-
 }  // namespace vfg

@@ -510,19 +510,157 @@ static double lanczos_lmax(const double *ab, int m) {
   return hi;
 }
 
-// Inner PCG in FP32 on A32 d = r (d0 = 0); returns iterations; lanczos
-// estimates of the extreme eigenvalues of M^-1 A are accumulated from the CG
-// coefficients when est != nullptr (used to size the Chebyshev interval).
-// alpha, beta and the breakdown flag of CG iteration k, kept for the host
-__global__ void k_ab_save(const double *sc, double *hist, int k) {
-  hist[3 * k] = sc[S_ALPHA];
-  hist[3 * k + 1] = sc[S_BETA];
-  hist[3 * k + 2] = sc[S_FLAG];
+// lambda_max(D^-1 A) of several operators at once by a fixed number of
+// Jacobi-PCG steps each (FP32 vectors, FP64 sums): the levels of a multigrid
+// hierarchy step together, and no scalar is passed between kernels -- each
+// workgroup sums the partials it needs itself, in the same order.  Three
+// launches and the applies per step for all operators; one kernel per vector
+// operation and operator was nine (first solve of 16 problems of 16 to 64
+// elements per side: 31 -> 15 ms; of one of 32: 2.9 -> 2.0 ms).
+struct LzOp {
+  const float *dinv;
+  float *r, *p, *q;
+  int64_t n;
+  int nb, b0;  // workgroups, and the first of them
+};
+struct LzOps {
+  LzOp op[MgHier::MAXL];
+  int L, nb;  // operators, workgroups of all
+  double *part, *hist;  // 3 nb partials (r.z before and after the step, p.q); alpha, beta, flag per step
+  int seed;             // r starts from a fixed pseudo-random vector
+};
+constexpr int LZ_MAX = 16;  // steps
+__device__ __forceinline__ int lz_find(const LzOps &T) {
+  int l = 0;
+  while (l + 1 < T.L && (int)blockIdx.x >= T.op[l + 1].b0) l++;
+  return l;
+}
+// the partials of one operator, summed by every workgroup alike
+__device__ __forceinline__ double lz_sum(const double *part, int nb) {
+  __shared__ double sh;
+  double a = 0.;
+  for (int i = threadIdx.x; i < nb; i += RB) a += part[i];
+  a = bsum(a);
+  if (threadIdx.x == 0) sh = a;
+  __syncthreads();
+  a = sh;
+  __syncthreads();
+  return a;
+}
+// deterministic start vector in [-1, 1)
+__device__ __forceinline__ float lz_seed(int64_t i) {
+  uint64_t z = (uint64_t)i * 0x9E3779B97F4A7C15ull + 0x632BE59BD9B4E019ull;
+  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+  z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+  z ^= z >> 31;
+  return (float)((double)(z >> 11) * (2.0 / 9007199254740992.0) - 1.0);
+}
+__global__ __launch_bounds__(RB) void k_lz_init(LzOps T) {
+  const LzOp o = T.op[lz_find(T)];
+  double rz = 0.;
+  for (int64_t i = (int64_t)(blockIdx.x - o.b0) * RB + threadIdx.x; i < o.n; i += (int64_t)o.nb * RB) {
+    const float r = T.seed ? lz_seed(i) : o.r[i], z = o.dinv[i] * r;
+    if (T.seed) o.r[i] = r;
+    o.p[i] = z;
+    rz += (double)r * (double)z;
+  }
+  rz = bsum(rz);
+  if (threadIdx.x == 0) T.part[blockIdx.x] = rz;
+}
+__global__ __launch_bounds__(RB) void k_lz_dot(LzOps T) {
+  const LzOp o = T.op[lz_find(T)];
+  double s = 0.;
+  for (int64_t i = (int64_t)(blockIdx.x - o.b0) * RB + threadIdx.x; i < o.n; i += (int64_t)o.nb * RB)
+    s += (double)o.p[i] * (double)o.q[i];
+  s = bsum(s);
+  if (threadIdx.x == 0) T.part[2 * T.nb + blockIdx.x] = s;
+}
+// r -= alpha q and the next r.z; step k
+__global__ __launch_bounds__(RB) void k_lz_r(LzOps T, int k) {
+  const int l = lz_find(T);
+  const LzOp o = T.op[l];
+  const double rz0 = lz_sum(T.part + (k & 1) * T.nb + o.b0, o.nb), pq = lz_sum(T.part + 2 * T.nb + o.b0, o.nb);
+  const bool ok = pq > 0. && isfinite(pq);
+  const double al = ok ? rz0 / pq : 0.;
+  double rz = 0.;
+  for (int64_t i = (int64_t)(blockIdx.x - o.b0) * RB + threadIdx.x; i < o.n; i += (int64_t)o.nb * RB) {
+    const float r = (float)((double)o.r[i] - al * o.q[i]), z = o.dinv[i] * r;
+    o.r[i] = r;
+    rz += (double)r * (double)z;
+  }
+  rz = bsum(rz);
+  if (threadIdx.x != 0) return;
+  T.part[((k + 1) & 1) * T.nb + blockIdx.x] = rz;
+  if ((int)blockIdx.x == o.b0) {
+    double *h = T.hist + 3 * (l * LZ_MAX + k);
+    h[0] = al;
+    h[2] = ok ? 0. : isfinite(pq) ? 1. : 2.;
+  }
+}
+// p = D^-1 r + beta p
+__global__ __launch_bounds__(RB) void k_lz_p(LzOps T, int k) {
+  const int l = lz_find(T);
+  const LzOp o = T.op[l];
+  const double rz0 = lz_sum(T.part + (k & 1) * T.nb + o.b0, o.nb),
+               rz1 = lz_sum(T.part + ((k + 1) & 1) * T.nb + o.b0, o.nb);
+  const double be = rz0 != 0. ? rz1 / rz0 : 0.;
+  for (int64_t i = (int64_t)(blockIdx.x - o.b0) * RB + threadIdx.x; i < o.n; i += (int64_t)o.nb * RB) {
+    const float z = o.dinv[i] * o.r[i];
+    o.p[i] = (float)((double)z + be * o.p[i]);
+  }
+  if (threadIdx.x == 0 && (int)blockIdx.x == o.b0) {
+    double *h = T.hist + 3 * (l * LZ_MAX + k);
+    h[1] = be;
+    if (!isfinite(rz1)) h[2] = 2.;
+  }
+}
+// enqueues m <= LZ_MAX steps; A(l): q_l = A_l p_l
+static int lz_begin(vfg_handle *h, LzOps &T, int m, const std::function<void(int)> &A) {
+  hipStream_t s = h->stream;
+  if (!h->abh && vfg_alloc(h, (void **)&h->abh, 8 * 3 * LZ_MAX * MgHier::MAXL)) return VFG_E_NOMEM;
+  T.part = h->part;  // at most 3 x 2048 per operator
+  T.hist = h->abh;
+  T.nb = 0;
+  for (int l = 0; l < T.L; l++) {
+    T.op[l].nb = red_blocks(T.op[l].n);
+    T.op[l].b0 = T.nb;
+    T.nb += T.op[l].nb;
+  }
+  hipLaunchKernelGGL(k_lz_init, dim3(T.nb), dim3(RB), 0, s, T);
+  for (int k = 0; k < m; k++) {
+    for (int l = 0; l < T.L; l++) A(l);
+    hipLaunchKernelGGL(k_lz_dot, dim3(T.nb), dim3(RB), 0, s, T);
+    hipLaunchKernelGGL(k_lz_r, dim3(T.nb), dim3(RB), 0, s, T, k);
+    hipLaunchKernelGGL(k_lz_p, dim3(T.nb), dim3(RB), 0, s, T, k);
+  }
+  return VFG_OK;
+}
+// reads the steps of L operators back; lmax[l], status[l] (VFG_E_NAN: not finite)
+static int lz_end(vfg_handle *h, int L, int m, double *lmax, int *status) {
+  double hist[3 * LZ_MAX * MgHier::MAXL], ab[2 * LZ_MAX];
+  if (hipMemcpyAsync(hist, h->abh, 8 * 3 * LZ_MAX * L, hipMemcpyDeviceToHost, h->stream) != hipSuccess ||
+      hipStreamSynchronize(h->stream) != hipSuccess)
+    return VFG_E_HIP;
+  for (int l = 0; l < L; l++) {
+    int n = 0;
+    status[l] = VFG_OK;
+    for (int k = 0; k < m; k++) {
+      const double *q = hist + 3 * (l * LZ_MAX + k);
+      if (q[2] == 2.) { status[l] = VFG_E_NAN; break; }
+      if (q[2] != 0.) break;  // breakdown: the steps before it stand
+      ab[2 * n] = q[0];
+      ab[2 * n + 1] = q[1];
+      n++;
+    }
+    lmax[l] = lanczos_lmax(ab, n);
+  }
+  return VFG_OK;
 }
 
+// Inner PCG in FP32 on A32 d = r (d0 = 0); returns iterations.
 static int pcg32(vfg_handle *h, int64_t n, const std::function<void(const float *, float *)> &A, const float *dinv,
                  float *x, float *r, float *z, float *p, float *q, float *w1, float *w2, const Cheb &cb,
-                 double rtol, int maxit, double *lmax_est, int *status) {
+                 double rtol, int maxit, int *status) {
   hipStream_t s = h->stream;
   double *sc = h->scal, *part = h->part;
   const int nb = red_blocks(n);
@@ -535,45 +673,9 @@ static int pcg32(vfg_handle *h, int64_t n, const std::function<void(const float 
     return 0;
   }
   const double rn0 = sqrt(hs[S_RR0]);
-  double rn = rn0, ab[128];
-  int it = 0, n_ab = 0;
+  double rn = rn0;
+  int it = 0;
   *status = VFG_OK;
-  if (lmax_est) {
-    // eigenvalue estimate: a fixed number of steps (at most 64), the
-    // coefficients recorded on the device and read once
-    if (!h->abh && vfg_alloc(h, (void **)&h->abh, 8 * 3 * 64)) {
-      *status = VFG_E_NOMEM;
-      return 0;
-    }
-    const int m = maxit < 64 ? maxit : 64;
-    for (int k = 0; k < m; k++) {
-      A(p, q);
-      hipLaunchKernelGGL(k_dotp32, dim3(nb), dim3(RB), 0, s, (const float *)p, (const float *)q, n, part);
-      hipLaunchKernelGGL(k_pcg_scalar, dim3(1), dim3(RB), 0, s, (const double *)part, nb, 1, sc);
-      hipLaunchKernelGGL(k_pcg32_xr, dim3(nb), dim3(RB), 0, s, x, r, (const float *)p, (const float *)q, n,
-                         (const double *)sc);
-      precond32(h, A, dinv, r, z, w1, w2, n, cb);
-      hipLaunchKernelGGL(k_rz32, dim3(nb), dim3(RB), 0, s, (const float *)r, (const float *)z, n, part);
-      hipLaunchKernelGGL(k_pcg_scalar, dim3(1), dim3(RB), 0, s, (const double *)part, nb, 2, sc);
-      hipLaunchKernelGGL(k_pcg32_p, dim3(nb), dim3(RB), 0, s, p, (const float *)z, n, (const double *)sc);
-      hipLaunchKernelGGL(k_ab_save, dim3(1), dim3(1), 0, s, (const double *)sc, h->abh, k);
-    }
-    double hist[3 * 64];
-    if (hipMemcpyAsync(hist, h->abh, 8 * 3 * m, hipMemcpyDeviceToHost, s) != hipSuccess ||
-        hipStreamSynchronize(s) != hipSuccess) {
-      *status = VFG_E_HIP;
-      return 0;
-    }
-    for (int k = 0; k < m; k++) {
-      if (hist[3 * k + 2] == 2.) { *status = VFG_E_NAN; break; }
-      if (hist[3 * k + 2] != 0.) break;  // breakdown: the steps before it stand
-      ab[2 * n_ab] = hist[3 * k];
-      ab[2 * n_ab + 1] = hist[3 * k + 1];
-      n_ab++;
-    }
-    *lmax_est = lanczos_lmax(ab, n_ab);
-    return m;
-  }
   const int check = 10;
   double rate = -1.;  // observed residual reduction per iteration
   while (rn > rtol * rn0 && it < maxit) {
@@ -672,8 +774,10 @@ int mg_build(vfg_handle *h) {
 
 // Refreshes the hierarchy from the current problem (V, E, properties, BCs):
 // coarse coefficients, FP32 inverse diagonals and the smoother intervals.
-// dinv64: the problem's FP64 inverse diagonal.
-int mg_setup(vfg_handle *h, const double *dinv64) {
+// dinv64: the problem's FP64 inverse diagonal.  _begin enqueues, _end reads the
+// estimates back where they were due (the set-ups of several problems overlap).
+constexpr int MG_LZ = 10;  // Lanczos steps
+int mg_setup_begin(vfg_handle *h, const double *dinv64) {
   int rc = mg_build(h);
   if (rc) return rc;
   MgHier &m = *h->mg;
@@ -704,23 +808,35 @@ int mg_setup(vfg_handle *h, const double *dinv64) {
   // Poisson ratio, not by V or E (measured: 2.55, 2.50, 2.30, 1.79 on the
   // levels of a cracked 32^3 problem against 2.5 for a uniform one), so the
   // estimates of the first set-up are reused and refreshed every 16th.
-  if (m.setups++ % 16 != 0) return VFG_OK;
-  float **w = h->wf;
-  for (int l = 0; l < m.L; l++) {
+  m.estimate = m.setups++ % 16 == 0;
+  if (!m.estimate) return VFG_OK;
+  LzOps T{};
+  T.L = m.L;
+  T.seed = 1;
+  for (int l = 0; l < m.L; l++) {  // the coarse levels' own vectors are free here
     MgLevel &lv = m.lv[l];
-    launch_mg_seed(w[1], lv.n, s);
-    launch_mg_fill32(w[0], 0.f, lv.n, s);
-    std::function<void(const float *, float *)> A = [&](const float *in, float *out) {
-      launch_u_apply_f32(lv.P, in, out, s);
-    };
-    double lmax = 0.;
-    int st = 0;
-    pcg32(h, lv.n, A, lv.dinv, w[0], w[1], w[2], w[3], w[4], w[5], w[6], Cheb{1, 0., 0.}, 0., 10, &lmax, &st);
-    if (st == VFG_E_HIP || st == VFG_E_NAN || !(lmax > 0.))
-      return vfg_fail(h, st ? st : VFG_E_NAN, "multigrid set-up: eigenvalue estimate failed on level %d", l);
-    lv.lmax = 1.1 * lmax;
+    if (l == 0) T.op[l] = LzOp{lv.dinv, h->wf[1], h->wf[3], h->wf[4], lv.n, 0, 0};
+    else T.op[l] = LzOp{lv.dinv, lv.b, lv.x, lv.y, lv.n, 0, 0};
+  }
+  return lz_begin(h, T, MG_LZ, [&](int l) { launch_u_apply_f32(m.lv[l].P, T.op[l].p, T.op[l].q, s); });
+}
+int mg_setup_end(vfg_handle *h) {
+  MgHier &m = *h->mg;
+  if (!m.estimate) return VFG_OK;
+  m.estimate = false;
+  double lmax[MgHier::MAXL];
+  int st[MgHier::MAXL];
+  int rc = lz_end(h, m.L, MG_LZ, lmax, st);
+  for (int l = 0; l < m.L; l++) {
+    if (rc || st[l] || !(lmax[l] > 0.))
+      return vfg_fail(h, rc ? rc : VFG_E_NAN, "multigrid set-up: eigenvalue estimate failed on level %d", l);
+    m.lv[l].lmax = 1.1 * lmax[l];
   }
   return VFG_OK;
+}
+int mg_setup(vfg_handle *h, const double *dinv64) {
+  const int rc = mg_setup_begin(h, dinv64);
+  return rc ? rc : mg_setup_end(h);
 }
 
 // Chebyshev coefficients of mg_cheb_entry's step i on [lo, hi]
@@ -1046,9 +1162,13 @@ static int u_solve_mixed(vfg_handle *h, double *x, double *r64, double *t64, con
       // lambda_max(D^-1 A) from 12 Jacobi-PCG steps on this residual, then restart
       double lmax = 0.;
       int st = 0;
-      pcg32(h, n, A32, dinv, d, r, z, p, q, w1, w2, cb, 0., 12, &lmax, &st);
+      LzOps T{};
+      T.L = 1;
+      T.op[0] = LzOp{dinv, r, p, q, n, 0, 0};
+      int e = lz_begin(h, T, 12, [&](int) { A32(p, q); });
+      if (!e) e = lz_end(h, 1, 12, &lmax, &st);
       inf->iterations += 12;
-      if (st == VFG_E_HIP) return st;
+      if (e) return e;
       cb.degree = o->cheb_degree > 1 ? o->cheb_degree : 4;
       cb.lmax = 1.1 * lmax;
       cb.lmin = cb.lmax / 30.;
@@ -1056,7 +1176,7 @@ static int u_solve_mixed(vfg_handle *h, double *x, double *r64, double *t64, con
       hipLaunchKernelGGL(k_fill32, dim3(nb_(n)), dim3(256), 0, s, d, n);
     }
     int st = 0;
-    int its = pcg32(h, n, A32, dinv, d, r, z, p, q, w1, w2, cb, inner_rtol, o->maxit, nullptr, &st);
+    int its = pcg32(h, n, A32, dinv, d, r, z, p, q, w1, w2, cb, inner_rtol, o->maxit, &st);
     inf->iterations += its * (cb.degree > 1 ? cb.degree : 1);  // a V-cycle step counts once
     if (st == VFG_E_HIP || st == VFG_E_NAN) return st;
     hipLaunchKernelGGL(k_axpy3264, dim3(nb_(n)), dim3(256), 0, s, x, (const float *)d, rn, n);
