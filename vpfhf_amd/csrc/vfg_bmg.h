@@ -52,6 +52,7 @@ int bmg_rebuild(BatchMG *g, hipStream_t s, bool *grew);
 int bmg_setup(BatchMG *g, const double *const *dinv64, hipStream_t s);
 // the same for member p alone
 int bmg_setup_member(BatchMG *g, int p, const double *dinv64, hipStream_t s);
+void bmg_idle(BatchMG *g);  // the stream of the uploads has been synchronised
 // z = V-cycle(r) for every member with flags[p * fstride] != 0
 void bmg_vcycle(BatchMG *g, const double *flags, int fstride, hipStream_t s);
 

@@ -18,6 +18,7 @@
 #include "vfg_mg.h"
 #include "vfg_batch_apply.h"
 #include "vfg_bmg.h"
+#include "vfg_stage.h"
 
 namespace vfg {
 
@@ -112,7 +113,8 @@ struct BatchMG {
   BmgPlan lv[BML];
   BmgVec *d_lvt = nullptr;
   BmgCoef *d_coef = nullptr;
-  std::vector<BmgVec> h_lvt;          // staging of the tables (kept: uploads are asynchronous)
+  Stage up;                           // uploads of the tables and lists
+  std::vector<BmgVec> h_lvt;          // the tables' host copies
   std::vector<BmgCoef> h_coef;
   std::vector<std::vector<char>> h_ops, h_pre, h_post;
   std::vector<void *> allocs;         // fixed allocations
@@ -151,11 +153,8 @@ static int grow(BatchMG *g, Grow<V> &a, bool *grew) {
   return VFG_OK;
 }
 template <typename V>
-static int push(Grow<V> &a, hipStream_t s) {
-  if (a.h.empty()) return VFG_OK;
-  return hipMemcpyAsync(a.d, a.h.data(), sizeof(V) * a.h.size(), hipMemcpyHostToDevice, s) == hipSuccess
-             ? VFG_OK
-             : VFG_E_HIP;
+static int push(BatchMG *g, Grow<V> &a, hipStream_t s) {
+  return g->up.put(a.d, a.h.data(), sizeof(V) * a.h.size(), s) ? VFG_OK : VFG_E_HIP;
 }
 
 static const Grid &level_grid(const BatchMG *g, int p, int l) { return g->m[p]->mg->lv[l].P.G; }
@@ -235,17 +234,16 @@ int bmg_rebuild(BatchMG *g, hipStream_t s, bool *grew) {
     if (cfit != P.cfit) *grew = true;  // the V-cycle's launches change
     P.cfit = cfit;
     for (int k = 0; k < 3 && !rc; k++)
-      if ((rc = push(ls[k]->items, s)) || (rc = push(ls[k]->ch, s))) break;
-    if (rc || (rc = push(P.rch, s)) || (rc = push(P.pch, s))) break;
-    if (hipMemcpyAsync(P.dcnt, P.hcnt, sizeof P.hcnt, hipMemcpyHostToDevice, s) != hipSuccess) rc = VFG_E_HIP;
+      if ((rc = push(g, ls[k]->items, s)) || (rc = push(g, ls[k]->ch, s))) break;
+    if (rc || (rc = push(g, P.rch, s)) || (rc = push(g, P.pch, s))) break;
+    if (!g->up.put(P.dcnt, P.hcnt, sizeof P.hcnt, s)) rc = VFG_E_HIP;
   }
   int Lcap = 0;
   for (int l = 0; l < BML; l++)
     if (g->lv[l].M.ch.cap > 0) Lcap = l + 1;
   if (Lcap != g->Lcap) *grew = true;
   g->Lcap = Lcap;
-  // the counts above are read from their host arrays when the copies run
-  if (!rc && hipStreamSynchronize(s) != hipSuccess) rc = VFG_E_HIP;
+  if (!rc && !g->up.flush(s)) rc = VFG_E_HIP;
   return rc;
 }
 
@@ -284,6 +282,7 @@ int bmg_create(const std::vector<vfg_handle *> &m, float *const *r32, float *con
   bool grew = false;
   hipStream_t s = m.empty() ? nullptr : m[0]->stream;
   if (!rc) rc = bmg_rebuild(g, s, &grew);
+  if (!rc && hipStreamSynchronize(s) != hipSuccess) rc = VFG_E_HIP;  // later uploads are on another stream
   if (rc) {
     bmg_destroy(g);
     return rc;
@@ -342,31 +341,33 @@ static void stage_member(BatchMG *g, int p) {
 }
 static int upload_member(BatchMG *g, int p, hipStream_t s) {
   const size_t ob = batch_op_bytes(1);
-  if (hipMemcpyAsync(g->d_lvt + (size_t)p * BML, &g->h_lvt[(size_t)p * BML], sizeof(BmgVec) * BML,
-                     hipMemcpyHostToDevice, s) != hipSuccess ||
-      hipMemcpyAsync(g->d_coef + (size_t)p * BML * 2 * BMK, &g->h_coef[(size_t)p * BML * 2 * BMK],
-                     sizeof(BmgCoef) * BML * 2 * BMK, hipMemcpyHostToDevice, s) != hipSuccess)
+  const size_t L = (size_t)g->L[p];
+  if (!g->up.put(g->d_lvt + (size_t)p * BML, &g->h_lvt[(size_t)p * BML], sizeof(BmgVec) * L, s) ||
+      !g->up.put(g->d_coef + (size_t)p * BML * 2 * BMK, &g->h_coef[(size_t)p * BML * 2 * BMK],
+                 sizeof(BmgCoef) * L * 2 * BMK, s))
     return VFG_E_HIP;
-  const size_t pb = mg_smooth_op_bytes(), qb = mg_smooth_op_bytes();
-  for (int l = 0; l < g->L[p]; l++)
-    if (!g->lv[l].ops || !g->lv[l].ops_pre || !g->lv[l].ops_post ||
-        hipMemcpyAsync((char *)g->lv[l].ops + ob * p, g->h_ops[l].data() + ob * p, ob, hipMemcpyHostToDevice, s) !=
-            hipSuccess ||
-        hipMemcpyAsync((char *)g->lv[l].ops_pre + pb * p, g->h_pre[l].data() + pb * p, pb, hipMemcpyHostToDevice,
-                       s) != hipSuccess ||
-        hipMemcpyAsync((char *)g->lv[l].ops_post + qb * p, g->h_post[l].data() + qb * p, qb, hipMemcpyHostToDevice,
-                       s) != hipSuccess)
+  const size_t pb = mg_smooth_op_bytes();
+  for (int l = 0; l < g->L[p]; l++) {
+    BmgPlan &P = g->lv[l];
+    if (!P.ops || !P.ops_pre || !P.ops_post || !g->up.put((char *)P.ops + ob * p, g->h_ops[l].data() + ob * p, ob, s) ||
+        !g->up.put((char *)P.ops_pre + pb * p, g->h_pre[l].data() + pb * p, pb, s) ||
+        !g->up.put((char *)P.ops_post + pb * p, g->h_post[l].data() + pb * p, pb, s))
       return VFG_E_HIP;
+  }
   return VFG_OK;
+}
+void bmg_idle(BatchMG *g) {
+  if (g) g->up.idle();
 }
 
 int bmg_setup(BatchMG *g, const double *const *dinv64, hipStream_t s) {
   if (hipStreamSynchronize(s) != hipSuccess) return VFG_E_HIP;  // dinv64 is written on the batch stream
+  g->up.idle();
   int rc;
   for (int p = 0; p < g->np; p++)
-    if (g->m[p] && (rc = mg_setup_begin(g->m[p], dinv64[p]))) return rc;
+    if (g->m[p] && (rc = mg_setup_begin(g->m[p], dinv64[p], g->m[p]->stream))) return rc;
   for (int p = 0; p < g->np; p++)
-    if (g->m[p] && (rc = mg_setup_end(g->m[p]))) return rc;
+    if (g->m[p] && (rc = mg_setup_end(g->m[p], g->m[p]->stream))) return rc;
   for (int p = 0; p < g->np; p++)
     if (g->m[p] && hipStreamSynchronize(g->m[p]->stream) != hipSuccess) return VFG_E_HIP;
   for (int p = 0; p < g->np; p++)
@@ -374,18 +375,17 @@ int bmg_setup(BatchMG *g, const double *const *dinv64, hipStream_t s) {
       stage_member(g, p);
       if ((rc = upload_member(g, p, s))) return rc;
     }
-  return hipStreamSynchronize(s) == hipSuccess ? VFG_OK : VFG_E_HIP;
+  return g->up.flush(s) ? VFG_OK : VFG_E_HIP;
 }
 
 int bmg_setup_member(BatchMG *g, int p, const double *dinv64, hipStream_t s) {
   if (p < 0 || p >= g->np || !g->m[p]) return VFG_E_ARG;
-  if (hipStreamSynchronize(s) != hipSuccess) return VFG_E_HIP;  // dinv64 and the fields are written on s
-  int rc = mg_setup(g->m[p], dinv64);
+  int rc = mg_setup_begin(g->m[p], dinv64, s);  // on s, where dinv64 and the fields are written
+  if (!rc) rc = mg_setup_end(g->m[p], s);
   if (rc) return rc;
-  if (hipStreamSynchronize(g->m[p]->stream) != hipSuccess) return VFG_E_HIP;
   stage_member(g, p);
   if ((rc = upload_member(g, p, s))) return rc;
-  return hipStreamSynchronize(s) == hipSuccess ? VFG_OK : VFG_E_HIP;  // the staging is reused
+  return g->up.flush(s) ? VFG_OK : VFG_E_HIP;
 }
 
 static void apply(BatchMG *g, int l, const BmgList &L, int which, const double *flags, int fstride, hipStream_t s) {

@@ -22,6 +22,7 @@
 #include <vector>
 #include "vfg_batch_apply.h"
 #include "vfg_bmg.h"
+#include "vfg_stage.h"
 #include "vfg_handle.h"
 
 namespace vfg {
@@ -360,6 +361,7 @@ struct vfg_engine {
   int h_cnt[C_N] = {0};
   double *d_part = nullptr;
   int cap_part = 0;
+  Stage up;  // uploads of the tables and lists
   bool dirty_lists = true, dirty_vt = true, dirty_uop = true, dirty_vop = true;
   hipGraphExec_t g = nullptr, g_mg = nullptr;  // replay graphs without / with the batched V-cycle
   int grid_apply = 0, grid_vapply = 0, grid_vec = 0;
@@ -701,6 +703,10 @@ static int advance(vfg_engine *e, int p) {
   }
 }
 
+// upload in stream order, by the next flush of e->up
+static int eput(vfg_engine *e, void *dst, const void *src, size_t bytes) {
+  return e->up.put(dst, src, bytes, e->s) ? VFG_OK : efail(e, VFG_E_HIP, "vfg_engine: staged upload failed");
+}
 // work lists of the requests in a CG phase
 static int rebuild_lists(vfg_engine *e) {
   for (int k = 0; k < 3; k++) e->h_it[k].clear();
@@ -744,16 +750,13 @@ static int rebuild_lists(vfg_engine *e) {
   e->h_cnt[C_F32] = (int)e->h_ch[0].size();
   e->h_cnt[C_F64] = (int)e->h_ch[1].size();
   for (int k = 0; k < 3; k++)
-    if (!e->h_it[k].empty())
-      ECHK(e, hipMemcpyAsync(e->d_it[k], e->h_it[k].data(), sizeof(BItem) * e->h_it[k].size(),
-                             hipMemcpyHostToDevice, e->s));
+    if ((rc = eput(e, e->d_it[k], e->h_it[k].data(), sizeof(BItem) * e->h_it[k].size()))) return rc;
   for (int k = 0; k < 2; k++)
-    if (!e->h_ch[k].empty())
-      ECHK(e, hipMemcpyAsync(e->d_ch[k], e->h_ch[k].data(), sizeof(EChunk) * e->h_ch[k].size(),
-                             hipMemcpyHostToDevice, e->s));
-  ECHK(e, hipMemcpyAsync(e->d_first, e->h_first.data(), sizeof(int) * e->ns, hipMemcpyHostToDevice, e->s));
-  ECHK(e, hipMemcpyAsync(e->d_nch, e->h_nch.data(), sizeof(int) * e->ns, hipMemcpyHostToDevice, e->s));
-  ECHK(e, hipMemcpyAsync(e->d_cnt, e->h_cnt, sizeof(int) * C_N, hipMemcpyHostToDevice, e->s));
+    if ((rc = eput(e, e->d_ch[k], e->h_ch[k].data(), sizeof(EChunk) * e->h_ch[k].size()))) return rc;
+  if ((rc = eput(e, e->d_first, e->h_first.data(), sizeof(int) * e->ns)) ||
+      (rc = eput(e, e->d_nch, e->h_nch.data(), sizeof(int) * e->ns)) ||
+      (rc = eput(e, e->d_cnt, e->h_cnt, sizeof(int) * C_N)))
+    return rc;
   e->dirty_lists = false;
   return VFG_OK;
 }
@@ -901,7 +904,7 @@ int vfg_engine_create(const vfg_engine_opts *o, vfg_engine **out) {
     return VFG_E_HIP;
   }
   int rc = rebuild_lists(e);  // empty lists, device counters = 0
-  if (!rc && hipStreamSynchronize(e->s) != hipSuccess) rc = VFG_E_HIP;
+  if (!rc && (!e->up.flush(e->s) || hipStreamSynchronize(e->s) != hipSuccess)) rc = VFG_E_HIP;
   if (rc) {
     vfg_engine_destroy(e);
     return rc;
@@ -966,25 +969,20 @@ int vfg_engine_step(vfg_engine *e) {
   if (!used) return 0;
   ECHK(e, hipMemcpyAsync(e->h_sc, e->d_sc, 8 * E_NS * (size_t)e->ns, hipMemcpyDeviceToHost, e->s));
   ECHK(e, hipStreamSynchronize(e->s));
+  e->up.idle();
+  bmg_idle(e->bmg);
   for (int p = 0; p < e->ns; p++) {
     if (e->slot[p].st == ST_FREE) continue;
     int rc = advance(e, p);
     if (rc) return rc;
   }
-  if (e->dirty_vt) {
-    ECHK(e, hipMemcpyAsync(e->d_vt, e->h_vt.data(), sizeof(EVec) * e->ns, hipMemcpyHostToDevice, e->s));
-    e->dirty_vt = false;
-  }
-  if (e->dirty_uop) {
-    ECHK(e, hipMemcpyAsync(e->d_uop, e->h_uop.data(), e->uop_sz * e->ns, hipMemcpyHostToDevice, e->s));
-    e->dirty_uop = false;
-  }
-  if (e->dirty_vop) {
-    ECHK(e, hipMemcpyAsync(e->d_vop, e->h_vop.data(), e->vop_sz * e->ns, hipMemcpyHostToDevice, e->s));
-    e->dirty_vop = false;
-  }
   int rc;
+  if (e->dirty_vt && (rc = eput(e, e->d_vt, e->h_vt.data(), sizeof(EVec) * e->ns))) return rc;
+  if (e->dirty_uop && (rc = eput(e, e->d_uop, e->h_uop.data(), e->uop_sz * e->ns))) return rc;
+  if (e->dirty_vop && (rc = eput(e, e->d_vop, e->h_vop.data(), e->vop_sz * e->ns))) return rc;
+  e->dirty_vt = e->dirty_uop = e->dirty_vop = false;
   if (e->dirty_lists && (rc = rebuild_lists(e))) return rc;
+  if (!e->up.flush(e->s)) return efail(e, VFG_E_HIP, "vfg_engine: staged upload failed");
   if ((rc = mg_lists(e))) return rc;
   bool any_cg = false;
   used = 0;

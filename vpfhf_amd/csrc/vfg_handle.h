@@ -62,8 +62,9 @@ namespace vfg {
 constexpr int MG_SMOOTH = 1, MG_COARSE_DEG = 6, MG_COARSEST = 8;
 int mg_build(vfg_handle *h);                      // hierarchy shape and buffers (once)
 int mg_setup(vfg_handle *h, const double *dinv64);  // coefficients, diagonals, bounds (per solve)
-int mg_setup_begin(vfg_handle *h, const double *dinv64);  // the same in two parts: enqueue, read back
-int mg_setup_end(vfg_handle *h);
+// the same in two parts on stream s: enqueue, read back
+int mg_setup_begin(vfg_handle *h, const double *dinv64, hipStream_t s);
+int mg_setup_end(vfg_handle *h, hipStream_t s);
 }  // namespace vfg
 
 int vfg_fail(vfg_handle *h, int code, const char *fmt, ...);

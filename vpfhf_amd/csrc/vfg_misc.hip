@@ -2,6 +2,7 @@
 // vector kernels of the solvers.  All reductions are two-stage with a fixed
 // summation order, so results are bitwise reproducible run to run.
 #include "vfg_modal.h"
+#include "vfg_stage.h"
 #include "vfg_kernels.h"
 
 namespace vfg {
@@ -472,6 +473,20 @@ void launch_crack_volume(const DevProblem &P, const double *U, const double *V, 
                      energy_ez(P.G));
   hipLaunchKernelGGL(k_reduce_partials<1>, dim3(1), dim3(256), 0, s, (const double *)partials, energy_blocks(P),
                      result);
+}
+
+// ------------------------------------------------------------ staged uploads
+// one segment per blockIdx.x
+__global__ __launch_bounds__(256) void k_stage(const StageSeg *__restrict__ seg) {
+  const StageSeg q = seg[blockIdx.x];
+  const size_t n = q.bytes / 4, st = (size_t)gridDim.y * 256;
+  uint32_t *__restrict__ d = (uint32_t *)q.dst;
+  const uint32_t *__restrict__ a = (const uint32_t *)q.src;
+  for (size_t i = (size_t)blockIdx.y * 256 + threadIdx.x; i < n; i += st) d[i] = a[i];
+}
+void launch_stage(const StageSeg *seg, int n, size_t max_bytes, hipStream_t s) {
+  const unsigned ny = (unsigned)((max_bytes + 4095) / 4096);
+  hipLaunchKernelGGL(k_stage, dim3(n, ny < 1 ? 1 : ny > 64 ? 64 : ny), dim3(256), 0, s, seg);
 }
 
 // ------------------------------------------------------------ penny crack

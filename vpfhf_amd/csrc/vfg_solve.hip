@@ -615,8 +615,7 @@ __global__ __launch_bounds__(RB) void k_lz_p(LzOps T, int k) {
   }
 }
 // enqueues m <= LZ_MAX steps; A(l): q_l = A_l p_l
-static int lz_begin(vfg_handle *h, LzOps &T, int m, const std::function<void(int)> &A) {
-  hipStream_t s = h->stream;
+static int lz_begin(vfg_handle *h, LzOps &T, int m, hipStream_t s, const std::function<void(int)> &A) {
   if (!h->abh && vfg_alloc(h, (void **)&h->abh, 8 * 3 * LZ_MAX * MgHier::MAXL)) return VFG_E_NOMEM;
   T.part = h->part;  // at most 3 x 2048 per operator
   T.hist = h->abh;
@@ -636,10 +635,10 @@ static int lz_begin(vfg_handle *h, LzOps &T, int m, const std::function<void(int
   return VFG_OK;
 }
 // reads the steps of L operators back; lmax[l], status[l] (VFG_E_NAN: not finite)
-static int lz_end(vfg_handle *h, int L, int m, double *lmax, int *status) {
+static int lz_end(vfg_handle *h, int L, int m, hipStream_t s, double *lmax, int *status) {
   double hist[3 * LZ_MAX * MgHier::MAXL], ab[2 * LZ_MAX];
-  if (hipMemcpyAsync(hist, h->abh, 8 * 3 * LZ_MAX * L, hipMemcpyDeviceToHost, h->stream) != hipSuccess ||
-      hipStreamSynchronize(h->stream) != hipSuccess)
+  if (hipMemcpyAsync(hist, h->abh, 8 * 3 * LZ_MAX * L, hipMemcpyDeviceToHost, s) != hipSuccess ||
+      hipStreamSynchronize(s) != hipSuccess)
     return VFG_E_HIP;
   for (int l = 0; l < L; l++) {
     int n = 0;
@@ -777,11 +776,10 @@ int mg_build(vfg_handle *h) {
 // dinv64: the problem's FP64 inverse diagonal.  _begin enqueues, _end reads the
 // estimates back where they were due (the set-ups of several problems overlap).
 constexpr int MG_LZ = 10;  // Lanczos steps
-int mg_setup_begin(vfg_handle *h, const double *dinv64) {
+int mg_setup_begin(vfg_handle *h, const double *dinv64, hipStream_t s) {
   int rc = mg_build(h);
   if (rc) return rc;
   MgHier &m = *h->mg;
-  hipStream_t s = h->stream;
   const int64_t nf = 3 * h->P.nn;
   for (int i = 0; i < 7; i++)
     if (!h->wf[i] && (rc = vfg_alloc(h, (void **)&h->wf[i], 4 * (size_t)nf))) return rc;
@@ -818,15 +816,15 @@ int mg_setup_begin(vfg_handle *h, const double *dinv64) {
     if (l == 0) T.op[l] = LzOp{lv.dinv, h->wf[1], h->wf[3], h->wf[4], lv.n, 0, 0};
     else T.op[l] = LzOp{lv.dinv, lv.b, lv.x, lv.y, lv.n, 0, 0};
   }
-  return lz_begin(h, T, MG_LZ, [&](int l) { launch_u_apply_f32(m.lv[l].P, T.op[l].p, T.op[l].q, s); });
+  return lz_begin(h, T, MG_LZ, s, [&](int l) { launch_u_apply_f32(m.lv[l].P, T.op[l].p, T.op[l].q, s); });
 }
-int mg_setup_end(vfg_handle *h) {
+int mg_setup_end(vfg_handle *h, hipStream_t s) {
   MgHier &m = *h->mg;
   if (!m.estimate) return VFG_OK;
   m.estimate = false;
   double lmax[MgHier::MAXL];
   int st[MgHier::MAXL];
-  int rc = lz_end(h, m.L, MG_LZ, lmax, st);
+  int rc = lz_end(h, m.L, MG_LZ, s, lmax, st);
   for (int l = 0; l < m.L; l++) {
     if (rc || st[l] || !(lmax[l] > 0.))
       return vfg_fail(h, rc ? rc : VFG_E_NAN, "multigrid set-up: eigenvalue estimate failed on level %d", l);
@@ -835,8 +833,8 @@ int mg_setup_end(vfg_handle *h) {
   return VFG_OK;
 }
 int mg_setup(vfg_handle *h, const double *dinv64) {
-  const int rc = mg_setup_begin(h, dinv64);
-  return rc ? rc : mg_setup_end(h);
+  const int rc = mg_setup_begin(h, dinv64, h->stream);
+  return rc ? rc : mg_setup_end(h, h->stream);
 }
 
 // Chebyshev coefficients of mg_cheb_entry's step i on [lo, hi]
@@ -1165,8 +1163,8 @@ static int u_solve_mixed(vfg_handle *h, double *x, double *r64, double *t64, con
       LzOps T{};
       T.L = 1;
       T.op[0] = LzOp{dinv, r, p, q, n, 0, 0};
-      int e = lz_begin(h, T, 12, [&](int) { A32(p, q); });
-      if (!e) e = lz_end(h, 1, 12, &lmax, &st);
+      int e = lz_begin(h, T, 12, s, [&](int) { A32(p, q); });
+      if (!e) e = lz_end(h, 1, 12, s, &lmax, &st);
       inf->iterations += 12;
       if (e) return e;
       cb.degree = o->cheb_degree > 1 ? o->cheb_degree : 4;
