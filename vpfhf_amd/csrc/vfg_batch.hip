@@ -40,7 +40,6 @@ template <typename T>
 __device__ __forceinline__ T *vec(const BVec *t, const BChunk &c, int slot) {
   return (T *)t[c.p].v[slot] + c.start;
 }
-constexpr int CH = 4096;  // vector elements per chunk
 constexpr int BRB = 256;
 
 enum { B_RZ = 0, B_PQ, B_ALPHA, B_BETA, B_RR, B_RR0, B_ACTIVE, B_STATUS, B_SCALE, B_ITS, B_NS = 16 };
@@ -57,14 +56,18 @@ __global__ __launch_bounds__(BRB) void k_binit(const BVec *vt, int o, const BChu
   const T *r = vec<T>(vt, c, o + VR), *dinv = vec<T>(vt, c, o + VD);
   T *z = vec<T>(vt, c, o + VZ), *p = vec<T>(vt, c, o + VP);
   double rz = 0., rr = 0.;
-  for (int k = threadIdx.x; k < c.len; k += BRB) {
-    double ri = r[k];
-    T zi = (T)(dinv[k] * r[k]);
-    z[k] = zi;
-    p[k] = zi;
-    rz += ri * (double)zi;
-    rr += ri * ri;
-  }
+  struct V {
+    T r, d;
+  };
+  chunk_walk<BRB>(c.len, [&](int k) { return V{r[k], dinv[k]}; },
+                  [&](int k, const V &v) {
+                    const double ri = v.r;
+                    const T zi = (T)(v.d * v.r);
+                    z[k] = zi;
+                    p[k] = zi;
+                    rz += ri * (double)zi;
+                    rr += ri * ri;
+                  });
   rz = bbsum(rz);
   rr = bbsum(rr);
   if (threadIdx.x == 0) { part[2 * blockIdx.x] = rz; part[2 * blockIdx.x + 1] = rr; }
@@ -78,7 +81,10 @@ __global__ __launch_bounds__(BRB) void k_bdot(const BVec *vt, int sa, int sb, co
   if (sc && sc[(int64_t)c.p * B_NS + B_ACTIVE] == 0.) return;  // frozen member
   const T *a = vec<T>(vt, c, sa), *b = vec<T>(vt, c, sb);
   double s = 0.;
-  for (int i = threadIdx.x; i < c.len; i += BRB) s += (double)a[i] * (double)b[i];
+  struct V {
+    T a, b;
+  };
+  chunk_walk<BRB>(c.len, [&](int k) { return V{a[k], b[k]}; }, [&](int, const V &v) { s += (double)v.a * (double)v.b; });
   s = bbsum(s);
   if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
@@ -134,15 +140,19 @@ __global__ __launch_bounds__(BRB) void k_bxr(const BVec *vt, int o, const BChunk
   const T *p = vec<T>(vt, c, o + VP), *q = vec<T>(vt, c, o + VQ), *dinv = vec<T>(vt, c, o + VD);
   const double al = sc[(int64_t)c.p * B_NS + B_ALPHA];
   double rz = 0., rr = 0.;
-  for (int k = threadIdx.x; k < c.len; k += BRB) {
-    x[k] = (T)((double)x[k] + al * (double)p[k]);
-    T ri = (T)((double)r[k] - al * (double)q[k]);
-    r[k] = ri;
-    T zi = (T)(dinv[k] * ri);
-    z[k] = zi;
-    rz += (double)ri * (double)zi;
-    rr += (double)ri * (double)ri;
-  }
+  struct V {
+    T x, p, r, q, d;
+  };
+  chunk_walk<BRB>(c.len, [&](int k) { return V{x[k], p[k], r[k], q[k], dinv[k]}; },
+                  [&](int k, const V &v) {
+                    x[k] = (T)((double)v.x + al * (double)v.p);
+                    const T ri = (T)((double)v.r - al * (double)v.q);
+                    r[k] = ri;
+                    const T zi = (T)(v.d * ri);
+                    z[k] = zi;
+                    rz += (double)ri * (double)zi;
+                    rr += (double)ri * (double)ri;
+                  });
   rz = bbsum(rz);
   rr = bbsum(rr);
   if (threadIdx.x == 0) { part[2 * blockIdx.x] = rz; part[2 * blockIdx.x + 1] = rr; }
@@ -157,10 +167,14 @@ __global__ __launch_bounds__(BRB) void k_bxr_mg(const BVec *vt, int o, const BCh
   T *x = vec<T>(vt, c, o + VX), *r = vec<T>(vt, c, o + VR);
   const T *p = vec<T>(vt, c, o + VP), *q = vec<T>(vt, c, o + VQ);
   const double al = sc[(int64_t)c.p * B_NS + B_ALPHA];
-  for (int k = threadIdx.x; k < c.len; k += BRB) {
-    x[k] = (T)((double)x[k] + al * (double)p[k]);
-    r[k] = (T)((double)r[k] - al * (double)q[k]);
-  }
+  struct V {
+    T x, p, r, q;
+  };
+  chunk_walk<BRB>(c.len, [&](int k) { return V{x[k], p[k], r[k], q[k]}; },
+                  [&](int k, const V &v) {
+                    x[k] = (T)((double)v.x + al * (double)v.p);
+                    r[k] = (T)((double)v.r - al * (double)v.q);
+                  });
 }
 // multigrid CG: partial sums of r.z and r.r (and p = z at the start); sc
 // (optional) skips frozen members
@@ -172,12 +186,16 @@ __global__ __launch_bounds__(BRB) void k_brz(const BVec *vt, int o, const BChunk
   const T *r = vec<T>(vt, c, o + VR), *z = vec<T>(vt, c, o + VZ);
   T *p = vec<T>(vt, c, o + VP);
   double rz = 0., rr = 0.;
-  for (int k = threadIdx.x; k < c.len; k += BRB) {
-    const double ri = r[k];
-    rz += ri * (double)z[k];
-    rr += ri * ri;
-    if (setp) p[k] = z[k];
-  }
+  struct V {
+    T r, z;
+  };
+  chunk_walk<BRB>(c.len, [&](int k) { return V{r[k], z[k]}; },
+                  [&](int k, const V &v) {
+                    const double ri = v.r;
+                    rz += ri * (double)v.z;
+                    rr += ri * ri;
+                    if (setp) p[k] = v.z;
+                  });
   rz = bbsum(rz);
   rr = bbsum(rr);
   if (threadIdx.x == 0) { part[2 * blockIdx.x] = rz; part[2 * blockIdx.x + 1] = rr; }
@@ -190,7 +208,11 @@ __global__ __launch_bounds__(BRB) void k_bp(const BVec *vt, int o, const BChunk 
   T *p = vec<T>(vt, c, o + VP);
   const T *z = vec<T>(vt, c, o + VZ);
   const double be = sc[(int64_t)c.p * B_NS + B_BETA];
-  for (int k = threadIdx.x; k < c.len; k += BRB) p[k] = (T)((double)z[k] + be * (double)p[k]);
+  struct V {
+    T z, p;
+  };
+  chunk_walk<BRB>(c.len, [&](int k) { return V{z[k], p[k]}; },
+                  [&](int k, const V &v) { p[k] = (T)((double)v.z + be * (double)v.p); });
 }
 
 // FP64 CG under the FP32 V-cycle (the single-problem default, batched):
@@ -202,12 +224,16 @@ __global__ __launch_bounds__(BRB) void k_bxr_mg64(const BVec *vt, const BChunk *
   const double *p = vec<double>(vt, c, VP), *q = vec<double>(vt, c, VQ);
   float *r32 = vec<float>(vt, c, VR32);
   const double al = sc[(int64_t)c.p * B_NS + B_ALPHA];
-  for (int k = threadIdx.x; k < c.len; k += BRB) {
-    x[k] += al * p[k];
-    const double ri = r[k] - al * q[k];
-    r[k] = ri;
-    r32[k] = (float)ri;
-  }
+  struct V {
+    double x, p, r, q;
+  };
+  chunk_walk<BRB>(c.len, [&](int k) { return V{x[k], p[k], r[k], q[k]}; },
+                  [&](int k, const V &v) {
+                    x[k] = v.x + al * v.p;
+                    const double ri = v.r - al * v.q;
+                    r[k] = ri;
+                    r32[k] = (float)ri;
+                  });
 }
 // r32 = r (before the first V-cycle)
 __global__ __launch_bounds__(BRB) void k_br32(const BVec *vt, const BChunk *__restrict__ ch) {
@@ -225,12 +251,17 @@ __global__ __launch_bounds__(BRB) void k_brz64(const BVec *vt, const BChunk *__r
   const float *z = vec<float>(vt, c, VZ32);
   double *p = vec<double>(vt, c, VP);
   double rz = 0., rr = 0.;
-  for (int k = threadIdx.x; k < c.len; k += BRB) {
-    const double ri = r[k], zi = (double)z[k];
-    rz += ri * zi;
-    rr += ri * ri;
-    if (setp) p[k] = zi;
-  }
+  struct V {
+    double r;
+    float z;
+  };
+  chunk_walk<BRB>(c.len, [&](int k) { return V{r[k], z[k]}; },
+                  [&](int k, const V &v) {
+                    const double zi = (double)v.z;
+                    rz += v.r * zi;
+                    rr += v.r * v.r;
+                    if (setp) p[k] = zi;
+                  });
   rz = bbsum(rz);
   rr = bbsum(rr);
   if (threadIdx.x == 0) { part[2 * blockIdx.x] = rz; part[2 * blockIdx.x + 1] = rr; }
@@ -242,7 +273,12 @@ __global__ __launch_bounds__(BRB) void k_bp64(const BVec *vt, const BChunk *__re
   double *p = vec<double>(vt, c, VP);
   const float *z = vec<float>(vt, c, VZ32);
   const double be = sc[(int64_t)c.p * B_NS + B_BETA];
-  for (int k = threadIdx.x; k < c.len; k += BRB) p[k] = (double)z[k] + be * p[k];
+  struct V {
+    float z;
+    double p;
+  };
+  chunk_walk<BRB>(c.len, [&](int k) { return V{z[k], p[k]}; },
+                  [&](int k, const V &v) { p[k] = (double)v.z + be * v.p; });
 }
 
 // R32 = R * scale_p ; X32 = 0
@@ -425,7 +461,8 @@ int vfg_batch_create(vfg_handle *const *members, int n, vfg_batch **out) {
   for (int p = 0; p < n; p++) {
     int64_t len = 3 * members[p]->P.nn;
     first[p] = (int)ch.size();
-    for (int64_t s = 0; s < len; s += CH) ch.push_back({p, s, (int)(len - s < CH ? len - s : CH)});
+    for (int64_t s = 0; s < len; s += chunk_entries(len))
+      ch.push_back({p, s, (int)(len - s < chunk_entries(len) ? len - s : chunk_entries(len))});
     nch[p] = (int)ch.size() - first[p];
   }
   b->nch = (int)ch.size();

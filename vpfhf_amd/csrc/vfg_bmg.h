@@ -16,7 +16,8 @@ struct BmgVec {
   const float *dinv;
   Grid G;
   BcMask bc;
-  int coarsest;  // 1 on the member's coarsest level
+  const void *op;  // the level's FP32 apply record (device)
+  int coarsest;    // 1 on the member's coarsest level
 };
 struct BmgChunk {
   int p;
@@ -27,12 +28,12 @@ struct BmgCoef {
   float c1, c2;
 };
 
-// the coarsest-level Chebyshev(MG_COARSE_DEG) solve, from x = 0, of every
-// member listed in ch[0, *dn) whose chunk starts its vector, one workgroup
-// each with the level in LDS (levels that satisfy mg_coarse_fits); ops: the
-// level's FP32 apply records, one per member
-void launch_bmg_coarse_cheb(const void *ops, const BmgVec *lvt, int level, const BmgChunk *ch, const int *dn,
-                            int grid, const BmgCoef *coef, const double *flags, int fstride, hipStream_t s);
+// the coarsest-level Chebyshev(MG_COARSE_DEG) solve, from x = 0, of the members
+// listed in ch[0, *dn), one workgroup each with the level in LDS (levels that
+// satisfy mg_coarse_fits): coarse = 1: {member, level (at least 1)}; coarse = 0:
+// level 0 of every member whose chunk starts its vector
+void launch_bmg_coarse_cheb(const BmgVec *lvt, int coarse, const BmgChunk *ch, const int *dn, int grid,
+                            const BmgCoef *coef, const double *flags, int fstride, hipStream_t s);
 
 struct BatchMG;
 // level plans of the members' hierarchies; r32[p] / z32[p]: the member's FP32

@@ -107,6 +107,8 @@ struct BatchMG {
   std::vector<vfg_handle *> m;        // per member (nullptr: empty slot)
   std::vector<float *> r32, z32;
   int np = 0, slots = 0;
+  Grow<BmgChunk> cch;                 // {member, coarsest level}: the one-launch coarsest solves
+  int *d_ccnt = nullptr;              // and their number
   int Lcap = 0;                       // levels whose lists have room (the V-cycle's launches)
   std::vector<int> L;                 // levels per member (0: empty)
   std::vector<std::vector<int>> oz;   // [p][l]
@@ -194,15 +196,27 @@ int bmg_set_member(BatchMG *g, int p, vfg_handle *h, float *r32, float *z32) {
   return VFG_OK;
 }
 
+// the coarsest level (below level 0) is solved in one workgroup
+static bool in_coarse_list(const BatchMG *g, int p) {
+  return g->L[p] > 1 && mg_coarse_fits(g->m[p]->mg->lv[g->L[p] - 1].P);
+}
+
 int bmg_rebuild(BatchMG *g, hipStream_t s, bool *grew) {
   int rc = VFG_OK;
+  g->cch.h.clear();
+  for (int p = 0; p < g->np; p++)
+    if (in_coarse_list(g, p)) g->cch.h.push_back({p, g->L[p] - 1, 1});
+  if (!g->d_ccnt && (rc = galloc(g, (void **)&g->d_ccnt, sizeof(int)))) return rc;
+  const int ccnt = (int)g->cch.h.size();
+  if ((rc = grow(g, g->cch, grew)) || (rc = push(g, g->cch, s))) return rc;
+  if (!g->up.put(g->d_ccnt, &ccnt, sizeof ccnt, s)) return VFG_E_HIP;
   int Lmax = 0;
   for (int p = 0; p < g->np; p++) Lmax = g->L[p] > Lmax ? g->L[p] : Lmax;
   for (int l = 0; l < BML && !rc; l++) {
     BmgPlan &P = g->lv[l];
     fill_list(g, l, [](int) { return true; }, P.M);
     fill_list(g, l, [&](int p) { return g->L[p] - 1 > l; }, P.D);
-    fill_list(g, l, [&](int p) { return g->L[p] - 1 == l; }, P.C);
+    fill_list(g, l, [&](int p) { return g->L[p] - 1 == l && !in_coarse_list(g, p); }, P.C);
     P.rch.h.clear();
     P.pch.h.clear();
     for (int p = 0; p < g->np; p++) {
@@ -228,7 +242,8 @@ int bmg_rebuild(BatchMG *g, hipStream_t s, bool *grew) {
     }
     P.hcnt[6] = (int)P.rch.h.size();
     P.hcnt[7] = (int)P.pch.h.size();
-    int cfit = P.C.ch.h.empty() ? 0 : 1;
+    // level 0 as the coarsest: the one-launch solve where all fit (or none is listed)
+    int cfit = l == 0;
     for (int p = 0; p < g->np && cfit; p++)
       if (g->m[p] && g->L[p] - 1 == l && !mg_coarse_fits(g->m[p]->mg->lv[l].P)) cfit = 0;
     if (cfit != P.cfit) *grew = true;  // the V-cycle's launches change
@@ -330,6 +345,7 @@ static void stage_member(BatchMG *g, int p) {
     BmgCoef *cf = &g->h_coef[((size_t)p * BML + l) * 2 * BMK];
     cheb_coefs(V.lmax / 11., V.lmax, MG_SMOOTH, cf);           // smoother
     cheb_coefs(V.lmax / 30., V.lmax, MG_COARSE_DEG, cf + BMK);  // coarsest level
+    v.op = (const char *)g->lv[l].ops + batch_op_bytes(1) * p;
     make_uop(V.P, v.x, v.y, 1, g->oz[p][l], g->h_ops[l].data() + batch_op_bytes(1) * p);
     // descending levels: pre-smoothing from 0 into d (b - A d into y), post-smoothing d -> x
     static_assert(MG_SMOOTH == 1, "the fused smoothing records do one Chebyshev step");
@@ -418,8 +434,8 @@ void bmg_vcycle(BatchMG *g, const double *flags, int fstride, hipStream_t s) {
     BmgPlan &P = g->lv[l];
     if (P.D.ch.cap) smooth(g, l, P.D, 0, flags, fstride, s);
     if (P.cfit) {
-      launch_bmg_coarse_cheb(P.ops, (const BmgVec *)g->d_lvt, l, (const BmgChunk *)P.C.ch.d,
-                             (const int *)(P.dcnt + 5), P.C.ch.cap, (const BmgCoef *)g->d_coef, flags, fstride, s);
+      launch_bmg_coarse_cheb((const BmgVec *)g->d_lvt, 0, (const BmgChunk *)P.C.ch.d, (const int *)(P.dcnt + 5),
+                             P.C.ch.cap, (const BmgCoef *)g->d_coef, flags, fstride, s);
     } else {
       for (int i = 0; i < BMK && P.C.ch.cap; i++) {
         if (i > 0) apply(g, l, P.C, 2, flags, fstride, s);
@@ -430,6 +446,9 @@ void bmg_vcycle(BatchMG *g, const double *flags, int fstride, hipStream_t s) {
       hipLaunchKernelGGL(k_bmg_restrict, dim3(P.rch.cap), dim3(256), 0, s, (const BmgVec *)g->d_lvt, l,
                          (const BmgChunk *)P.rch.d, (const int *)(P.dcnt + 6), flags, fstride);
   }
+  // the members' coarsest levels, whichever they are, at once
+  launch_bmg_coarse_cheb((const BmgVec *)g->d_lvt, 1, (const BmgChunk *)g->cch.d, (const int *)g->d_ccnt, g->cch.cap,
+                         (const BmgCoef *)g->d_coef, flags, fstride, s);
   for (int l = g->Lcap - 2; l >= 0; l--) {
     BmgPlan &P = g->lv[l];
     if (!P.D.ch.cap) continue;

@@ -35,7 +35,6 @@ enum {
   E_MGON,  // the V-cycle runs for the slot in this iteration (E_MG and E_ACTIVE)
   E_NS
 };
-constexpr int ECH = 4096;  // vector entries per chunk
 constexpr int ERB = 256;
 
 // vector slots of a request (its handle's solver work vectors, or U)
@@ -62,7 +61,10 @@ template <typename T>
 __device__ __forceinline__ double chunk_dot(const EVec &t, int sa, int sb, const EChunk &c) {
   const T *a = (const T *)t.v[sa] + c.start, *b = (const T *)t.v[sb] + c.start;
   double s = 0.;
-  for (int i = threadIdx.x; i < c.len; i += ERB) s += (double)a[i] * (double)b[i];
+  struct V {
+    T a, b;
+  };
+  chunk_walk<ERB>(c.len, [&](int k) { return V{a[k], b[k]}; }, [&](int, const V &v) { s += (double)v.a * (double)v.b; });
   return s;
 }
 
@@ -89,16 +91,20 @@ __device__ __forceinline__ void chunk_xr(const EVec &t, int o, const EChunk &c, 
   const T *p = (const T *)t.v[o + QP] + c.start, *q = (const T *)t.v[o + QQ] + c.start;
   const T *dinv = (const T *)t.v[o + QD] + c.start;
   float *rf = (float *)t.v[QR32] + c.start;  // FP32 copy of r for the V-cycle (an FP64 multigrid CG)
-  for (int k = threadIdx.x; k < c.len; k += ERB) {
-    x[k] = (T)((double)x[k] + al * (double)p[k]);
-    T ri = (T)((double)r[k] - al * (double)q[k]);
-    r[k] = ri;
-    if (r32) rf[k] = (float)ri;
-    T zi = (T)(dinv[k] * ri);
-    z[k] = zi;
-    rz += (double)ri * (double)zi;
-    rr += (double)ri * (double)ri;
-  }
+  struct V {
+    T x, p, r, q, d;
+  };
+  chunk_walk<ERB>(c.len, [&](int k) { return V{x[k], p[k], r[k], q[k], dinv[k]}; },
+                  [&](int k, const V &v) {
+                    x[k] = (T)((double)v.x + al * (double)v.p);
+                    const T ri = (T)((double)v.r - al * (double)v.q);
+                    r[k] = ri;
+                    if (r32) rf[k] = (float)ri;
+                    const T zi = (T)(v.d * ri);
+                    z[k] = zi;
+                    rz += (double)ri * (double)zi;
+                    rr += (double)ri * (double)ri;
+                  });
 }
 
 // x += alpha p; r -= alpha q; z = dinv r; part[2 pi] = r.z, part[2 pi + 1] = r.r
@@ -128,7 +134,11 @@ template <typename T>
 __device__ __forceinline__ void chunk_p(const EVec &t, int o, const EChunk &c, double be) {
   T *p = (T *)t.v[o + QP] + c.start;
   const T *z = (const T *)t.v[o + QZ] + c.start;
-  for (int k = threadIdx.x; k < c.len; k += ERB) p[k] = (T)((double)z[k] + be * (double)p[k]);
+  struct V {
+    T z, p;
+  };
+  chunk_walk<ERB>(c.len, [&](int k) { return V{z[k], p[k]}; },
+                  [&](int k, const V &v) { p[k] = (T)((double)v.z + be * (double)v.p); });
 }
 
 // p = z + beta p
@@ -167,11 +177,16 @@ __global__ __launch_bounds__(ERB) void k_e_rz(const EVec *__restrict__ vt, const
       const float *z32 = (const float *)t.v[QZ32] + k.start;
       double *z = (double *)t.v[QZ] + k.start;
       rz = 0.;
-      for (int i = threadIdx.x; i < k.len; i += ERB) {
-        const double zi = (double)z32[i];
-        z[i] = zi;
-        rz += r[i] * zi;
-      }
+      struct V {
+        double r;
+        float z;
+      };
+      chunk_walk<ERB>(k.len, [&](int i) { return V{r[i], z32[i]}; },
+                      [&](int i, const V &v) {
+                        const double zi = (double)v.z;
+                        z[i] = zi;
+                        rz += v.r * zi;
+                      });
     }
     rz = esum(rz);
     if (threadIdx.x == 0) part[2 * k.pi] = rz;
@@ -722,8 +737,9 @@ static int rebuild_lists(vfg_engine *e) {
       if ((pass == 0) != f32) continue;
       const int64_t len = q.kind == K_V64 ? q.h->P.nn : 3 * q.h->P.nn;
       e->h_first[p] = pi;
-      for (int64_t st = 0; st < len; st += ECH)
-        e->h_ch[f32 ? 0 : 1].push_back({p, pi++, st, (int)(len - st < ECH ? len - st : ECH), 0});
+      const int cl = chunk_entries(len);
+      for (int64_t st = 0; st < len; st += cl)
+        e->h_ch[f32 ? 0 : 1].push_back({p, pi++, st, (int)(len - st < cl ? len - st : cl), 0});
       e->h_nch[p] = pi - e->h_first[p];
     }
   for (int p = 0; p < e->ns; p++) {
@@ -877,7 +893,7 @@ int vfg_engine_create(const vfg_engine_opts *o, vfg_engine **out) {
   if (hipGetDeviceProperties(&prop, dev) == hipSuccess) cus = prop.multiProcessorCount;
   e->grid_apply = batch_slots(o->precision == VFG_PREC_MIXED);
   e->grid_vapply = v_apply_slots();
-  e->grid_vec = 4 * cus;
+  e->grid_vec = 8 * cus;
   bool ok = hipStreamCreateWithFlags(&e->s, hipStreamNonBlocking) == hipSuccess &&
             hipMalloc((void **)&e->d_sc, 8 * E_NS * (size_t)e->ns) == hipSuccess &&
             hipHostMalloc((void **)&e->h_sc, 8 * E_NS * (size_t)e->ns, hipHostMallocDefault) == hipSuccess &&

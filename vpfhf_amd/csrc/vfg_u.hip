@@ -1259,7 +1259,10 @@ __device__ __forceinline__ void mg_coarse_cheb_body(const UModOp<float, UNIT> &o
     const int c = t / nn, n = t - c * nn, ni = n % G.nx, nj = (n / G.nx) % G.ny, nk = n / (G.nx * G.ny);
     eb[q] = b[3 * n + c];
     ed[q] = dinv[3 * n + c];
-    fixed[q] = on_dirichlet(G, op.bc.face[c], op.bc.vert[c], ni, nj, nk);
+    // (selected: an index into the record would put it in scratch memory)
+    const uint8_t fc = c == 0 ? op.bc.face[0] : c == 1 ? op.bc.face[1] : op.bc.face[2];
+    const uint8_t vc = c == 0 ? op.bc.vert[0] : c == 1 ? op.bc.vert[1] : op.bc.vert[2];
+    fixed[q] = on_dirichlet(G, fc, vc, ni, nj, nk);
 #pragma unroll
     for (int a = 0; a < 8; a++) {
       const int ei = ni - (a & 1), ej = nj - ((a >> 1) & 1), ek = nk - (a >> 2);  // the node is its corner a
@@ -1345,22 +1348,22 @@ __global__ __launch_bounds__(MGC_T) void k_mg_coarse_cheb(UModOp<float, true> op
   mg_coarse_cheb_body<true>(op, b, dinv, xout, cc.k, [&](int i) { return BmgCoef{cc.c1[i], cc.c2[i]}; });
 }
 
-// the batched form: one workgroup per listed member (its first chunk), the
-// member's level operator, vectors and coarsest-level coefficients from the
-// engine's tables
-template <bool UNIT>
-__global__ __launch_bounds__(MGC_T) void k_bmg_coarse_cheb(const BApply<float> *__restrict__ ops,
-                                                           const BmgVec *__restrict__ lvt, int level,
+// the batched form: one workgroup per listed member (COARSE: at the level its
+// entry names; else level 0, its first chunk), the member's level operator,
+// vectors and coarsest-level coefficients from the engine's tables
+template <bool COARSE>
+__global__ __launch_bounds__(MGC_T) void k_bmg_coarse_cheb(const BmgVec *__restrict__ lvt,
                                                            const BmgChunk *__restrict__ ch, const int *__restrict__ dn,
                                                            const BmgCoef *__restrict__ coef,
                                                            const double *__restrict__ flags, int fstride) {
   if ((int)blockIdx.x >= *dn) return;
   const BmgChunk c = ch[blockIdx.x];
-  if (c.start != 0 || flags[(int64_t)c.p * fstride] == 0.) return;  // uniform in the workgroup
+  if ((!COARSE && c.start != 0) || flags[(int64_t)c.p * fstride] == 0.) return;  // uniform in the workgroup
+  const int level = COARSE ? (int)c.start : 0;
   const BmgVec &v = lvt[c.p * BML + level];
   const BmgCoef *__restrict__ cf = coef + ((c.p * BML + level) * 2 + 1) * BMK;
-  mg_coarse_cheb_body<UNIT>(op_of<UModOp<float, UNIT>>(ops[c.p].op), v.b, v.dinv, v.x, MG_COARSE_DEG,
-                            [&](int i) { return cf[i]; });
+  mg_coarse_cheb_body<COARSE>(op_of<UModOp<float, COARSE>>(((const BApply<float> *)v.op)->op), v.b, v.dinv, v.x,
+                              MG_COARSE_DEG, [&](int i) { return cf[i]; });
 }
 
 bool mg_coarse_fits(const DevProblem &P) {
@@ -1374,16 +1377,11 @@ void launch_mg_coarse_cheb(const DevProblem &P, const float *b, const float *din
   hipLaunchKernelGGL(k_mg_coarse_cheb, dim3(1), dim3(MGC_T), 0, s, op, b, dinv, x, cc);
 }
 
-void launch_bmg_coarse_cheb(const void *ops, const BmgVec *lvt, int level, const BmgChunk *ch, const int *dn,
-                            int grid, const BmgCoef *coef, const double *flags, int fstride, hipStream_t s) {
+void launch_bmg_coarse_cheb(const BmgVec *lvt, int coarse, const BmgChunk *ch, const int *dn, int grid,
+                            const BmgCoef *coef, const double *flags, int fstride, hipStream_t s) {
   if (grid <= 0) return;
-  // level 0: a problem small enough to be its own coarsest level
-  if (level > 0)
-    hipLaunchKernelGGL(k_bmg_coarse_cheb<true>, dim3(grid), dim3(MGC_T), 0, s, (const BApply<float> *)ops, lvt, level,
-                       ch, dn, coef, flags, fstride);
-  else
-    hipLaunchKernelGGL(k_bmg_coarse_cheb<false>, dim3(grid), dim3(MGC_T), 0, s, (const BApply<float> *)ops, lvt,
-                       level, ch, dn, coef, flags, fstride);
+  auto go = [&](auto k) { hipLaunchKernelGGL(k, dim3(grid), dim3(MGC_T), 0, s, lvt, ch, dn, coef, flags, fstride); };
+  coarse ? go(k_bmg_coarse_cheb<true>) : go(k_bmg_coarse_cheb<false>);
 }
 
 void launch_u_apply(const DevProblem &P, const double *x, double *y, hipStream_t s) {
