@@ -185,8 +185,12 @@ int bmg_set_member(BatchMG *g, int p, vfg_handle *h, float *r32, float *z32) {
   g->z32[p] = z32;
   g->L[p] = 0;
   if (!h) return VFG_OK;
+  const bool fresh = !h->mg;
   int rc = mg_build(h);
   if (rc) return rc;
+  // the coarse levels' v = 1 is written on the handle's stream, the engine's
+  // set-ups run on its own
+  if (fresh && hipStreamSynchronize(h->stream) != hipSuccess) return VFG_E_HIP;
   g->L[p] = h->mg->L;
   for (int l = 0; l < g->L[p]; l++) {
     const Grid &G = level_grid(g, p, l);
