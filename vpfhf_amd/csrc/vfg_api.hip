@@ -43,6 +43,27 @@ int vfg_alloc(vfg_handle *h, void **p, size_t bytes) {
   return VFG_OK;
 }
 
+// several arrays in one allocation (an allocation or a release costs tens of
+// microseconds each, and a release waits for the device); arrays that exist stay
+int vfg_alloc_group(vfg_handle *h, const std::vector<VfgAlloc> &a) {
+  size_t sum = 0;
+  const auto up = [](size_t b) { return (b + 255) / 256 * 256; };
+  for (const VfgAlloc &q : a)
+    if (!*q.p) sum += up(q.bytes);
+  if (!sum) return VFG_OK;
+  char *base = nullptr;
+  const hipError_t e = hipMalloc((void **)&base, sum);
+  if (e != hipSuccess) return vfg_fail(h, VFG_E_NOMEM, "hipMalloc(%zu): %s", sum, hipGetErrorString(e));
+  h->allocs.push_back(base);
+  for (const VfgAlloc &q : a) {
+    if (*q.p) continue;
+    *q.p = base;
+    base += up(q.bytes);
+    h->bytes += q.bytes;
+  }
+  return VFG_OK;
+}
+
 static void bcmask_from(const vfg_bc *bc, int dof, BcMask *m) {
   for (int c = 0; c < dof; c++) {
     uint8_t f = 0, v = 0;
@@ -141,12 +162,11 @@ int vfg_create(const vfg_grid *g, const vfg_props *pr, vfg_handle **out) {
     return vfg_fail(nullptr, VFG_E_HIP, "vfg_create: hipStreamCreate failed");
   }
   int rc;
-  if ((rc = vfg_alloc(h, (void **)&P.V, 8 * P.nn)) || (rc = vfg_alloc(h, (void **)&P.VIrrev, 8 * P.nn)) ||
-      (rc = vfg_alloc(h, (void **)&P.dth, 8 * P.nn)) || (rc = vfg_alloc(h, (void **)&P.p, 8 * P.nn)) ||
-      (rc = vfg_alloc(h, (void **)&P.V32, 4 * P.nn)) || (rc = vfg_alloc(h, (void **)&P.zero3, 24 * P.nn)) ||
-      (rc = vfg_alloc(h, (void **)&P.vfix, P.nn)) || (rc = vfg_alloc(h, (void **)&P.bV, 8 * P.nn)) ||
-      (rc = vfg_alloc(h, (void **)&h->part, 8 * 4 * 65536)) || (rc = vfg_alloc(h, (void **)&h->scal, 8 * 64)) ||
-      (rc = vfg_alloc(h, (void **)&P.cmask, 4 * P.ne))) {
+  const size_t nn = (size_t)P.nn;
+  if ((rc = vfg_alloc_group(h, {{(void **)&P.V, 8 * nn}, {(void **)&P.VIrrev, 8 * nn}, {(void **)&P.dth, 8 * nn},
+                                {(void **)&P.p, 8 * nn}, {(void **)&P.V32, 4 * nn}, {(void **)&P.zero3, 24 * nn},
+                                {(void **)&P.vfix, nn}, {(void **)&P.bV, 8 * nn}, {(void **)&h->part, 8 * 4 * 65536},
+                                {(void **)&h->scal, 8 * 64}, {(void **)&P.cmask, 4 * (size_t)P.ne}}))) {
     snprintf(g_err, sizeof g_err, "%s", h->err.c_str());
     vfg_destroy(h);
     return rc;

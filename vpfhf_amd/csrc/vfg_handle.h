@@ -73,6 +73,11 @@ int vfg_fail(vfg_handle *h, int code, const char *fmt, ...);
 int vfg_u_prepare(vfg_handle *h);
 inline void vfg_u_invalidate(vfg_handle *h) { h->P.uq = nullptr; }
 int vfg_alloc(vfg_handle *h, void **p, size_t bytes);
+struct VfgAlloc {
+  void **p;
+  size_t bytes;
+};
+int vfg_alloc_group(vfg_handle *h, const std::vector<VfgAlloc> &a);  // several arrays in one allocation
 int vfg_scratch(vfg_handle *h, int64_t ndoubles);
 // solver work vectors of 3*nn entries: w[0..n64) FP64 and wf[0..n32) FP32
 int vfg_work(vfg_handle *h, int n64, int n32);

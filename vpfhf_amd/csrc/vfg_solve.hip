@@ -282,20 +282,17 @@ static int pcg_fused(vfg_handle *h, int64_t n, const FusedFn &A, const double *d
   return status;
 }
 
-static int work(vfg_handle *h, int nvec, int64_t n) {
-  for (int i = 0; i < nvec; i++) {
-    if (h->w[i]) continue;
-    int rc = vfg_alloc(h, (void **)&h->w[i], 8 * (size_t)n);
-    if (rc) return rc;
-  }
-  return VFG_OK;
+// work vectors w[0..n64) of n doubles and wf[0..n32) of n floats
+static int work(vfg_handle *h, int n64, int64_t n, int n32 = 0) {
+  std::vector<VfgAlloc> a;
+  for (int i = 0; i < n64; i++) a.push_back({(void **)&h->w[i], 8 * (size_t)n});
+  for (int i = 0; i < n32; i++) a.push_back({(void **)&h->wf[i], 4 * (size_t)n});
+  return vfg_alloc_group(h, a);
 }
 }  // namespace vfg
 int vfg_work(vfg_handle *h, int n64, int n32) {
   const int64_t n = 3 * h->P.nn;
-  int rc = vfg::work(h, n64, n);
-  for (int i = 0; i < n32 && !rc; i++) rc = vfg_alloc(h, (void **)&h->wf[i], 4 * (size_t)n);
-  return rc;
+  return vfg::work(h, n64, n, n32);
 }
 namespace vfg {
 
@@ -729,13 +726,12 @@ int mg_build(vfg_handle *h) {
   l0.P = h->P;
   l0.P.uq = nullptr;  // level 0 runs the FP32 apply only
   l0.n = 3 * h->P.nn;
-  rc = vfg_alloc(h, (void **)&l0.dinv, 4 * (size_t)l0.n);
-  if (!rc) rc = vfg_alloc(h, (void **)&l0.y, 4 * (size_t)l0.n);
-  if (!rc) rc = vfg_alloc(h, (void **)&l0.d, 4 * (size_t)l0.n);
+  std::vector<VfgAlloc> al;
+  for (float **f : {&l0.dinv, &l0.y, &l0.d}) al.push_back({(void **)f, 4 * (size_t)l0.n});
   int L = 1;
   Grid G = h->P.G;
   auto halve = [](int n) { return n > MG_COARSEST ? (n + 1) / 2 : n; };
-  while (!rc && L < MgHier::MAXL) {
+  while (L < MgHier::MAXL) {
     Grid Gc;
     Gc.nex = halve(G.nex); Gc.ney = halve(G.ney); Gc.nez = halve(G.nez);
     if (Gc.nex == G.nex && Gc.ney == G.ney && Gc.nez == G.nez) break;
@@ -749,19 +745,20 @@ int mg_build(vfg_handle *h) {
     Pc.ne = (int64_t)Gc.nex * Gc.ney * Gc.nez;
     Pc.unit = 1;
     lc.n = 3 * Pc.nn;
-    if ((rc = vfg_alloc(h, (void **)&Pc.E_elem, 8 * (size_t)Pc.ne)) ||
-        (rc = vfg_alloc(h, (void **)&Pc.V, 8 * (size_t)Pc.nn)) ||
-        (rc = vfg_alloc(h, (void **)&Pc.V32, 4 * (size_t)Pc.nn)))
-      break;
-    float **fv[5] = {&lc.dinv, &lc.b, &lc.x, &lc.y, &lc.d};
-    for (int i = 0; i < 5 && !rc; i++) rc = vfg_alloc(h, (void **)fv[i], 4 * (size_t)lc.n);
-    if (rc) break;
-    launch_fill(Pc.V, 1., Pc.nn, h->stream);
-    launch_mg_fill32(Pc.V32, 1.f, Pc.nn, h->stream);
+    al.push_back({(void **)&Pc.E_elem, 8 * (size_t)Pc.ne});
+    al.push_back({(void **)&Pc.V, 8 * (size_t)Pc.nn});
+    al.push_back({(void **)&Pc.V32, 4 * (size_t)Pc.nn});
+    for (float **f : {&lc.dinv, &lc.b, &lc.x, &lc.y, &lc.d}) al.push_back({(void **)f, 4 * (size_t)lc.n});
     G = Gc;
     L++;
   }
-  if (!rc && L > 1) rc = vfg_alloc(h, (void **)&m->dtmp, 8 * (size_t)m->lv[1].n);
+  if (L > 1) al.push_back({(void **)&m->dtmp, 8 * (size_t)m->lv[1].n});
+  rc = vfg_alloc_group(h, al);
+  for (int l = 1; l < L && !rc; l++) {
+    const DevProblem &Pc = m->lv[l].P;
+    launch_fill(Pc.V, 1., Pc.nn, h->stream);
+    launch_mg_fill32(Pc.V32, 1.f, Pc.nn, h->stream);
+  }
   if (rc) {
     delete m;
     return rc;
@@ -781,9 +778,7 @@ int mg_setup_begin(vfg_handle *h, const double *dinv64, hipStream_t s) {
   if (rc) return rc;
   MgHier &m = *h->mg;
   const int64_t nf = 3 * h->P.nn;
-  for (int i = 0; i < 7; i++)
-    if (!h->wf[i] && (rc = vfg_alloc(h, (void **)&h->wf[i], 4 * (size_t)nf))) return rc;
-  if (m.L > 1 && (rc = work(h, 8, nf))) return rc;  // w[7]: per-element coefficients of the problem
+  if ((rc = work(h, m.L > 1 ? 8 : 0, nf, 7))) return rc;  // w[7]: per-element coefficients of the problem
   m.lv[0].P = h->P;
   launch_copy_d2f(dinv64, m.lv[0].dinv, nf, s);
   for (int l = 1; l < m.L; l++) {
