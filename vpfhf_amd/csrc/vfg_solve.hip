@@ -114,14 +114,6 @@ __global__ __launch_bounds__(RB) void k_pcg_p(double *__restrict__ p, const doub
     p[i] = z[i] + be * p[i];
 }
 
-// p = z + beta p with z the FP32 preconditioner output (exact in FP64)
-__global__ __launch_bounds__(RB) void k_pcg_p32(double *__restrict__ p, const float *__restrict__ z32, int64_t n,
-                                                const double *sc) {
-  const double be = sc[S_BETA];
-  for (int64_t i = (int64_t)blockIdx.x * RB + threadIdx.x; i < n; i += (int64_t)gridDim.x * RB)
-    p[i] = (double)z32[i] + be * p[i];
-}
-
 __global__ void k_recip(const double *d, double *dinv, int64_t n) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) dinv[i] = d[i] != 0. ? 1. / d[i] : 1.;
@@ -906,48 +898,72 @@ static int mg_apply(vfg_handle *h, const float *r, float *z, const double *r64, 
   return mg_vcycle(h, 0, r64, part);
 }
 
-// x += alpha p ; r -= alpha q ; r32 = r; with part, one partial of r.r per block
-__global__ __launch_bounds__(RB) void k_mg_xr(double *__restrict__ x, double *__restrict__ r,
-                                              const double *__restrict__ p, const double *__restrict__ q,
-                                              float *__restrict__ r32, int64_t n, const double *sc, double *part) {
-  const double al = sc[S_ALPHA];
+// The vector updates of an iteration.  Each workgroup sums the partials of the
+// inner products itself, in the same order (a scalar kernel between them costs
+// 3.5 us and a launch gap; a 32^3 solve 1.61 -> 1.53 ms), and the first one keeps
+// the scalars.  r.z alternates between two places, so that none is read and
+// written by one launch.  x is updated with the next direction, which reads p
+// anyway (128^3: 84 -> 75 us for both).
+__device__ __forceinline__ int rz_slot(int k) { return k & 1 ? (int)S_TMP0 : (int)S_RZ; }
+// alpha = r.z / p.q (partials ppq[0, na)); r -= alpha q; r32 = r; partials of r.r
+__global__ __launch_bounds__(RB) void k_mg_r(double *__restrict__ r, const double *__restrict__ q,
+                                             float *__restrict__ r32, int64_t n, const double *__restrict__ ppq, int na,
+                                             int k, double *sc, double *__restrict__ prr) {
+  const double pq = lz_sum(ppq, na);
+  const bool ok = pq > 0. && isfinite(pq);
+  const double al = ok ? sc[rz_slot(k)] / pq : 0.;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    sc[S_PQ] = pq;
+    sc[S_ALPHA] = al;
+    if (!ok) sc[S_FLAG] = isfinite(pq) ? 1. : 2.;
+  }
   double rr = 0.;
   for (int64_t i = (int64_t)blockIdx.x * RB + threadIdx.x; i < n; i += (int64_t)gridDim.x * RB) {
-    x[i] += al * p[i];
     const double ri = r[i] - al * q[i];
     r[i] = ri;
     r32[i] = (float)ri;
     rr += ri * ri;
   }
-  if (part) {
-    rr = bsum(rr);
-    if (threadIdx.x == 0) part[blockIdx.x] = rr;
+  rr = bsum(rr);
+  if (threadIdx.x == 0) prr[blockIdx.x] = rr;
+}
+// beta from the partials of r.z; x += alpha p; p = z32 + beta p
+__global__ __launch_bounds__(RB) void k_mg_xp(double *__restrict__ x, double *__restrict__ p,
+                                              const float *__restrict__ z32, int64_t n, const double *__restrict__ prz,
+                                              int nrz, const double *__restrict__ prr, int nrr, int k, double *sc) {
+  const double rz = lz_sum(prz, nrz), old = sc[rz_slot(k)], al = sc[S_ALPHA];
+  const double be = old != 0. ? rz / old : 0.;
+  if (blockIdx.x == 0) {
+    const double rr = lz_sum(prr, nrr);
+    if (threadIdx.x == 0) {
+      sc[S_BETA] = be;
+      sc[rz_slot(k + 1)] = rz;
+      sc[S_RR] = rr;
+      if (!isfinite(rz) || !isfinite(rr)) sc[S_FLAG] = 2.;
+    }
+  }
+  for (int64_t i = (int64_t)blockIdx.x * RB + threadIdx.x; i < n; i += (int64_t)gridDim.x * RB) {
+    const double pi = p[i];
+    x[i] += al * pi;
+    p[i] = (double)z32[i] + be * pi;
   }
 }
-// op 2 of k_pcg_scalar (beta, rz, rr) from separate partials: rz from prz[0, nrz), rr from prr[0, nrr)
-__global__ __launch_bounds__(RB) void k_pcg_beta_split(const double *prz, int nrz, const double *prr, int nrr,
-                                                       double *sc) {
-  double a = 0., b = 0.;
-  for (int i = threadIdx.x; i < nrz; i += RB) a += prz[i];
-  for (int i = threadIdx.x; i < nrr; i += RB) b += prr[i];
-  a = bsum(a);
-  b = bsum(b);
-  if (threadIdx.x != 0 || sc[S_DONE] != 0.) return;
-  const double rz = sc[S_RZ];
-  sc[S_BETA] = rz != 0. ? a / rz : 0.;
-  sc[S_RZ] = a;
-  sc[S_RR] = b;
-  sc[S_ITS] += 1.;
-  if (!isfinite(a) || !isfinite(b)) sc[S_FLAG] = 2.;
-  else if (sc[S_TOL2] > 0. && b <= sc[S_TOL2]) sc[S_DONE] = 1.;
+// partials of r.z with z = z32
+__global__ __launch_bounds__(RB) void k_mg_dot(const double *__restrict__ r, const float *__restrict__ z32, int64_t n,
+                                               double *part) {
+  double s = 0.;
+  for (int64_t i = (int64_t)blockIdx.x * RB + threadIdx.x; i < n; i += (int64_t)gridDim.x * RB)
+    s += r[i] * (double)z32[i];
+  s = bsum(s);
+  if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
-// partial sums of r.z and r.r with z = z32 (and p = z when p != nullptr)
+// partial sums of r.z and r.r with z = z32, and p = z
 __global__ __launch_bounds__(RB) void k_mg_rz(const double *__restrict__ r, const float *__restrict__ z32,
                                               double *__restrict__ p, int64_t n, double *part) {
   double rz = 0., rr = 0.;
   for (int64_t i = (int64_t)blockIdx.x * RB + threadIdx.x; i < n; i += (int64_t)gridDim.x * RB) {
     const double ri = r[i], zi = (double)z32[i];
-    if (p) p[i] = zi;
+    p[i] = zi;
     rz += ri * zi;
     rr += ri * ri;
   }
@@ -992,22 +1008,18 @@ static int pcg_mg(vfg_handle *h, int64_t n, const ApplyFn &A, double *x, double 
         hipLaunchKernelGGL(k_dotp, dim3(nb), dim3(RB), 0, s, (const double *)p, (const double *)q, n, part);
         na = nb;
       }
-      hipLaunchKernelGGL(k_pcg_scalar, dim3(1), dim3(RB), 0, s, (const double *)part, na, 1, sc);
       // r.r partials from the update, r.z partials from the V-cycle's last
       // kernel (in two regions of part past the apply's partials)
       double *prr = part + 65536, *prz = part + 2 * 65536;
-      hipLaunchKernelGGL(k_mg_xr, dim3(nb), dim3(RB), 0, s, x, r, (const double *)p, (const double *)q, r32, n,
-                         (const double *)sc, prr);
-      const int nrz = mg_apply(h, r32, z32, r, prz);  // at most 2 x 65536 partials
-      if (nrz > 0) {
-        hipLaunchKernelGGL(k_pcg_beta_split, dim3(1), dim3(RB), 0, s, (const double *)prz, nrz, (const double *)prr,
-                           nb, sc);
-      } else {
-        hipLaunchKernelGGL(k_mg_rz, dim3(nb), dim3(RB), 0, s, (const double *)r, (const float *)z32,
-                           (double *)nullptr, n, part);
-        hipLaunchKernelGGL(k_pcg_scalar, dim3(1), dim3(RB), 0, s, (const double *)part, nb, 2, sc);
+      hipLaunchKernelGGL(k_mg_r, dim3(nb), dim3(RB), 0, s, r, (const double *)q, r32, n, (const double *)part, na,
+                         it + k, sc, prr);
+      int nrz = mg_apply(h, r32, z32, r, prz);  // at most 2 x 65536 partials
+      if (!nrz) {
+        hipLaunchKernelGGL(k_mg_dot, dim3(nb), dim3(RB), 0, s, (const double *)r, (const float *)z32, n, prz);
+        nrz = nb;
       }
-      hipLaunchKernelGGL(k_pcg_p32, dim3(nb), dim3(RB), 0, s, p, (const float *)z32, n, (const double *)sc);
+      hipLaunchKernelGGL(k_mg_xp, dim3(nb), dim3(RB), 0, s, x, p, (const float *)z32, n, (const double *)prz, nrz,
+                         (const double *)prr, nb, it + k, sc);
     }
     it += todo;
     if (hipMemcpyAsync(hs, sc, 64, hipMemcpyDeviceToHost, s) != hipSuccess || hipStreamSynchronize(s) != hipSuccess)
