@@ -95,25 +95,37 @@ void launch_v_chunk_list(const DevProblem &P, const uint8_t *mask, uint32_t *fla
 // element with a listed node, where K x changes when x changes on the listed
 // nodes only
 void launch_v_dilated_list(const DevProblem &P, const uint32_t *flag, uint32_t *flag2, int *list2, hipStream_t s);
+// scalars of a CG (vfg_handle::scal)
+enum { S_RZ = 0, S_PQ, S_ALPHA, S_BETA, S_RR, S_RR0, S_FLAG, S_TMP0, S_TMP1, S_TMP2, S_TOL2, S_DONE, S_ITS };
+// Iteration k of the V-CG as its kernels see it: every workgroup sums the
+// partials of the previous launch itself, the first one keeps the scalars, each
+// of which is written by one launch and read by the next.
+struct VCgStep {
+  const double *pairs;  // (r.z, r.r) of the current residual
+  int npairs, k;
+  double tol2;          // > 0: r.r <= tol2 ends the solve
+  double *sc;
+};
+// partials a list can hold: its chunks, or the blocks of a reduction
+size_t vcg_partials(const Grid &G);
 // CG-fused masked V apply (mask: fixed or active nodes) over the listed
-// chunks: p = z + beta p_old staged, q = K p, p and q written on the chunks'
-// owned nodes (p, q must be zero on the other chunks), one partial of p.q per
-// chunk; returns the number of partials (= count)
-int launch_v_apply_cg_list(const DevProblem &P, const double *pold, double *p, const double *z, const double *beta,
-                           double *q, double *part, const uint8_t *mask, const int *list, int count, hipStream_t s,
-                           const double *done = nullptr);
+// chunks: beta from the step's r.z, p = z + beta p_old staged, q = K p, p and q
+// written on the chunks' owned nodes (p, q must be zero on the other chunks),
+// one partial of p.q per chunk.  Marks the solve done, and does nothing, once
+// r.r has reached tol2.
+void launch_v_apply_cg_list(const DevProblem &P, const double *pold, double *p, const double *z, double *q, double *part,
+                            const uint8_t *mask, const int *list, int count, const VCgStep &c, hipStream_t s);
 // launch_v_apply and launch_v_diag over the listed chunks' owned nodes (the
 // other entries of y, d are left as they are)
 void launch_v_apply_list(const DevProblem &P, const double *x, double *y, int mode, const int *list, int count,
                          hipStream_t s, const uint8_t *mask = nullptr);
 void launch_v_diag_list(const DevProblem &P, double *d, const uint8_t *mask, const int *list, int count,
                         hipStream_t s);
-// the CG update x += a p, r -= a q, z = dinv r over the listed chunks, with
-// (r.z, r.r) partial pairs; returns their number (= count)
-int launch_v_xr_list(const Grid &G, const int *list, int count, double *x, double *r, double *z, const double *p,
-                     const double *q, const double *dinv, const double *alpha, double *part, hipStream_t s,
-                     const double *done = nullptr);
-// (both: the launch does nothing once *done != 0, a device-side stop of the CG)
+// the CG update x += a p, r -= a q, z = dinv r over the listed chunks, a = r.z /
+// p.q from ppq[0, count), with the next (r.z, r.r) in pairs (one per chunk)
+void launch_v_xr_list(const Grid &G, const int *list, int count, double *x, double *r, double *z, const double *p,
+                      const double *q, const double *dinv, const double *ppq, double *pairs, const VCgStep &c,
+                      hipStream_t s);
 
 // misc (vfg_misc.hip)
 void launch_bc_mask(const DevProblem &P, int which, uint8_t *mask, hipStream_t s);

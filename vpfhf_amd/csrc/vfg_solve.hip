@@ -23,7 +23,6 @@
 
 namespace vfg {
 
-enum { S_RZ = 0, S_PQ, S_ALPHA, S_BETA, S_RR, S_RR0, S_FLAG, S_TMP0, S_TMP1, S_TMP2, S_TOL2, S_DONE, S_ITS };
 constexpr int RB = 256;
 
 __device__ __forceinline__ double bsum(double v) {
@@ -61,9 +60,6 @@ __global__ __launch_bounds__(RB) void k_pcg_scalar(const double *part, int nb, i
   if (threadIdx.x != 0) return;
   if (op == 0) {
     sc[S_RZ] = a; sc[S_RR] = b; sc[S_RR0] = b; sc[S_FLAG] = 0.;
-    sc[S_TOL2] = 0.; sc[S_DONE] = 0.; sc[S_ITS] = 0.;
-  } else if (sc[S_DONE] != 0.) {
-    return;  // converged: the rest of the iteration batch does nothing
   } else if (op == 1) {
     sc[S_PQ] = a;
     if (!(a > 0.) || !isfinite(a)) { sc[S_ALPHA] = 0.; sc[S_FLAG] = isfinite(a) ? 1. : 2.; }
@@ -73,9 +69,7 @@ __global__ __launch_bounds__(RB) void k_pcg_scalar(const double *part, int nb, i
     sc[S_BETA] = rz != 0. ? a / rz : 0.;
     sc[S_RZ] = a;
     sc[S_RR] = b;
-    sc[S_ITS] += 1.;
     if (!isfinite(a) || !isfinite(b)) sc[S_FLAG] = 2.;
-    else if (sc[S_TOL2] > 0. && b <= sc[S_TOL2]) sc[S_DONE] = 1.;  // only solvers whose kernels all check S_DONE set S_TOL2
   }
 }
 
@@ -129,21 +123,6 @@ typedef std::function<void(const double *, double *)> ApplyFn;
 // apply with the x.y partials written to h->part: (x, y) -> their number, 0
 // when the operator has no such kernel (nothing launched then)
 typedef std::function<int(const double *, double *)> DotApplyFn;
-// fused apply: (p_old, p, q) -> number of p.q partials written to h->part
-typedef std::function<int(const double *, double *, double *)> FusedFn;
-// CG update over a subset of the nodes: (p, q) -> number of (r.z, r.r)
-// partial pairs written to h->part
-typedef std::function<int(const double *, const double *)> XrFn;
-
-
-// Preconditioned CG with the direction update and the p.q product fused into
-// the operator apply (launch_v_apply_cg_list): per iteration
-// one apply, one vector update of x, r, z and two scalar steps.  p alternates
-// between two arrays.  Same convergence test and reporting as pcg().
-static int pcg_fused(vfg_handle *h, int64_t n, const FusedFn &A, const double *dinv, double *x, double *r,
-                     double *z, double *p, double *p2, double *q, double rtol, double atol, int maxit, int check,
-                     vfg_solve_info *info, const XrFn *xr = nullptr, double rn0_known = -1., int first = 0);
-
 // Preconditioned CG on the device.  On entry x is the initial guess and r the
 // initial residual b - A x.  Converged when ||r|| <= max(rtol*||r0||, atol).
 static int pcg(vfg_handle *h, int64_t n, const ApplyFn &A, const double *dinv, double *x, double *r, double *z,
@@ -206,60 +185,96 @@ static int pcg(vfg_handle *h, int64_t n, const ApplyFn &A, const double *dinv, d
   return status;
 }
 
-__global__ void k_set_scalar(double *sc, int i, double v) { sc[i] = v; }
 // two device counts next to a scalar, so that one copy reads all three
 __global__ void k_pack_counts(const int *a, const int *b, double *out) {
   out[0] = (double)*a;
   out[1] = (double)*b;
 }
 
-static int pcg_fused(vfg_handle *h, int64_t n, const FusedFn &A, const double *dinv, double *x, double *r,
-                     double *z, double *p, double *p2, double *q, double rtol, double atol, int maxit, int check,
-                     vfg_solve_info *info, const XrFn *xr, double rn0_known, int first) {
+// start of the V-CG: z = dinv r, p = z (finite where the first direction reads
+// it), pairs (r.z, r.r); the scalars of the solve
+__global__ __launch_bounds__(RB) void k_vcg_init(const double *__restrict__ r, double *__restrict__ z,
+                                                 double *__restrict__ p, const double *__restrict__ dinv, int64_t n,
+                                                 double *pairs, double *sc) {
+  double rz = 0., rr = 0.;
+  for (int64_t i = (int64_t)blockIdx.x * RB + threadIdx.x; i < n; i += (int64_t)gridDim.x * RB) {
+    const double ri = r[i], zi = dinv[i] * ri;
+    z[i] = zi;
+    p[i] = zi;
+    rz += ri * zi;
+    rr += ri * ri;
+  }
+  rz = bsum(rz);
+  rr = bsum(rr);
+  if (threadIdx.x != 0) return;
+  pairs[2 * blockIdx.x] = rz;
+  pairs[2 * blockIdx.x + 1] = rr;
+  if (blockIdx.x == 0) sc[S_FLAG] = sc[S_DONE] = sc[S_ITS] = 0.;
+}
+// end of a batch after iteration k - 1: what the next apply would decide
+__global__ __launch_bounds__(RB) void k_vcg_final(VCgStep c) {
+  if (c.sc[S_DONE] != 0.) return;
+  double rz = 0., rr = 0.;
+  for (int i = threadIdx.x; i < c.npairs; i += RB) {
+    rz += c.pairs[2 * i];
+    rr += c.pairs[2 * i + 1];
+  }
+  rz = bsum(rz);
+  rr = bsum(rr);
+  if (threadIdx.x != 0) return;
+  c.sc[S_RR] = rr;
+  c.sc[S_ITS] = (double)c.k;
+  if (!isfinite(rz) || !isfinite(rr)) c.sc[S_FLAG] = 2.;
+  else if (c.tol2 > 0. && rr <= c.tol2) c.sc[S_DONE] = 1.;
+}
+
+// Preconditioned CG of the reduced V system over the listed chunks, two
+// launches per iteration: the apply with the direction update and p.q, and the
+// update of x, r, z with (r.z, r.r).  Each forms the scalars it needs from the
+// partials of the one before (VCgStep).  The iteration that reaches tol marks
+// the solve done on the device and the rest of its batch exits at once.  p
+// alternates between p and p2, the pairs between two buffers of h->vpart (after
+// its p.q partials).  rn0: ||r0||; first > 0: the caller's estimate of the
+// iterations needed (launches after the stop cost a launch each, for nothing).
+// Same convergence test and reporting as pcg().
+static int pcg_v(vfg_handle *h, const uint8_t *mask, const int *list, int count, const double *dinv, double *x,
+                 double *r, double *z, double *p, double *p2, double *q, double rtol, double rn0, int maxit, int check,
+                 int first, vfg_solve_info *info) {
   hipStream_t s = h->stream;
-  double *sc = h->scal, *part = h->part;
-  const int nb = red_blocks(n);
-  hipLaunchKernelGGL(k_pcg_init, dim3(nb), dim3(RB), 0, s, r, z, p, dinv, n, part);
-  hipLaunchKernelGGL(k_pcg_scalar, dim3(1), dim3(RB), 0, s, (const double *)part, nb, 0, sc);
-  hipLaunchKernelGGL(k_set_scalar, dim3(1), dim3(1), 0, s, sc, (int)S_BETA, 0.);  // first direction p = z
-  double hs[13];
-  // ||r0|| from the caller when it has just read it back; else read here
-  if (rn0_known < 0. &&
-      (hipMemcpyAsync(hs, sc, 64, hipMemcpyDeviceToHost, s) != hipSuccess || hipStreamSynchronize(s) != hipSuccess))
-    return vfg_fail(h, VFG_E_HIP, "pcg: initial reduction failed");
-  const double rn0 = rn0_known < 0. ? sqrt(hs[S_RR0]) : rn0_known;
-  double rn = rn0;
+  const DevProblem &P = h->P;
+  const int64_t n = P.nn;
+  const size_t cap = vcg_partials(P.G);
+  double *sc = h->scal, *ppq = h->vpart, *pairs[2] = {h->vpart + cap, h->vpart + 3 * cap};
+  double rn = rn0, hs[13];
   int it = 0, status = VFG_OK;
-  const double tol = fmax(rtol * rn0, atol);
+  const double tol = rtol * rn0;
   if (!isfinite(rn0)) status = VFG_E_NAN;
-  // with xr (the listed kernels), the iteration that reaches tol marks the
-  // solve done on the device and the rest of its batch exits at once
-  if (xr) hipLaunchKernelGGL(k_set_scalar, dim3(1), dim3(1), 0, s, sc, (int)S_TOL2, tol * tol);
+  VCgStep c;
+  c.pairs = pairs[0];
+  c.npairs = red_blocks(n);
+  c.k = 0;
+  c.tol2 = tol * tol;
+  c.sc = sc;
+  hipLaunchKernelGGL(k_vcg_init, dim3(c.npairs), dim3(RB), 0, s, (const double *)r, z, p, dinv, n, pairs[0], sc);
   double *pa = p, *pb = p2;  // previous / current direction
-  bool first_batch = true;
   while (status == VFG_OK && rn > tol && it < maxit) {
     int todo = check < maxit - it ? check : maxit - it;
-    // first > 0: the caller's estimate of the iterations needed (launches
-    // after the device-side stop cost a launch each, for nothing)
-    if (first_batch && first > 0 && first < todo) todo = first;
-    first_batch = false;
-    for (int k = 0; k < todo; k++) {
-      const int na = A(pa, pb, q);  // pb = z + beta pa, q = A pb, part = p.q per workgroup
-      hipLaunchKernelGGL(k_pcg_scalar, dim3(1), dim3(RB), 0, s, (const double *)part, na, 1, sc);
-      int nx = nb;
-      if (xr) nx = (*xr)(pb, q);
-      else
-        hipLaunchKernelGGL(k_pcg_xr, dim3(nb), dim3(RB), 0, s, x, r, z, (const double *)pb, (const double *)q, dinv,
-                           n, (const double *)sc, part);
-      hipLaunchKernelGGL(k_pcg_scalar, dim3(1), dim3(RB), 0, s, (const double *)part, nx, 2, sc);
+    if (c.k == 0 && first > 0 && first < todo) todo = first;
+    for (int i = 0; i < todo; i++, c.k++) {
+      launch_v_apply_cg_list(P, pa, pb, z, q, ppq, mask, list, count, c, s);
+      double *nx = pairs[(c.k + 1) & 1];
+      launch_v_xr_list(P.G, list, count, x, r, z, pb, q, dinv, ppq, nx, c, s);
+      c.pairs = nx;
+      c.npairs = count;
       double *t = pa;
       pa = pb;
       pb = t;
     }
+    hipLaunchKernelGGL(k_vcg_final, dim3(1), dim3(RB), 0, s, c);
     if (hipMemcpyAsync(hs, sc, 8 * 13, hipMemcpyDeviceToHost, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess)
       return vfg_fail(h, VFG_E_HIP, "pcg: iteration failed");
-    it = (int)hs[S_ITS];  // iterations that ran (with xr the batch stops at convergence)
+    it = (int)hs[S_ITS];  // iterations that ran (the batch stops at convergence)
     rn = sqrt(hs[S_RR]);
     if (hs[S_FLAG] == 2. || !isfinite(rn)) status = VFG_E_NAN;
     else if (hs[S_FLAG] == 1.) status = rn <= tol ? VFG_OK : VFG_E_BREAKDOWN;
@@ -1312,12 +1327,13 @@ int vfg_v_solve(vfg_handle *h, const double *U, double *V, const double *ub, con
   hipStream_t s = h->stream;
   int rc;
   if ((rc = work(h, 13, 3 * n))) return rc;
-  if ((rc = vfg_alloc(h, (void **)&h->act, n))) return rc;
   const int vcap = v_chunk_cap(P.G);
-  if ((rc = vfg_alloc(h, (void **)&h->vflag, 4 * (size_t)vcap)) ||
-      (rc = vfg_alloc(h, (void **)&h->vlist, 4 * (size_t)(vcap + 2))) ||
-      (rc = vfg_alloc(h, (void **)&h->vflag2, 4 * (size_t)vcap)) ||
-      (rc = vfg_alloc(h, (void **)&h->vlist2, 4 * (size_t)(vcap + 2))))
+  if ((rc = vfg_alloc_group(h, {{(void **)&h->act, (size_t)n},
+                                {(void **)&h->vflag, 4 * (size_t)vcap},
+                                {(void **)&h->vlist, 4 * (size_t)(vcap + 2)},
+                                {(void **)&h->vflag2, 4 * (size_t)vcap},
+                                {(void **)&h->vlist2, 4 * (size_t)(vcap + 2)},
+                                {(void **)&h->vpart, 8 * 5 * vcg_partials(P.G)}})))
     return rc;
   double *x = h->w[0], *r = h->w[1], *z = h->w[2], *p = h->w[3], *q = h->w[4], *dinv = h->w[5];
   double *Vd = h->w[6], *g = h->w[7], *Vn = h->w[8], *D = h->w[9], *KD = h->w[10], *ubd = nullptr;
@@ -1384,20 +1400,12 @@ int vfg_v_solve(vfg_handle *h, const double *U, double *V, const double *ub, con
     hipLaunchKernelGGL(k_recip, dim3(nb_(n)), dim3(256), 0, s, (const double *)q, dinv, n);
     launch_fill(x, 0., n, s);
     launch_fill(h->w[12], 0., n, s);
-    FusedFn A = [&](const double *pold, double *pn, double *qq) {
-      return launch_v_apply_cg_list(P, pold, pn, z, h->scal + S_BETA, qq, h->part, act, vlist, nlist, s,
-                                    h->scal + S_DONE);
-    };
-    XrFn XR = [&](const double *pc, const double *qc) {
-      return launch_v_xr_list(P.G, vlist, nlist, x, r, z, pc, qc, dinv, h->scal + S_ALPHA, h->part, s,
-                              h->scal + S_DONE);
-    };
     const double inner_rtol = fmax(inner_floor, fmin(0.1, 0.1 * pg / pg0));
     // r = -g on the free nodes, so ||r0|| = pg; the first batch holds two
     // iterations more than the previous Newton step's solve took
     const int its0 = inf.iterations;
-    int prc = pcg_fused(h, n, A, dinv, x, r, z, p, h->w[12], q, inner_rtol, 0., 20000, 20, &inf, &XR, pg,
-                        last_cg > 0 ? last_cg + 2 : 0);
+    int prc = pcg_v(h, act, vlist, nlist, dinv, x, r, z, p, h->w[12], q, inner_rtol, pg, 20000, 20,
+                    last_cg > 0 ? last_cg + 2 : 0, &inf);
     last_cg = inf.iterations - its0;
     if (prc == VFG_E_HIP || prc == VFG_E_NAN) { status = prc; break; }
     // projected step with Armijo backtracking on f(V) = 1/2 V.KV - b.V

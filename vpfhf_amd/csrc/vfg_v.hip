@@ -336,10 +336,9 @@ struct VApplyOp : VApplyRec {
 // arrays (neighbouring workgroups still read p_old at their halo nodes)
 struct VApplyCgOp : VApplyOp<0> {
   const double *z;
-  const double *beta;
   double *pw;
   double *part;
-  double bval;  // *beta, read once by the kernel
+  double bval;  // beta, formed by the kernel
   struct Raw {
     double z, x;
     uint8_t fix;
@@ -388,10 +387,43 @@ __device__ __forceinline__ VChunk chunk_at(const Grid &G, const int *__restrict_
   const int c = __builtin_amdgcn_readfirstlane(list[w]), t = c % txy;  // uniform: the moments' base address too
   return VChunk{t % gx, t / gx, c / txy, __builtin_amdgcn_readfirstlane(list[cap + 1])};
 }
+// the sums of n pairs, or of n values in the first of them, in every thread
+template <int W>
+__device__ __forceinline__ void vcg_sums(const double *__restrict__ part, int n, double (&s)[W]) {
+  __shared__ double sh[4], bc[W];
+  double a[W] = {};
+  for (int i = threadIdx.x; i < n; i += 256)
+#pragma unroll
+    for (int w = 0; w < W; w++) a[w] += part[W * i + w];
+#pragma unroll
+  for (int w = 0; w < W; w++) {
+    const double v = block_sum<256>(a[w], sh);
+    if (threadIdx.x == 0) bc[w] = v;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < W; w++) s[w] = bc[w];
+}
 __global__ __launch_bounds__(256, 2) void k_v_apply_cg_list(VApplyCgOp op, const int *__restrict__ list, int cap,
-                                                           const double *__restrict__ done) {
-  if (done && *done != 0.) return;  // the CG has converged
-  op.bval = *op.beta;
+                                                           VCgStep c) {
+  if (c.sc[S_DONE] != 0.) return;  // the CG has converged
+  double s[2];
+  vcg_sums<2>(c.pairs, c.npairs, s);
+  const bool first = blockIdx.x == 0 && threadIdx.x == 0;
+  if (c.k > 0 && c.tol2 > 0. && s[1] <= c.tol2) {  // in every workgroup alike
+    if (first) {
+      c.sc[S_DONE] = 1.;
+      c.sc[S_RR] = s[1];
+      c.sc[S_ITS] = (double)c.k;
+    }
+    return;
+  }
+  const double old = c.sc[S_RZ];
+  op.bval = c.k > 0 && old != 0. ? s[0] / old : 0.;
+  if (first) {
+    c.sc[S_TMP0] = s[0];
+    if (!isfinite(s[0]) || !isfinite(s[1])) c.sc[S_FLAG] = 2.;
+  }
   const VChunk q = chunk_at(op.G, list, cap, blockIdx.x);
   march_modal<16, 16>(op.G, op, q.L, q.bx, q.by, q.bz, blockIdx.x);
 }
@@ -508,16 +540,23 @@ __global__ __launch_bounds__(256) void k_v_xr_list(Grid G, const int *__restrict
                                                    double *__restrict__ x, double *__restrict__ r,
                                                    double *__restrict__ z, const double *__restrict__ p,
                                                    const double *__restrict__ q, const double *__restrict__ dinv,
-                                                   const double *__restrict__ alpha, double *__restrict__ part,
-                                                   const double *__restrict__ done) {
-  if (done && *done != 0.) return;  // the CG has converged
+                                                   const double *__restrict__ ppq, double *__restrict__ part,
+                                                   VCgStep cg) {
+  if (cg.sc[S_DONE] != 0.) return;  // the CG has converged
   __shared__ double sh[4];
   const int gx = (G.nx + 14) / 15, txy = gx * ((G.ny + 14) / 15);
   const int c = list[blockIdx.x], L = list[cap + 1], t = c % txy;
   const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
   const int i = (t % gx) * 15 + tx, j = (t / gx) * 15 + ty, k0 = (c / txy) * L;
   const int k1 = k0 + L < G.nz ? k0 + L : G.nz;
-  const double al = *alpha;
+  double pq[1];
+  vcg_sums<1>(ppq, (int)gridDim.x, pq);
+  const bool ok = pq[0] > 0. && isfinite(pq[0]);
+  const double old = cg.sc[S_TMP0], al = ok ? old / pq[0] : 0.;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    cg.sc[S_RZ] = old;
+    if (!ok) cg.sc[S_FLAG] = isfinite(pq[0]) ? 1. : 2.;
+  }
   double rz = 0., rr = 0.;
   if (tx < 15 && ty < 15 && i < G.nx && j < G.ny)
     for (int k = k0; k < k1; k++) {
@@ -799,11 +838,11 @@ void launch_engine_v_apply(const void *d_ops, const BItem *items, const int *dco
                      fstride);
 }
 
-static VApplyCgOp make_vcg_op(const DevProblem &P, const double *pold, double *p, const double *z,
-                              const double *beta, double *q, double *part, const uint8_t *mask) {
+static VApplyCgOp make_vcg_op(const DevProblem &P, const double *pold, double *p, const double *z, double *q,
+                              double *part, const uint8_t *mask) {
   VApplyCgOp op;
   vapply_fill(op, P, pold, q, mask);
-  op.z = z; op.beta = beta; op.pw = p; op.part = part;
+  op.z = z; op.pw = p; op.part = part;
   return op;
 }
 
@@ -828,22 +867,25 @@ void launch_v_dilated_list(const DevProblem &P, const uint32_t *flag, uint32_t *
                      1024, list2, cap);
 }
 
-int launch_v_apply_cg_list(const DevProblem &P, const double *pold, double *p, const double *z, const double *beta,
-                           double *q, double *part, const uint8_t *mask, const int *list, int count, hipStream_t s,
-                           const double *done) {
-  if (count <= 0) return 0;
-  const VApplyCgOp op = make_vcg_op(P, pold, p, z, beta, q, part, mask);
-  hipLaunchKernelGGL(k_v_apply_cg_list, dim3((unsigned)count), dim3(256), 0, s, op, list, v_chunk_cap(P.G), done);
-  return count;
+size_t vcg_partials(const Grid &G) {
+  // launch_v_chunk_list: at most 32768 + one per tile
+  const size_t cap = (size_t)v_chunk_cap(G), most = 32768 + cap / (size_t)G.nz, n = cap < most ? cap : most;
+  return n < 2048 ? 2048 : n;
 }
 
-int launch_v_xr_list(const Grid &G, const int *list, int count, double *x, double *r, double *z, const double *p,
-                     const double *q, const double *dinv, const double *alpha, double *part, hipStream_t s,
-                     const double *done) {
-  if (count <= 0) return 0;
+void launch_v_apply_cg_list(const DevProblem &P, const double *pold, double *p, const double *z, double *q, double *part,
+                            const uint8_t *mask, const int *list, int count, const VCgStep &c, hipStream_t s) {
+  if (count <= 0) return;
+  const VApplyCgOp op = make_vcg_op(P, pold, p, z, q, part, mask);
+  hipLaunchKernelGGL(k_v_apply_cg_list, dim3((unsigned)count), dim3(256), 0, s, op, list, v_chunk_cap(P.G), c);
+}
+
+void launch_v_xr_list(const Grid &G, const int *list, int count, double *x, double *r, double *z, const double *p,
+                      const double *q, const double *dinv, const double *ppq, double *pairs, const VCgStep &c,
+                      hipStream_t s) {
+  if (count <= 0) return;
   hipLaunchKernelGGL(k_v_xr_list, dim3((unsigned)count), dim3(256), 0, s, G, list, v_chunk_cap(G), x, r, z, p, q,
-                     dinv, alpha, part, done);
-  return count;
+                     dinv, ppq, pairs, c);
 }
 
 void launch_v_diag(const DevProblem &P, double *d, hipStream_t s, const uint8_t *mask) {
