@@ -378,7 +378,7 @@ struct UModRec {
 };
 // the parts of the march's interface that every moment-form operator shares
 // (Rec: UModRec<T> or a record derived from it)
-template <typename T_, bool UNIT, class Rec>
+template <typename T_, bool UNIT, class Rec, bool CUBIC>
 struct UModBase : Rec {
   using T = T_;
   using Record = Rec;
@@ -411,7 +411,7 @@ struct UModBase : Rec {
     return this->E_elem ? T(this->E_elem[cell_id(this->G, ex, ey, ek)]) : this->E;
   }
   __device__ void element(T Ee, const Face &B, const Face &F, T (&tot)[3][4], T (&carry)[3][4]) const {
-    um_layer<T, UNIT>(B.f, F.f, B.v, F.v, Ee, this->m, tot, carry);
+    um_layer<T, UNIT, CUBIC>(B.f, F.f, B.v, F.v, Ee, this->m, tot, carry);
   }
   // A x of a node: the displacement itself on the Dirichlet rows (a wavefront
   // without a boundary node skips the tests)
@@ -426,9 +426,9 @@ struct UModBase : Rec {
     }
   }
 };
-template <typename T, bool UNIT>
-struct UModOp : UModBase<T, UNIT, UModRec<T>> {
-  using typename UModBase<T, UNIT, UModRec<T>>::Own;
+template <typename T, bool UNIT, bool CUBIC = false>
+struct UModOp : UModBase<T, UNIT, UModRec<T>, CUBIC> {
+  using typename UModBase<T, UNIT, UModRec<T>, CUBIC>::Own;
   __device__ T load(int f, int64_t n) const { return f < 3 ? this->x[3 * n + f] : this->v[n]; }
   __device__ void store(int64_t n, uint32_t fb, const T (&acc)[3], const Own &own) const {
     T yv[3];
@@ -452,8 +452,8 @@ static void umod_fill(UModRec<T> &r, const DevProblem &P, const T *x, T *y) {
 // waves per SIMD asked of the compiler: FP64 two (256 registers), FP32 three
 template <typename T>
 constexpr int um_waves() { return sizeof(T) == 8 ? 2 : 3; }
-template <typename T, int TX, int TY, bool UNIT>
-__global__ __launch_bounds__(TX *TY, um_waves<T>()) void k_u_apply(UModOp<T, UNIT> op, int OZ) {
+template <typename T, int TX, int TY, bool UNIT, bool CUBIC>
+__global__ __launch_bounds__(TX *TY, um_waves<T>()) void k_u_apply(UModOp<T, UNIT, CUBIC> op, int OZ) {
   march_modal<TX, TY>(op.G, op, OZ, xcd_block());
 }
 
@@ -473,9 +473,9 @@ struct UMgRec : UModRec<float> {
   const double *r64;  // rz form
   double *part;       // rz form
 };
-template <bool UNIT>
-struct UMgPreOp : UModBase<float, UNIT, UMgRec> {
-  using typename UModBase<float, UNIT, UMgRec>::Own;
+template <bool UNIT, bool CUBIC = false>
+struct UMgPreOp : UModBase<float, UNIT, UMgRec, CUBIC> {
+  using typename UModBase<float, UNIT, UMgRec, CUBIC>::Own;
   struct Raw {
     float b, di;
   };
@@ -507,9 +507,9 @@ struct MgOwnR {
   float b[3], di[3];
   double r[3];
 };
-template <bool UNIT, bool RZ>
-struct UMgPostOp : UModBase<float, UNIT, UMgRec> {
-  using typename UModBase<float, UNIT, UMgRec>::Own;
+template <bool UNIT, bool RZ, bool CUBIC = false>
+struct UMgPostOp : UModBase<float, UNIT, UMgRec, CUBIC> {
+  using typename UModBase<float, UNIT, UMgRec, CUBIC>::Own;
   __device__ float load(int f, int64_t n) const { return f < 3 ? this->x[3 * n + f] : this->v[n]; }
   __device__ auto own_load(int64_t n) const {
     std::conditional_t<RZ, MgOwnR, MgOwn> o;
@@ -535,8 +535,9 @@ struct UMgPostOp : UModBase<float, UNIT, UMgRec> {
     if constexpr (RZ) return rz;
   }
 };
-struct UMgPostRzOp : UMgPostOp<false, true> {
-  __device__ void partial(int slot, double v) const { part[slot] = v; }
+template <bool CUBIC>
+struct UMgPostRzOp : UMgPostOp<false, true, CUBIC> {
+  __device__ void partial(int slot, double v) const { this->part[slot] = v; }
 };
 template <class Op, int TX, int TY>
 __global__ __launch_bounds__(TX *TY, 3) void k_u_mg(Op op, int OZ) {
@@ -545,21 +546,24 @@ __global__ __launch_bounds__(TX *TY, 3) void k_u_mg(Op op, int OZ) {
 
 // the FP64 apply also reducing p.q (p = the input, q = the output, every
 // row) to one partial per workgroup: the CG's p.q without another pass
-struct UApplyDotOp : UModOp<double, false> {
+template <bool CUBIC>
+struct UApplyDotOp : UModOp<double, false, CUBIC> {
+  using typename UModOp<double, false, CUBIC>::Own;
   double *part;
   __device__ double store(int64_t n, uint32_t fb, const double (&acc)[3], const Own &own) const {
     double d = 0., yv[3];
-    rows(fb, acc, own, yv);
+    this->rows(fb, acc, own, yv);
 #pragma unroll
     for (int c = 0; c < 3; c++) {
-      y[3 * n + c] = yv[c];
+      this->y[3 * n + c] = yv[c];
       d += own.x[c] * yv[c];
     }
     return d;
   }
   __device__ void partial(int slot, double v) const { part[slot] = v; }
 };
-__global__ __launch_bounds__(256, 2) void k_u_apply_dot(UApplyDotOp op, int OZ) {
+template <bool CUBIC>
+__global__ __launch_bounds__(256, 2) void k_u_apply_dot(UApplyDotOp<CUBIC> op, int OZ) {
   march_modal<16, 16>(op.G, op, OZ, xcd_block(),
                       blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));
 }
@@ -1156,13 +1160,20 @@ static void launch_u_apply_uni(const DevProblem &P, const T *x, T *y, const T *v
   const int OZ = choose_oz(P.G, tiles, slots);
   hipLaunchKernelGGL((k_u_apply_uni<T, 16, 16>), march_grid(P.G, 16, 16, OZ), dim3(256), 0, s, op, OZ);
 }
+template <typename T, int W, bool UNIT, bool CUBIC>
+static void launch_u_apply_c(const UModRec<T> &r, hipStream_t s) {
+  UModOp<T, UNIT, CUBIC> op;
+  static_cast<UModRec<T> &>(op) = r;
+  const Grid &G = r.G;
+  static int slots = device_slots(k_u_apply<T, W, W, UNIT, CUBIC>, W * W);
+  const int OZ = choose_oz(G, ((G.nx + W - 2) / (W - 1)) * ((G.ny + W - 2) / (W - 1)), slots);
+  hipLaunchKernelGGL((k_u_apply<T, W, W, UNIT, CUBIC>), march_grid(G, W, W, OZ), dim3(W * W), 0, s, op, OZ);
+}
 template <typename T, int W, bool UNIT>
 static void launch_u_apply_w(const DevProblem &P, const T *x, T *y, hipStream_t s) {
-  UModOp<T, UNIT> op;
-  umod_fill<T>(op, P, x, y);
-  static int slots = device_slots(k_u_apply<T, W, W, UNIT>, W * W);
-  const int OZ = choose_oz(P.G, ((P.G.nx + W - 2) / (W - 1)) * ((P.G.ny + W - 2) / (W - 1)), slots);
-  hipLaunchKernelGGL((k_u_apply<T, W, W, UNIT>), march_grid(P.G, W, W, OZ), dim3(W * W), 0, s, op, OZ);
+  UModRec<T> r;
+  umod_fill<T>(r, P, x, y);
+  r.m.cubic ? launch_u_apply_c<T, W, UNIT, true>(r, s) : launch_u_apply_c<T, W, UNIT, false>(r, s);
 }
 
 template <typename T>
@@ -1391,11 +1402,20 @@ void launch_u_apply(const DevProblem &P, const double *x, double *y, hipStream_t
   launch_u_apply_t<double>(P, x, y, P.V, s);
 }
 
+template <bool CUBIC>
+static int launch_u_apply_dot_c(const UModRec<double> &r, double *part, hipStream_t s) {
+  UApplyDotOp<CUBIC> op;
+  static_cast<UModRec<double> &>(op) = r;
+  op.part = part;
+  const Grid &G = r.G;
+  static int slots = device_slots(k_u_apply_dot<CUBIC>, 256);
+  const int OZ = choose_oz(G, ((G.nx + 14) / 15) * ((G.ny + 14) / 15), slots);
+  const dim3 g = march_grid(G, 16, 16, OZ);
+  hipLaunchKernelGGL(k_u_apply_dot<CUBIC>, g, dim3(256), 0, s, op, OZ);
+  return (int)(g.x * g.y * g.z);
+}
 int launch_u_apply_dot(const DevProblem &P, const double *x, double *y, double *part, hipStream_t s) {
   if (P.unilateral) return 0;
-  UApplyDotOp op;
-  umod_fill<double>(op, P, x, y);
-  op.part = part;
   if (P.uq) {
     UApplyLdsqDotOp q;
     q.x = x; q.y = y; q.part = part; q.uq = P.uq;
@@ -1408,12 +1428,9 @@ int launch_u_apply_dot(const DevProblem &P, const double *x, double *y, double *
     hipLaunchKernelGGL(k_u_apply_ldsq_dot, g, dim3(256), 0, s, q, OZ);
     return (int)(g.x * g.y * g.z);
   }
-  static int slots = device_slots(k_u_apply_dot, 256);
-  const int tiles = ((P.G.nx + 14) / 15) * ((P.G.ny + 14) / 15);
-  const int OZ = choose_oz(P.G, tiles, slots);
-  const dim3 g = march_grid(P.G, 16, 16, OZ);
-  hipLaunchKernelGGL(k_u_apply_dot, g, dim3(256), 0, s, op, OZ);
-  return (int)(g.x * g.y * g.z);
+  UModRec<double> r;
+  umod_fill<double>(r, P, x, y);
+  return r.m.cubic ? launch_u_apply_dot_c<true>(r, part, s) : launch_u_apply_dot_c<false>(r, part, s);
 }
 void launch_u_apply_f32(const DevProblem &P, const float *x, float *y, hipStream_t s) {
   launch_u_apply_t<float>(P, x, y, P.V32, s);
@@ -1448,8 +1465,8 @@ void launch_mg_presmooth(const DevProblem &P, const float *b, const float *dinv,
   UMgRec op;
   mg_op_fill(op, P, b, dinv, c2);
   op.xo = x; op.ro = r;
-  if (P.unit) mg_launch<UMgPreOp<true>>(P, op, s);
-  else mg_launch<UMgPreOp<false>>(P, op, s);
+  if (op.m.cubic) P.unit ? mg_launch<UMgPreOp<true, true>>(P, op, s) : mg_launch<UMgPreOp<false, true>>(P, op, s);
+  else P.unit ? mg_launch<UMgPreOp<true>>(P, op, s) : mg_launch<UMgPreOp<false>>(P, op, s);
 }
 int launch_mg_postsmooth(const DevProblem &P, const float *b, const float *dinv, float c2, const float *x, float *xo,
                          const double *r64, double *part, hipStream_t s) {
@@ -1457,9 +1474,12 @@ int launch_mg_postsmooth(const DevProblem &P, const float *b, const float *dinv,
   mg_op_fill(op, P, b, dinv, c2);
   op.x = x; op.xo = xo; op.r64 = r64; op.part = part;
   if (r64) {
-    const int n = mg_launch<UMgPostRzOp>(P, op, s, 2 * 65536);
+    const int n = op.m.cubic ? mg_launch<UMgPostRzOp<true>>(P, op, s, 2 * 65536)
+                             : mg_launch<UMgPostRzOp<false>>(P, op, s, 2 * 65536);
     if (n) return n;  // else too many workgroups for the partials: the plain form
   }
+  if (op.m.cubic)
+    return P.unit ? mg_launch<UMgPostOp<true, false, true>>(P, op, s) : mg_launch<UMgPostOp<false, false, true>>(P, op, s);
   return P.unit ? mg_launch<UMgPostOp<true, false>>(P, op, s) : mg_launch<UMgPostOp<false, false>>(P, op, s);
 }
 

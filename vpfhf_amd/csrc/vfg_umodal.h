@@ -29,6 +29,7 @@ struct UModal {
   T eta4;        // 4 eta
   // hx^2 / (h_d h_e) times 1 (kx), lam / mu (kl), and for d = e lam / mu + 2 (k2)
   T kx[3][3], kl[3][3], k2[3];
+  int cubic;     // all of kx are 1: the products by them are left out, with the same results
 };
 template <typename T>
 inline UModal<T> make_umodal(const Grid &G, double lam1, double mu1, double eta, bool unit) {
@@ -43,6 +44,12 @@ inline UModal<T> make_umodal(const Grid &G, double lam1, double mu1, double eta,
       m.kl[d][e] = T(lr * h[0] * h[0] / (h[d] * h[e]));
     }
     m.k2[d] = T((lr + 2) * h[0] * h[0] / (h[d] * h[d]));
+  }
+  m.cubic = 1;
+  for (int d = 0; d < 3; d++) {
+    for (int e = 0; e < 3; e++)
+      if (m.kx[d][e] != T(1) || m.kl[d][e] != m.kl[0][0]) m.cubic = 0;
+    if (m.k2[d] != m.k2[0]) m.cubic = 0;
   }
   return m;
 }
@@ -154,7 +161,8 @@ __device__ __forceinline__ void um_modes(const UFace<T> &B, const UFace<T> &F, T
 // component c (its four modes holding variable d):
 //   test d of component d:  M_dd k2_d D_dd + sum_{e != d} M_de kl_de D_ee
 //   test d of component c:  M_dd kx_dd D_cd + M_dc kx_dc D_dc
-template <typename T>
+// CUBIC: kx = 1, one kl, one k2.
+template <bool CUBIC, typename T>
 __device__ __forceinline__ void um_force(const T (&M)[3][3][3], const T (&U)[3][8], const UModal<T> &m, int c,
                                          T (&R)[8]) {
 #pragma unroll
@@ -170,7 +178,9 @@ __device__ __forceinline__ void um_force(const T (&M)[3][3][3], const T (&U)[3][
 #pragma unroll
       for (int j = 0; j < 8; j++) {
         if (!um_pow(j, e)) continue;
-        const T t = (c != d ? m.kx[d][e] : e == d ? m.k2[d] : m.kl[d][e]) * U[cu][j];
+        const T t = CUBIC && c != d ? U[cu][j]
+                    : CUBIC         ? (e == d ? m.k2[0] : m.kl[0][0]) * U[cu][j]
+                                    : (c != d ? m.kx[d][e] : e == d ? m.k2[d] : m.kl[d][e]) * U[cu][j];
 #pragma unroll
         for (int i = 0; i < 8; i++)
           if (um_pow(i, d))
@@ -181,7 +191,7 @@ __device__ __forceinline__ void um_force(const T (&M)[3][3][3], const T (&U)[3][
 // The same for s = 1 (the coarse multigrid levels): the odd moments vanish and
 // the even ones are constants, so each block is diagonal (60 FMAs); Ek = E kap
 // with the unit form's kap.
-template <typename T>
+template <bool CUBIC, typename T>
 __device__ __forceinline__ void um_force_unit(T Ek, const T (&U)[3][8], const UModal<T> &m, int c, T (&R)[8]) {
 #pragma unroll
   for (int i = 0; i < 8; i++) R[i] = T(0);
@@ -200,7 +210,9 @@ __device__ __forceinline__ void um_force_unit(T Ek, const T (&U)[3][8], const UM
           const int q0 = um_exp(i, d, j, e, 0), q1 = um_exp(i, d, j, e, 1), q2 = um_exp(i, d, j, e, 2);
           if ((q0 & 1) || (q1 & 1) || (q2 & 1)) continue;
           const T w = T((q0 ? 1. / 3. : 1.) * (q1 ? 1. / 3. : 1.) * (q2 ? 1. / 3. : 1.));
-          R[i] += (w * (c != d ? m.kx[d][e] : e == d ? m.k2[d] : m.kl[d][e])) * U[cu][j];
+          const T k = CUBIC ? (c != d ? T(1) : e == d ? m.k2[0] : m.kl[0][0])
+                            : (c != d ? m.kx[d][e] : e == d ? m.k2[d] : m.kl[d][e]);
+          R[i] += (w * k) * U[cu][j];
         }
       }
     }
@@ -210,13 +222,18 @@ __device__ __forceinline__ void um_force_unit(T Ek, const T (&U)[3][8], const UM
 
 // One layer of an element column: the modal forces of the bottom face added to
 // tot, those of the top face set in carry (per component s, x, y, w).
-// UNIT: s = 1 (vb, vt unused).
+// UNIT: s = 1 (vb, vt unused).  CUBIC: elements whose three spacings agree
+// (UModal::cubic): 60 of the multiplications are by 1 or shared; results are
+// bitwise those of the general form.  A branch inside the element would keep
+// all of it live at once (FP64: 23 registers spilled), so the kernels come in
+// both forms (FP64 94 -> 86 us at 128^3, 620 -> 560 us at 256^3; FP32
+// smoothing 72 -> 66 us at 128^3).
 // Bound by instruction issue: about 690 FP64 and 140 other vector instructions
 // per element and layer, 0.75 of the issue peak at 256^3 (two waves per SIMD in
-// FP64, three to four in FP32).  Against the 27-point form on the same tiles:
-// FP64 176 -> 94 us at 128^3 and 1299 -> 666 us at 256^3, FP32 98 -> 59 us and
-// 776 -> 391 us.
-template <typename T, bool UNIT>
+// FP64, three to four in FP32).  Against the 27-point form on the same tiles,
+// general elements: FP64 176 -> 94 us at 128^3 and 1299 -> 640 us at 256^3, FP32
+// 98 -> 59 us and 776 -> 391 us.
+template <typename T, bool UNIT, bool CUBIC = false>
 __device__ __forceinline__ void um_layer(const UFace<T> &B, const UFace<T> &F, const T *vb, const T *vt, T Ee,
                                          const UModal<T> &m, T (&tot)[3][4], T (&carry)[3][4]) {
   T U[3][8], M[3][3][3];
@@ -226,8 +243,8 @@ __device__ __forceinline__ void um_layer(const UFace<T> &B, const UFace<T> &F, c
 #pragma unroll
   for (int c = 0; c < 3; c++) {
     T R[8];
-    if constexpr (UNIT) um_force_unit<T>(Ek, U, m, c, R);
-    else um_force<T>(M, U, m, c, R);
+    if constexpr (UNIT) um_force_unit<CUBIC>(Ek, U, m, c, R);
+    else um_force<CUBIC>(M, U, m, c, R);
     tot[c][0] -= R[4];
     tot[c][1] += R[1] - R[5];
     tot[c][2] += R[2] - R[6];
