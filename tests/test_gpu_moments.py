@@ -103,3 +103,28 @@ def test_v_setup_moment_form(oracle, n, unilateral):
         y, ry = P.VIJacobian_mult(s["xv"]), oracle.v_jacobian(op, F, s["U"]) @ s["xv"]
         assert np.abs(y - ry).max() <= 1e-12 * np.abs(ry).max()
         P.close()
+
+
+def test_batch_forms(oracle):
+    """Members with equal spacings, and mixed with one without: the batched
+    solves give each member what it gives alone, in either form."""
+    from vpfhf_amd.batch import Batch
+    boxes = [((9, 9, 9), (1.0, 1.0, 1.0)), ((18, 10, 12), (17 / 8, 9 / 8, 11 / 8)), ((11, 12, 9), (1.0, 2.3, 0.6))]
+    sc = [S.make(n=n, l=l, seed=i, nu=0.3) for i, (n, l) in enumerate(boxes)]
+    alone = {}
+    for pick in ([0], [1], [2], [0, 1], [0, 1, 2]):
+        P = [S.to_gpu(sc[i]) for i in pick]
+        B = Batch(P)
+        y = B.u_apply([sc[i]["x"] for i in pick])
+        for i, yi in zip(pick, y):
+            op, F = S.to_oracle(oracle, sc[i])
+            ref = oracle.u_jacobian(op, F) @ sc[i]["x"]
+            # one apply: 1e-12 as above; the forms differ by exact factors of 1 only
+            assert np.abs(yi - ref).max() <= 1e-12 * np.abs(ref).max()
+            if len(pick) == 1:
+                alone[i] = yi
+            else:
+                assert np.array_equal(yi, alone[i])
+        B.close()
+        for p in P:
+            p.close()

@@ -357,6 +357,7 @@ struct vfg_batch {
   double *d_part = nullptr, *d_sc = nullptr, *d_scale = nullptr, *d_iscale = nullptr;
   void *d_ops = nullptr, *d_ops32 = nullptr, *d_opsx = nullptr;
   int grid = 0;  // persistent grid size (0: one block per item)
+  int form = 0;   // FORM_CUBIC where it holds for every member
   int sched = 0;  // persistent-apply schedule (batch_tile_x, BATCH_SCHEDS)
   double oz_scale = 1.;
   std::vector<vfg_tune_point> tune;  // the last autotuning's measurements
@@ -437,6 +438,9 @@ int vfg_batch_create(vfg_handle *const *members, int n, vfg_batch **out) {
   for (int i = 0; i < n; i++)
     if (!members[i] || members[i]->P.unilateral) return VFG_E_ARG;  // linear u-problems only
   vfg_batch *b = new vfg_batch();
+  b->form = FORM_CUBIC;
+  for (int i = 0; i < n; i++)
+    if (!cubic_grid(members[i]->P.G)) b->form = 0;
   b->np = n;
   b->m.assign(members, members + n);
   if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess) {
@@ -507,7 +511,7 @@ int vfg_batch_u_apply(vfg_batch *b, const double *const *x, double *const *y) {
   if (!b || !x || !y) return VFG_E_ARG;
   std::vector<const void *> xs(x, x + b->np), ys(y, y + b->np);
   fill_ops(b->m, xs.data(), (void *const *)ys.data(), 0, b->oz, b->d_opsx, b->stream);
-  launch_batch_apply(0, b->sched, b->d_opsx, b->d_items, b->nitems, b->grid, b->stream);
+  launch_batch_apply(0, b->sched, b->form, b->d_opsx, b->d_items, b->nitems, b->grid, b->stream);
   BCHK(b, hipStreamSynchronize(b->stream));
   BCHK(b, hipGetLastError());
   return VFG_OK;
@@ -517,7 +521,7 @@ int vfg_batch_u_apply_f32(vfg_batch *b, const float *const *x, float *const *y) 
   if (!b || !x || !y) return VFG_E_ARG;
   std::vector<const void *> xs(x, x + b->np), ys(y, y + b->np);
   fill_ops(b->m, xs.data(), (void *const *)ys.data(), 1, b->oz, b->d_ops32, b->stream);
-  launch_batch_apply(1, b->sched, b->d_ops32, b->d_items, b->nitems, b->grid, b->stream);
+  launch_batch_apply(1, b->sched, b->form, b->d_ops32, b->d_items, b->nitems, b->grid, b->stream);
   BCHK(b, hipStreamSynchronize(b->stream));
   BCHK(b, hipGetLastError());
   return VFG_OK;
@@ -538,7 +542,7 @@ int vfg_batch_time_u_apply(vfg_batch *b, int fp32, int nrep, double *ms) {
   BCHK(b, hipEventCreate(&e0));
   BCHK(b, hipEventCreate(&e1));
   hipEventRecord(e0, b->stream);
-  for (int i = 0; i < nrep; i++) launch_batch_apply(fp32, b->sched, ops, b->d_items, b->nitems, b->grid, b->stream);
+  for (int i = 0; i < nrep; i++) launch_batch_apply(fp32, b->sched, b->form, ops, b->d_items, b->nitems, b->grid, b->stream);
   hipEventRecord(e1, b->stream);
   hipEventSynchronize(e1);
   float t = 0.f;
@@ -622,7 +626,7 @@ static void cg_iter(vfg_batch *b, int o, void *ops, int fp32, double rtol, int m
   const BChunk *ch = b->d_ch;
   // frozen members are skipped by the apply and the vector kernels
   const int g = b->grid > 0 && b->grid < b->nitems ? b->grid : b->nitems;
-  launch_engine_u_apply(fp32, b->sched, 0, ops, b->d_items, 0, b->d_nitems, g, b->d_sc + B_ACTIVE, B_NS, s);
+  launch_engine_u_apply(fp32, b->sched, b->form, ops, b->d_items, 0, b->d_nitems, g, b->d_sc + B_ACTIVE, B_NS, s);
   hipLaunchKernelGGL(k_bdot<T>, dim3(b->nch), dim3(BRB), 0, s, (const BVec *)b->d_vt, o + VP, o + VQ, ch,
                      (const double *)b->d_sc, b->d_part);
   hipLaunchKernelGGL(k_bscalar, dim3(b->np), dim3(BRB), 0, s, (const double *)b->d_part, (const int *)b->d_first,

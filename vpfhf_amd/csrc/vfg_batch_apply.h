@@ -18,24 +18,27 @@ int choose_oz_pub(const Grid &G, int tiles_xy, int slots);
 // writes one {operator, OZ} record per member (x[p] -> y[p]) into d_ops
 void fill_ops(const std::vector<vfg_handle *> &m, const void *const *x, void *const *y, int fp32,
               const std::vector<int> &oz, void *d_ops, hipStream_t s);
+// forms of the persistent kernels: coarse multigrid levels (s = 1; FP32, schedule
+// 0 only); every listed member has equal spacings (UModal::cubic)
+enum { FORM_UNIT = 1, FORM_CUBIC = 2 };
+inline bool cubic_grid(const Grid &G) { return G.hx == G.hy && G.hy == G.hz; }
 // grid == 0: one workgroup per item; otherwise a persistent grid striding the items
-void launch_batch_apply(int fp32, int sched, const void *d_ops, const BItem *items, int nitems, int grid,
+void launch_batch_apply(int fp32, int sched, int form, const void *d_ops, const BItem *items, int nitems, int grid,
                         hipStream_t s);
 
 // persistent applies over (device-counted, when dcount is given) work lists;
-// items of members whose flags[p * fstride] is 0 are skipped; unit: FP32
-// records of coarse multigrid levels (s = 1), schedule 0
-void launch_engine_u_apply(int fp32, int sched, int unit, const void *d_ops, const BItem *items, int nitems,
+// items of members whose flags[p * fstride] is 0 are skipped
+void launch_engine_u_apply(int fp32, int sched, int form, const void *d_ops, const BItem *items, int nitems,
                            const int *dcount, int grid, const double *flags, int fstride, hipStream_t s);
 void make_uop(const DevProblem &P, const void *x, void *y, int fp32, int OZ, void *out);  // host record
 // multigrid smoothing fused with the level apply, one record per member
 // (launch_mg_presmooth / launch_mg_postsmooth of every listed member at once;
 // 16 x 16 tiles): post = 0: x = c2 D^-1 b into xo, b - A x
-// (0 on the Dirichlet rows) into ro; post = 1: xo = xin + c2 D^-1 (b - A xin); unit: coarse levels
+// (0 on the Dirichlet rows) into ro; post = 1: xo = xin + c2 D^-1 (b - A xin)
 size_t mg_smooth_op_bytes();
 void make_mg_smooth_op(const DevProblem &P, int post, const float *b, const float *dinv, float c2, const float *xin,
                        float *xo, float *ro, int OZ, void *out);  // host record
-void launch_batch_mg_smooth(int post, int unit, const void *d_ops, const BItem *items, const int *dcount, int grid,
+void launch_batch_mg_smooth(int post, int form, const void *d_ops, const BItem *items, const int *dcount, int grid,
                             const double *flags, int fstride, hipStream_t s);
 size_t vop_bytes();
 int v_oz(const Grid &G);

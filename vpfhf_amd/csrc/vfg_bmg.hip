@@ -101,6 +101,7 @@ struct BmgPlan {
   // live counts: M items, M chunks, D items, D chunks, C items, C chunks, rch, pch
   int *dcnt = nullptr;
   int hcnt[8] = {0};
+  int form = 0;  // FORM_UNIT, FORM_CUBIC
   int cfit = 0;  // every member whose coarsest level this is fits the one-launch solve
 };
 struct BatchMG {
@@ -250,8 +251,17 @@ int bmg_rebuild(BatchMG *g, hipStream_t s, bool *grew) {
     int cfit = l == 0;
     for (int p = 0; p < g->np && cfit; p++)
       if (g->m[p] && g->L[p] - 1 == l && !mg_coarse_fits(g->m[p]->mg->lv[l].P)) cfit = 0;
-    if (cfit != P.cfit) *grew = true;  // the V-cycle's launches change
+    int form = (l > 0 ? FORM_UNIT : 0) | FORM_CUBIC;
+    bool listed = false;
+    for (int p = 0; p < g->np; p++)
+      if (g->m[p] && g->L[p] > l) {
+        listed = true;
+        if (!cubic_grid(level_grid(g, p, l))) form &= ~FORM_CUBIC;
+      }
+    if (!listed) form = P.form;  // nothing to apply: the captured launches may stay
+    if (cfit != P.cfit || form != P.form) *grew = true;  // the V-cycle's launches change
     P.cfit = cfit;
+    P.form = form;
     for (int k = 0; k < 3 && !rc; k++)
       if ((rc = push(g, ls[k]->items, s)) || (rc = push(g, ls[k]->ch, s))) break;
     if (rc || (rc = push(g, P.rch, s)) || (rc = push(g, P.pch, s))) break;
@@ -411,7 +421,7 @@ int bmg_setup_member(BatchMG *g, int p, const double *dinv64, hipStream_t s) {
 static void apply(BatchMG *g, int l, const BmgList &L, int which, const double *flags, int fstride, hipStream_t s) {
   if (!L.items.cap) return;
   const int grid = L.items.cap < g->slots ? L.items.cap : g->slots;
-  launch_engine_u_apply(1, 0, l > 0, g->lv[l].ops, L.items.d, 0, g->lv[l].dcnt + 2 * which, grid, flags, fstride, s);
+  launch_engine_u_apply(1, 0, g->lv[l].form, g->lv[l].ops, L.items.d, 0, g->lv[l].dcnt + 2 * which, grid, flags, fstride, s);
 }
 static void cheb(BatchMG *g, int l, const BmgList &L, int which, int step, int use_y, int xzero, const double *flags,
                  int fstride, hipStream_t s) {
@@ -424,7 +434,7 @@ static void cheb(BatchMG *g, int l, const BmgList &L, int which, int step, int u
 static void smooth(BatchMG *g, int l, const BmgList &L, int post, const double *flags, int fstride, hipStream_t s) {
   if (!L.items.cap) return;
   const int grid = L.items.cap < g->slots ? L.items.cap : g->slots;
-  launch_batch_mg_smooth(post, l > 0, post ? g->lv[l].ops_post : g->lv[l].ops_pre, L.items.d, g->lv[l].dcnt + 2, grid, flags,
+  launch_batch_mg_smooth(post, g->lv[l].form, post ? g->lv[l].ops_post : g->lv[l].ops_pre, L.items.d, g->lv[l].dcnt + 2, grid, flags,
                          fstride, s);
 }
 

@@ -380,6 +380,7 @@ struct vfg_engine {
   bool dirty_lists = true, dirty_vt = true, dirty_uop = true, dirty_vop = true;
   hipGraphExec_t g = nullptr, g_mg = nullptr;  // replay graphs without / with the batched V-cycle
   int grid_apply = 0, grid_vapply = 0, grid_vec = 0;
+  int form = FORM_CUBIC;  // of the resident requests
   int64_t ticks = 0, replays = 0;
   // multigrid of the mixed engine: one member per slot; d_one: flags of an
   // eager V-cycle of a single slot
@@ -783,9 +784,9 @@ static void e_iter(vfg_engine *e, bool with_mg) {
   hipStream_t s = e->s;
   const double *fl = e->d_sc + E_ACTIVE;
   if (e->o.precision == VFG_PREC_MIXED)
-    launch_engine_u_apply(1, 0, 0, e->d_uop, e->d_it[0], 0, e->d_cnt + C_U32, e->grid_apply, fl, E_NS, s);
+    launch_engine_u_apply(1, 0, e->form, e->d_uop, e->d_it[0], 0, e->d_cnt + C_U32, e->grid_apply, fl, E_NS, s);
   else
-    launch_engine_u_apply(0, 0, 0, e->d_uop, e->d_it[1], 0, e->d_cnt + C_U64, e->grid_apply, fl, E_NS, s);
+    launch_engine_u_apply(0, 0, e->form, e->d_uop, e->d_it[1], 0, e->d_cnt + C_U64, e->grid_apply, fl, E_NS, s);
   launch_engine_v_apply(e->d_vop, e->d_it[2], e->d_cnt + C_V, e->grid_vapply, fl, E_NS, s);
   hipLaunchKernelGGL(k_e_dot, dim3(e->grid_vec), dim3(ERB), 0, s, (const EVec *)e->d_vt, (const EChunk *)e->d_ch[0],
                      (const EChunk *)e->d_ch[1], (const int *)e->d_cnt, (const double *)e->d_sc, e->d_part);
@@ -1000,6 +1001,16 @@ int vfg_engine_step(vfg_engine *e) {
   if (e->dirty_lists && (rc = rebuild_lists(e))) return rc;
   if (!e->up.flush(e->s)) return efail(e, VFG_E_HIP, "vfg_engine: staged upload failed");
   if ((rc = mg_lists(e))) return rc;
+  int form = FORM_CUBIC, resident = 0;
+  for (const ESlot &q : e->slot) {
+    if (q.st == ST_FREE) continue;
+    resident++;
+    if (!cubic_grid(q.h->P.G)) form = 0;
+  }
+  if (resident && form != e->form) {
+    drop_graphs(e);
+    e->form = form;
+  }
   bool any_cg = false;
   used = 0;
   for (const ESlot &q : e->slot) {

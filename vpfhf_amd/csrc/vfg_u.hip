@@ -1556,7 +1556,7 @@ namespace vfg {
 // flags (optional) skip items of members whose flags[p * fstride] is 0.
 // Schedules (the autotuner's choice): TX x TY element tiles of (TX-1) x (TY-1)
 // owned node columns.  UNIT: the records are coarse multigrid levels.
-template <typename T, int TX, int TY, bool UNIT>
+template <typename T, int TX, int TY, bool UNIT, bool CUBIC>
 __global__ __launch_bounds__(TX *TY, um_waves<T>()) void k_batch_u_apply(
     const BApply<T> *__restrict__ probs, const BItem *__restrict__ items, int nitems, const int *__restrict__ dcount,
     const double *__restrict__ flags, int fstride) {
@@ -1564,7 +1564,7 @@ __global__ __launch_bounds__(TX *TY, um_waves<T>()) void k_batch_u_apply(
   for (int it = blockIdx.x; it < n; it += gridDim.x) {
     const BItem w = items[it];
     if (flags && flags[(int64_t)w.p * fstride] == 0.) continue;  // uniform per block
-    const auto op = op_of<UModOp<T, UNIT>>(probs[w.p].op);
+    const auto op = op_of<UModOp<T, UNIT, CUBIC>>(probs[w.p].op);
     const int OZ = probs[w.p].OZ;
     __syncthreads();  // LDS of the previous item is free
     march_modal<TX, TY>(op.G, op, OZ, w.bx, w.by, w.bz);
@@ -1576,9 +1576,9 @@ int batch_tile_x(int sched) { return sched == 1 ? 8 : 16; }
 int batch_tile_y(int sched) { return sched == 0 ? 16 : 8; }
 template <typename T>
 static int batch_slots_t(int sched) {
-  if (sched == 1) return device_slots(k_batch_u_apply<T, 8, 8, false>, 64);
-  if (sched == 2) return device_slots(k_batch_u_apply<T, 16, 8, false>, 128);
-  return device_slots(k_batch_u_apply<T, 16, 16, false>, 256);
+  if (sched == 1) return device_slots(k_batch_u_apply<T, 8, 8, false, false>, 64);
+  if (sched == 2) return device_slots(k_batch_u_apply<T, 16, 8, false, false>, 128);
+  return device_slots(k_batch_u_apply<T, 16, 16, false, false>, 256);
 }
 int batch_slots_s(int fp32, int sched) {
   static int cache[2][BATCH_SCHEDS] = {{0}};
@@ -1612,30 +1612,34 @@ void fill_ops(const std::vector<vfg_handle *> &m, const void *const *x, void *co
   else fill_ops_t<double>(m, x, y, oz, d_ops, s);
 }
 
-void launch_batch_apply(int fp32, int sched, const void *d_ops, const BItem *items, int nitems, int grid,
+void launch_batch_apply(int fp32, int sched, int form, const void *d_ops, const BItem *items, int nitems, int grid,
                         hipStream_t s) {
   const int g = grid > 0 && grid < nitems ? grid : nitems;
-  launch_engine_u_apply(fp32, sched, 0, d_ops, items, nitems, nullptr, g, nullptr, 0, s);
+  launch_engine_u_apply(fp32, sched, form, d_ops, items, nitems, nullptr, g, nullptr, 0, s);
 }
 
 template <typename T, int TX, int TY, bool UNIT>
-static void launch_batch_t(const void *d_ops, const BItem *items, int nitems, const int *dcount, int grid,
+static void launch_batch_t(bool cubic, const void *d_ops, const BItem *items, int nitems, const int *dcount, int grid,
                            const double *flags, int fstride, hipStream_t s) {
-  hipLaunchKernelGGL((k_batch_u_apply<T, TX, TY, UNIT>), dim3(grid), dim3(TX * TY), 0, s, (const BApply<T> *)d_ops,
-                     items, nitems, dcount, flags, fstride);
+  auto go = [&](auto k) {
+    hipLaunchKernelGGL(k, dim3(grid), dim3(TX * TY), 0, s, (const BApply<T> *)d_ops, items, nitems, dcount, flags,
+                       fstride);
+  };
+  cubic ? go(k_batch_u_apply<T, TX, TY, UNIT, true>) : go(k_batch_u_apply<T, TX, TY, UNIT, false>);
 }
 template <typename T>
-static void launch_batch_s(int sched, const void *d_ops, const BItem *items, int nitems, const int *dcount, int grid,
-                           const double *flags, int fstride, hipStream_t s) {
-  if (sched == 1) launch_batch_t<T, 8, 8, false>(d_ops, items, nitems, dcount, grid, flags, fstride, s);
-  else if (sched == 2) launch_batch_t<T, 16, 8, false>(d_ops, items, nitems, dcount, grid, flags, fstride, s);
-  else launch_batch_t<T, 16, 16, false>(d_ops, items, nitems, dcount, grid, flags, fstride, s);
+static void launch_batch_s(int sched, bool cubic, const void *d_ops, const BItem *items, int nitems, const int *dcount,
+                           int grid, const double *flags, int fstride, hipStream_t s) {
+  if (sched == 1) launch_batch_t<T, 8, 8, false>(cubic, d_ops, items, nitems, dcount, grid, flags, fstride, s);
+  else if (sched == 2) launch_batch_t<T, 16, 8, false>(cubic, d_ops, items, nitems, dcount, grid, flags, fstride, s);
+  else launch_batch_t<T, 16, 16, false>(cubic, d_ops, items, nitems, dcount, grid, flags, fstride, s);
 }
-void launch_engine_u_apply(int fp32, int sched, int unit, const void *d_ops, const BItem *items, int nitems,
+void launch_engine_u_apply(int fp32, int sched, int form, const void *d_ops, const BItem *items, int nitems,
                            const int *dcount, int grid, const double *flags, int fstride, hipStream_t s) {
-  if (unit) launch_batch_t<float, 16, 16, true>(d_ops, items, nitems, dcount, grid, flags, fstride, s);
-  else if (fp32) launch_batch_s<float>(sched, d_ops, items, nitems, dcount, grid, flags, fstride, s);
-  else launch_batch_s<double>(sched, d_ops, items, nitems, dcount, grid, flags, fstride, s);
+  const bool cubic = form & FORM_CUBIC;
+  if (form & FORM_UNIT) launch_batch_t<float, 16, 16, true>(cubic, d_ops, items, nitems, dcount, grid, flags, fstride, s);
+  else if (fp32) launch_batch_s<float>(sched, cubic, d_ops, items, nitems, dcount, grid, flags, fstride, s);
+  else launch_batch_s<double>(sched, cubic, d_ops, items, nitems, dcount, grid, flags, fstride, s);
 }
 
 // multigrid smoothing records and their persistent launch
@@ -1669,13 +1673,23 @@ void make_mg_smooth_op(const DevProblem &P, int post, const float *b, const floa
   r.OZ = OZ;
   *(BSmooth *)out = r;
 }
-void launch_batch_mg_smooth(int post, int unit, const void *d_ops, const BItem *items, const int *dcount, int grid,
+void launch_batch_mg_smooth(int post, int form, const void *d_ops, const BItem *items, const int *dcount, int grid,
                             const double *flags, int fstride, hipStream_t s) {
   auto go = [&](auto k) {
     hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, s, (const BSmooth *)d_ops, items, dcount, flags, fstride);
   };
-  if (post) unit ? go(k_batch_mg_smooth<UMgPostOp<true, false>>) : go(k_batch_mg_smooth<UMgPostOp<false, false>>);
-  else unit ? go(k_batch_mg_smooth<UMgPreOp<true>>) : go(k_batch_mg_smooth<UMgPreOp<false>>);
+  const int f = form & (FORM_UNIT | FORM_CUBIC);
+  if (post) {
+    if (f == (FORM_UNIT | FORM_CUBIC)) go(k_batch_mg_smooth<UMgPostOp<true, false, true>>);
+    else if (f == FORM_UNIT) go(k_batch_mg_smooth<UMgPostOp<true, false>>);
+    else if (f == FORM_CUBIC) go(k_batch_mg_smooth<UMgPostOp<false, false, true>>);
+    else go(k_batch_mg_smooth<UMgPostOp<false, false>>);
+  } else {
+    if (f == (FORM_UNIT | FORM_CUBIC)) go(k_batch_mg_smooth<UMgPreOp<true, true>>);
+    else if (f == FORM_UNIT) go(k_batch_mg_smooth<UMgPreOp<true>>);
+    else if (f == FORM_CUBIC) go(k_batch_mg_smooth<UMgPreOp<false, true>>);
+    else go(k_batch_mg_smooth<UMgPreOp<false>>);
+  }
 }
 
 // one member's operator entry for a persistent list (host memory `out`)
