@@ -22,7 +22,6 @@ struct MgHier {
   MgLevel lv[MAXL];
   int setups = 0;          // smoother bounds are re-estimated on every 16th set-up
   bool estimate = false;   // and are on their way in this one
-  double *dtmp = nullptr;  // FP64 diagonal of level 1 (largest coarse level)
 };
 }  // namespace vfg
 

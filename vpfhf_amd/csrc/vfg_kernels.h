@@ -149,7 +149,7 @@ void launch_mg_prolong(const Grid &Gf, const Grid &Gc, const BcMask &bc, const f
                        hipStream_t s);
 void launch_mg_cheb(const float *b, const float *y, const float *dinv, float *d, float *x, float c1, float c2,
                     int dfirst, int xzero, int64_t n, hipStream_t s);
-void launch_mg_recip32(const double *d, float *dinv, int64_t n, hipStream_t s);
+void launch_mg_diag32(const DevProblem &P, float *dinv, hipStream_t s);  // of a coarse level (P.unit)
 void launch_mg_fill32(float *x, float v, int64_t n, hipStream_t s);
 void launch_cell_to_node(const DevProblem &P, double lx, double ly, double lz, const double *cell, double *node,
                          int dof, hipStream_t s);

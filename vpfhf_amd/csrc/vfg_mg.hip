@@ -17,6 +17,7 @@
 #include "vfg_internal.h"
 #include "vfg_kernels.h"
 #include "vfg_mg.h"
+#include "vfg_modal.h"
 
 namespace vfg {
 
@@ -26,64 +27,108 @@ namespace vfg {
 // the factor that gives the isotropic coarse operator the point's P-wave
 // modulus: c_g = (kappa (1 + eta) + 4/3 mu s_g) / (lam + 2 mu), kappa =
 // lam + 2/3 mu (the spherical part there is not degraded)
-__global__ void k_mg_elem_coef(Grid G, const double *__restrict__ V, const double *__restrict__ E_elem, double E,
-                               double eta, const uint32_t *__restrict__ cmask, double lam1, double mu1,
-                               double *__restrict__ out) {
+// The mean of s = v^2 + eta over an element from the modal sums of v, orthogonal
+// on it; UNI: at the Gauss points, compressed ones with their own weight.
+template <bool UNI>
+__global__ __launch_bounds__(256) void k_mg_elem_coef(Grid G, const double *__restrict__ V,
+                                                      const double *__restrict__ E_elem, double E, double eta,
+                                                      const uint32_t *__restrict__ cmask, double lam1, double mu1,
+                                                      double *__restrict__ out) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= (int64_t)G.nex * G.ney * G.nez) return;
   const int ei = (int)(e % G.nex), ej = (int)((e / G.nex) % G.ney), ek = (int)(e / ((int64_t)G.nex * G.ney));
-  double v[8];
+  double v[8], m[8];
+#pragma unroll
   for (int a = 0; a < 8; a++) v[a] = V[node_id(G, ei + (a & 1), ej + ((a >> 1) & 1), ek + (a >> 2))];
-  const uint32_t cm = cmask ? cmask[e] : 0u;
-  const double kap1 = lam1 + 2. * mu1 / 3., pw = 1. / (lam1 + 2. * mu1);
+  modal_sums([&](int a) { return v[a]; }, m);
   double s = 0.;
-  for (int gz = 0; gz < 3; gz++)
-    for (int gy = 0; gy < 3; gy++)
-      for (int gx = 0; gx < 3; gx++) {
-        double vg = 0.;
-        for (int a = 0; a < 8; a++)
-          vg += ((a & 1) ? gP1(gx) : gP0(gx)) * (((a >> 1) & 1) ? gP1(gy) : gP0(gy)) * ((a >> 2) ? gP1(gz) : gP0(gz)) *
-                v[a];
-        const double sg = vg * vg + eta;
-        const bool comp = (cm >> ((gz * 3 + gy) * 3 + gx)) & 1u;
-        s += gW(gx) * gW(gy) * gW(gz) * (comp ? (kap1 * (1. + eta) + 4. * mu1 * sg / 3.) * pw : sg);
+  if constexpr (UNI) {
+    const uint32_t cm = cmask[e];
+    const double kap1 = lam1 + 2. * mu1 / 3., pw = 1. / (lam1 + 2. * mu1);
+#pragma unroll
+    for (int gz = 0; gz < 3; gz++)
+#pragma unroll
+      for (int gy = 0; gy < 3; gy++) {
+        double r[2];
+#pragma unroll
+        for (int x = 0; x < 2; x++)
+          r[x] = at_gauss(gy, at_gauss(gz, m[x], m[x + 4]), at_gauss(gz, m[x + 2], m[x + 6]));
+#pragma unroll
+        for (int gx = 0; gx < 3; gx++) {
+          const double vg = .125 * at_gauss(gx, r[0], r[1]), sg = vg * vg + eta;
+          const bool comp = (cm >> ((gz * 3 + gy) * 3 + gx)) & 1u;
+          s += gW(gx) * gW(gy) * gW(gz) * (comp ? (kap1 * (1. + eta) + 4. * mu1 * sg / 3.) * pw : sg);
+        }
       }
+  } else {
+#pragma unroll
+    for (int i = 7; i >= 0; i--) {
+      const int o = __builtin_popcount(i);
+      s += (o == 0 ? 1. : o == 1 ? 1. / 3. : o == 2 ? 1. / 9. : 1. / 27.) / 64. * (m[i] * m[i]);
+    }
+    s += eta;
+  }
   out[e] = (E_elem ? E_elem[e] : E) * s;
 }
 
-// fine elements e overlapping coarse element C along one axis, with overlaps
-__device__ __forceinline__ int mg_overlap(int C, int nf, int nc, int *e0, double *ov) {
-  const double a = (double)C * nf / nc, b = (double)(C + 1) * nf / nc;
-  const int lo = (int)floor(a);
-  int m = 0;
-  for (int e = lo; e < nf && (double)e < b && m < 4; e++) {
-    const double o = fmin((double)(e + 1), b) - fmax((double)e, a);
-    if (o > 0.) {
-      if (m == 0) *e0 = e;
-      ov[m++] = o;
-    }
+// Coarse coefficients: the mean of the fine elements under a coarse one, by
+// overlap.  Along one axis the fine elements lo .. lo + M - 1 meet coarse element
+// C (nf / nc <= 2: at most three, two where the grids are nested or equal), with
+// integer overlaps in units of 1 / nc that sum to nf (0 off the axis).
+template <int M>
+__device__ __forceinline__ void mg_overlap(int C, int nf, int nc, int (&e)[M], double (&w)[M]) {
+  const int lo = C * nf / nc;
+#pragma unroll
+  for (int q = 0; q < M; q++) {
+    const int a = (lo + q) * nc > C * nf ? (lo + q) * nc : C * nf;
+    const int b = (lo + q + 1) * nc < (C + 1) * nf ? (lo + q + 1) * nc : (C + 1) * nf;
+    w[q] = b > a && lo + q < nf ? (double)(b - a) : 0.;
+    e[q] = lo + q < nf ? lo + q : nf - 1;
   }
-  return m;
 }
-
-__global__ void k_mg_coarsen(Grid Gf, const double *__restrict__ cf, Grid Gc, double *__restrict__ cc) {
+template <int M>
+__global__ __launch_bounds__(256) void k_mg_coarsen(Grid Gf, const double *__restrict__ cf, Grid Gc,
+                                                    double *__restrict__ cc) {
   const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= (int64_t)Gc.nex * Gc.ney * Gc.nez) return;
   const int ci = (int)(c % Gc.nex), cj = (int)((c / Gc.nex) % Gc.ney), ck = (int)(c / ((int64_t)Gc.nex * Gc.ney));
-  int x0 = 0, y0 = 0, z0 = 0;
-  double ox[4], oy[4], oz[4];
-  const int mx = mg_overlap(ci, Gf.nex, Gc.nex, &x0, ox);
-  const int my = mg_overlap(cj, Gf.ney, Gc.ney, &y0, oy);
-  const int mz = mg_overlap(ck, Gf.nez, Gc.nez, &z0, oz);
-  double acc = 0., wsum = 0.;
-  for (int k = 0; k < mz; k++)
-    for (int j = 0; j < my; j++)
-      for (int i = 0; i < mx; i++) {
-        const double w = ox[i] * oy[j] * oz[k];
-        acc += w * cf[cell_id(Gf, x0 + i, y0 + j, z0 + k)];
-        wsum += w;
-      }
-  cc[c] = acc / wsum;
+  int x[M], y[M], z[M];
+  double wx[M], wy[M], wz[M];
+  mg_overlap<M>(ci, Gf.nex, Gc.nex, x, wx);
+  mg_overlap<M>(cj, Gf.ney, Gc.ney, y, wy);
+  mg_overlap<M>(ck, Gf.nez, Gc.nez, z, wz);
+  double acc = 0.;
+#pragma unroll
+  for (int k = 0; k < M; k++)
+#pragma unroll
+    for (int j = 0; j < M; j++) {
+      const double w = wy[j] * wz[k];
+#pragma unroll
+      for (int i = 0; i < M; i++) acc += (wx[i] * w) * cf[cell_id(Gf, x[i], y[j], z[k])];
+    }
+  cc[c] = acc / ((double)Gf.nex * Gf.ney * Gf.nez);
+}
+// FP32 inverse diagonal of a coarse level (s = 1): every element corner has
+// E vol / 9 [(lam + mu) / h_c^2 + mu sum_d 1 / h_d^2] = E kc; 1 on the Dirichlet
+// rows.  With the coefficients of its level about 8 us per level of a 32^3
+// problem, 21 us with the marching diagonal kernel and a reciprocal pass.
+__global__ __launch_bounds__(256) void k_mg_diag32(Grid G, const double *__restrict__ E, BcMask bc, double kx, double ky,
+                                                   double kz, float *__restrict__ dinv) {
+  const int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (n >= (int64_t)G.nx * G.ny * G.nz) return;
+  const int i = (int)(n % G.nx), j = (int)((n / G.nx) % G.ny), k = (int)(n / ((int64_t)G.nx * G.ny));
+  double s = 0.;
+#pragma unroll
+  for (int a = 0; a < 8; a++) {
+    const int ei = i - (a & 1), ej = j - ((a >> 1) & 1), ek = k - (a >> 2);
+    if (ei >= 0 && ei < G.nex && ej >= 0 && ej < G.ney && ek >= 0 && ek < G.nez) s += E[cell_id(G, ei, ej, ek)];
+  }
+  const double kc[3] = {kx, ky, kz};
+#pragma unroll
+  for (int c = 0; c < 3; c++) {
+    const double d = kc[c] * s;
+    dinv[3 * n + c] = on_dirichlet(G, bc.face[c], bc.vert[c], i, j, k) || d == 0. ? 1.f : (float)(1. / d);
+  }
 }
 
 // Transfers, plane blockIdx.y (so that indices are 32-bit): restriction one
@@ -126,11 +171,6 @@ __global__ void k_mg_cheb(const float *__restrict__ b, const float *__restrict__
   if (i < n) mg_cheb_entry(b, y, dinv, d, x, c1, c2, dfirst, xzero, i);
 }
 
-__global__ void k_mg_recip32(const double *__restrict__ d, float *__restrict__ dinv, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) dinv[i] = d[i] != 0. ? (float)(1. / d[i]) : 1.f;
-}
-
 __global__ void k_mg_fill32(float *x, float v, int64_t n) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) x[i] = v;
@@ -139,13 +179,17 @@ __global__ void k_mg_fill32(float *x, float v, int64_t n) {
 static unsigned nbm(int64_t n) { return (unsigned)((n + 255) / 256); }
 
 void launch_mg_elem_coef(const DevProblem &P, double *out, hipStream_t s) {
-  hipLaunchKernelGGL(k_mg_elem_coef, dim3(nbm(P.ne)), dim3(256), 0, s, P.G, (const double *)P.V,
-                     (const double *)P.E_elem, P.E, P.eta, (const uint32_t *)(P.unilateral ? P.cmask : nullptr),
-                     P.lam1, P.mu1, out);
+  auto go = [&](auto k) {
+    hipLaunchKernelGGL(k, dim3(nbm(P.ne)), dim3(256), 0, s, P.G, (const double *)P.V, (const double *)P.E_elem, P.E, P.eta,
+                       (const uint32_t *)P.cmask, P.lam1, P.mu1, out);
+  };
+  P.unilateral ? go(k_mg_elem_coef<true>) : go(k_mg_elem_coef<false>);
 }
 void launch_mg_coarsen(const Grid &Gf, const double *cf, const Grid &Gc, double *cc, hipStream_t s) {
   const int64_t ne = (int64_t)Gc.nex * Gc.ney * Gc.nez;
-  hipLaunchKernelGGL(k_mg_coarsen, dim3(nbm(ne)), dim3(256), 0, s, Gf, cf, Gc, cc);
+  auto two = [](int f, int c) { return f == c || f == 2 * c; };
+  auto go = [&](auto k) { hipLaunchKernelGGL(k, dim3(nbm(ne)), dim3(256), 0, s, Gf, cf, Gc, cc); };
+  two(Gf.nex, Gc.nex) && two(Gf.ney, Gc.ney) && two(Gf.nez, Gc.nez) ? go(k_mg_coarsen<2>) : go(k_mg_coarsen<3>);
 }
 void launch_mg_restrict(const Grid &Gf, const Grid &Gc, const BcMask &bc, const float *r, float *bcoarse,
                         hipStream_t s) {
@@ -166,8 +210,13 @@ void launch_mg_cheb(const float *b, const float *y, const float *dinv, float *d,
                     int dfirst, int xzero, int64_t n, hipStream_t s) {
   hipLaunchKernelGGL(k_mg_cheb, dim3(nbm(n)), dim3(256), 0, s, b, y, dinv, d, x, c1, c2, dfirst, xzero, n);
 }
-void launch_mg_recip32(const double *d, float *dinv, int64_t n, hipStream_t s) {
-  hipLaunchKernelGGL(k_mg_recip32, dim3(nbm(n)), dim3(256), 0, s, d, dinv, n);
+void launch_mg_diag32(const DevProblem &P, float *dinv, hipStream_t s) {
+  const Grid &G = P.G;
+  const double vol = G.hx * G.hy * G.hz / 9., i2[3] = {1. / (G.hx * G.hx), 1. / (G.hy * G.hy), 1. / (G.hz * G.hz)};
+  double kc[3];
+  for (int c = 0; c < 3; c++) kc[c] = vol * ((P.lam1 + P.mu1) * i2[c] + P.mu1 * (i2[0] + i2[1] + i2[2]));
+  hipLaunchKernelGGL(k_mg_diag32, dim3(nbm(P.nn)), dim3(256), 0, s, G, (const double *)P.E_elem, P.bcU, kc[0], kc[1],
+                     kc[2], dinv);
 }
 void launch_mg_fill32(float *x, float v, int64_t n, hipStream_t s) {
   hipLaunchKernelGGL(k_mg_fill32, dim3(nbm(n)), dim3(256), 0, s, x, v, n);

@@ -759,7 +759,6 @@ int mg_build(vfg_handle *h) {
     G = Gc;
     L++;
   }
-  if (L > 1) al.push_back({(void **)&m->dtmp, 8 * (size_t)m->lv[1].n});
   rc = vfg_alloc_group(h, al);
   for (int l = 1; l < L && !rc; l++) {
     const DevProblem &Pc = m->lv[l].P;
@@ -800,8 +799,7 @@ int mg_setup_begin(vfg_handle *h, const double *dinv64, hipStream_t s) {
     } else {
       launch_mg_coarsen(lf.P.G, lf.P.E_elem, Pc.G, Pc.E_elem, s);
     }
-    launch_u_diag(Pc, m.dtmp, s);
-    launch_mg_recip32(m.dtmp, lc.dinv, lc.n, s);
+    launch_mg_diag32(Pc, lc.dinv, s);
   }
   // lambda_max(D^-1 A) per level from 10 Jacobi-PCG steps (Lanczos).  The
   // top of the Jacobi-scaled spectrum is set by the element geometry and the
