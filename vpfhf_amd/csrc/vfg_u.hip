@@ -562,9 +562,9 @@ struct UApplyDotOp : UModOp<double, false, CUBIC> {
   }
   __device__ void partial(int slot, double v) const { part[slot] = v; }
 };
-template <bool CUBIC>
-__global__ __launch_bounds__(256, 2) void k_u_apply_dot(UApplyDotOp<CUBIC> op, int OZ) {
-  march_modal<16, 16>(op.G, op, OZ, xcd_block(),
+template <int W, bool CUBIC>
+__global__ __launch_bounds__(W *W, 2) void k_u_apply_dot(UApplyDotOp<CUBIC> op, int OZ) {
+  march_modal<W, W>(op.G, op, OZ, xcd_block(),
                       blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));
 }
 
@@ -1089,8 +1089,9 @@ struct ULoadsOp {
     return t == 3 ? BCU[3 * n + c] : t == 2 ? 1. : 0.;
   }
 };
-__global__ __launch_bounds__(256, 2) void k_u_loads(ULoadsOp op, int OZ) {
-  march_modal<16, 16>(op.G, op, OZ, xcd_block());
+template <int W>
+__global__ __launch_bounds__(W *W, 2) void k_u_loads(ULoadsOp op, int OZ) {
+  march_modal<W, W>(op.G, op, OZ, xcd_block());
 }
 
 __global__ __launch_bounds__(256) void k_u_rhs(URhsOp op, int OZ) {
@@ -1145,6 +1146,11 @@ static int device_slots(K kernel, int threads) {
 // FP32 grids of 16-64 nodes in x (coarse multigrid levels) march 8 x 8 tiles
 // of 7 x 7 owned nodes: more, shorter workgroups
 constexpr int SMALL_NX_LO = 16, SMALL_NX_HI = 64;
+// FP64 grids whose 8 x 8 tiles all run at once in chunks of one node plane take
+// them: the one-wavefront workgroups start and synchronise faster (cubes of 16
+// elements 11.1 -> 6.2 us, 32 9.0 -> 6.7, 40 equal; 44 and 56, which no longer
+// fit, 9.3 -> 11.9 and 12.8 -> 15.4 us)
+static bool small_fp64(const Grid &G);
 template <typename T>
 static void launch_u_apply_uni(const DevProblem &P, const T *x, T *y, const T *v, hipStream_t s) {
   UApplyUniOp<T> op;
@@ -1194,12 +1200,17 @@ static void launch_u_apply_t(const DevProblem &P, const T *x, T *y, const T *v, 
       hipLaunchKernelGGL(k_u_apply_ldsq, march_grid(P.G, 16, 16, OZ), dim3(256), 0, s, q, OZ);
       return;
     }
-    launch_u_apply_w<T, 16, false>(P, x, y, s);
+    small_fp64(P.G) ? launch_u_apply_w<T, 8, false>(P, x, y, s) : launch_u_apply_w<T, 16, false>(P, x, y, s);
   } else {
     const bool small = P.G.nx >= SMALL_NX_LO && P.G.nx <= SMALL_NX_HI;
     if (P.unit) small ? launch_u_apply_w<T, 8, true>(P, x, y, s) : launch_u_apply_w<T, 16, true>(P, x, y, s);
     else small ? launch_u_apply_w<T, 8, false>(P, x, y, s) : launch_u_apply_w<T, 16, false>(P, x, y, s);
   }
+}
+
+static bool small_fp64(const Grid &G) {
+  static int slots = device_slots(k_u_apply<double, 8, 8, false, false>, 64);
+  return (int64_t)((G.nx + 6) / 7) * ((G.ny + 6) / 7) * G.nz <= slots;
 }
 
 // per element: the Gauss points where tr(eps(U)) < 0
@@ -1402,16 +1413,16 @@ void launch_u_apply(const DevProblem &P, const double *x, double *y, hipStream_t
   launch_u_apply_t<double>(P, x, y, P.V, s);
 }
 
-template <bool CUBIC>
+template <int W, bool CUBIC>
 static int launch_u_apply_dot_c(const UModRec<double> &r, double *part, hipStream_t s) {
   UApplyDotOp<CUBIC> op;
   static_cast<UModRec<double> &>(op) = r;
   op.part = part;
   const Grid &G = r.G;
-  static int slots = device_slots(k_u_apply_dot<CUBIC>, 256);
-  const int OZ = choose_oz(G, ((G.nx + 14) / 15) * ((G.ny + 14) / 15), slots);
-  const dim3 g = march_grid(G, 16, 16, OZ);
-  hipLaunchKernelGGL(k_u_apply_dot<CUBIC>, g, dim3(256), 0, s, op, OZ);
+  static int slots = device_slots(k_u_apply_dot<W, CUBIC>, W * W);
+  const int OZ = choose_oz(G, ((G.nx + W - 2) / (W - 1)) * ((G.ny + W - 2) / (W - 1)), slots);
+  const dim3 g = march_grid(G, W, W, OZ);
+  hipLaunchKernelGGL((k_u_apply_dot<W, CUBIC>), g, dim3(W * W), 0, s, op, OZ);
   return (int)(g.x * g.y * g.z);
 }
 int launch_u_apply_dot(const DevProblem &P, const double *x, double *y, double *part, hipStream_t s) {
@@ -1430,7 +1441,9 @@ int launch_u_apply_dot(const DevProblem &P, const double *x, double *y, double *
   }
   UModRec<double> r;
   umod_fill<double>(r, P, x, y);
-  return r.m.cubic ? launch_u_apply_dot_c<true>(r, part, s) : launch_u_apply_dot_c<false>(r, part, s);
+  if (small_fp64(P.G))
+    return r.m.cubic ? launch_u_apply_dot_c<8, true>(r, part, s) : launch_u_apply_dot_c<8, false>(r, part, s);
+  return r.m.cubic ? launch_u_apply_dot_c<16, true>(r, part, s) : launch_u_apply_dot_c<16, false>(r, part, s);
 }
 void launch_u_apply_f32(const DevProblem &P, const float *x, float *y, hipStream_t s) {
   launch_u_apply_t<float>(P, x, y, P.V32, s);
@@ -1513,6 +1526,13 @@ static void launch_u_rhs_uni(const DevProblem &P, const double *U, const double 
   hipLaunchKernelGGL(k_u_rhs, march_grid(P.G, 16, 16, OZ), dim3(256), 0, s, op, OZ);
 }
 
+template <int W>
+static void launch_u_loads_w(const ULoadsOp &op, hipStream_t s) {
+  const Grid &G = op.G;
+  static int slots = device_slots(k_u_loads<W>, W * W);
+  const int OZ = choose_oz(G, ((G.nx + W - 2) / (W - 1)) * ((G.ny + W - 2) / (W - 1)), slots);
+  hipLaunchKernelGGL(k_u_loads<W>, march_grid(G, W, W, OZ), dim3(W * W), 0, s, op, OZ);
+}
 void launch_u_rhs(const DevProblem &P, const double *U, const double *BCU, double *out, int mode,
                   hipStream_t s) {
   if (P.unilateral) {  // (mode 2 is not used with NOCOMPRESSION: its load depends on U)
@@ -1539,10 +1559,7 @@ void launch_u_rhs(const DevProblem &P, const double *U, const double *BCU, doubl
     op.kt[d][2] = k * .6;
     op.kp[d] = w / (256. * h[d]);
   }
-  const int tiles = ((P.G.nx + 14) / 15) * ((P.G.ny + 14) / 15);
-  static int slots = device_slots(k_u_loads, 256);
-  const int OZ = choose_oz(P.G, tiles, slots);
-  hipLaunchKernelGGL(k_u_loads, march_grid(P.G, 16, 16, OZ), dim3(256), 0, s, op, OZ);
+  small_fp64(P.G) ? launch_u_loads_w<8>(op, s) : launch_u_loads_w<16>(op, s);
 }
 
 }  // namespace vfg
