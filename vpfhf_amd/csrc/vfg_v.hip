@@ -734,9 +734,6 @@ static int v_slots() {
 static int oz_for(const Grid &G) { return choose_oz(G, ((G.nx + 14) / 15) * ((G.ny + 14) / 15), v_slots()); }
 
 void launch_v_setup(const DevProblem &P, const double *U, hipStream_t s) {
-  const dim3 g((P.G.nx + 14) / 15, (P.G.ny + 14) / 15, P.G.nez);
-  if (P.unilateral) hipLaunchKernelGGL(k_v_setup<true>, g, dim3(256), 0, s, P, make_vsetup(P), U);
-  else hipLaunchKernelGGL(k_v_setup<false>, g, dim3(256), 0, s, P, make_vsetup(P), U);
   VRhsOp op;
   op.U = U; op.p = P.p; op.b = P.bV; op.G = P.G;
   const double h[3] = {P.G.hx, P.G.hy, P.G.hz}, vol = h[0] * h[1] * h[2];
@@ -745,6 +742,10 @@ void launch_v_setup(const DevProblem &P, const double *U, hipStream_t s) {
   op.crack = P.hasCrackPressure;
   int OZ = oz_for(P.G);
   hipLaunchKernelGGL(k_v_rhs, mgrid(P.G, OZ), dim3(256), 0, s, op, OZ);
+  // after the load: the moments are what the next product reads, and the last written
+  const dim3 g((P.G.nx + 14) / 15, (P.G.ny + 14) / 15, P.G.nez);
+  if (P.unilateral) hipLaunchKernelGGL(k_v_setup<true>, g, dim3(256), 0, s, P, make_vsetup(P), U);
+  else hipLaunchKernelGGL(k_v_setup<false>, g, dim3(256), 0, s, P, make_vsetup(P), U);
 }
 
 void launch_v_fixmask(const DevProblem &P, hipStream_t s) {
