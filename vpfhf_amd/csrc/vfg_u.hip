@@ -1245,132 +1245,133 @@ __device__ __forceinline__ Op op_of(const typename Op::Record &r) {
 }
 
 // Chebyshev-Jacobi solve of a small FP32 level from x = 0 in one workgroup
-// (the coarsest multigrid level, at most MGC_NE elements).  A thread owns one
-// element (its modulus, face sums of v and place are read once) and up to MGC_Q
-// entries (node, component), whose b, D^-1, x and direction stay in its
-// registers; only the iterate and the element forces go through LDS, component
-// by component so that consecutive lanes touch consecutive words.  A step is an
-// element pass and an entry pass that adds each node's eight element forces in
-// a fixed order (x-pairs, then y-pairs, the lower element layer before the
-// upper); the step itself is mg_cheb_entry's.  Latency-bound on one CU: 9^3
-// nodes 15 us, 27 us with E, b and D^-1 re-read from memory in every step and
-// the forces interleaved by element (eight-way bank conflicts).
-constexpr int MGC_T = 512, MGC_NE = 512, MGC_NN = 729;
-constexpr int MGC_Q = (3 * MGC_NN + MGC_T - 1) / MGC_T;
+// (the coarsest multigrid level, at most 8 elements per direction).  A thread
+// owns one element (its modulus and place are read once) and up to MGC_Q nodes,
+// whose b, D^-1, x and direction stay in its registers; only the iterate and the
+// element forces go through LDS, component by component so that consecutive
+// lanes touch consecutive words.  A step is an element pass and a node pass that
+// adds each node's eight element forces in a fixed order (x-pairs, then y-pairs,
+// the lower element layer before the upper); the step itself is
+// mg_cheb_entry's.  LDS is laid out for 8^3 elements whatever the level has, the
+// forces with a border of elements that stay zero: every address is a thread's
+// base plus a constant (a table of the forces' places, formed with divisions by
+// the level's extents, cost a quarter of the time).  Latency-bound on one CU:
+// 9^3 nodes 15 -> 11.7 us.
+constexpr int MGC_E = 8, MGC_N = MGC_E + 1, MGC_P = MGC_E + 2;  // elements, nodes, bordered elements per direction
+constexpr int MGC_T = MGC_E * MGC_E * MGC_E, MGC_NN = MGC_N * MGC_N * MGC_N, MGC_NP = MGC_P * MGC_P * MGC_P;
+constexpr int MGC_Q = (MGC_NN + MGC_T - 1) / MGC_T;
+struct MgcLds {
+  float x[3 * MGC_NN];
+  alignas(16) float r[24 * MGC_NP];  // [corner * 3 + component][bordered element]
+};
 
 // coef(i): the step's coefficients {c1, c2}
-template <bool UNIT, class Coef>
-__device__ __forceinline__ void mg_coarse_cheb_body(const UModOp<float, UNIT> &op, const float *__restrict__ b,
+template <bool UNIT, bool CUBIC, class Coef>
+__device__ __forceinline__ void mg_coarse_cheb_body(MgcLds &S, const UModRec<float> &rec, const float *__restrict__ b,
                                                     const float *__restrict__ dinv, float *__restrict__ xout,
                                                     int steps, const Coef &coef) {
-  __shared__ float sx[3 * MGC_NN];
-  __shared__ float sr[24 * MGC_NE + 1];  // [corner * 3 + component][element]; the last word stays 0
-  const Grid &G = op.G;
+  const Grid &G = rec.G;
   const int tid = threadIdx.x;
-  const int nn = G.nx * G.ny * G.nz, ne = G.nex * G.ney * G.nez;
-  if (tid == 0) sr[24 * MGC_NE] = 0.f;
-  // the entries t = tid + q MGC_T, component t / nn
-  float eb[MGC_Q], ed[MGC_Q], ex_[MGC_Q], dir[MGC_Q];
-  int src[MGC_Q][8];  // where the eight forces of the entry lie in sr
-  bool fixed[MGC_Q];
+  // the nodes tid + q MGC_T of a 9^3 grid
+  float eb[MGC_Q][3], ed[MGC_Q][3], xe[MGC_Q][3], dir[MGC_Q][3];
+  uint32_t fixed[MGC_Q];  // components on Dirichlet rows
+  int node[MGC_Q];        // of the level, -1: none
+  int src[MGC_Q];         // bordered element above the node
 #pragma unroll
   for (int q = 0; q < MGC_Q; q++) {
-    const int t = tid + q * MGC_T;
-    eb[q] = ed[q] = ex_[q] = dir[q] = 0.f;
-    fixed[q] = false;
+    const int t = tid + q * MGC_T, i = t % MGC_N, j = t / MGC_N % MGC_N, k = t / (MGC_N * MGC_N);
+    const bool in = t < MGC_NN && i < G.nx && j < G.ny && k < G.nz;
+    node[q] = in ? i + G.nx * (j + G.ny * k) : -1;
+    src[q] = in ? (i + 1) + MGC_P * ((j + 1) + MGC_P * (k + 1)) : MGC_NP - 1;
+    fixed[q] = 0u;
+    const uint32_t fb = face_bits_xy(G, i, j) | (k == 0 ? 16u : 0u) | (k == G.nz - 1 ? 32u : 0u);
 #pragma unroll
-    for (int a = 0; a < 8; a++) src[q][a] = 24 * MGC_NE;
-    if (t >= 3 * nn) continue;
-    const int c = t / nn, n = t - c * nn, ni = n % G.nx, nj = (n / G.nx) % G.ny, nk = n / (G.nx * G.ny);
-    eb[q] = b[3 * n + c];
-    ed[q] = dinv[3 * n + c];
-    // (selected: an index into the record would put it in scratch memory)
-    const uint8_t fc = c == 0 ? op.bc.face[0] : c == 1 ? op.bc.face[1] : op.bc.face[2];
-    const uint8_t vc = c == 0 ? op.bc.vert[0] : c == 1 ? op.bc.vert[1] : op.bc.vert[2];
-    fixed[q] = on_dirichlet(G, fc, vc, ni, nj, nk);
-#pragma unroll
-    for (int a = 0; a < 8; a++) {
-      const int ei = ni - (a & 1), ej = nj - ((a >> 1) & 1), ek = nk - (a >> 2);  // the node is its corner a
-      if (ei >= 0 && ei < G.nex && ej >= 0 && ej < G.ney && ek >= 0 && ek < G.nez)
-        src[q][a] = (a * 3 + c) * MGC_NE + ei + G.nex * (ej + G.ney * ek);
+    for (int c = 0; c < 3; c++) {
+      eb[q][c] = in ? b[3 * node[q] + c] : 0.f;
+      ed[q][c] = in ? dinv[3 * node[q] + c] : 0.f;
+      xe[q][c] = dir[q][c] = 0.f;
+      if (face_dirichlet(rec.bc.face[c], rec.bc.vert[c], fb)) fixed[q] |= 1u << c;
     }
   }
   // the thread's element
-  const bool el = tid < ne;
+  const int ex = tid % MGC_E, ey = tid / MGC_E % MGC_E, ez = tid / (MGC_E * MGC_E);
+  const bool el = ex < G.nex && ey < G.ney && ez < G.nez;
+  const int n0 = ex + MGC_N * (ey + MGC_N * ez), e0 = (ex + 1) + MGC_P * ((ey + 1) + MGC_P * (ez + 1));
   float E = 0.f, vb[4] = {}, vt[4] = {};
-  int n0 = 0;
-  const int nr = G.nx, np = G.nx * G.ny;
   if (el) {
-    const int ex = tid % G.nex, ey = (tid / G.nex) % G.ney, ez = tid / (G.nex * G.ney);
-    n0 = ex + nr * ey + np * ez;
-    E = op.aux(ex, ey, ez, 0, 0);
+    E = rec.E_elem ? (float)rec.E_elem[cell_id(G, ex, ey, ez)] : rec.E;
     if constexpr (!UNIT)
 #pragma unroll
       for (int q = 0; q < 4; q++) {
-        vb[q] = op.v[n0 + (q >> 1) * nr + (q & 1)];
-        vt[q] = op.v[n0 + np + (q >> 1) * nr + (q & 1)];
+        vb[q] = rec.v[node_id(G, ex + (q & 1), ey + (q >> 1), ez)];
+        vt[q] = rec.v[node_id(G, ex + (q & 1), ey + (q >> 1), ez + 1)];
       }
   }
+  for (int i = tid; i < 24 * MGC_NP / 4; i += MGC_T) ((float4 *)S.r)[i] = make_float4(0.f, 0.f, 0.f, 0.f);
   for (int i = 0; i < steps; i++) {
     const BmgCoef cf = coef(i);
     if (i > 0) {
 #pragma unroll
       for (int q = 0; q < MGC_Q; q++)
-        if (tid + q * MGC_T < 3 * nn) sx[tid + q * MGC_T] = ex_[q];
+        if (tid + q * MGC_T < MGC_NN)
+#pragma unroll
+          for (int c = 0; c < 3; c++) S.x[c * MGC_NN + tid + q * MGC_T] = xe[q][c];
       __syncthreads();
       if (el) {
         UFace<float> fb, ft;
         float t[2][3][4] = {};
 #pragma unroll
         for (int c = 0; c < 3; c++) {
-          const float *xb = sx + c * nn + n0, *xt = xb + np;
-          uface_set<float>(fb, c, xb[0], xb[1], xb[nr], xb[nr + 1]);
-          uface_set<float>(ft, c, xt[0], xt[1], xt[nr], xt[nr + 1]);
+          const float *xb = S.x + c * MGC_NN + n0, *xt = xb + MGC_N * MGC_N;
+          uface_set<float>(fb, c, xb[0], xb[1], xb[MGC_N], xb[MGC_N + 1]);
+          uface_set<float>(ft, c, xt[0], xt[1], xt[MGC_N], xt[MGC_N + 1]);
         }
-        um_layer<float, UNIT>(fb, ft, vb, vt, E, op.m, t[0], t[1]);
+        um_layer<float, UNIT, CUBIC>(fb, ft, vb, vt, E, rec.m, t[0], t[1]);
 #pragma unroll
         for (int kz = 0; kz < 2; kz++)
 #pragma unroll
           for (int c = 0; c < 3; c++) {
             const float(&u)[4] = t[kz][c];
-            const float e0 = u[0] - u[1], e1 = u[0] + u[1], f0 = u[2] - u[3], f1 = u[2] + u[3];
-            float *o = sr + (kz * 12 + c) * MGC_NE + tid;
-            o[0] = e0 - f0;
-            o[3 * MGC_NE] = e1 - f1;
-            o[6 * MGC_NE] = e0 + f0;
-            o[9 * MGC_NE] = e1 + f1;
+            const float p0 = u[0] - u[1], p1 = u[0] + u[1], f0 = u[2] - u[3], f1 = u[2] + u[3];
+            float *o = S.r + (kz * 12 + c) * MGC_NP + e0;
+            o[0] = p0 - f0;
+            o[3 * MGC_NP] = p1 - f1;
+            o[6 * MGC_NP] = p0 + f0;
+            o[9 * MGC_NP] = p1 + f1;
           }
       }
       __syncthreads();
     }
 #pragma unroll
-    for (int q = 0; q < MGC_Q; q++) {
-      float res = eb[q];
-      if (i > 0) {
-        const int(&s)[8] = src[q];
-        // corners a = 4 K + 2 J + I: the element layer below (K = 1), then the layer above
-        const float lo = (sr[s[7]] + sr[s[6]]) + (sr[s[5]] + sr[s[4]]);
-        const float y = lo + ((sr[s[3]] + sr[s[2]]) + (sr[s[1]] + sr[s[0]]));
-        res -= fixed[q] ? ex_[q] : y;
+    for (int q = 0; q < MGC_Q; q++)
+#pragma unroll
+      for (int c = 0; c < 3; c++) {
+        float res = eb[q][c];
+        if (i > 0) {
+          // corner a = 4 K + 2 J + I of the element below by (I, J, K): the layer below (K = 1), then the layer above
+          const float *s = S.r + c * MGC_NP + src[q];
+          auto at = [&](int a) { return s[a * 3 * MGC_NP - ((a & 1) + MGC_P * ((a >> 1 & 1) + MGC_P * (a >> 2)))]; };
+          const float lo = (at(7) + at(6)) + (at(5) + at(4));
+          const float y = lo + ((at(3) + at(2)) + (at(1) + at(0)));
+          res -= fixed[q] >> c & 1u ? xe[q][c] : y;
+        }
+        dir[q][c] = (i > 0 ? cf.c1 * dir[q][c] : 0.f) + cf.c2 * ed[q][c] * res;
+        xe[q][c] += dir[q][c];
       }
-      dir[q] = (i > 0 ? cf.c1 * dir[q] : 0.f) + cf.c2 * ed[q] * res;
-      ex_[q] += dir[q];
-    }
   }
 #pragma unroll
-  for (int q = 0; q < MGC_Q; q++) {
-    const int t = tid + q * MGC_T;
-    if (t < 3 * nn) {
-      const int c = t / nn;
-      xout[3 * (t - c * nn) + c] = ex_[q];
-    }
-  }
+  for (int q = 0; q < MGC_Q; q++)
+    if (node[q] >= 0)
+#pragma unroll
+      for (int c = 0; c < 3; c++) xout[3 * node[q] + c] = xe[q][c];
 }
 
-__global__ __launch_bounds__(MGC_T) void k_mg_coarse_cheb(UModOp<float, true> op, const float *__restrict__ b,
+template <bool CUBIC>
+__global__ __launch_bounds__(MGC_T) void k_mg_coarse_cheb(UModRec<float> rec, const float *__restrict__ b,
                                                           const float *__restrict__ dinv, float *__restrict__ xout,
                                                           MgChebCoefs cc) {
-  mg_coarse_cheb_body<true>(op, b, dinv, xout, cc.k, [&](int i) { return BmgCoef{cc.c1[i], cc.c2[i]}; });
+  __shared__ MgcLds S;
+  mg_coarse_cheb_body<true, CUBIC>(S, rec, b, dinv, xout, cc.k, [&](int i) { return BmgCoef{cc.c1[i], cc.c2[i]}; });
 }
 
 // the batched form: one workgroup per listed member (COARSE: at the level its
@@ -1387,19 +1388,23 @@ __global__ __launch_bounds__(MGC_T) void k_bmg_coarse_cheb(const BmgVec *__restr
   const int level = COARSE ? (int)c.start : 0;
   const BmgVec &v = lvt[c.p * BML + level];
   const BmgCoef *__restrict__ cf = coef + ((c.p * BML + level) * 2 + 1) * BMK;
-  mg_coarse_cheb_body<COARSE>(op_of<UModOp<float, COARSE>>(((const BApply<float> *)v.op)->op), v.b, v.dinv, v.x,
-                              MG_COARSE_DEG, [&](int i) { return cf[i]; });
+  __shared__ MgcLds S;
+  const UModRec<float> &rec = ((const BApply<float> *)v.op)->op;
+  auto co = [&](int i) { return cf[i]; };
+  if (rec.m.cubic) mg_coarse_cheb_body<COARSE, true>(S, rec, v.b, v.dinv, v.x, MG_COARSE_DEG, co);  // uniform
+  else mg_coarse_cheb_body<COARSE, false>(S, rec, v.b, v.dinv, v.x, MG_COARSE_DEG, co);
 }
 
 bool mg_coarse_fits(const DevProblem &P) {
-  return !P.unilateral && P.ne <= MGC_NE && P.nn <= MGC_NN;
+  return !P.unilateral && P.G.nex <= MGC_E && P.G.ney <= MGC_E && P.G.nez <= MGC_E;
 }
 
 void launch_mg_coarse_cheb(const DevProblem &P, const float *b, const float *dinv, float *x, const MgChebCoefs &cc,
                            hipStream_t s) {
-  UModOp<float, true> op;  // a coarse level: s = 1
-  umod_fill<float>(op, P, nullptr, nullptr);
-  hipLaunchKernelGGL(k_mg_coarse_cheb, dim3(1), dim3(MGC_T), 0, s, op, b, dinv, x, cc);
+  UModRec<float> rec;
+  umod_fill<float>(rec, P, nullptr, nullptr);
+  auto go = [&](auto k) { hipLaunchKernelGGL(k, dim3(1), dim3(MGC_T), 0, s, rec, b, dinv, x, cc); };
+  rec.m.cubic ? go(k_mg_coarse_cheb<true>) : go(k_mg_coarse_cheb<false>);
 }
 
 void launch_bmg_coarse_cheb(const BmgVec *lvt, int coarse, const BmgChunk *ch, const int *dn, int grid,
