@@ -156,33 +156,6 @@ template <class Op, class = void>
 struct has_aux : std::false_type {};
 template <class Op>
 struct has_aux<Op, std::void_t<decltype(&Op::aux)>> : std::true_type {};
-// Ops that keep per-element data in a tile-blocked layout (one 16x16 slot
-// block per workgroup tile and element layer; halo elements stored in every
-// tile that computes them) declare TILED and take (tile, slot, ek) instead of
-// (ex, ey, ek): a wavefront then reads each coefficient as one aligned,
-// contiguous 512-byte segment.
-template <class Op, class = void>
-struct is_tiled : std::false_type {};
-template <class Op>
-struct is_tiled<Op, std::void_t<decltype(Op::TILED)>> : std::true_type {};
-// Ops whose store also reads data of the owned node that is not staged define
-//   __device__ O own_load(int i, int j, int k)      (O trivially copyable)
-//   store(i, j, k, acc, own, O o)
-// the register march loads it one node plane ahead, beside the staged plane,
-// so its latency is not exposed at the store.
-template <class Op, class = void>
-struct has_own : std::false_type {};
-template <class Op>
-struct has_own<Op, std::void_t<decltype(&Op::own_load)>> : std::true_type {};
-template <class Op, class = void>
-struct own_of {
-  using type = int;
-};
-template <class Op>
-struct own_of<Op, std::void_t<decltype(&Op::own_load)>> {
-  using type = decltype(std::declval<const Op &>().own_load(0, 0, 0));
-};
-
 // Ops that also reduce over their owned nodes define
 //   __device__ double store(...)      (returns the node's contribution)
 //   __device__ void partial(int slot, double sum)
@@ -203,13 +176,11 @@ struct aux_of<Op, std::void_t<decltype(&Op::aux)>> {
 };
 
 template <typename T, int TX, int TY, class Op>
-__device__ __forceinline__ void march(const Grid &G, const Op &op, int OZ, int bx, int by, int bz, int rslot = 0) {
+__device__ __forceinline__ void march(const Grid &G, const Op &op, int OZ, int bx, int by, int bz) {
   constexpr int NF = Op::NF, NC = Op::NC;
   constexpr int NT = TX * TY, OX = TX - 1, OY = TY - 1, SX = TX + 1, SY = TY + 1;
   constexpr int NPF = (SX * SY + NT - 1) / NT;  // staged nodes per thread
   constexpr bool AUX = has_aux<Op>::value;
-  constexpr bool TILED = is_tiled<Op>::value;
-  constexpr bool RED = has_red<Op>::value;
   __shared__ T s_in[NF][SY * SX];
   __shared__ T s_red[2 * NC][NT];
   const int tid = threadIdx.x, tx = tid % TX, ty = tid / TX;
@@ -218,7 +189,6 @@ __device__ __forceinline__ void march(const Grid &G, const Op &op, int OZ, int b
   const bool exy_ok = ex >= 0 && ex < G.nex && ey >= 0 && ey < G.ney;
   const bool owner = tx < OX && ty < OY && (ox0 + tx) < G.nx && (oy0 + ty) < G.ny;
   const int64_t plane = (int64_t)G.nx * G.ny;
-  const int tile = bx + ((G.nx + OX - 1) / OX) * by;  // workgroup tile, for tiled ops
 
   // staged nodes of this thread: in-plane offsets, fixed for the whole march
   int64_t soff[NPF];
@@ -257,10 +227,7 @@ __device__ __forceinline__ void march(const Grid &G, const Op &op, int OZ, int b
   auto aux_at = [&](int ek) -> AuxT {
     AuxT a{};
     if constexpr (AUX) {
-      if (exy_ok && ek >= 0 && ek < G.nez) {
-        if constexpr (TILED) a = op.aux(tile, tid, ek);
-        else a = op.aux(ex, ey, ek);
-      }
+      if (exy_ok && ek >= 0 && ek < G.nez) a = op.aux(ex, ey, ek);
     }
     return a;
   };
@@ -273,24 +240,13 @@ __device__ __forceinline__ void march(const Grid &G, const Op &op, int OZ, int b
   T carry[NC];
 #pragma unroll
   for (int c = 0; c < NC; c++) carry[c] = T(0);
-  double racc = 0.;  // owned-node contributions (reducing ops)
-  using OwnT = typename own_of<Op>::type;
-  auto own_at = [&](int k) -> OwnT {
-    OwnT o{};
-    if constexpr (has_own<Op>::value)
-      if (owner && k >= oz0 && k >= 0 && k < G.nz) o = op.own_load(ox0 + tx, oy0 + ty, k);
-    return o;
-  };
-
   // one element layer: bottom plane xb (node plane ek), top plane xt (ek + 1)
-  auto layer = [&](int ek, const T (&xb)[4][NF], T (&xt)[4][NF], AuxT &aux_next, OwnT &own_next) {
+  auto layer = [&](int ek, const T (&xb)[4][NF], T (&xt)[4][NF], AuxT &aux_next) {
     const AuxT aux_cur = aux_next;
-    const OwnT own_cur = own_next;
     __syncthreads();
     commit();       // plane ek + 1
     fetch(ek + 2);  // in flight during this layer
     aux_next = aux_at(ek + 1);
-    own_next = own_at(ek + 1);
     __syncthreads();
     read_plane(xt);
     T r[8][NC];
@@ -307,9 +263,8 @@ __device__ __forceinline__ void march(const Grid &G, const Op &op, int OZ, int b
           xin[0][q][f] = xb[q][f];
           xin[1][q][f] = xt[q][f];
         }
-      const int e0 = TILED ? tile : ex, e1 = TILED ? tid : ey;
-      if constexpr (AUX) op.element(e0, e1, ek, xin, aux_cur, r);
-      else op.element(e0, e1, ek, xin, r);
+      if constexpr (AUX) op.element(ex, ey, ek, xin, aux_cur, r);
+      else op.element(ex, ey, ek, xin, r);
     }
     // x-combine: node (ex+1) gets corner i=1 of this element and corner i=0
     // of the element to the right (next lane inside the 16-lane row).
@@ -337,15 +292,7 @@ __device__ __forceinline__ void march(const Grid &G, const Op &op, int OZ, int b
         bot[c] = carry[c] + (cx[0][1][c] + s_red[c][tid + TX]);
         carry[c] = cx[1][1][c] + s_red[NC + c][tid + TX];
       }
-      if (ek >= oz0 && ek >= 0) {
-        if constexpr (has_own<Op>::value) {
-          if constexpr (RED) racc += op.store(ox0 + tx, oy0 + ty, ek, bot, xb[3], own_cur);
-          else op.store(ox0 + tx, oy0 + ty, ek, bot, xb[3], own_cur);
-        } else {
-          if constexpr (RED) racc += op.store(ox0 + tx, oy0 + ty, ek, bot, xb[3]);
-          else op.store(ox0 + tx, oy0 + ty, ek, bot, xb[3]);
-        }
-      }
+      if (ek >= oz0 && ek >= 0) op.store(ox0 + tx, oy0 + ty, ek, bot, xb[3]);
     }
   };
 
@@ -354,19 +301,13 @@ __device__ __forceinline__ void march(const Grid &G, const Op &op, int OZ, int b
   commit();
   fetch(oz0);
   AuxT aux_next = aux_at(oz0 - 1);
-  OwnT own_next = own_at(oz0 - 1);
   __syncthreads();
   read_plane(xa);
   const int ek_end = min(oz0 + OZ - 1, G.nz - 1);
   for (int ek = oz0 - 1; ek <= ek_end; ek += 2) {
-    layer(ek, xa, xb2, aux_next, own_next);
+    layer(ek, xa, xb2, aux_next);
     if (ek + 1 > ek_end) break;
-    layer(ek + 1, xb2, xa, aux_next, own_next);
-  }
-  if constexpr (RED) {
-    __shared__ double s_rs[NT / 64];
-    const double v = block_sum<NT>(racc, s_rs);
-    if (tid == 0) op.partial(rslot, v);
+    layer(ek + 1, xb2, xa, aux_next);
   }
 }
 
@@ -375,21 +316,17 @@ __device__ __forceinline__ void march(const Grid &G, const Op &op, int OZ, int b
 // for the next layer), so the element computation can re-read its corners
 // instead of keeping them in registers:
 //   __device__ void element_lds(int ex, int ey, int ek, const XS &xs, A aux, T (&r)[8][NC])
-// with xs(k, q, f) the value of staged field f at corner (k, q = j*2+i).  The
-// next plane is prefetched through registers as in march; the combination of
+// with xs(k, q, f) the value of staged field f at corner (k, q = j*2+i).  The combination of
 // the element results (x by lane shuffles, y through LDS, z carried) and the
-// stores are those of march.  Two barriers per layer.  No tiled or reducing
-// ops.  PF: the next plane is loaded one layer ahead into registers (held
-// during the element computation); without PF it is loaded at the start of
-// its layer and its latency is left to the other resident workgroup.
-template <typename T, int TX, int TY, bool PF, class Op>
+// stores are those of march.  Two barriers per layer.  The next plane is loaded
+// at the start of its layer; its latency is left to the other resident workgroup.
+template <typename T, int TX, int TY, class Op>
 __device__ __forceinline__ void march_lds(const Grid &G, const Op &op, int OZ, int bx, int by, int bz,
                                           int rslot = 0) {
   constexpr int NF = Op::NF, NC = Op::NC;
   constexpr int NT = TX * TY, OX = TX - 1, OY = TY - 1, SX = TX + 1, SY = TY + 1, PL = SX * SY;
   constexpr int NPF = (PL + NT - 1) / NT;
   constexpr bool RED = has_red<Op>::value;
-  static_assert(!is_tiled<Op>::value, "march_lds: untiled ops only");
   double racc = 0.;  // owned-node contributions (reducing ops)
   __shared__ T s_in[3][NF][PL];
   __shared__ T s_red[2 * NC][NT];
@@ -445,20 +382,14 @@ __device__ __forceinline__ void march_lds(const Grid &G, const Op &op, int OZ, i
   int bb = 0, bt = 1, bn = 2;
   fetch(oz0 - 1);
   commit(bb);
-  if constexpr (PF) fetch(oz0);
   AuxT aux_next = aux_at(oz0 - 1);
   const int ek_end = min(oz0 + OZ - 1, G.nz - 1);
   for (int ek = oz0 - 1; ek <= ek_end; ek++) {
     const AuxT aux_cur = aux_next;
     // buffer bt last held a plane read two layers ago; the barriers since
     // then order this write after those reads
-    if constexpr (PF) {
-      commit(bt);     // plane ek + 1
-      fetch(ek + 2);  // in flight during this layer
-    } else {
-      fetch(ek + 1);
-      commit(bt);
-    }
+    fetch(ek + 1);
+    commit(bt);
     aux_next = aux_at(ek + 1);
     __syncthreads();
     T r[8][NC];
@@ -515,94 +446,15 @@ __device__ __forceinline__ void march_lds(const Grid &G, const Op &op, int OZ, i
   }
 }
 
-// ------------------------------------------------- Gauss-point walk
-// Values (and, for the first NG fields, gradients) of trilinear nodal fields
-// at the 27 Gauss points of one element, by sum factorisation one axis at a
-// time: the 8 corner values f[a], a = (k*2+j)*2+i, are interpolated along z
-// for each Gauss layer, then along y, then along x, with each derivative
-// taken at the stage of its axis (d/dz of the corner pairs, constant in z).
-// f(gx, gy, gz, val[NG+NV], grad[NG][3]) is called for every point in the
-// order gz, gy, gx.  About 11 operations per point and gradient field and 3
-// per value-only field, against 32 and 8 for the direct 8-corner sums.
-// The corner values come from cv(q, a) (field q, corner a), read where they
-// are used: from LDS, the array need not stay in registers for the walk.
-// UZ, UY: unroll factors of the Gauss-layer and Gauss-row loops (1 keeps one
-// layer's or row's values live, for walks with many fields).  With UZ = 1 the
-// corners are re-read in every layer (a compiler barrier keeps the reads from
-// being hoisted out of the loop, which would hold them all in registers).
-template <int NG, int NV, int UZ = 3, int UY = 3, typename CV, typename F>
-__device__ __forceinline__ void gauss_walk_cv(const CV &cv, double ihx, double ihy, double ihz, const F &f) {
-  constexpr int NF = NG + NV;
-  double dz[NG > 0 ? NG : 1][4];  // d/dz at the 4 (x, y) corners
-#pragma unroll
-  for (int q = 0; q < NG; q++)
-#pragma unroll
-    for (int c = 0; c < 4; c++) dz[q][c] = (cv(q, c + 4) - cv(q, c)) * ihz;
-#pragma unroll UZ
-  for (int gz = 0; gz < 3; gz++) {
-    if constexpr (UZ == 1) __asm__ __volatile__("" ::: "memory");
-    const double pz = gP1(gz);
-    double z[NF][4];
-#pragma unroll
-    for (int q = 0; q < NF; q++)
-#pragma unroll
-      for (int c = 0; c < 4; c++) {
-        const double f0 = cv(q, c);
-        z[q][c] = f0 + pz * (cv(q, c + 4) - f0);
-      }
-#pragma unroll UY
-    for (int gy = 0; gy < 3; gy++) {
-      const double py = gP1(gy);
-      double y[NF][2], dyv[NG > 0 ? NG : 1][2], dzy[NG > 0 ? NG : 1][2];
-#pragma unroll
-      for (int q = 0; q < NF; q++)
-#pragma unroll
-        for (int i = 0; i < 2; i++) {
-          const double d = z[q][i + 2] - z[q][i];
-          y[q][i] = z[q][i] + py * d;
-          if (q < NG) {
-            dyv[q][i] = d * ihy;
-            dzy[q][i] = dz[q][i] + py * (dz[q][i + 2] - dz[q][i]);
-          }
-        }
-#pragma unroll
-      for (int gx = 0; gx < 3; gx++) {
-        const double px = gP1(gx);
-        double val[NF], grad[NG > 0 ? NG : 1][3];
-#pragma unroll
-        for (int q = 0; q < NF; q++) {
-          const double d = y[q][1] - y[q][0];
-          val[q] = y[q][0] + px * d;
-          if (q < NG) {
-            grad[q][0] = d * ihx;
-            grad[q][1] = dyv[q][0] + px * (dyv[q][1] - dyv[q][0]);
-            grad[q][2] = dzy[q][0] + px * (dzy[q][1] - dzy[q][0]);
-          }
-        }
-        f(gx, gy, gz, val, grad);
-      }
-    }
-  }
-}
-template <int NG, int NV, typename F>
-__device__ __forceinline__ void gauss_walk(const double (&fld)[NG + NV][8], double ihx, double ihy, double ihz,
-                                           const F &f) {
-  gauss_walk_cv<NG, NV>([&](int q, int a) { return fld[q][a]; }, ihx, ihy, ihz, f);
-}
-
 template <typename T>
 __device__ __forceinline__ T interp(int g, T f0, T f1) {
   return T(gP0(g)) * f0 + T(gP1(g)) * f1;
 }
 
-// the marches at a renumbered block (xcd_block)
+// the march at a renumbered block (xcd_block)
 template <typename T, int TX, int TY, class Op>
-__device__ __forceinline__ void march(const Grid &G, const Op &op, int OZ, Blk3 b, int rslot = 0) {
-  march<T, TX, TY>(G, op, OZ, b.x, b.y, b.z, rslot);
-}
-template <typename T, int TX, int TY, bool PF, class Op>
-__device__ __forceinline__ void march_lds(const Grid &G, const Op &op, int OZ, Blk3 b, int rslot = 0) {
-  march_lds<T, TX, TY, PF>(G, op, OZ, b.x, b.y, b.z, rslot);
+__device__ __forceinline__ void march(const Grid &G, const Op &op, int OZ, Blk3 b) {
+  march<T, TX, TY>(G, op, OZ, b.x, b.y, b.z);
 }
 
 }  // namespace vfg

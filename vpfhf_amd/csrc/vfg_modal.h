@@ -131,6 +131,10 @@ __device__ __forceinline__ bool face_dirichlet(uint8_t face, uint8_t vert, uint3
 //   store(n, fb, acc, own[, o])       fb: face bits of the node
 //   partial(slot, sum)                (optional) the workgroup's sum of what store returned
 template <class Op, class = void>
+struct has_own : std::false_type {};
+template <class Op>
+struct has_own<Op, std::void_t<decltype(&Op::own_load)>> : std::true_type {};
+template <class Op, class = void>
 struct ownm_of {
   using type = int;
 };

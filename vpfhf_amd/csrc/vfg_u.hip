@@ -610,10 +610,10 @@ struct UApplyLdsqDotOp : UApplyLdsqOp<true> {
   __device__ void partial(int slot, double v) const { part[slot] = v; }
 };
 __global__ __launch_bounds__(256, 2) void k_u_apply_ldsq(UApplyLdsqOp<false> op, int OZ) {
-  march_lds<double, 16, 16, false>(op.G, op, OZ, blockIdx.x, blockIdx.y, blockIdx.z);
+  march_lds<double, 16, 16>(op.G, op, OZ, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 __global__ __launch_bounds__(256, 2) void k_u_apply_ldsq_dot(UApplyLdsqDotOp op, int OZ) {
-  march_lds<double, 16, 16, false>(op.G, op, OZ, blockIdx.x, blockIdx.y, blockIdx.z,
+  march_lds<double, 16, 16>(op.G, op, OZ, blockIdx.x, blockIdx.y, blockIdx.z,
                                    blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));
 }
 // q of the node-owned tiles: block (bx, by, ek), thread = slot
