@@ -46,7 +46,7 @@ def test_vcycle_transfers(n):
 
 
 @pytest.mark.parametrize("unilateral", [0, 1], ids=["linear", "nocompression"])
-@pytest.mark.parametrize("n", [(2, 2, 2), (17, 18, 3), (18, 33, 20), (115, 114, 10)], ids=lambda n: "x".join(map(str, n)))
+@pytest.mark.parametrize("n", [(2, 2, 2), (17, 18, 3), (18, 33, 20), (115, 114, 10), (18, 18, 1101)], ids=lambda n: "x".join(map(str, n)))
 def test_energies_modal_form(oracle, n, unilateral):
     """Element tiles that are full, have one element or end in a ragged layer
     group, on both sides of the layer-group switch; AT1 and AT2."""

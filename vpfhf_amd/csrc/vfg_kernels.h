@@ -134,6 +134,9 @@ void launch_vec_apply_dirichlet(const DevProblem &P, int which, double *vec, con
                                 hipStream_t s);
 // partial sums per block: out[b*4 + {elastic, pressure work, surface, crack volume}]
 int energy_blocks(const DevProblem &P);
+// blocks of 16 x 16 element columns by 8 layers (2 on grids of fewer than 64
+// such columns): the unit in which vfg_energies_static states its limit
+int64_t energy_cell_blocks(const DevProblem &P);
 void launch_energies(const DevProblem &P, const double *U, const double *V, double *partials,
                      double *cellfield, double *efield, double *result4, hipStream_t s);
 // crack volume alone (one partial per block of energy_blocks)

@@ -91,25 +91,13 @@ void launch_vec_apply_dirichlet(const DevProblem &P, int which, double *vec, con
 //   pressure work = sum_g W p (u . grad v)
 //   surface = Gc/(4 atCv) sum_g W [(1-v)^k/eps + eps |grad v|^2], k = 1 (AT1), 2 (AT2)
 //   crack volume = sum_g W u . grad v
-// A workgroup takes a 16 x 16 tile of element columns over EZ element layers:
+// A workgroup takes a 16 x 16 tile of element columns over EZ element layers
+// (energy_layers):
 // the node planes (u, v, p, theta - thetaRef) are staged in LDS two at a time,
 // the next one loaded into registers meanwhile, and each thread evaluates its
 // element from the modal sums of its corners (vfg_modal.h).  One group of 4
 // partials per workgroup, in a fixed order.
 constexpr int EB = 256, ET = 16, EP = ET + 1;
-static int energy_ez(const Grid &G) {
-  const int tiles = ((G.nex + ET - 1) / ET) * ((G.ney + ET - 1) / ET);
-  return tiles >= 64 ? 8 : 2;
-}
-static dim3 energy_grid(const Grid &G) {
-  const int ez = energy_ez(G);
-  return dim3((G.nex + ET - 1) / ET, (G.ney + ET - 1) / ET, (G.nez + ez - 1) / ez);
-}
-int energy_blocks(const DevProblem &P) {
-  const dim3 g = energy_grid(P.G);
-  return (int)(g.x * g.y * g.z);
-}
-
 // the operators' constants, formed once on the host (kernel arguments sit in
 // scalar registers; formed in the kernel they take vector ones)
 struct EnergyConst {
@@ -278,7 +266,7 @@ __device__ __forceinline__ double spherical(const double (&R)[7], const double (
 
 // Bound by FP64 issue at two waves per SIMD: about 1350 operations per element
 // against 2900 when every field and gradient is interpolated from the corners
-// at each of the 27 points.  113 x 126 x 98: 116 us on first touch, 300 us so.
+// at each of the 27 points.  113 x 126 x 98: 99 us, 300 us so (eight layers).
 // Registers decide here: at three waves per SIMD 86 of them spill (254 us).
 template <bool UNI>
 __global__ __launch_bounds__(EB, 2) void k_energies(DevProblem P, EnergyConst C, const double *__restrict__ U,
@@ -457,21 +445,60 @@ __global__ __launch_bounds__(256) void k_reduce_partials(const double *__restric
   }
 }
 
+int device_slots_of(const void *kernel, int threads);  // vfg_u.hip
+static int64_t element_tiles(const Grid &G) { return (int64_t)((G.nex + ET - 1) / ET) * ((G.ney + ET - 1) / ET); }
+static dim3 layer_grid(const Grid &G, int ez) {
+  return dim3((G.nex + ET - 1) / ET, (G.ney + ET - 1) / ET, (G.nez + ez - 1) / ez);
+}
+// layers per workgroup of the crack volume, which is bound by memory
+static int volume_layers(const Grid &G) { return element_tiles(G) >= 64 ? 8 : 2; }
+// of the energies: the fewest whole rounds of resident workgroups times layers
+// (and one for the first plane and the sums), as for the marches.  Eight layers
+// whatever the grid left a second round of 113 x 126 x 98 elements half empty:
+// 115 us against 99 (thirteen layers; 3 to 14 layers 95 to 120).
+// Chunks under eight layers only while their partials fit a handle's own array.
+static int energy_layers(const DevProblem &P) {
+  static const int slots_uni = device_slots_of((const void *)k_energies<true>, EB);
+  static const int slots_lin = device_slots_of((const void *)k_energies<false>, EB);
+  const int slots = P.unilateral ? slots_uni : slots_lin;
+  const int64_t tiles = element_tiles(P.G);
+  int best = 8;
+  int64_t best_cost = INT64_MAX;
+  for (int ez = 1; ez <= P.G.nez; ez++) {
+    const int chunks = (P.G.nez + ez - 1) / ez;
+    if (ez > 1 && (P.G.nez + ez - 2) / (ez - 1) == chunks) continue;  // same chunk count, shorter is free
+    if (ez < 8 && tiles * chunks > 65536) continue;
+    const int64_t cost = (tiles * chunks + slots - 1) / slots * (ez + 1);
+    if (cost < best_cost) best_cost = cost, best = ez;
+  }
+  return best;
+}
+int64_t energy_cell_blocks(const DevProblem &P) {
+  const dim3 g = layer_grid(P.G, volume_layers(P.G));
+  return (int64_t)g.x * g.y * g.z;
+}
+int energy_blocks(const DevProblem &P) {
+  const dim3 g = layer_grid(P.G, energy_layers(P));
+  return (int)std::max((int64_t)g.x * g.y * g.z, energy_cell_blocks(P));
+}
+
 void launch_energies(const DevProblem &P, const double *U, const double *V, double *partials,
                      double *cellfield, double *efield, double *result4, hipStream_t s) {
-  const int nb = energy_blocks(P), ez = energy_ez(P.G);
+  const int ez = energy_layers(P);
+  const dim3 g = layer_grid(P.G, ez);
   auto go = [&](auto k) {
-    hipLaunchKernelGGL(k, energy_grid(P.G), dim3(EB), 0, s, P, energy_const(P), U, V, partials, cellfield, efield,
-                       ez);
+    hipLaunchKernelGGL(k, g, dim3(EB), 0, s, P, energy_const(P), U, V, partials, cellfield, efield, ez);
   };
   P.unilateral ? go(k_energies<true>) : go(k_energies<false>);
-  hipLaunchKernelGGL(k_reduce_partials<4>, dim3(1), dim3(256), 0, s, (const double *)partials, nb, result4);
+  hipLaunchKernelGGL(k_reduce_partials<4>, dim3(1), dim3(256), 0, s, (const double *)partials, (int)(g.x * g.y * g.z),
+                     result4);
 }
 void launch_crack_volume(const DevProblem &P, const double *U, const double *V, double *partials, double *cellfield,
                          double *result, hipStream_t s) {
-  hipLaunchKernelGGL(k_crack_volume, energy_grid(P.G), dim3(EB), 0, s, P.G, energy_const(P), U, V, partials, cellfield,
-                     energy_ez(P.G));
-  hipLaunchKernelGGL(k_reduce_partials<1>, dim3(1), dim3(256), 0, s, (const double *)partials, energy_blocks(P),
+  const int ez = volume_layers(P.G);
+  const dim3 g = layer_grid(P.G, ez);
+  hipLaunchKernelGGL(k_crack_volume, g, dim3(EB), 0, s, P.G, energy_const(P), U, V, partials, cellfield, ez);
+  hipLaunchKernelGGL(k_reduce_partials<1>, dim3(1), dim3(256), 0, s, (const double *)partials, (int)(g.x * g.y * g.z),
                      result);
 }
 
@@ -707,12 +734,13 @@ int scratch_address(vfg_handle *h, double **out) {
 extern "C" int vfg_energies_static(vfg_handle *h, const double *U, const double *V, double out[4]) {
   if (!h) return vfg_fail(nullptr, VFG_E_ARG, "NULL handle");
   if (!U || !V || !out) return vfg_fail(h, VFG_E_ARG, "vfg_energies_static: NULL array");
-  const int nb = vfg::energy_blocks(h->P);
+  // (the groups that are written are no more than these, or than 65536)
+  const int64_t nb = vfg::energy_cell_blocks(h->P);
   if (nb > ENERGY_STATIC_BLOCKS)
     return vfg_fail(h, VFG_E_ARG,
-                    "vfg_energies_static: %lld cells need %d partial groups, more than the %d of the "
+                    "vfg_energies_static: %lld cells need %lld partial groups, more than the %d of the "
                     "static scratch array (use vfg_energies)",
-                    (long long)h->P.ne, nb, ENERGY_STATIC_BLOCKS);
+                    (long long)h->P.ne, (long long)nb, ENERGY_STATIC_BLOCKS);
   double *part = nullptr;
   int rc = scratch_address(h, &part);
   if (rc) return rc;
