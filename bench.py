@@ -26,9 +26,10 @@ sys.path.insert(0, ROOT)
 
 PEAK_HBM_GBS = 8000.0
 PEAK_FP64_TFLOPS = 78.6  # MI355X FP64 vector (dense)
-# FP64 operations of the apply's element routine (u_elem_apply_lds), counted
-# in the compiled kernel's AMD assembly: 978 FMA + 123 MUL + 261 ADD per element
-FP64_FLOPS_PER_ELEMENT = 2 * 978 + 123 + 261
+# FP64 operations of the apply per element (the moment form for cubic elements,
+# with the combination of its neighbours), counted in the compiled kernel's AMD
+# assembly: 366 FMA + 69 MUL + 155 ADD
+FP64_FLOPS_PER_ELEMENT = 2 * 366 + 69 + 155
 
 
 def apply_bytes(nn, ne, fp32=False, hetero=True, stored=False):

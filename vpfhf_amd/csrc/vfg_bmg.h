@@ -44,7 +44,7 @@ int bmg_create_slots(int np, BatchMG **out);
 void bmg_destroy(BatchMG *g);
 // sets (h != nullptr) or clears member p; the work lists change at the next bmg_rebuild
 int bmg_set_member(BatchMG *g, int p, vfg_handle *h, float *r32, float *z32);
-// rebuilds the work lists of the current members on stream s (synchronised);
+// rebuilds the work lists of the current members (uploads queued on stream s);
 // *grew is set when a device list moved or the level count changed, i.e.
 // when a graph that captured bmg_vcycle must be captured again
 int bmg_rebuild(BatchMG *g, hipStream_t s, bool *grew);

@@ -2,8 +2,9 @@
 //
 // Element basis: trilinear Q1 on an axis-aligned box, 3-point Gauss-Legendre
 // per direction (27 points), exactly the rule of VFCartFEElement3DInit
-// (VFCartFE.c:90-116, 216-269).  The 27-point tables are never stored: every
-// quantity is evaluated by sum factorisation with the 1-D tables below.
+// (VFCartFE.c:90-116, 216-269).  The 27-point tables are never stored: what
+// visits the points does so by sum factorisation with the 1-D tables below, the
+// rest works on polynomial moments (vfg_modal.h).
 //
 // Node accumulation ("gather") without atomics: a workgroup owns a tile of
 // (TX-1) x (TY-1) node columns and marches upward through a z-chunk of node
@@ -58,8 +59,8 @@ __device__ __forceinline__ Blk3 xcd_block() {
 
 // tr(eps(u)) at Gauss point (gx, gy, gz) of an element from its 8 nodal
 // displacements (local node a = (k*2+j)*2+i), accumulated per component over
-// the nodes and summed as (d1u1 + d2u2) + d3u3: every kernel that branches on
-// its sign (UNILATERAL_NOCOMPRESSION) evaluates it this way.
+// the nodes and summed as (d1u1 + d2u2) + d3u3: the u operator, its diagonal and
+// its loads branch on the sign of this value (UNILATERAL_NOCOMPRESSION).
 __device__ __forceinline__ double tr_eps_at(const double (&u)[8][3], int gx, int gy, int gz, double ihx,
                                             double ihy, double ihz) {
   double h0 = 0., h1 = 0., h2 = 0.;

@@ -1295,9 +1295,9 @@ int vfg_u_solve(vfg_handle *h, double *U, const double *BCU, const vfg_solve_opt
     if (!rc) rc = pcg_mg(h, n, A, x, r, p, q, h->wf[0], h->wf[1], o->rtol, o->atol, o->maxit, 4, &inf, &Ad);
     inf.outer = 1;
   } else {
-    // the u-operator is issue-bound at one wave per SIMD: fusing the direction
-    // update into its staging, as the V-solve does, measured slower than the
-    // separate vector kernels (282 us against 215 + 33 us at 128^3)
+    // the u-operator is issue-bound: fusing the direction update into its
+    // staging, as the V-solve does, measured slower than the separate vector
+    // kernels (with a 27-point product 282 us against 215 + 33 us at 128^3)
     ApplyFn A = [&](const double *in, double *out) { launch_u_apply(P, in, out, s); };
     DotApplyFn Ad = [&](const double *in, double *out) { return launch_u_apply_dot(P, in, out, h->part, s); };
     rc = pcg(h, n, A, dinv, x, r, z, p, q, o->rtol, o->atol, o->maxit, 20, &inf, &Ad);

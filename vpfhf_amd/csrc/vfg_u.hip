@@ -7,9 +7,10 @@
 //   s_g = v_g^2 + eta.
 // Applied matrix-free: (Ke x)_{a,c} = sum_g sum_d sigma_cd(g) d_d phi_a(g) with
 //   sigma = W s (lam tr(H) I + mu (H + H^T)),  H_cd = d_d u_c  (displacement
-//   gradient of x).  All 27-point quantities are obtained by sum
-// factorisation with the 1-D Gauss tables; d_x u_c is constant along x, so it
-// takes 9 distinct values per component.
+//   gradient of x).  Without compression the sum over the 27 points is taken
+// in closed form from polynomial moments of s and the modal sums of x
+// (vfg_umodal.h); the compressed and the stored-coefficient forms visit the
+// points by sum factorisation with the 1-D Gauss tables.
 #include "vfg_internal.h"
 #include "vfg_umodal.h"
 #include "vfg_kernels.h"
