@@ -128,3 +128,15 @@ def test_batch_forms(oracle):
         B.close()
         for p in P:
             p.close()
+
+
+@pytest.mark.parametrize("n", [(2, 2, 2), (8, 15, 4), (9, 16, 31), (46, 17, 3), (47, 46, 30)], ids=lambda n: "x".join(map(str, n)))
+def test_u_diag_moment_form(oracle, n):
+    # 8 elements of some 30 positive terms each: 240 eps = 5e-14, 1e-12 as for
+    # the other operators, entry by entry
+    s = S.make(n=n, l=(1.0, 2.3, 0.6), seed=3 * sum(n), nu=0.3, bcU=S.MIXED_U)
+    op, F = S.to_oracle(oracle, s)
+    P = S.to_gpu(s)
+    ref = oracle.u_jacobian(op, F).diagonal()
+    assert np.all(np.abs(P.u_diag() - ref) <= 1e-12 * np.abs(ref))
+    P.close()

@@ -658,7 +658,7 @@ struct UDiagOp {
   const double *v;
   double *d;
   const double *E_elem;
-  const uint32_t *cmask;  // UNILATERAL_NOCOMPRESSION state (nullptr: none)
+  const uint32_t *cmask;  // UNILATERAL_NOCOMPRESSION state
   Grid G;
   BcMask bc;
   double E, lam1, mu1, eta, vol;
@@ -671,7 +671,7 @@ struct UDiagOp {
   __device__ void element(int ex, int ey, int ek, const double (&xin)[2][4][1], double (&r)[8][3]) const {
     double Ee = E_elem ? E_elem[cell_id(G, ex, ey, ek)] : E;
     double cE = Ee * vol;
-    const uint32_t cm = cmask ? cmask[cell_id(G, ex, ey, ek)] : 0u;
+    const uint32_t cm = cmask[cell_id(G, ex, ey, ek)];
     const double kap1 = (lam1 + 2. * mu1 / 3.) * (1. + eta);
     const double i2[3] = {1. / (G.hx * G.hx), 1. / (G.hy * G.hy), 1. / (G.hz * G.hz)};
     double vx[2][2][3];  // v along x on the (j, k) lines
@@ -741,7 +741,88 @@ struct UDiagOp {
   }
 };
 
-__global__ __launch_bounds__(256) void k_u_diag(UDiagOp op, int OZ) { march<double, 16, 16>(op.G, op, OZ, xcd_block()); }
+__global__ __launch_bounds__(256) void k_u_diag_uni(UDiagOp op, int OZ) {
+  march<double, 16, 16>(op.G, op, OZ, xcd_block());
+}
+
+// The same without compression, from the moments of s = v^2 + eta: (d_x phi_a)^2
+// = (1 +- y)^2 (1 +- z)^2 / (16 hx^2) in the element's variables, so its integral
+// is a sum of moments without x, in modal form: 1, y, z and yz parts.  Bound by
+// FP64 issue on large grids, by latency on small ones: 128^3 114 -> 46 us, a
+// cube of 32 elements 13 -> 5.7 us.
+struct UDiagModOp {
+  using T = double;
+  static constexpr int NF = 1, NC = 3;
+  const double *v;
+  double *d;
+  const double *E_elem;
+  Grid G;
+  BcMask bc;
+  double E, eta4, lr1;  // 4 eta; (lam + mu) / mu
+  double kd[3];         // vol mu / (16 h_d^2), per 144 times a moment
+  struct Face {
+    double v[4];
+  };
+  struct Own {};
+  using Aux = double;  // E_e
+  using Raw = double;
+  static __device__ double off() { return 0.; }
+  __device__ double load(int, int64_t n) const { return v[n]; }
+  __device__ double stage(int, double x) const { return x; }
+  template <class RD>
+  __device__ void face(const RD &rd, Face &F) const {
+#pragma unroll
+    for (int q = 0; q < 4; q++) F.v[q] = rd(0, q);
+  }
+  __device__ Own own(const Face &) const { return Own{}; }
+  __device__ double aux(int ex, int ey, int ek, int, int) const {
+    return E_elem ? E_elem[cell_id(G, ex, ey, ek)] : E;
+  }
+  __device__ void element(double Ee, const Face &B, const Face &F, double (&tot)[3][4], double (&carry)[3][4]) const {
+    double M[3][3][3], I[3][8], sum[8];  // I: of (d_d phi)^2, by modes
+    um_moments<double>(B.v, F.v, Ee, eta4, M);
+#pragma unroll
+    for (int i = 0; i < 8; i++) sum[i] = 0.;
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+      const int o1 = d == 0 ? 1 : 0, o2 = d == 2 ? 1 : 2;
+      double s[3], o[3];
+#pragma unroll
+      for (int b = 0; b < 3; b++) {
+        auto m = [&](int c) { return d == 0 ? M[0][b][c] : d == 1 ? M[b][0][c] : M[b][c][0]; };
+        s[b] = m(0) + m(2);
+        o[b] = 2. * m(1);
+      }
+#pragma unroll
+      for (int i = 0; i < 8; i++) I[d][i] = 0.;
+      I[d][0] = kd[d] * (s[0] + s[2]);
+      I[d][1 << o1] = kd[d] * (2. * s[1]);
+      I[d][1 << o2] = kd[d] * (o[0] + o[2]);
+      I[d][1 << o1 | 1 << o2] = kd[d] * (2. * o[1]);
+#pragma unroll
+      for (int i = 0; i < 8; i++) sum[i] += I[d][i];
+    }
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      double R[8];
+#pragma unroll
+      for (int i = 0; i < 8; i++) R[i] = sum[i] + lr1 * I[c][i];
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        tot[c][q] += R[q] - R[q + 4];
+        carry[c][q] = R[q] + R[q + 4];
+      }
+    }
+  }
+  __device__ void store(int64_t n, uint32_t fb, const double (&acc)[3], const Own &) const {
+#pragma unroll
+    for (int c = 0; c < 3; c++) d[3 * n + c] = face_dirichlet(bc.face[c], bc.vert[c], fb) ? 1. : acc[c];
+  }
+};
+template <int W>
+__global__ __launch_bounds__(W *W, 2) void k_u_diag(UDiagModOp op, int OZ) {
+  march_modal<W, W>(op.G, op, OZ, xcd_block());
+}
 
 // ------------------------------------------------------- load vector / residual
 // b_{a,c} = sum_g W d_c phi_a [(3lam+2mu) alpha dth s + beta p v]          (thermo-poro)
@@ -1502,16 +1583,33 @@ int launch_mg_postsmooth(const DevProblem &P, const float *b, const float *dinv,
   return P.unit ? mg_launch<UMgPostOp<true, false>>(P, op, s) : mg_launch<UMgPostOp<false, false>>(P, op, s);
 }
 
-void launch_u_diag(const DevProblem &P, double *d, hipStream_t s) {
+static void launch_u_diag_uni(const DevProblem &P, double *d, hipStream_t s) {
   UDiagOp op;
   op.v = P.V; op.d = d; op.E_elem = P.E_elem; op.G = P.G; op.bc = P.bcU;
-  op.cmask = P.unilateral ? P.cmask : nullptr;
+  op.cmask = P.cmask;
   op.E = P.E; op.lam1 = P.lam1; op.mu1 = P.mu1; op.eta = P.eta;
   op.vol = P.G.hx * P.G.hy * P.G.hz;
-  int tiles = ((P.G.nx + 14) / 15) * ((P.G.ny + 14) / 15);
-  static int slots = device_slots(k_u_diag, 256);
-  int OZ = choose_oz(P.G, tiles, slots);
-  hipLaunchKernelGGL(k_u_diag, march_grid(P.G, 16, 16, OZ), dim3(256), 0, s, op, OZ);
+  const int tiles = ((P.G.nx + 14) / 15) * ((P.G.ny + 14) / 15);
+  static int slots = device_slots(k_u_diag_uni, 256);
+  const int OZ = choose_oz(P.G, tiles, slots);
+  hipLaunchKernelGGL(k_u_diag_uni, march_grid(P.G, 16, 16, OZ), dim3(256), 0, s, op, OZ);
+}
+template <int W>
+static void launch_u_diag_w(const UDiagModOp &op, hipStream_t s) {
+  const Grid &G = op.G;
+  static int slots = device_slots(k_u_diag<W>, W * W);
+  const int OZ = choose_oz(G, ((G.nx + W - 2) / (W - 1)) * ((G.ny + W - 2) / (W - 1)), slots);
+  hipLaunchKernelGGL(k_u_diag<W>, march_grid(G, W, W, OZ), dim3(W * W), 0, s, op, OZ);
+}
+void launch_u_diag(const DevProblem &P, double *d, hipStream_t s) {
+  if (P.unilateral) return launch_u_diag_uni(P, d, s);
+  UDiagModOp op;
+  const Grid &G = P.G;
+  op.v = P.V; op.d = d; op.E_elem = P.E_elem; op.G = G; op.bc = P.bcU;
+  op.E = P.E; op.eta4 = 4. * P.eta; op.lr1 = (P.lam1 + P.mu1) / P.mu1;
+  const double h[3] = {G.hx, G.hy, G.hz};
+  for (int k = 0; k < 3; k++) op.kd[k] = h[0] * h[1] * h[2] * P.mu1 / (16. * 144. * h[k] * h[k]);
+  small_fp64(G) ? launch_u_diag_w<8>(op, s) : launch_u_diag_w<16>(op, s);
 }
 
 static void launch_u_rhs_uni(const DevProblem &P, const double *U, const double *BCU, double *out, int mode,
