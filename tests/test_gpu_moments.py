@@ -45,6 +45,19 @@ def test_vcycle_transfers(n):
     P.close()
 
 
+def test_vcycle_long_column():
+    """More node planes than a launch has block rows (65535)."""
+    s = S.make(n=(3, 2, 66001), l=(1.0, 0.5, 33000.0), seed=7, bcU=S.MIXED_U)
+    P = S.to_gpu(s)
+    free = 1.0 - P.bc_mask("U")
+    rng = np.random.default_rng(7)
+    a, b = (rng.standard_normal(3 * P.nn) * free for _ in range(2))
+    Ma, Mb = P.u_pc_apply(a), P.u_pc_apply(b)
+    # FP32 throughout: 1e-5 of the norms, as for one FP32 apply
+    assert abs(a @ Mb - b @ Ma) <= 1e-5 * (np.linalg.norm(a) * np.linalg.norm(Mb) + np.linalg.norm(b) * np.linalg.norm(Ma))
+    P.close()
+
+
 @pytest.mark.parametrize("unilateral", [0, 1], ids=["linear", "nocompression"])
 @pytest.mark.parametrize("n", [(2, 2, 2), (17, 18, 3), (18, 33, 20), (115, 114, 10), (18, 18, 1101)], ids=lambda n: "x".join(map(str, n)))
 def test_energies_modal_form(oracle, n, unilateral):

@@ -15,7 +15,18 @@ namespace vfg {
 //   coefficients: the overlap-weighted mean of the fine elements under each
 //     coarse element.
 // The weights are formed from integers, (nf - |i nc - I nf|) / nf, and written
-// out (1/2, 1, 1/2) where the grids are nested.
+// out (1/2, 1, 1/2) where the grids are nested.  A product of two counts passes
+// 31 bits on an axis of more than 65535 elements, so quotients are written out
+// for the pairs in use (nc = nf or ceil(nf / 2)) and differences of products,
+// which are a few nf at most, are formed modulo 2^32.
+// floor(C nf / nc), 0 <= C < nc
+__device__ __forceinline__ int mg_floor(int C, int nf, int nc) {
+  return nf == nc ? C : 2 * C - (nf < 2 * nc && C > 0 ? 1 : 0);
+}
+// i nc - I nf
+__device__ __forceinline__ int mg_diff(int i, int nc, int I, int nf) {
+  return (int)((unsigned)i * (unsigned)nc - (unsigned)I * (unsigned)nf);
+}
 __device__ __forceinline__ bool mg_nested_grids(const Grid &Gf, const Grid &Gc) {
   return Gf.nex == 2 * Gc.nex && Gf.ney == 2 * Gc.ney && Gf.nez == 2 * Gc.nez;
 }
@@ -35,11 +46,11 @@ __device__ __forceinline__ void mg_gather(int I, int nf, int nc, int (&i)[M], fl
       w[q] = i[q] < 0 || i[q] > nf ? 0.f : q == 1 ? 1.f : .5f;
     }
   } else {
-    const int lo = I > 0 ? (I - 1) * nf / nc + 1 : 0;  // first i with i nc > (I - 1) nf
+    const int lo = I > 0 ? mg_floor(I - 1, nf, nc) + 1 : 0;  // first i with i nc > (I - 1) nf
 #pragma unroll
     for (int q = 0; q < M; q++) {
       i[q] = lo + q;
-      const int m = i[q] * nc - I * nf, n = nf - (m < 0 ? -m : m);
+      const int m = mg_diff(i[q], nc, I, nf), n = nf - (m < 0 ? -m : m);
       w[q] = n <= 0 || i[q] > nf ? 0.f : mg_wt(n, nf);
     }
   }
@@ -104,7 +115,7 @@ __device__ __forceinline__ void mg_bracket(int i, int nf, int nc, int (&I)[2], f
     w[0] = i & 1 ? .5f : 1.f;
     w[1] = i & 1 ? .5f : 0.f;
   } else {
-    const int q = i * nc / nf, m = i * nc - q * nf;
+    const int q = nf == nc ? i : i == nf ? nc : i >> 1, m = mg_diff(i, nc, q, nf);
     I[0] = q;
     I[1] = q + (m > 0);
     w[0] = mg_wt(nf - m, nf);

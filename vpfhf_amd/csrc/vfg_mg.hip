@@ -77,11 +77,11 @@ __global__ __launch_bounds__(256) void k_mg_elem_coef(Grid G, const double *__re
 // integer overlaps in units of 1 / nc that sum to nf (0 off the axis).
 template <int M>
 __device__ __forceinline__ void mg_overlap(int C, int nf, int nc, int (&e)[M], double (&w)[M]) {
-  const int lo = C * nf / nc;
+  const int lo = mg_floor(C, nf, nc);
 #pragma unroll
   for (int q = 0; q < M; q++) {
-    const int a = (lo + q) * nc > C * nf ? (lo + q) * nc : C * nf;
-    const int b = (lo + q + 1) * nc < (C + 1) * nf ? (lo + q + 1) * nc : (C + 1) * nf;
+    const int d = mg_diff(lo + q, nc, C, nf);  // start of the fine element in the coarse one
+    const int a = d > 0 ? d : 0, b = d + nc < nf ? d + nc : nf;
     w[q] = b > a && lo + q < nf ? (double)(b - a) : 0.;
     e[q] = lo + q < nf ? lo + q : nf - 1;
   }
@@ -131,7 +131,14 @@ __global__ __launch_bounds__(256) void k_mg_diag32(Grid G, const double *__restr
   }
 }
 
-// Transfers, plane blockIdx.y (so that indices are 32-bit): restriction one
+constexpr int PLANE_ROWS = 1 << 15;
+__device__ __forceinline__ int plane_of_block() { return (int)(blockIdx.y + gridDim.y * blockIdx.z); }
+static dim3 plane_grid(unsigned x, int nz) {
+  return dim3(x, nz < PLANE_ROWS ? nz : PLANE_ROWS, (nz + PLANE_ROWS - 1) / PLANE_ROWS);
+}
+
+// Transfers, one plane of nodes per block row (so that indices are 32-bit; rows
+// beyond a grid's 65535 go on in z): restriction one
 // thread per (coarse node, component), on small levels (latency-bound) four,
 // one per fine plane of the gather; prolongation one thread per fine node.
 // Restriction, mean of the 129^3 -> 65^3 -> 33^3 nodes 9.7 us (25 us as three
@@ -142,8 +149,9 @@ template <int M, int LANES>
 __global__ __launch_bounds__(256) void k_mg_restrict(Grid Gf, Grid Gc, BcMask bc, const float *__restrict__ r,
                                                      float *__restrict__ bcoarse) {
   const int g = blockIdx.x * 256 + threadIdx.x, t = g / LANES, np = 3 * Gc.nx * Gc.ny;
-  const bool ok = t < np;
-  const int N = ok ? t / 3 : 0, c = ok ? t - 3 * N : 0, J = N / Gc.nx, I = N - J * Gc.nx, K = blockIdx.y;
+  const int pl = plane_of_block(), K = pl < Gc.nz ? pl : 0;
+  const bool ok = t < np && pl < Gc.nz;
+  const int N = ok ? t / 3 : 0, c = ok ? t - 3 * N : 0, J = N / Gc.nx, I = N - J * Gc.nx;
   if constexpr (LANES == 1) {
     if (ok) bcoarse[t + (int64_t)np * K] = mg_restrict_entry<M>(Gf, Gc, bc, r, I, J, K, c);
   } else {
@@ -154,10 +162,10 @@ __global__ __launch_bounds__(256) void k_mg_restrict(Grid Gf, Grid Gc, BcMask bc
 template <bool NESTED>
 __global__ __launch_bounds__(256) void k_mg_prolong(Grid Gf, Grid Gc, BcMask bc, const float *__restrict__ xc,
                                                     float *__restrict__ xf) {
-  const int t = blockIdx.x * 256 + threadIdx.x;
-  if (t >= Gf.nx * Gf.ny) return;
+  const int t = blockIdx.x * 256 + threadIdx.x, k = plane_of_block();
+  if (t >= Gf.nx * Gf.ny || k >= Gf.nz) return;
   const int j = t / Gf.nx;
-  mg_prolong_node<NESTED>(Gf, Gc, bc, xc, xf, t - j * Gf.nx, j, (int)blockIdx.y);
+  mg_prolong_node<NESTED>(Gf, Gc, bc, xc, xf, t - j * Gf.nx, j, k);
 }
 static bool mg_nested(const Grid &Gf, const Grid &Gc) {
   return Gf.nex == 2 * Gc.nex && Gf.ney == 2 * Gc.ney && Gf.nez == 2 * Gc.nez;
@@ -195,14 +203,14 @@ void launch_mg_restrict(const Grid &Gf, const Grid &Gc, const BcMask &bc, const 
                         hipStream_t s) {
   const int64_t np = 3 * (int64_t)Gc.nx * Gc.ny;
   const bool small = np * Gc.nz <= (1 << 16);  // few entries: split each over its fine planes
-  const dim3 g(nbm(small ? 4 * np : np), Gc.nz);
+  const dim3 g = plane_grid(nbm(small ? 4 * np : np), Gc.nz);
   auto go = [&](auto k) { hipLaunchKernelGGL(k, g, dim3(256), 0, s, Gf, Gc, bc, r, bcoarse); };
   if (mg_nested(Gf, Gc)) small ? go(k_mg_restrict<3, 4>) : go(k_mg_restrict<3, 1>);
   else small ? go(k_mg_restrict<4, 4>) : go(k_mg_restrict<4, 1>);
 }
 void launch_mg_prolong(const Grid &Gf, const Grid &Gc, const BcMask &bc, const float *xc, float *xf,
                        hipStream_t s) {
-  const dim3 g(nbm((int64_t)Gf.nx * Gf.ny), Gf.nz);
+  const dim3 g = plane_grid(nbm((int64_t)Gf.nx * Gf.ny), Gf.nz);
   if (mg_nested(Gf, Gc)) hipLaunchKernelGGL(k_mg_prolong<true>, g, dim3(256), 0, s, Gf, Gc, bc, xc, xf);
   else hipLaunchKernelGGL(k_mg_prolong<false>, g, dim3(256), 0, s, Gf, Gc, bc, xc, xf);
 }
