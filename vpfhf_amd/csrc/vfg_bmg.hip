@@ -393,13 +393,19 @@ void bmg_idle(BatchMG *g) {
 int bmg_setup(BatchMG *g, const double *const *dinv64, hipStream_t s) {
   if (hipStreamSynchronize(s) != hipSuccess) return VFG_E_HIP;  // dinv64 is written on the batch stream
   g->up.idle();
-  int rc;
-  for (int p = 0; p < g->np; p++)
-    if (g->m[p] && (rc = mg_setup_begin(g->m[p], dinv64[p], g->m[p]->stream))) return rc;
-  for (int p = 0; p < g->np; p++)
-    if (g->m[p] && (rc = mg_setup_end(g->m[p], g->m[p]->stream))) return rc;
-  for (int p = 0; p < g->np; p++)
-    if (g->m[p] && hipStreamSynchronize(g->m[p]->stream) != hipSuccess) return VFG_E_HIP;
+  // every member's set-up that was begun is finished, whatever another member's
+  // came to: none is left with work queued or without its bounds
+  int rc = VFG_OK, begun = 0;
+  for (; begun < g->np && !rc; begun++)
+    if (g->m[begun]) rc = mg_setup_begin(g->m[begun], dinv64[begun], g->m[begun]->stream);
+  const int ended = rc ? begun - 1 : begun;  // not the one that could not begin
+  for (int p = 0; p < begun; p++) {
+    if (!g->m[p]) continue;
+    int e = p < ended ? mg_setup_end(g->m[p], g->m[p]->stream) : VFG_OK;
+    if (hipStreamSynchronize(g->m[p]->stream) != hipSuccess && !e) e = VFG_E_HIP;
+    if (!rc) rc = e;
+  }
+  if (rc) return rc;
   for (int p = 0; p < g->np; p++)
     if (g->m[p]) {
       stage_member(g, p);

@@ -20,8 +20,8 @@ struct MgHier {
   static constexpr int MAXL = 12;
   int L = 0;
   MgLevel lv[MAXL];
-  int setups = 0;          // smoother bounds are re-estimated on every 16th set-up
-  bool estimate = false;   // and are on their way in this one
+  int setups = 0;          // complete ones; smoother bounds are re-estimated on every 16th
+  bool estimate = false;   // the estimates of the set-up that was begun are on their way
 };
 }  // namespace vfg
 

@@ -805,8 +805,10 @@ int mg_setup_begin(vfg_handle *h, const double *dinv64, hipStream_t s) {
   // top of the Jacobi-scaled spectrum is set by the element geometry and the
   // Poisson ratio, not by V or E (measured: 2.55, 2.50, 2.30, 1.79 on the
   // levels of a cracked 32^3 problem against 2.5 for a uniform one), so the
-  // estimates of the first set-up are reused and refreshed every 16th.
-  m.estimate = m.setups++ % 16 == 0;
+  // estimates of the first set-up are reused and refreshed every 16th.  A set-up
+  // counts once its estimates have been read back (mg_setup_end): one that fails,
+  // or that another member's failure leaves unfinished, is due again.
+  m.estimate = m.setups % 16 == 0;
   if (!m.estimate) return VFG_OK;
   LzOps T{};
   T.L = m.L;
@@ -820,16 +822,17 @@ int mg_setup_begin(vfg_handle *h, const double *dinv64, hipStream_t s) {
 }
 int mg_setup_end(vfg_handle *h, hipStream_t s) {
   MgHier &m = *h->mg;
-  if (!m.estimate) return VFG_OK;
-  m.estimate = false;
-  double lmax[MgHier::MAXL];
-  int st[MgHier::MAXL];
-  int rc = lz_end(h, m.L, MG_LZ, s, lmax, st);
-  for (int l = 0; l < m.L; l++) {
-    if (rc || st[l] || !(lmax[l] > 0.))
-      return vfg_fail(h, rc ? rc : VFG_E_NAN, "multigrid set-up: eigenvalue estimate failed on level %d", l);
-    m.lv[l].lmax = 1.1 * lmax[l];
+  if (m.estimate) {
+    m.estimate = false;
+    double lmax[MgHier::MAXL];
+    int st[MgHier::MAXL];
+    int rc = lz_end(h, m.L, MG_LZ, s, lmax, st);
+    for (int l = 0; l < m.L; l++)
+      if (rc || st[l] || !(lmax[l] > 0.))
+        return vfg_fail(h, rc ? rc : VFG_E_NAN, "multigrid set-up: eigenvalue estimate failed on level %d", l);
+    for (int l = 0; l < m.L; l++) m.lv[l].lmax = 1.1 * lmax[l];
   }
+  m.setups++;
   return VFG_OK;
 }
 int mg_setup(vfg_handle *h, const double *dinv64) {
