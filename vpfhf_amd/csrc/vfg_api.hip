@@ -165,7 +165,7 @@ int vfg_create(const vfg_grid *g, const vfg_props *pr, vfg_handle **out) {
   const size_t nn = (size_t)P.nn;
   if ((rc = vfg_alloc_group(h, {{(void **)&P.V, 8 * nn}, {(void **)&P.VIrrev, 8 * nn}, {(void **)&P.dth, 8 * nn},
                                 {(void **)&P.p, 8 * nn}, {(void **)&P.V32, 4 * nn}, {(void **)&P.zero3, 24 * nn},
-                                {(void **)&P.vfix, nn}, {(void **)&P.bV, 8 * nn}, {(void **)&h->part, 8 * 4 * 65536},
+                                {(void **)&P.vfix, nn}, {(void **)&P.bV, 8 * nn}, {(void **)&h->part, 8 * (size_t)PART_N},
                                 {(void **)&h->scal, 8 * 64}, {(void **)&P.cmask, 4 * (size_t)P.ne}}))) {
     snprintf(g_err, sizeof g_err, "%s", h->err.c_str());
     vfg_destroy(h);

@@ -23,6 +23,10 @@ struct MgHier {
   int setups = 0;          // complete ones; smoother bounds are re-estimated on every 16th
   bool estimate = false;   // the estimates of the set-up that was begun are on their way
 };
+// vfg_handle::part.  The multigrid CG's vector updates sum one set of partials
+// while they write another, so its three sets are apart: p.q in [0, PART_RR), r.r
+// (at most 2048) in [PART_RR, PART_RZ), r.z in [PART_RZ, PART_N)
+constexpr int PART_N = 4 * 65536, PART_RZ = 2 * 65536, PART_RR = PART_RZ - 2048;
 }  // namespace vfg
 
 struct vfg_handle {
@@ -35,7 +39,7 @@ struct vfg_handle {
   size_t bytes = 0;
   double *stage = nullptr;  // staging for host-pointer calls
   int64_t stage_n = 0;
-  double *part = nullptr;      // reduction partials (4 x 65536)
+  double *part = nullptr;      // reduction partials (PART_N)
   double *part_big = nullptr;  // partials for very large grids
   double *scal = nullptr;      // device scalars (64)
   double *abh = nullptr;       // CG coefficient histories of eigenvalue estimates

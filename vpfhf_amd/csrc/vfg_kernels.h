@@ -46,14 +46,16 @@ void launch_u_apply_f32(const DevProblem &P, const float *x, float *y, hipStream
 // apply (x = c2 D^-1 b, r = b - A x, 0 on the Dirichlet rows: what the
 // restriction reads), and one step from x fused with its apply (xo = x + c2 D^-1 (b - A x));
 // xo must not alias x.  With r64 the post-smoothing also writes one partial of
-// r64 . xo per workgroup to part and returns their number (else 0 partials).
+// r64 . xo per workgroup to part and returns their number (else 0 partials), for
+// at most max_part workgroups.
 void launch_mg_presmooth(const DevProblem &P, const float *b, const float *dinv, float c2, float *x, float *r,
                          hipStream_t s);
 int launch_mg_postsmooth(const DevProblem &P, const float *b, const float *dinv, float c2, const float *x, float *xo,
-                         const double *r64, double *part, hipStream_t s);
+                         const double *r64, double *part, int max_part, hipStream_t s);
 // FP64 y = A x (no NOCOMPRESSION) with one x.y partial per workgroup in part;
-// returns the number of partials (0, and nothing launched, for NOCOMPRESSION)
-int launch_u_apply_dot(const DevProblem &P, const double *x, double *y, double *part, hipStream_t s);
+// returns the number of partials (0, and nothing launched, for NOCOMPRESSION and
+// for more than max_part workgroups)
+int launch_u_apply_dot(const DevProblem &P, const double *x, double *y, double *part, int max_part, hipStream_t s);
 // Chebyshev(k)-Jacobi from x = 0 on a small FP32 level in one launch (k <= 8;
 // step i: coefficients c1[i], c2[i] of mg_cheb_entry); mg_coarse_fits tells
 // whether the level qualifies (at most 8^3 elements, no NOCOMPRESSION)

@@ -121,7 +121,7 @@ static unsigned nb_(int64_t n) { return (unsigned)((n + 255) / 256); }
 
 typedef std::function<void(const double *, double *)> ApplyFn;
 // apply with the x.y partials written to h->part: (x, y) -> their number, 0
-// when the operator has no such kernel (nothing launched then)
+// when the operator has no such kernel or too many workgroups (nothing launched then)
 typedef std::function<int(const double *, double *)> DotApplyFn;
 // Preconditioned CG on the device.  On entry x is the initial guess and r the
 // initial residual b - A x.  Converged when ||r|| <= max(rtol*||r0||, atol).
@@ -901,7 +901,7 @@ static int mg_vcycle(vfg_handle *h, int l, const double *r64 = nullptr, double *
   launch_mg_restrict(L.P.G, C.P.G, L.P.bcU, L.y, C.b, s);
   mg_vcycle(h, l + 1);
   launch_mg_prolong(L.P.G, C.P.G, L.P.bcU, C.x, L.d, s);
-  return launch_mg_postsmooth(L.P, L.b, L.dinv, c2[0], L.d, L.x, r64, part, s);
+  return launch_mg_postsmooth(L.P, L.b, L.dinv, c2[0], L.d, L.x, r64, part, PART_N - PART_RZ, s);
 }
 
 // z = V-cycle(r) on the problem's grid (r: FP32, zero on Dirichlet rows);
@@ -1024,12 +1024,11 @@ static int pcg_mg(vfg_handle *h, int64_t n, const ApplyFn &A, double *x, double 
         hipLaunchKernelGGL(k_dotp, dim3(nb), dim3(RB), 0, s, (const double *)p, (const double *)q, n, part);
         na = nb;
       }
-      // r.r partials from the update, r.z partials from the V-cycle's last
-      // kernel (in two regions of part past the apply's partials)
-      double *prr = part + 65536, *prz = part + 2 * 65536;
+      // r.r partials from the update, r.z partials from the V-cycle's last kernel
+      double *prr = part + PART_RR, *prz = part + PART_RZ;
       hipLaunchKernelGGL(k_mg_r, dim3(nb), dim3(RB), 0, s, r, (const double *)q, r32, n, (const double *)part, na,
                          it + k, sc, prr);
-      int nrz = mg_apply(h, r32, z32, r, prz);  // at most 2 x 65536 partials
+      int nrz = mg_apply(h, r32, z32, r, prz);
       if (!nrz) {
         hipLaunchKernelGGL(k_mg_dot, dim3(nb), dim3(RB), 0, s, (const double *)r, (const float *)z32, n, prz);
         nrz = nb;
@@ -1293,7 +1292,7 @@ int vfg_u_solve(vfg_handle *h, double *U, const double *BCU, const vfg_solve_opt
     rc = vfg_fail(h, VFG_E_ARG, "vfg_u_solve: the Chebyshev preconditioner is provided for the mixed-precision solve");
   } else if (o->pc == VFG_PC_MG) {
     ApplyFn A = [&](const double *in, double *out) { launch_u_apply(P, in, out, s); };
-    DotApplyFn Ad = [&](const double *in, double *out) { return launch_u_apply_dot(P, in, out, h->part, s); };
+    DotApplyFn Ad = [&](const double *in, double *out) { return launch_u_apply_dot(P, in, out, h->part, PART_RR, s); };
     rc = mg_setup(h, dinv);
     if (!rc) rc = pcg_mg(h, n, A, x, r, p, q, h->wf[0], h->wf[1], o->rtol, o->atol, o->maxit, 4, &inf, &Ad);
     inf.outer = 1;
@@ -1302,7 +1301,7 @@ int vfg_u_solve(vfg_handle *h, double *U, const double *BCU, const vfg_solve_opt
     // staging, as the V-solve does, measured slower than the separate vector
     // kernels (with a 27-point product 282 us against 215 + 33 us at 128^3)
     ApplyFn A = [&](const double *in, double *out) { launch_u_apply(P, in, out, s); };
-    DotApplyFn Ad = [&](const double *in, double *out) { return launch_u_apply_dot(P, in, out, h->part, s); };
+    DotApplyFn Ad = [&](const double *in, double *out) { return launch_u_apply_dot(P, in, out, h->part, PART_N, s); };
     rc = pcg(h, n, A, dinv, x, r, z, p, q, o->rtol, o->atol, o->maxit, 20, &inf, &Ad);
     inf.outer = 1;
   }

@@ -1501,7 +1501,7 @@ void launch_u_apply(const DevProblem &P, const double *x, double *y, hipStream_t
 }
 
 template <int W, bool CUBIC>
-static int launch_u_apply_dot_c(const UModRec<double> &r, double *part, hipStream_t s) {
+static int launch_u_apply_dot_c(const UModRec<double> &r, double *part, int max_part, hipStream_t s) {
   UApplyDotOp<CUBIC> op;
   static_cast<UModRec<double> &>(op) = r;
   op.part = part;
@@ -1509,10 +1509,12 @@ static int launch_u_apply_dot_c(const UModRec<double> &r, double *part, hipStrea
   static int slots = device_slots(k_u_apply_dot<W, CUBIC>, W * W);
   const int OZ = choose_oz(G, ((G.nx + W - 2) / (W - 1)) * ((G.ny + W - 2) / (W - 1)), slots);
   const dim3 g = march_grid(G, W, W, OZ);
+  const int64_t nwg = (int64_t)g.x * g.y * g.z;
+  if (nwg > max_part) return 0;
   hipLaunchKernelGGL((k_u_apply_dot<W, CUBIC>), g, dim3(W * W), 0, s, op, OZ);
-  return (int)(g.x * g.y * g.z);
+  return (int)nwg;
 }
-int launch_u_apply_dot(const DevProblem &P, const double *x, double *y, double *part, hipStream_t s) {
+int launch_u_apply_dot(const DevProblem &P, const double *x, double *y, double *part, int max_part, hipStream_t s) {
   if (P.unilateral) return 0;
   if (P.uq) {
     UApplyLdsqDotOp q;
@@ -1523,14 +1525,18 @@ int launch_u_apply_dot(const DevProblem &P, const double *x, double *y, double *
     const int tiles = ((P.G.nx + 14) / 15) * ((P.G.ny + 14) / 15);
     const int OZ = choose_oz(P.G, tiles, lqslots);
     const dim3 g = march_grid(P.G, 16, 16, OZ);
+    const int64_t nwg = (int64_t)g.x * g.y * g.z;
+    if (nwg > max_part) return 0;
     hipLaunchKernelGGL(k_u_apply_ldsq_dot, g, dim3(256), 0, s, q, OZ);
-    return (int)(g.x * g.y * g.z);
+    return (int)nwg;
   }
   UModRec<double> r;
   umod_fill<double>(r, P, x, y);
   if (small_fp64(P.G))
-    return r.m.cubic ? launch_u_apply_dot_c<8, true>(r, part, s) : launch_u_apply_dot_c<8, false>(r, part, s);
-  return r.m.cubic ? launch_u_apply_dot_c<16, true>(r, part, s) : launch_u_apply_dot_c<16, false>(r, part, s);
+    return r.m.cubic ? launch_u_apply_dot_c<8, true>(r, part, max_part, s)
+                     : launch_u_apply_dot_c<8, false>(r, part, max_part, s);
+  return r.m.cubic ? launch_u_apply_dot_c<16, true>(r, part, max_part, s)
+                   : launch_u_apply_dot_c<16, false>(r, part, max_part, s);
 }
 void launch_u_apply_f32(const DevProblem &P, const float *x, float *y, hipStream_t s) {
   launch_u_apply_t<float>(P, x, y, P.V32, s);
@@ -1569,13 +1575,13 @@ void launch_mg_presmooth(const DevProblem &P, const float *b, const float *dinv,
   else P.unit ? mg_launch<UMgPreOp<true>>(P, op, s) : mg_launch<UMgPreOp<false>>(P, op, s);
 }
 int launch_mg_postsmooth(const DevProblem &P, const float *b, const float *dinv, float c2, const float *x, float *xo,
-                         const double *r64, double *part, hipStream_t s) {
+                         const double *r64, double *part, int max_part, hipStream_t s) {
   UMgRec op;
   mg_op_fill(op, P, b, dinv, c2);
   op.x = x; op.xo = xo; op.r64 = r64; op.part = part;
   if (r64) {
-    const int n = op.m.cubic ? mg_launch<UMgPostRzOp<true>>(P, op, s, 2 * 65536)
-                             : mg_launch<UMgPostRzOp<false>>(P, op, s, 2 * 65536);
+    const int n = op.m.cubic ? mg_launch<UMgPostRzOp<true>>(P, op, s, max_part)
+                             : mg_launch<UMgPostRzOp<false>>(P, op, s, max_part);
     if (n) return n;  // else too many workgroups for the partials: the plain form
   }
   if (op.m.cubic)
