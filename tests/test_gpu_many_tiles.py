@@ -20,9 +20,9 @@ def _bar(nx):
     return P, rng.uniform(-1e-3, 1e-3, 3 * P.nn)
 
 
-# tiles: 66,669; 262,669 (partials: 129,024 of p.q under multigrid and 262,144
-# under Jacobi)
-@pytest.mark.parametrize("nx,pc,rtol", [(1000021, "mg", 1e-9), (3940021, "jacobi", 1e-6)])
+# tiles: 66,669; 131,337; 262,669 (partials: 129,024 of p.q under multigrid and
+# 262,144 under Jacobi, 131,072 of r.z)
+@pytest.mark.parametrize("nx,pc,rtol", [(1000021, "mg", 1e-9), (1970041, "mg", 1e-9), (3940021, "jacobi", 1e-6)])
 def test_u_solve_of_many_tiles(nx, pc, rtol):
     from vpfhf_amd import _lib
     pc = _lib.PC_MG if pc == "mg" else _lib.PC_JACOBI

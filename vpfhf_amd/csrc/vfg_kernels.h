@@ -46,8 +46,8 @@ void launch_u_apply_f32(const DevProblem &P, const float *x, float *y, hipStream
 // apply (x = c2 D^-1 b, r = b - A x, 0 on the Dirichlet rows: what the
 // restriction reads), and one step from x fused with its apply (xo = x + c2 D^-1 (b - A x));
 // xo must not alias x.  With r64 the post-smoothing also writes one partial of
-// r64 . xo per workgroup to part and returns their number (else 0 partials), for
-// at most max_part workgroups.
+// r64 . xo per workgroup to part and returns their number (0: none written,
+// without r64 and for more than max_part workgroups).
 void launch_mg_presmooth(const DevProblem &P, const float *b, const float *dinv, float c2, float *x, float *r,
                          hipStream_t s);
 int launch_mg_postsmooth(const DevProblem &P, const float *b, const float *dinv, float c2, const float *x, float *xo,

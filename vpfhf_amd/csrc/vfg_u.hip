@@ -1585,8 +1585,9 @@ int launch_mg_postsmooth(const DevProblem &P, const float *b, const float *dinv,
     if (n) return n;  // else too many workgroups for the partials: the plain form
   }
   if (op.m.cubic)
-    return P.unit ? mg_launch<UMgPostOp<true, false, true>>(P, op, s) : mg_launch<UMgPostOp<false, false, true>>(P, op, s);
-  return P.unit ? mg_launch<UMgPostOp<true, false>>(P, op, s) : mg_launch<UMgPostOp<false, false>>(P, op, s);
+    P.unit ? mg_launch<UMgPostOp<true, false, true>>(P, op, s) : mg_launch<UMgPostOp<false, false, true>>(P, op, s);
+  else P.unit ? mg_launch<UMgPostOp<true, false>>(P, op, s) : mg_launch<UMgPostOp<false, false>>(P, op, s);
+  return 0;
 }
 
 static void launch_u_diag_uni(const DevProblem &P, double *d, hipStream_t s) {
