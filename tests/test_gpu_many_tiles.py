@@ -1,6 +1,7 @@
-"""Grids of more workgroup tiles than the solvers keep reduction partials for:
-long bars of one element in y and z, one 15-node tile per 15 nodes.  The
-products and the post-smoothing then reduce in a pass of their own."""
+"""Long bars: grids of more workgroup tiles than the solvers keep reduction
+partials for (one element in y and z, one 15-node tile per 15 nodes; the products
+and the post-smoothing then reduce in a pass of their own), and axes of more than
+65535 elements, whose products of two counts pass 31 bits."""
 import numpy as np
 import pytest
 
@@ -39,3 +40,43 @@ def test_u_solve_of_many_tiles(nx, pc, rtol):
         P.close()
     # the extremes of a larger sample cost a step or two; the batch lengths round it up
     assert its[1] <= 1.25 * its[0] + 4, its
+
+
+def _held_bar(axis, m):
+    """m elements along axis, short ones, so that the coarse levels carry the
+    convergence; E over three decades along it, so that they need its means."""
+    import vpfhf_amd as V
+    n, l = [3, 3, 3], [1.0, 1.0, 1.0]
+    n[axis], l[axis] = m + 1, 0.05 * m
+    P = V.Problem(tuple(n), tuple(l), nu=0.3, eta=1e-5, atnum=1)
+    P.set_bc([V.make_bc({2 * ((axis + 1) % 3): V.ZERO})] * 3, V.make_bc())
+    shape = [q - 1 for q in n[::-1]]
+    along = np.exp(1.5 * np.log(10.0) * np.sin(2 * np.pi * (np.arange(m) + 0.5) / 1000))
+    E = np.broadcast_to(along.reshape([-1 if 2 - d == axis else 1 for d in range(3)]), shape)
+    P.set_fields(V=np.ones(P.nn), E_elem=np.ascontiguousarray(E).ravel())
+    return P
+
+
+@pytest.mark.parametrize("axis", [0, 2], ids="xz")
+def test_multigrid_coefficients_of_long_axes(axis):
+    """Coarse coefficients and transfers beyond 65535 elements along an axis: the
+    solve takes the iterations of the same bar at half the length, a third of
+    Jacobi's or fewer, and the V-cycle is positive."""
+    from vpfhf_amd import _lib
+    its = []
+    for m in (33000, 66000):
+        P = _held_bar(axis, m)
+        rng = np.random.default_rng(m)
+        Z, U0 = np.zeros(3 * P.nn), rng.uniform(-1e-3, 1e-3, 3 * P.nn)
+        _, info = P.VF_StepU(U0, Z, rtol=1e-9, pc=_lib.PC_MG)
+        assert info.status == 0
+        its.append(info.iterations)
+        if m == 33000:
+            _, jac = P.VF_StepU(U0, Z, rtol=1e-9, pc=_lib.PC_JACOBI)
+            assert 3 * info.iterations < jac.iterations, (info.iterations, jac.iterations)
+        free = 1.0 - P.bc_mask("U")
+        a = rng.standard_normal(3 * P.nn) * free
+        assert a @ P.u_pc_apply(a) > 0.0
+        P.close()
+    # two samples of the same statistics: a step or two, rounded up to a batch of four
+    assert abs(its[1] - its[0]) <= 4, its
