@@ -21,19 +21,21 @@ struct VConst {
   double crhs;      // Gc/atCv/eps * (.5 AT2 | .25 AT1), VFMech.c:2350-2384
 };
 
+// the launch constants are formed in extended precision and rounded once: a
+// constant's error is the same in every element, so it does not average out
 static VConst make_vconst(const DevProblem &P) {
   VConst C;
-  const double h[3] = {P.G.hx, P.G.hy, P.G.hz}, c = P.Gc / P.atcv * .5;
+  const long double h[3] = {P.G.hx, P.G.hy, P.G.hz}, c = .5L * P.Gc / P.atcv;
   for (int i = 0; i < 8; i++) {
-    double t = 0.;
+    long double t = 0.;
     for (int d = 0; d < 3; d++) {
       if (!um_pow(i, d)) continue;
-      double w = 1. / (h[d] * h[d]);
+      long double w = 1. / (h[d] * h[d]);
       for (int e = 0; e < 3; e++)
         if (e != d && um_pow(i, e)) w /= 3.;
       t += w;
     }
-    C.ks[i] = c * P.eps * h[0] * h[1] * h[2] / 16. * t;
+    C.ks[i] = (double)(c * P.eps * h[0] * h[1] * h[2] / 16. * t);
   }
   C.crhs = P.atnum == 2 ? P.Gc / P.atcv / P.eps * .5 : P.Gc / P.atcv / P.eps * .25;
   return C;
@@ -50,15 +52,15 @@ struct VSetup {
 };
 static VSetup make_vsetup(const DevProblem &P) {
   const Grid &G = P.G;
-  const double s = 16. * G.hz * G.hz;
+  const long double s = 16.L * G.hz * G.hz;
   VSetup C;
   C.kx = G.hz / G.hx;
   C.ky = G.hz / G.hy;
   C.kth = P.alpha * G.hz / 2.;
-  C.lam = P.lam1 / s;
-  C.mu2 = 2. * P.mu1 / s;
-  C.cm = P.atnum == 2 ? P.Gc / P.atcv * .5 / P.eps : 0.;
-  C.vol = G.hx * G.hy * G.hz / 64.;
+  C.lam = (double)(P.lam1 / s);
+  C.mu2 = (double)(2. * P.mu1 / s);
+  C.cm = P.atnum == 2 ? (double)(.5L * P.Gc / P.atcv / P.eps) : 0.;
+  C.vol = (double)((long double)G.hx * G.hy * G.hz / 64.);
   return C;
 }
 
