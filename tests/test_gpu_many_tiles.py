@@ -80,3 +80,57 @@ def test_multigrid_coefficients_of_long_axes(axis):
         P.close()
     # two samples of the same statistics: a step or two, rounded up to a batch of four
     assert abs(its[1] - its[0]) <= 4, its
+
+
+def _plate(n):
+    import vpfhf_amd as V
+    P = V.Problem((n, n, 2), ((n - 1) / 128, (n - 1) / 128, 1 / 128), nu=0.2, atnum=2, epsilon=4 / 128, eta=1e-5,
+                  alpha=0.0, beta=0.0)
+    P.set_fields(V=np.ones(P.nn), VIrrev=np.ones(P.nn))
+    rng = np.random.default_rng(n)
+    return P, 1e-2 * rng.random(3 * P.nn), 0.5 + 0.5 * rng.random(P.nn)
+
+
+def test_v_solve_of_many_chunks():
+    """More chunks in the reduced system than its launches sum directly: the
+    iterations of a small plate (same statistics), and the gradient asked for."""
+    its = []
+    for n in (201, 1001):  # 196 and 4489 chunks
+        P, U, V0 = _plate(n)
+        V, info = P.VF_StepV(U, V0, rtol=1e-8)
+        assert info.status == 0
+        its.append(info.iterations)
+        P.VIJacobian_setup(U)
+        g, g0 = (np.linalg.norm(P.VF_VResidual(v)) for v in (V, V0))
+        assert g <= 1.01e-8 * g0, (g, g0)
+        P.close()
+    # a larger sample's extremes cost a step or two in each of the few Newton steps
+    assert its[1] <= 1.25 * its[0] + 4, its
+
+
+def test_v_solve_time_follows_the_grid():
+    """A CG iteration reads the coupling once, whatever the number of chunks
+    (71,289 here): a few products' time each, all else included."""
+    import ctypes as C
+    import time
+    import vpfhf_amd as vf
+    from vpfhf_amd import DeviceBuffer, _lib
+    P, U, V0 = _plate(4001)
+    dU, dV, dy = DeviceBuffer(8 * U.size).upload(U), DeviceBuffer(8 * V0.size), DeviceBuffer(8 * V0.size)
+    L, o, info = vf.load(), P.opts(rtol=1e-8), _lib.SolveInfo()
+
+    def timed(f, n):
+        t = []
+        for _ in range(n):
+            dV.upload(V0)
+            t0 = time.perf_counter()
+            vf.check(f(), P.h)
+            t.append(time.perf_counter() - t0)
+        return sorted(t)[n // 2]
+
+    solve = timed(lambda: L.vfg_v_solve(P.h, dU.ptr, dV.ptr, None, C.byref(o), C.byref(info), vf.DEVICE), 3)
+    product = timed(lambda: L.vfg_v_apply(P.h, dV.ptr, dy.ptr, vf.DEVICE), 9)
+    # an iteration: the product and an update of three of its eight vector passes
+    # (the product itself is bound by the coupling, 27 values per element)
+    assert solve <= 6 * product * info.iterations, (solve, product, info.iterations)
+    P.close()

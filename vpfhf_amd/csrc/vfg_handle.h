@@ -47,7 +47,7 @@ struct vfg_handle {
   int *vlist = nullptr;        //          and their list, count and chunk length (v_chunk_cap + 2)
   uint32_t *vflag2 = nullptr;  // the same dilated by one tile and one plane,
   int *vlist2 = nullptr;       //          and its list
-  double *vpart = nullptr;     // partials of the V-CG (5 x vcg_partials)
+  double *vpart = nullptr;     // partials of the V-CG (5 x vcg_partials + 3 x VCG_FOLD)
   bool v_ready = false;
   // solver work space (allocated on first use)
   double *w[16] = {nullptr};

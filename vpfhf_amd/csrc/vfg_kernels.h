@@ -110,6 +110,13 @@ struct VCgStep {
 };
 // partials a list can hold: its chunks, or the blocks of a reduction
 size_t vcg_partials(const Grid &G);
+// Lists of more than VCG_DIRECT chunks (wide bands of grids with many tiles): the
+// partials of a launch, n groups of w, are folded to VCG_FOLD groups before every
+// workgroup of the next one sums them; summed by every workgroup the work is the
+// square of the count.  V-solves of plates with everything free, folded and not:
+// 1681 chunks 22.0 and 22.1 ms, 2209 28.5 and 29.4, 4489 54 and 60, 40401 253 and 777.
+constexpr int VCG_DIRECT = 2048, VCG_FOLD = 128;
+void launch_vcg_fold(const double *part, int w, int n, double *out, hipStream_t s);
 // CG-fused masked V apply (mask: fixed or active nodes) over the listed
 // chunks: beta from the step's r.z, p = z + beta p_old staged, q = K p, p and q
 // written on the chunks' owned nodes (p, q must be zero on the other chunks),
@@ -124,9 +131,9 @@ void launch_v_apply_list(const DevProblem &P, const double *x, double *y, int mo
 void launch_v_diag_list(const DevProblem &P, double *d, const uint8_t *mask, const int *list, int count,
                         hipStream_t s);
 // the CG update x += a p, r -= a q, z = dinv r over the listed chunks, a = r.z /
-// p.q from ppq[0, count), with the next (r.z, r.r) in pairs (one per chunk)
+// p.q from ppq[0, npq), with the next (r.z, r.r) in pairs (one per chunk)
 void launch_v_xr_list(const Grid &G, const int *list, int count, double *x, double *r, double *z, const double *p,
-                      const double *q, const double *dinv, const double *ppq, double *pairs, const VCgStep &c,
+                      const double *q, const double *dinv, const double *ppq, int npq, double *pairs, const VCgStep &c,
                       hipStream_t s);
 
 // misc (vfg_misc.hip)

@@ -245,6 +245,8 @@ static int pcg_v(vfg_handle *h, const uint8_t *mask, const int *list, int count,
   const int64_t n = P.nn;
   const size_t cap = vcg_partials(P.G);
   double *sc = h->scal, *ppq = h->vpart, *pairs[2] = {h->vpart + cap, h->vpart + 3 * cap};
+  double *fpq = h->vpart + 5 * cap, *fpairs = fpq + VCG_FOLD;
+  const bool fold = count > VCG_DIRECT;
   double rn = rn0, hs[13];
   int it = 0, status = VFG_OK;
   const double tol = rtol * rn0;
@@ -263,9 +265,11 @@ static int pcg_v(vfg_handle *h, const uint8_t *mask, const int *list, int count,
     for (int i = 0; i < todo; i++, c.k++) {
       launch_v_apply_cg_list(P, pa, pb, z, q, ppq, mask, list, count, c, s);
       double *nx = pairs[(c.k + 1) & 1];
-      launch_v_xr_list(P.G, list, count, x, r, z, pb, q, dinv, ppq, nx, c, s);
-      c.pairs = nx;
-      c.npairs = count;
+      if (fold) launch_vcg_fold(ppq, 1, count, fpq, s);
+      launch_v_xr_list(P.G, list, count, x, r, z, pb, q, dinv, fold ? fpq : ppq, fold ? VCG_FOLD : count, nx, c, s);
+      if (fold) launch_vcg_fold(nx, 2, count, fpairs, s);
+      c.pairs = fold ? fpairs : nx;
+      c.npairs = fold ? VCG_FOLD : count;
       double *t = pa;
       pa = pb;
       pb = t;
@@ -1333,7 +1337,7 @@ int vfg_v_solve(vfg_handle *h, const double *U, double *V, const double *ub, con
                                 {(void **)&h->vlist, 4 * (size_t)(vcap + 2)},
                                 {(void **)&h->vflag2, 4 * (size_t)vcap},
                                 {(void **)&h->vlist2, 4 * (size_t)(vcap + 2)},
-                                {(void **)&h->vpart, 8 * 5 * vcg_partials(P.G)}})))
+                                {(void **)&h->vpart, 8 * (5 * vcg_partials(P.G) + 3 * VCG_FOLD)}})))
     return rc;
   double *x = h->w[0], *r = h->w[1], *z = h->w[2], *p = h->w[3], *q = h->w[4], *dinv = h->w[5];
   double *Vd = h->w[6], *g = h->w[7], *Vn = h->w[8], *D = h->w[9], *KD = h->w[10], *ubd = nullptr;

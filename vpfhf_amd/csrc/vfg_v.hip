@@ -406,6 +406,16 @@ __device__ __forceinline__ void vcg_sums(const double *__restrict__ part, int n,
 #pragma unroll
   for (int w = 0; w < W; w++) s[w] = bc[w];
 }
+// group b of the output sums the b-th part of the n groups
+template <int W>
+__global__ __launch_bounds__(256) void k_vcg_fold(const double *__restrict__ part, int n, double *__restrict__ out) {
+  const int per = (n + VCG_FOLD - 1) / VCG_FOLD, lo = blockIdx.x * per, hi = lo + per < n ? lo + per : n;
+  double s[W];
+  vcg_sums<W>(part + (int64_t)W * lo, hi - lo, s);
+  if (threadIdx.x == 0)
+#pragma unroll
+    for (int w = 0; w < W; w++) out[W * blockIdx.x + w] = s[w];
+}
 __global__ __launch_bounds__(256, 2) void k_v_apply_cg_list(VApplyCgOp op, const int *__restrict__ list, int cap,
                                                            VCgStep c) {
   if (c.sc[S_DONE] != 0.) return;  // the CG has converged
@@ -542,7 +552,7 @@ __global__ __launch_bounds__(256) void k_v_xr_list(Grid G, const int *__restrict
                                                    double *__restrict__ x, double *__restrict__ r,
                                                    double *__restrict__ z, const double *__restrict__ p,
                                                    const double *__restrict__ q, const double *__restrict__ dinv,
-                                                   const double *__restrict__ ppq, double *__restrict__ part,
+                                                   const double *__restrict__ ppq, int npq, double *__restrict__ part,
                                                    VCgStep cg) {
   if (cg.sc[S_DONE] != 0.) return;  // the CG has converged
   __shared__ double sh[4];
@@ -552,7 +562,7 @@ __global__ __launch_bounds__(256) void k_v_xr_list(Grid G, const int *__restrict
   const int i = (t % gx) * 15 + tx, j = (t / gx) * 15 + ty, k0 = (c / txy) * L;
   const int k1 = k0 + L < G.nz ? k0 + L : G.nz;
   double pq[1];
-  vcg_sums<1>(ppq, (int)gridDim.x, pq);
+  vcg_sums<1>(ppq, npq, pq);
   const bool ok = pq[0] > 0. && isfinite(pq[0]);
   const double old = cg.sc[S_TMP0], al = ok ? old / pq[0] : 0.;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -884,11 +894,15 @@ void launch_v_apply_cg_list(const DevProblem &P, const double *pold, double *p, 
 }
 
 void launch_v_xr_list(const Grid &G, const int *list, int count, double *x, double *r, double *z, const double *p,
-                      const double *q, const double *dinv, const double *ppq, double *pairs, const VCgStep &c,
+                      const double *q, const double *dinv, const double *ppq, int npq, double *pairs, const VCgStep &c,
                       hipStream_t s) {
   if (count <= 0) return;
   hipLaunchKernelGGL(k_v_xr_list, dim3((unsigned)count), dim3(256), 0, s, G, list, v_chunk_cap(G), x, r, z, p, q,
-                     dinv, ppq, pairs, c);
+                     dinv, ppq, npq, pairs, c);
+}
+void launch_vcg_fold(const double *part, int w, int n, double *out, hipStream_t s) {
+  auto go = [&](auto k) { hipLaunchKernelGGL(k, dim3(VCG_FOLD), dim3(256), 0, s, part, n, out); };
+  w == 2 ? go(k_vcg_fold<2>) : go(k_vcg_fold<1>);
 }
 
 void launch_v_diag(const DevProblem &P, double *d, hipStream_t s, const uint8_t *mask) {
