@@ -316,7 +316,7 @@ __device__ __forceinline__ void march(const Grid &G, const Op &op, int OZ, int b
 // (bottom and top of the current element layer, and the one being committed
 // for the next layer), so the element computation can re-read its corners
 // instead of keeping them in registers:
-//   __device__ void element_lds(int ex, int ey, int ek, const XS &xs, A aux, T (&r)[8][NC])
+//   __device__ void element_lds(int ex, int ey, int ek, const XS &xs, T (&r)[8][NC])
 // with xs(k, q, f) the value of staged field f at corner (k, q = j*2+i).  The combination of
 // the element results (x by lane shuffles, y through LDS, z carried) and the
 // stores are those of march.  Two barriers per layer.  The next plane is loaded
@@ -367,13 +367,6 @@ __device__ __forceinline__ void march_lds(const Grid &G, const Op &op, int OZ, i
         for (int f = 0; f < NF; f++) s_in[b][f][n] = pf[q][f];
     }
   };
-  using AuxT = typename aux_of<Op>::type;
-  auto aux_at = [&](int ek) -> AuxT {
-    AuxT a{};
-    if constexpr (has_aux<Op>::value)
-      if (exy_ok && ek >= 0 && ek < G.nez) a = op.aux(ex, ey, ek);
-    return a;
-  };
   const int c0 = ty * SX + tx;  // corner (j, i) = (0, 0) of this thread's element in a plane
   T carry[NC];
 #pragma unroll
@@ -383,15 +376,12 @@ __device__ __forceinline__ void march_lds(const Grid &G, const Op &op, int OZ, i
   int bb = 0, bt = 1, bn = 2;
   fetch(oz0 - 1);
   commit(bb);
-  AuxT aux_next = aux_at(oz0 - 1);
   const int ek_end = min(oz0 + OZ - 1, G.nz - 1);
   for (int ek = oz0 - 1; ek <= ek_end; ek++) {
-    const AuxT aux_cur = aux_next;
     // buffer bt last held a plane read two layers ago; the barriers since
     // then order this write after those reads
     fetch(ek + 1);
     commit(bt);
-    aux_next = aux_at(ek + 1);
     __syncthreads();
     T r[8][NC];
 #pragma unroll
@@ -403,8 +393,7 @@ __device__ __forceinline__ void march_lds(const Grid &G, const Op &op, int OZ, i
       auto xs = [pb, pt](int k, int q, int f) -> T {
         return (k ? pt : pb)[f * PL + (q >> 1) * SX + (q & 1)];
       };
-      if constexpr (has_aux<Op>::value) op.element_lds(ex, ey, ek, xs, aux_cur, r);
-      else op.element_lds(ex, ey, ek, xs, r);
+      op.element_lds(ex, ey, ek, xs, r);
     }
     T cx[2][2][NC];
 #pragma unroll

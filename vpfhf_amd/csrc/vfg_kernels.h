@@ -97,8 +97,9 @@ void launch_v_chunk_list(const DevProblem &P, const uint8_t *mask, uint32_t *fla
 // element with a listed node, where K x changes when x changes on the listed
 // nodes only
 void launch_v_dilated_list(const DevProblem &P, const uint32_t *flag, uint32_t *flag2, int *list2, hipStream_t s);
-// scalars of a CG (vfg_handle::scal)
-enum { S_RZ = 0, S_PQ, S_ALPHA, S_BETA, S_RR, S_RR0, S_FLAG, S_TMP0, S_TMP1, S_TMP2, S_TOL2, S_DONE, S_ITS };
+// scalars of a CG (vfg_handle::scal); S_RZ1: a second place of r.z, for kernels that
+// read the one before while the next is written
+enum { S_RZ = 0, S_PQ, S_ALPHA, S_BETA, S_RR, S_RR0, S_FLAG, S_RZ1, S_DONE, S_ITS, S_COUNT };
 // Iteration k of the V-CG as its kernels see it: every workgroup sums the
 // partials of the previous launch itself, the first one keeps the scalars, each
 // of which is written by one launch and read by the next.

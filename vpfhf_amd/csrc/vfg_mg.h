@@ -27,7 +27,7 @@ __device__ __forceinline__ int mg_floor(int C, int nf, int nc) {
 __device__ __forceinline__ int mg_diff(int i, int nc, int I, int nf) {
   return (int)((unsigned)i * (unsigned)nc - (unsigned)I * (unsigned)nf);
 }
-__device__ __forceinline__ bool mg_nested_grids(const Grid &Gf, const Grid &Gc) {
+__host__ __device__ __forceinline__ bool mg_nested_grids(const Grid &Gf, const Grid &Gc) {
   return Gf.nex == 2 * Gc.nex && Gf.ney == 2 * Gc.ney && Gf.nez == 2 * Gc.nez;
 }
 

@@ -167,10 +167,6 @@ __global__ __launch_bounds__(256) void k_mg_prolong(Grid Gf, Grid Gc, BcMask bc,
   const int j = t / Gf.nx;
   mg_prolong_node<NESTED>(Gf, Gc, bc, xc, xf, t - j * Gf.nx, j, k);
 }
-static bool mg_nested(const Grid &Gf, const Grid &Gc) {
-  return Gf.nex == 2 * Gc.nex && Gf.ney == 2 * Gc.ney && Gf.nez == 2 * Gc.nez;
-}
-
 // ----------------------------------------------------------------- smoother
 __global__ void k_mg_cheb(const float *__restrict__ b, const float *__restrict__ y, const float *__restrict__ dinv,
                           float *__restrict__ d, float *__restrict__ x, float c1, float c2, int dfirst, int xzero,
@@ -205,13 +201,13 @@ void launch_mg_restrict(const Grid &Gf, const Grid &Gc, const BcMask &bc, const 
   const bool small = np * Gc.nz <= (1 << 16);  // few entries: split each over its fine planes
   const dim3 g = plane_grid(nbm(small ? 4 * np : np), Gc.nz);
   auto go = [&](auto k) { hipLaunchKernelGGL(k, g, dim3(256), 0, s, Gf, Gc, bc, r, bcoarse); };
-  if (mg_nested(Gf, Gc)) small ? go(k_mg_restrict<3, 4>) : go(k_mg_restrict<3, 1>);
+  if (mg_nested_grids(Gf, Gc)) small ? go(k_mg_restrict<3, 4>) : go(k_mg_restrict<3, 1>);
   else small ? go(k_mg_restrict<4, 4>) : go(k_mg_restrict<4, 1>);
 }
 void launch_mg_prolong(const Grid &Gf, const Grid &Gc, const BcMask &bc, const float *xc, float *xf,
                        hipStream_t s) {
   const dim3 g = plane_grid(nbm((int64_t)Gf.nx * Gf.ny), Gf.nz);
-  if (mg_nested(Gf, Gc)) hipLaunchKernelGGL(k_mg_prolong<true>, g, dim3(256), 0, s, Gf, Gc, bc, xc, xf);
+  if (mg_nested_grids(Gf, Gc)) hipLaunchKernelGGL(k_mg_prolong<true>, g, dim3(256), 0, s, Gf, Gc, bc, xc, xf);
   else hipLaunchKernelGGL(k_mg_prolong<false>, g, dim3(256), 0, s, Gf, Gc, bc, xc, xf);
 }
 void launch_mg_cheb(const float *b, const float *y, const float *dinv, float *d, float *x, float c1, float c2,

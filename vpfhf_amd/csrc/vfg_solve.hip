@@ -247,7 +247,7 @@ static int pcg_v(vfg_handle *h, const uint8_t *mask, const int *list, int count,
   double *sc = h->scal, *ppq = h->vpart, *pairs[2] = {h->vpart + cap, h->vpart + 3 * cap};
   double *fpq = h->vpart + 5 * cap, *fpairs = fpq + VCG_FOLD;
   const bool fold = count > VCG_DIRECT;
-  double rn = rn0, hs[13];
+  double rn = rn0, hs[S_COUNT];
   int it = 0, status = VFG_OK;
   const double tol = rtol * rn0;
   if (!isfinite(rn0)) status = VFG_E_NAN;
@@ -275,7 +275,7 @@ static int pcg_v(vfg_handle *h, const uint8_t *mask, const int *list, int count,
       pb = t;
     }
     hipLaunchKernelGGL(k_vcg_final, dim3(1), dim3(RB), 0, s, c);
-    if (hipMemcpyAsync(hs, sc, 8 * 13, hipMemcpyDeviceToHost, s) != hipSuccess ||
+    if (hipMemcpyAsync(hs, sc, 8 * S_COUNT, hipMemcpyDeviceToHost, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess)
       return vfg_fail(h, VFG_E_HIP, "pcg: iteration failed");
     it = (int)hs[S_ITS];  // iterations that ran (the batch stops at convergence)
@@ -924,7 +924,7 @@ static int mg_apply(vfg_handle *h, const float *r, float *z, const double *r64, 
 // the scalars.  r.z alternates between two places, so that none is read and
 // written by one launch.  x is updated with the next direction, which reads p
 // anyway (128^3: 84 -> 75 us for both).
-__device__ __forceinline__ int rz_slot(int k) { return k & 1 ? (int)S_TMP0 : (int)S_RZ; }
+__device__ __forceinline__ int rz_slot(int k) { return k & 1 ? (int)S_RZ1 : (int)S_RZ; }
 // alpha = r.z / p.q (partials ppq[0, na)); r -= alpha q; r32 = r; partials of r.r
 __global__ __launch_bounds__(RB) void k_mg_r(double *__restrict__ r, const double *__restrict__ q,
                                              float *__restrict__ r32, int64_t n, const double *__restrict__ ppq, int na,

@@ -433,7 +433,7 @@ __global__ __launch_bounds__(256, 2) void k_v_apply_cg_list(VApplyCgOp op, const
   const double old = c.sc[S_RZ];
   op.bval = c.k > 0 && old != 0. ? s[0] / old : 0.;
   if (first) {
-    c.sc[S_TMP0] = s[0];
+    c.sc[S_RZ1] = s[0];
     if (!isfinite(s[0]) || !isfinite(s[1])) c.sc[S_FLAG] = 2.;
   }
   const VChunk q = chunk_at(op.G, list, cap, blockIdx.x);
@@ -564,7 +564,7 @@ __global__ __launch_bounds__(256) void k_v_xr_list(Grid G, const int *__restrict
   double pq[1];
   vcg_sums<1>(ppq, npq, pq);
   const bool ok = pq[0] > 0. && isfinite(pq[0]);
-  const double old = cg.sc[S_TMP0], al = ok ? old / pq[0] : 0.;
+  const double old = cg.sc[S_RZ1], al = ok ? old / pq[0] : 0.;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     cg.sc[S_RZ] = old;
     if (!ok) cg.sc[S_FLAG] = isfinite(pq[0]) ? 1. : 2.;
