@@ -134,3 +134,41 @@ def test_v_solve_time_follows_the_grid():
     # (the product itself is bound by the coupling, 27 values per element)
     assert solve <= 6 * product * info.iterations, (solve, product, info.iterations)
     P.close()
+
+
+@pytest.mark.parametrize("mixed", [False, True], ids=["fp64", "mixed"])
+def test_batched_multigrid_of_long_axes(mixed):
+    """Members whose last level still has more than eight elements along an axis
+    (the hierarchy ends at twelve levels), beside one whose last level is solved in
+    one workgroup: each as alone, and as by itself outside the batch."""
+    from vpfhf_amd import _lib
+    from vpfhf_amd.batch import Batch
+    boxes = [(0, 20000), (2, 33000), (1, 40), (0, 20000)]
+    rng = np.random.default_rng(8)
+    U0 = [rng.uniform(-1e-3, 1e-3, 27 * (m + 1)) for _, m in boxes]  # 3 x 3 nodes across
+
+    def solve(pick):
+        P = [_held_bar(*boxes[i]) for i in pick]
+        B = Batch(P)
+        Z = [np.zeros(3 * p.nn) for p in P]
+        U, infos = B.u_solve([U0[i] for i in pick], Z, rtol=1e-9, mixed=mixed, pc=_lib.PC_MG)
+        assert all(q.status == 0 for q in infos)
+        B.close()
+        single = []
+        for i, p, z in zip(pick, P, Z):
+            u, info = p.VF_StepU(U0[i], z, rtol=1e-9, pc=_lib.PC_MG)
+            assert info.status == 0
+            # both solves end within rtol of a zero load's solution, 0: their
+            # residuals are what can be compared
+            r0 = np.linalg.norm(p.VF_UResidual(p.VecApplyDirichletBC(U0[i], z), z))
+            for v in (u, U[pick.index(i)]):
+                assert np.linalg.norm(p.VF_UResidual(v, z)) <= 1.01e-9 * r0
+            single.append(info.iterations)
+            p.close()
+        return U, [q.iterations for q in infos], single
+
+    mix, its, single = solve([0, 1, 2, 3])
+    if not mixed:  # the same algorithm; the single solve looks at its residual every few steps
+        assert all(abs(a - b) <= 4 for a, b in zip(its, single)), (its, single)
+    for i in range(4):
+        assert np.array_equal(solve([i])[0][0], mix[i]), i
