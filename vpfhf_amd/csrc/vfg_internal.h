@@ -139,7 +139,10 @@ __device__ __forceinline__ void chunk_walk(int len, const L &load, const W &work
 // alone: its partial sums do not depend on the others).  1024 = one round of
 // loads in flight per workgroup of 256; the update of x and r in an engine of 8
 // requests took 14.7 us in chunks of 4096, one entry in flight, and 5.2 us so.
-// Long vectors fill the device either way, and each chunk is a partial to sum.
+// Long vectors fill the device either way, and each chunk is a partial to sum:
+// batched u-solve of one cube in chunks of 1024 and 4096, 33^3 nodes 1.51 and 1.58
+// ms, 65^3 2.42 and 2.43, 89^3 (2.1 M entries) 3.47 and 3.46, 97^3 3.96 and 3.91,
+// 113^3 5.15 and 5.03.
 inline int chunk_entries(int64_t n) { return n <= (1 << 21) ? 1024 : 4096; }
 
 // ---------------------------------------------------------------- marching

@@ -137,9 +137,9 @@ static dim3 plane_grid(unsigned x, int nz) {
   return dim3(x, nz < PLANE_ROWS ? nz : PLANE_ROWS, (nz + PLANE_ROWS - 1) / PLANE_ROWS);
 }
 
-// Transfers, one plane of nodes per block row (so that indices are 32-bit; rows
-// beyond a grid's 65535 go on in z): restriction one
-// thread per (coarse node, component), on small levels (latency-bound) four,
+// Transfers, one plane of nodes per block row (so that indices are 32-bit; after
+// PLANE_ROWS rows, under a launch's limit of 65535, they go on in z): restriction
+// one thread per (coarse node, component), on small levels (latency-bound) four,
 // one per fine plane of the gather; prolongation one thread per fine node.
 // Restriction, mean of the 129^3 -> 65^3 -> 33^3 nodes 9.7 us (25 us as three
 // separable passes that formed b - A x and the Dirichlet tests themselves), of

@@ -1226,7 +1226,13 @@ static int device_slots(K kernel, int threads) {
 }
 
 // FP32 grids of 16-64 nodes in x (coarse multigrid levels) march 8 x 8 tiles
-// of 7 x 7 owned nodes: more, shorter workgroups
+// of 7 x 7 owned nodes: more, shorter workgroups, and no row of 15-node tiles whose
+// last owns a node or two.  Apply in 16 x 16 and 8 x 8 tiles, cubes of nodes: 9
+// 6.1 and 6.6 us, 15 6.3 and 6.0, 17 11.6 and 6.1, 22 6.3 and 7.0, 25 6.3 and 6.3, 31
+// 10.8 and 6.3, 33 7.8 and 6.4, 49 9.9 and 9.7, 57 9.9 and 12.8, 64 and 65 15.2 and
+// 15.0, 129 52.3 and 56.9; 17 x 513 x 513 153 and 118, 33 x 257 x 257 64 and 58,
+// 129 x 129 x 9 9.4 and 9.9.  Outside the range the two are within 8 % (the
+// narrowest, 129 x 17 x 17 and 257 x 9 x 9: 7.5 and 6.3, 6.7 and 6.2).
 constexpr int SMALL_NX_LO = 16, SMALL_NX_HI = 64;
 // FP64 grids whose 8 x 8 tiles all run at once in chunks of one node plane take
 // them: the one-wavefront workgroups start and synchronise faster (cubes of 16

@@ -10,7 +10,7 @@
 // of which the 23 with no more than two of the exponents at 2 and the rest
 // matching a product of two derivatives occur.  A product of the element
 // matrix then takes 21 4 x 4 blocks of moments (336 FMAs) instead of 27 Gauss
-// points with nine stress entries each: about 680 operations per element
+// points with nine stress entries each: 686 FP64 instructions per element
 // against 1390.  The moments themselves are Simpson sums of s over the
 // 3 x 3 x 3 points {-1, 0, 1} (z in closed form), where v needs additions only.
 //
@@ -223,14 +223,15 @@ __device__ __forceinline__ void um_force_unit(T Ek, const T (&U)[3][8], const UM
 // One layer of an element column: the modal forces of the bottom face added to
 // tot, those of the top face set in carry (per component s, x, y, w).
 // UNIT: s = 1 (vb, vt unused).  CUBIC: elements whose three spacings agree
-// (UModal::cubic): 60 of the multiplications are by 1 or shared; results are
-// bitwise those of the general form.  A branch inside the element would keep
+// (UModal::cubic): products by 1 and shared ones are left out, 590 FP64
+// instructions per element and layer against 686; results are bitwise those of
+// the general form.  A branch inside the element would keep
 // all of it live at once (FP64: 23 registers spilled), so the kernels come in
 // both forms (FP64 94 -> 86 us at 128^3, 620 -> 560 us at 256^3; FP32
 // smoothing 72 -> 66 us at 128^3).
-// Bound by instruction issue: about 690 FP64 and 140 other vector instructions
-// per element and layer, 0.75 of the issue peak at 256^3 (two waves per SIMD in
-// FP64, three to four in FP32).  Against the 27-point form on the same tiles,
+// Bound by instruction issue: with about 90 other vector instructions (counted in
+// the assembly) the cubic form takes 0.64 of the issue slots at 128^3 and 0.67 at
+// 256^3 (SQ counters; two waves per SIMD in FP64, three to four in FP32).  Against the 27-point form on the same tiles,
 // general elements: FP64 176 -> 94 us at 128^3 and 1299 -> 640 us at 256^3, FP32
 // 98 -> 59 us and 776 -> 391 us.
 template <typename T, bool UNIT, bool CUBIC = false>

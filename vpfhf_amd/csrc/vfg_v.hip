@@ -362,9 +362,12 @@ struct VApplyCgOp : VApplyOp<0> {
 // slots at 128^3): 128^3 120 us = 5.1 TB/s, 141 us for the 27 Gauss weights read
 // a plane at a time.  All 27 of the next layer are in flight during a layer;
 // the 176 registers that takes leave two waves per SIMD (three spill: 151 us).
-// NT: a moment array well over the 256 MB last-level cache is streamed past
-// it (128^3, 579 MB: 120 against 127 us); one that fits is kept there for the
-// next product (96^3, 260 MB: 46 against 56 us).
+// NT: a moment array well over the 256 MB last-level cache is streamed past it,
+// one that fits is kept there for the next product.  Kept and streamed, back to
+// back, 105 x 105 nodes by 60 to 220 elements: 163 MB 33.4 and 38.8 us, 284 MB 55.3
+// and 65.7, 325 MB 70.6 and 72.5, 352 MB 80.3 and 79.7, 406 MB 90.8 and 88.8, 515 MB
+// 118.5 and 111.1, 596 MB 137.3 and 128.2.  They cross near 340 MB; up to the line
+// the choice loses 2 % at most.
 constexpr int64_t V_STREAM_BYTES = 400ll << 20;
 template <int MODE, bool NT>
 struct VApplyStreamOp : VApplyOp<MODE> {
