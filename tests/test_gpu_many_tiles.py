@@ -108,6 +108,18 @@ def test_v_solve_of_many_chunks():
     assert its[1] <= 1.25 * its[0] + 4, its
 
 
+@pytest.mark.parametrize("n", [201, 501, 1001])
+def test_v_solve_of_many_chunks_is_reproducible(n):
+    """196 chunks (all resident at once), 1156 and 4489 (late workgroups start after
+    the first has decided whether the CG goes on): bitwise the same every time."""
+    P, U, V0 = _plate(n)
+    V, info = P.VF_StepV(U, V0, rtol=1e-8)
+    for _ in range(3):
+        W, again = P.VF_StepV(U, V0, rtol=1e-8)
+        assert again.iterations == info.iterations and np.array_equal(V, W)
+    P.close()
+
+
 def test_v_solve_time_follows_the_grid():
     """A CG iteration reads the coupling once, whatever the number of chunks
     (71,289 here): a few products' time each, all else included."""

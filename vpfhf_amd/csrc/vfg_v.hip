@@ -421,7 +421,12 @@ __global__ __launch_bounds__(256) void k_vcg_fold(const double *__restrict__ par
 }
 __global__ __launch_bounds__(256, 2) void k_v_apply_cg_list(VApplyCgOp op, const int *__restrict__ list, int cap,
                                                            VCgStep c) {
-  if (c.sc[S_DONE] != 0.) return;  // the CG has converged
+  // the CG has converged: read by one thread, since the first workgroup may set it
+  // meanwhile (below) and a workgroup has to leave or stay as a whole
+  __shared__ int done;
+  if (threadIdx.x == 0) done = c.sc[S_DONE] != 0.;
+  __syncthreads();
+  if (done) return;
   double s[2];
   vcg_sums<2>(c.pairs, c.npairs, s);
   const bool first = blockIdx.x == 0 && threadIdx.x == 0;
