@@ -122,14 +122,15 @@ __device__ __forceinline__ double block_sum(double v, double *sh /* NT/64 */) {
 }
 
 // Vector chunks: the entries k = tid + u B of [0, len), four of a thread in
-// flight at once (load(k), then work(k, value) in order).
+// flight at once (load(k), then work(k, value) in order).  Past the end a thread
+// loads its first entry again: no other thread writes that.
 template <int B, class L, class W>
 __device__ __forceinline__ void chunk_walk(int len, const L &load, const W &work) {
   using R = decltype(load(0));
   for (int k0 = threadIdx.x; k0 < len; k0 += 4 * B) {
     R v[4];
 #pragma unroll
-    for (int u = 0; u < 4; u++) v[u] = load(k0 + u * B < len ? k0 + u * B : len - 1);
+    for (int u = 0; u < 4; u++) v[u] = load(k0 + u * B < len ? k0 + u * B : k0);
 #pragma unroll
     for (int u = 0; u < 4; u++)
       if (k0 + u * B < len) work(k0 + u * B, v[u]);
